@@ -764,7 +764,7 @@ __device__ __forceinline__ void trace_queue(const DevAccel& acc, const SegIn& in
     if (leaf_phase<STATS, false>(tk, tris, lane, ~static_cast<uint32_t>(leaf) >> 3, ca, ~static_cast<uint32_t>(node) >> 3,
                                  cb, rb.o, kxyz, shear, tmin, r.t, r.prim, kNoInstance, kNoInstance, better, kf,
                                  stats, acc.touch_tris) &&
-        ca + cb != 0) {
+        (leaf != 0 || node_leaf)) {  // not ca + cb != 0: an empty child's leaf holds no triangle
       if (better) {  // the barycentrics stay in tk.bary[lane] until the ray finishes
         r.t = key_t(kf);
         r.prim = static_cast<uint32_t>(kf);
@@ -951,7 +951,7 @@ __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& i
     if (leaf_phase<STATS, true>(tk, tris, lane, ~static_cast<uint32_t>(leaf) >> 3, ca, ~static_cast<uint32_t>(node) >> 3,
                                 cb, rb.o, kxyz, shear, tmin, r.t, r.prim, r.inst, cur_id, better, kf, stats,
                                 acc.touch_tris) &&
-        ca + cb != 0) {
+        (leaf != 0 || node_leaf)) {
       if (better) {  // the barycentrics stay in tk.bary[lane] until the ray finishes
         r.t = key_t(kf);
         r.prim = static_cast<uint32_t>(kf);
