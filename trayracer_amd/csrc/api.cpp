@@ -1357,6 +1357,12 @@ trt_status trt_backward(trt_context* ctx, const trt_render_opts* o, const float*
   ShadowQueue sq{ctx->s_o[0].as<float4>(), ctx->s_d[0].as<float4>(), ctx->s_c[0].as<float4>(), nullptr};
   hipStream_t stm = ctx->stream;
   const uint32_t cap = ctx->seg_cap;
+  // As in the forward frame, Shadow of bounce d runs on the second stream beside Extend of
+  // bounce d + 1 (it has the second spill area; they share no buffer); Shade of bounce
+  // d + 1 needs the radiance that Shadow took off its paths, so it waits.
+  DevAccel acc_sh = acc;
+  acc_sh.spill = acc.spill + ctx->spill_half;
+  hipStream_t stm2 = ctx->stream2;
   launch_zero_counters(ctr, stm);
   launch_raygen_adj(rp, uint32_t(n), cap, q[0], ctx->radiance.as<float4>(), ab, ctr, stm);
   for (uint32_t d = 0; d < D; ++d) {
@@ -1364,12 +1370,17 @@ trt_status trt_backward(trt_context* ctx, const trt_render_opts* o, const float*
     const int di = int(d);
     launch_extend(acc, q[cur], hb, SegIn{ctr + seg_ctr(kSegExt, di), ctr + seg_ctr(kSegWorkExt, di), cap}, ctr,
                   ctx->grid_trace, false, stm);
+    if (d > 0) HIPC(hipStreamWaitEvent(stm, ctx->ev2[2 * (d - 1) + 1], 0), "wait");
     launch_shade_adj(sv, sampling_mats(ctx), rp, q[cur], hb, q[nxt], sq, ab,
                      SegIn{ctr + seg_ctr(kSegExt, di), ctr + seg_ctr(kSegWorkShade, di), cap},
                      ctr + seg_ctr(kSegExt, di + 1), ctr + seg_ctr(kSegShadow, di), ctr, d, ctx->grid_shade, stm);
-    launch_shadow_adj(acc, sq, ab, SegIn{ctr + seg_ctr(kSegShadow, di), ctr + seg_ctr(kSegWorkShadow, di), cap}, ctr,
-                      d, ctx->grid_trace, stm);
+    HIPC(hipEventRecord(ctx->ev[4 + 4 * d + 1], stm), "event");
+    HIPC(hipStreamWaitEvent(stm2, ctx->ev[4 + 4 * d + 1], 0), "wait");
+    launch_shadow_adj(acc_sh, sq, ab, SegIn{ctr + seg_ctr(kSegShadow, di), ctr + seg_ctr(kSegWorkShadow, di), cap},
+                      ctr, d, ctx->grid_trace, stm2);
+    HIPC(hipEventRecord(ctx->ev2[2 * d + 1], stm2), "event");
   }
+  HIPC(hipStreamWaitEvent(stm, ctx->ev2[2 * (D - 1) + 1], 0), "wait");
   for (uint32_t lo = 0; lo < nm; lo += kGradMatsPerPass) {
     const uint32_t cnt = std::min(kGradMatsPerPass, nm - lo);
     launch_grad_reduce(ab, lo, cnt, ctx->a_partial.as<float>(), ctx->a_out.as<float>() + size_t(lo) * kNumParams, stm);

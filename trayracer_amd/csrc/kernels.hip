@@ -232,93 +232,14 @@ __device__ __forceinline__ void load_node(const DevNode48* __restrict__ nodes, i
   c = make_int4(row_child_ref(r0), row_child_ref(r1), 0, 0);
 }
 
-// BVH2 traversal of one bottom-level tree (or the single-level scene) for an
-// (object-space) ray. Stack lives in LDS: stk[k * 64] for entry k. Returns true on the
-// first hit when ANY. Updates tbest/pbest/ibest with the (t, inst, prim) order.
-template <bool ANY, bool STATS>
-__device__ __forceinline__ bool traverse_bvh(const DevNode48* __restrict__ nodes, const float4* __restrict__ tris,
-                                             int32_t root, V3 o, V3 d, float tmin, uint32_t inst, uint32_t* stk,
-                                             int sp0, int cap, TraceOut& r, uint32_t* overflow) {
-  const RayTri rt = ray_tri_setup(o, d);
-  const RayBox rb = ray_box_setup(o, d);
-  int sp = sp0;
-  int32_t node = root;
-  for (;;) {
-    if (node >= 0) {
-      float4 r0, r1, r2;
-      int4 c;
-      load_node(nodes, node, r0, r1, r2, c);
-      if (STATS) r.nodes++;
-      float t0, t1;
-      const bool h0 = slab_ch(r0.x, r0.y, r0.z, r0.w, r2.x, r2.y, rb, tmin, r.t, t0);
-      const bool h1 = slab_ch(r1.x, r1.y, r1.z, r1.w, r2.z, r2.w, rb, tmin, r.t, t1);
-      if (h0 && h1) {
-        int32_t nearc = c.x, farc = c.y;
-        if (t1 < t0) {
-          nearc = c.y;
-          farc = c.x;
-        }
-        if (sp < cap) {
-          stk[sp * 64] = static_cast<uint32_t>(farc);
-          ++sp;
-        } else {
-          atomicOr(overflow, 1u);
-        }
-        node = nearc;
-        continue;
-      }
-      if (h0) {
-        node = c.x;
-        continue;
-      }
-      if (h1) {
-        node = c.y;
-        continue;
-      }
-    } else {
-      const uint32_t code = ~static_cast<uint32_t>(node);
-      const uint32_t first = code >> 3, cnt = code & 7u;
-      for (uint32_t k = 0; k < cnt; ++k) {
-        const float4* tp = tris + static_cast<size_t>(first + k) * 3u;
-        const float4 a = tp[0], b = tp[1], cc = tp[2];
-        if (STATS) r.tests++;
-        TriHit th;
-        if (intersect_triangle(rt, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), v3(cc.x, cc.y, cc.z), tmin, r.t, th)) {
-          const uint32_t prim = __float_as_uint(a.w);
-          if (ANY) {
-            r.t = th.t;
-            r.prim = prim;
-            r.inst = inst;
-            return true;
-          }
-          if (th.t < r.t || inst < r.inst || (inst == r.inst && prim < r.prim)) {
-            r.t = th.t;
-            r.b1 = th.b1;
-            r.b2 = th.b2;
-            r.prim = prim;
-            r.inst = inst;
-          }
-        }
-      }
-    }
-    if (sp == sp0) break;
-    --sp;
-    node = static_cast<int32_t>(stk[sp * 64]);
-  }
-  return false;
-}
-
 // Sentinel of an exhausted traversal (never a leaf code: leaf first indices are < 2^28).
 constexpr int32_t kTravDone = static_cast<int32_t>(0x80000000u);
 
-// The while-while node loops end once at most kSearchBreak of the lanes still walking
+// The traversal's node loop ends once at most kSearchBreakSpread of the lanes still walking
 // have no leaf parked, instead of none: the last few searching lanes would otherwise
 // hold the wave for a long tail of iterations in which most lanes idle. They keep their
-// state and go on walking in the next round. With per-lane leaf loops (traverse_ww), 4
-// to 8 lanes traced 9% more rays per second than 0 on the 1M-triangle soup (16 slightly
-// worse); the queue loops, whose leaf phase is spread over the wave and so costs less
-// per round, measured best at 16 (soup: 8 -1.5%, 32 -6%; instanced: 8 -2%).
-constexpr uint32_t kSearchBreak = 8;
+// state and go on walking in the next round. 16 measured best on the 1M-triangle soup
+// (8 -1.5%, 32 -6%; instanced: 8 -2%).
 constexpr uint32_t kSearchBreakSpread = 16;
 
 // End of a queue traversal's node loop, evaluated by all lanes after each iteration as a
@@ -341,107 +262,16 @@ __device__ __forceinline__ uint32_t searching_lanes(int32_t leaf) {
          static_cast<uint32_t>(__builtin_popcount(static_cast<uint32_t>(m >> 32)));
 }
 
-// Single-level BVH2 traversal in the "speculative while-while" form of Aila & Laine
-// (2009, "Understanding the efficiency of ray traversal on GPUs"): lanes walk inner
-// nodes until (nearly) every lane of the wave holds a leaf (a lane that meets its first
-// leaf parks it and keeps walking), then the wave intersects leaves together. Triangle
-// tests are the costly step; this keeps them from running for a handful of lanes at
-// every iteration. The result does not depend on the visiting order (closest hit under
-// the (t, inst, prim) order, or any hit), so it equals traverse_bvh's.
-template <bool ANY, bool STATS>
-__device__ __forceinline__ bool traverse_ww(const DevNode48* __restrict__ nodes, const float4* __restrict__ tris, V3 o,
-                                            V3 d, float tmin, uint32_t* stk, int cap, TraceOut& r,
-                                            uint32_t* overflow) {
-  const RayTri rt = ray_tri_setup(o, d);
-  const RayBox rb = ray_box_setup(o, d);
-  int sp = 0;
-  int32_t node = 0;  // next node: inner index, leaf code, or kTravDone
-  int32_t leaf = 0;  // parked leaf code (0 = none)
-  auto pop = [&]() -> int32_t {
-    if (sp == 0) return kTravDone;
-    --sp;
-    return static_cast<int32_t>(stk[sp * 64]);
-  };
-  while (node != kTravDone || leaf != 0) {
-    // inner nodes
-    while (node >= 0) {
-      float4 r0, r1, r2;
-      int4 c;
-      load_node(nodes, node, r0, r1, r2, c);
-      if (STATS) r.nodes++;
-      float t0, t1;
-      const bool h0 = slab_ch(r0.x, r0.y, r0.z, r0.w, r2.x, r2.y, rb, tmin, r.t, t0);
-      const bool h1 = slab_ch(r1.x, r1.y, r1.z, r1.w, r2.z, r2.w, rb, tmin, r.t, t1);
-      if (h0 && h1) {
-        int32_t nearc = c.x, farc = c.y;
-        if (t1 < t0) {
-          nearc = c.y;
-          farc = c.x;
-        }
-        if (sp < cap) {
-          stk[sp * 64] = static_cast<uint32_t>(farc);
-          ++sp;
-        } else {
-          atomicOr(overflow, 1u);
-        }
-        node = nearc;
-      } else if (h0) {
-        node = c.x;
-      } else if (h1) {
-        node = c.y;
-      } else {
-        node = pop();
-      }
-      if (node < 0 && node != kTravDone && leaf == 0) {  // park the first leaf, keep walking
-        leaf = node;
-        node = pop();
-      }
-      if (searching_lanes(leaf) <= kSearchBreak) break;
-    }
-    // leaves
-    while (leaf != 0) {
-      const uint32_t code = ~static_cast<uint32_t>(leaf);
-      const uint32_t first = code >> 3, cnt = code & 7u;
-      for (uint32_t k = 0; k < cnt; ++k) {
-        const float4* tp = tris + static_cast<size_t>(first + k) * 3u;
-        const float4 a = tp[0], b = tp[1], cc = tp[2];
-        if (STATS) r.tests++;
-        TriHit th;
-        if (intersect_triangle(rt, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), v3(cc.x, cc.y, cc.z), tmin, r.t, th)) {
-          const uint32_t prim = __float_as_uint(a.w);
-          if (ANY) {
-            r.t = th.t;
-            r.prim = prim;
-            r.inst = kNoInstance;
-            return true;
-          }
-          if (th.t < r.t || prim < r.prim) {
-            r.t = th.t;
-            r.b1 = th.b1;
-            r.b2 = th.b2;
-            r.prim = prim;
-            r.inst = kNoInstance;
-          }
-        }
-      }
-      if (node < 0 && node != kTravDone) {
-        leaf = node;
-        node = pop();
-      } else {
-        leaf = 0;
-      }
-    }
-  }
-  return false;
-}
-
-// Persistent single-level traversal of a segmented ray queue with lane refill
-// ("dynamic fetch", Aila & Laine 2009): the wave runs rounds of the speculative
-// while-while loop above, and before each round lanes whose ray has finished take new
-// rays from the queue once at least kRefill of them are idle, so a few long rays no
-// longer hold the whole wave (40 of 64 measured best on MI355X with the early end of
-// the node loop and the spread leaf phase, 24 and 48 about 1-3% slower; 64, i.e. no
-// refill, was 18% slower with per-lane leaf loops).
+// Persistent single-level BVH2 traversal of a segmented ray queue, in rounds of the
+// "speculative while-while" form of Aila & Laine (2009, "Understanding the efficiency of
+// ray traversal on GPUs"): lanes walk inner nodes until (nearly) every lane of the wave
+// holds a leaf (a lane that meets its first leaf parks it and keeps walking), then the
+// wave intersects leaves together. Before each round lanes whose ray has finished take new
+// rays from the queue ("dynamic fetch", same paper) once at least kRefill of them are
+// idle, so a few long rays do not hold the whole wave (40 of 64 measured best on MI355X
+// with the early end of the node loop and the spread leaf phase, 24 and 48 about 1-3%
+// slower). The result does not depend on the visiting order (closest hit under the
+// (t, inst, prim) order, or any hit).
 // load(slot, o, d, tmin, tmax) reads a ray;
 // finish(slot, r, hit) consumes a result (hit: a hit was found).
 constexpr uint32_t kRefill = 40;
@@ -977,67 +807,6 @@ __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& i
   }
 }
 
-// Full trace (single or two-level). r.t must hold tmax on entry.
-template <bool ANY, bool STATS>
-__device__ __forceinline__ bool trace_ray(const DevAccel& acc, V3 o, V3 d, float tmin, uint32_t* stk,
-                                          TraceOut& r, uint32_t* overflow) {
-  if (!acc.two_level) return traverse_ww<ANY, STATS>(acc.nodes, acc.tris, o, d, tmin, stk, acc.stack_cap, r, overflow);
-  // top level: leaf ranges index the instance array in TLAS build order
-  const RayBox rb = ray_box_setup(o, d);
-  int sp = 0;
-  int32_t node = 0;
-  const int cap = acc.stack_cap;
-  for (;;) {
-    if (node >= 0) {
-      float4 r0, r1, r2;
-      int4 c;
-      load_node(acc.tlas, node, r0, r1, r2, c);
-      if (STATS) r.nodes++;
-      float t0, t1;
-      const bool h0 = slab_ch(r0.x, r0.y, r0.z, r0.w, r2.x, r2.y, rb, tmin, r.t, t0);
-      const bool h1 = slab_ch(r1.x, r1.y, r1.z, r1.w, r2.z, r2.w, rb, tmin, r.t, t1);
-      if (h0 && h1) {
-        int32_t nearc = c.x, farc = c.y;
-        if (t1 < t0) {
-          nearc = c.y;
-          farc = c.x;
-        }
-        if (sp < cap) {
-          stk[sp * 64] = static_cast<uint32_t>(farc);
-          ++sp;
-        } else {
-          atomicOr(overflow, 1u);
-        }
-        node = nearc;
-        continue;
-      }
-      if (h0) {
-        node = c.x;
-        continue;
-      }
-      if (h1) {
-        node = c.y;
-        continue;
-      }
-    } else {
-      const uint32_t code = ~static_cast<uint32_t>(node);
-      const uint32_t first = code >> 3, cnt = code & 7u;
-      for (uint32_t k = 0; k < cnt; ++k) {
-        const Instance& in = acc.inst[first + k];
-        const V3 oo = xform_point(in.w2o, o);
-        const V3 od = xform_vector(in.w2o, d);
-        if (traverse_bvh<ANY, STATS>(acc.nodes, acc.tris, static_cast<int32_t>(in.blas_root), oo, od, tmin, in.id,
-                                     stk, sp, cap, r, overflow))
-          return true;
-      }
-    }
-    if (sp == 0) break;
-    --sp;
-    node = static_cast<int32_t>(stk[sp * 64]);
-  }
-  return false;
-}
-
 // ------------------------------------------------------------------------------------
 __global__ __launch_bounds__(kBlock) void k_zero_counters(uint32_t* ctr) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
@@ -1141,28 +910,42 @@ __global__ __launch_bounds__(kBlock) void k_raygen(RenderParams rp, uint32_t n_p
 }
 
 
+// The calling wave's stack ring (this lane's first slot) and leaf-task area in the
+// traversal kernels' dynamic LDS: the block's rings, then its task areas.
+__device__ __forceinline__ uint32_t* wave_ring(uint32_t* lds) {
+  return lds + (threadIdx.x >> 6) * kRingEntries * 64 + lane_id();
+}
+__device__ __forceinline__ uint32_t* wave_tasks(uint32_t* lds) {
+  return lds + kWavesPerBlock * kRingEntries * 64 + (threadIdx.x >> 6) * kTaskWords;
+}
+
+// A ray from its (origin, tmin) and (direction, tmax) records.
+struct RayLoad {
+  const float4* o_tmin;
+  const float4* d_tmax;
+  __device__ __forceinline__ void operator()(uint32_t slot, V3& o, V3& d, float& tmin, float& tmax) const {
+    const float4 a = o_tmin[slot];
+    const float4 b = d_tmax[slot];
+    o = v3(a.x, a.y, a.z);
+    d = v3(b.x, b.y, b.z);
+    tmin = a.w;
+    tmax = b.w;
+  }
+};
+
 // Single-level scenes: Extend and Shadow through trace_queue. Both are held to 72
 // VGPRs, 7 waves per SIMD (the allocator otherwise settles just above, at 6 waves,
 // which measured 5% slower).
 template <bool STATS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_extend_sl(DevAccel acc, RayQueue q, HitBuf h, SegIn in, uint32_t* ctr) {
   extern __shared__ uint32_t lds[];
-  uint32_t* stk = lds + (threadIdx.x >> 6) * kRingEntries * 64 + lane_id();
-  uint32_t* tsk = lds + kWavesPerBlock * kRingEntries * 64 + (threadIdx.x >> 6) * kTaskWords;
   TraceOut st;
   st.nodes = 0;
   st.tests = 0;
   st.spills = 0;
   trace_queue<false, STATS>(
-      acc, in, stk, tsk, &ctr[kCtrOverflow], st,
-      [&](uint32_t slot, V3& o, V3& d, float& tmin, float& tmax) {
-        const float4 a = q.o_tmin[slot];
-        const float4 b = q.d_tmax[slot];
-        o = v3(a.x, a.y, a.z);
-        d = v3(b.x, b.y, b.z);
-        tmin = a.w;
-        tmax = b.w;
-      },
+      acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st,
+      RayLoad{q.o_tmin, q.d_tmax},
       [&](uint32_t slot, const TraceOut& r, bool) {
         h.thit[slot] = make_float4(r.t, r.b1, r.b2, __uint_as_float(r.prim));
       });
@@ -1177,22 +960,13 @@ template <bool STATS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_shadow_sl(DevAccel acc, ShadowQueue sq, float4* radiance, SegIn in,
                                                        uint32_t* ctr) {
   extern __shared__ uint32_t lds[];
-  uint32_t* stk = lds + (threadIdx.x >> 6) * kRingEntries * 64 + lane_id();
-  uint32_t* tsk = lds + kWavesPerBlock * kRingEntries * 64 + (threadIdx.x >> 6) * kTaskWords;
   TraceOut st;
   st.nodes = 0;
   st.tests = 0;
   st.spills = 0;
   trace_queue<true, STATS>(
-      acc, in, stk, tsk, &ctr[kCtrOverflow], st,
-      [&](uint32_t slot, V3& o, V3& d, float& tmin, float& tmax) {
-        const float4 a = sq.o_tmin[slot];
-        const float4 b = sq.d_tmax[slot];
-        o = v3(a.x, a.y, a.z);
-        d = v3(b.x, b.y, b.z);
-        tmin = a.w;
-        tmax = b.w;
-      },
+      acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st,
+      RayLoad{sq.o_tmin, sq.d_tmax},
       [&](uint32_t slot, const TraceOut&, bool occluded) {
         if (!occluded) {
           const float4 c = sq.contrib[slot];
@@ -1216,22 +990,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
 template <bool STATS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_extend_tl(DevAccel acc, RayQueue q, HitBuf h, SegIn in, uint32_t* ctr) {
   extern __shared__ uint32_t lds[];
-  uint32_t* stk = lds + (threadIdx.x >> 6) * kRingEntries * 64 + lane_id();
-  uint32_t* tsk = lds + kWavesPerBlock * kRingEntries * 64 + (threadIdx.x >> 6) * kTaskWords;
   TraceOut st;
   st.nodes = 0;
   st.tests = 0;
   st.spills = 0;
   trace_queue2<false, STATS>(
-      acc, in, stk, tsk, &ctr[kCtrOverflow], st,
-      [&](uint32_t slot, V3& o, V3& d, float& tmin, float& tmax) {
-        const float4 a = q.o_tmin[slot];
-        const float4 b = q.d_tmax[slot];
-        o = v3(a.x, a.y, a.z);
-        d = v3(b.x, b.y, b.z);
-        tmin = a.w;
-        tmax = b.w;
-      },
+      acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st,
+      RayLoad{q.o_tmin, q.d_tmax},
       [&](uint32_t slot, const TraceOut& r, bool) {
         h.thit[slot] = make_float4(r.t, r.b1, r.b2, __uint_as_float(r.prim));
         h.inst[slot] = r.inst;
@@ -1247,22 +1012,13 @@ template <bool STATS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_shadow_tl(DevAccel acc, ShadowQueue sq, float4* radiance, SegIn in,
                                                        uint32_t* ctr) {
   extern __shared__ uint32_t lds[];
-  uint32_t* stk = lds + (threadIdx.x >> 6) * kRingEntries * 64 + lane_id();
-  uint32_t* tsk = lds + kWavesPerBlock * kRingEntries * 64 + (threadIdx.x >> 6) * kTaskWords;
   TraceOut st;
   st.nodes = 0;
   st.tests = 0;
   st.spills = 0;
   trace_queue2<true, STATS>(
-      acc, in, stk, tsk, &ctr[kCtrOverflow], st,
-      [&](uint32_t slot, V3& o, V3& d, float& tmin, float& tmax) {
-        const float4 a = sq.o_tmin[slot];
-        const float4 b = sq.d_tmax[slot];
-        o = v3(a.x, a.y, a.z);
-        d = v3(b.x, b.y, b.z);
-        tmin = a.w;
-        tmax = b.w;
-      },
+      acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st,
+      RayLoad{sq.o_tmin, sq.d_tmax},
       [&](uint32_t slot, const TraceOut&, bool occluded) {
         if (!occluded) {
           const float4 c = sq.contrib[slot];
@@ -1618,47 +1374,47 @@ __global__ __launch_bounds__(kBlock) void k_shade_adj(SceneView sv, const Materi
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_shadow_adj(DevAccel acc, ShadowQueue sq, AdjBuffers ab, SegIn in,
-                                                        uint32_t* ctr, uint32_t depth) {
-  extern __shared__ uint32_t lds[];
-  const uint32_t lane = lane_id();
-  uint32_t* stk = lds + (threadIdx.x >> 6) * acc.stack_cap * 64 + lane;
+// Shadow rays of the adjoint, through the render's own traversal: an unoccluded ray's
+// contribution leaves the path's unattributed radiance, and its next-event gradient goes
+// to the vertex's record. (With one ray per lane held until the wave's longest had
+// finished, four launches took 4.0 ms on 512 x 512 x 64 spp of the Cornell box.)
+__device__ __forceinline__ void finish_shadow_adj(const ShadowQueue& sq, const AdjBuffers& ab, uint32_t depth,
+                                                  uint32_t slot, bool occluded) {
+  if (occluded) return;
+  const float4 c = sq.contrib[slot];
+  const uint32_t path = __float_as_uint(c.w);
+  float4 lr = ab.lrem[path];
+  lr.x -= c.x;
+  lr.y -= c.y;
+  lr.z -= c.z;
+  ab.lrem[path] = lr;
+  const float4 ga = ab.s_ga[slot];
+  const float gb = ab.s_gb[slot];
   const size_t R = ab.n_records;
-  const uint32_t n_seg = seg_counts(in), home = wave_home();
-  uint64_t done = seg_empty(n_seg);
-  uint32_t slot0, n_valid;
-  while (seg_fetch(in, n_seg, home, done, slot0, n_valid)) {
-    const uint32_t slot = slot0 + lane;
-    if (lane < n_valid) {
-      const float4 a = sq.o_tmin[slot];
-      const float4 b = sq.d_tmax[slot];
-      TraceOut r;
-      r.t = b.w;
-      r.prim = kNoHit;
-      r.inst = kNoInstance;
-      r.nodes = 0;
-      r.tests = 0;
-      const bool occ =
-          trace_ray<true, false>(acc, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, stk, r, &ctr[kCtrOverflow]);
-      if (!occ) {
-        const float4 c = sq.contrib[slot];
-        const uint32_t path = __float_as_uint(c.w);
-        float4 lr = ab.lrem[path];
-        lr.x -= c.x;
-        lr.y -= c.y;
-        lr.z -= c.z;
-        ab.lrem[path] = lr;
-        const float4 ga = ab.s_ga[slot];
-        const float gb = ab.s_gb[slot];
-        const size_t rr = static_cast<size_t>(path) * ab.depth + depth;
-        ab.rec_g[0 * R + rr] += ga.x;
-        ab.rec_g[1 * R + rr] += ga.y;
-        ab.rec_g[2 * R + rr] += ga.z;
-        ab.rec_g[3 * R + rr] += ga.w;
-        ab.rec_g[4 * R + rr] += gb;
-      }
-    }
-  }
+  const size_t rr = static_cast<size_t>(path) * ab.depth + depth;
+  ab.rec_g[0 * R + rr] += ga.x;
+  ab.rec_g[1 * R + rr] += ga.y;
+  ab.rec_g[2 * R + rr] += ga.z;
+  ab.rec_g[3 * R + rr] += ga.w;
+  ab.rec_g[4 * R + rr] += gb;
+}
+
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_shadow_adj_sl(
+    DevAccel acc, ShadowQueue sq, AdjBuffers ab, SegIn in, uint32_t* ctr, uint32_t depth) {
+  extern __shared__ uint32_t lds[];
+  TraceOut st;
+  trace_queue<true, false>(
+      acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st, RayLoad{sq.o_tmin, sq.d_tmax},
+      [&](uint32_t slot, const TraceOut&, bool occluded) { finish_shadow_adj(sq, ab, depth, slot, occluded); });
+}
+
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_shadow_adj_tl(
+    DevAccel acc, ShadowQueue sq, AdjBuffers ab, SegIn in, uint32_t* ctr, uint32_t depth) {
+  extern __shared__ uint32_t lds[];
+  TraceOut st;
+  trace_queue2<true, false>(
+      acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st, RayLoad{sq.o_tmin, sq.d_tmax},
+      [&](uint32_t slot, const TraceOut&, bool occluded) { finish_shadow_adj(sq, ab, depth, slot, occluded); });
 }
 
 // Deterministic reduction of records into per-material gradients, materials
@@ -1720,7 +1476,6 @@ __global__ __launch_bounds__(kBlock) void k_grad_final(const float* partial, uin
   out[i] = t;
 }
 
-size_t stack_lds_bytes(const DevAccel& acc) { return static_cast<size_t>(acc.stack_cap) * 64u * 4u * kWavesPerBlock; }
 size_t ring_lds_bytes() { return static_cast<size_t>(kRingEntries) * 64u * 4u * kWavesPerBlock; }
 // queue traversals: rings, then each wave's leaf-task area
 size_t trace_lds_bytes() { return ring_lds_bytes() + static_cast<size_t>(kTaskWords) * 4u * kWavesPerBlock; }
@@ -1749,7 +1504,8 @@ bool traversal_lds_check() {
   const void* ks[] = {reinterpret_cast<const void*>(k_extend_sl<false>), reinterpret_cast<const void*>(k_extend_sl<true>),
                       reinterpret_cast<const void*>(k_shadow_sl<false>), reinterpret_cast<const void*>(k_shadow_sl<true>),
                       reinterpret_cast<const void*>(k_extend_tl<false>), reinterpret_cast<const void*>(k_extend_tl<true>),
-                      reinterpret_cast<const void*>(k_shadow_tl<false>), reinterpret_cast<const void*>(k_shadow_tl<true>)};
+                      reinterpret_cast<const void*>(k_shadow_tl<false>), reinterpret_cast<const void*>(k_shadow_tl<true>),
+                      reinterpret_cast<const void*>(k_shadow_adj_sl), reinterpret_cast<const void*>(k_shadow_adj_tl)};
   for (const void* k : ks) {
     hipFuncAttributes a{};
     if (hipFuncGetAttributes(&a, k) != hipSuccess || a.sharedSizeBytes != 0) return false;
@@ -1862,8 +1618,10 @@ void launch_shade_adj(const SceneView& sv, const Material* sampling_mats, const 
 
 void launch_shadow_adj(const DevAccel& acc, ShadowQueue sq, const AdjBuffers& ab, SegIn in, uint32_t* ctr,
                        uint32_t depth, int grid, hipStream_t stream) {
-  hipLaunchKernelGGL(k_shadow_adj, dim3(grid), dim3(kBlock), stack_lds_bytes(acc), stream, acc, sq, ab, in, ctr,
-                     depth);
+  if (acc.two_level)
+    hipLaunchKernelGGL(k_shadow_adj_tl, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, sq, ab, in, ctr, depth);
+  else
+    hipLaunchKernelGGL(k_shadow_adj_sl, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, sq, ab, in, ctr, depth);
 }
 
 void launch_grad_reduce(const AdjBuffers& ab, uint32_t mat_lo, uint32_t n_mat, float* partial, float* out,
