@@ -145,7 +145,7 @@ struct trt_context {
   uint64_t frame_id = 0;       // frames rendered by this context
   trt_render_opts last_opts{};
   uint32_t last_sample_offset = 0;
-  DevBuf a_lrem, a_pend, a_key, a_g, a_sga, a_sgb, a_dldi, a_partial, a_out;
+  DevBuf a_lrem, a_pend, a_key, a_ga, a_gb, a_sga, a_sgb, a_dldi, a_partial, a_out;
 
   // denoiser
   std::unique_ptr<Unet> unet;
@@ -1323,7 +1323,8 @@ trt_status trt_backward(trt_context* ctx, const trt_render_opts* o, const float*
   HIPC(ctx->a_lrem.ensure(n * 16), "alloc adjoint");
   HIPC(ctx->a_pend.ensure(n * 64), "alloc adjoint");
   HIPC(ctx->a_key.ensure(R * 4), "alloc adjoint");
-  HIPC(ctx->a_g.ensure(R * 4 * kNumParams), "alloc adjoint");
+  HIPC(ctx->a_ga.ensure(R * 16), "alloc adjoint");
+  HIPC(ctx->a_gb.ensure(R * 4), "alloc adjoint");
   HIPC(ctx->a_sga.ensure(ctx->queue_slots * 16), "alloc adjoint");  // per shadow-queue slot
   HIPC(ctx->a_sgb.ensure(ctx->queue_slots * 4), "alloc adjoint");
   HIPC(ctx->a_dldi.ensure(uint64_t(W) * H * 12), "alloc adjoint");
@@ -1341,7 +1342,8 @@ trt_status trt_backward(trt_context* ctx, const trt_render_opts* o, const float*
   ab.lrem = ctx->a_lrem.as<float4>();
   ab.pend = ctx->a_pend.as<float4>();
   ab.rec_key = ctx->a_key.as<uint32_t>();
-  ab.rec_g = ctx->a_g.as<float>();
+  ab.rec_a = ctx->a_ga.as<float4>();
+  ab.rec_b = ctx->a_gb.as<float>();
   ab.s_ga = ctx->a_sga.as<float4>();
   ab.s_gb = ctx->a_sgb.as<float>();
   ab.n_records = R;

@@ -115,14 +115,19 @@ struct FrameBuffers {
 };
 
 // Adjoint (path replay) state. Records: one per (path, depth) slot r = path*depth + d,
-// key = material id of the vertex (0xffffffff = none), rec_g[k * n_records + r] =
-// gradient of parameter k (SoA so a wave's loads coalesce).
+// key = material id of the vertex (0xffffffff = none), gradient of parameters 0..3 in
+// rec_a[r] and of parameter 4 in rec_b[r] (valid where the key is). A vertex's record is
+// written whole by one kernel and read whole by the next, at an address that its queue
+// neighbours do not share, so the five parameters sit in two arrays (two lines per
+// record), not five.
 struct AdjBuffers {
   const float* dldi;   // dLoss/dImage, 3 floats per pixel
   float4* lrem;        // per path: radiance not yet attributed to earlier vertices
-  float4* pend;        // per path: 4 float4 = (d f / d theta)/f of the pending continuation + material
+  float4* pend;        // per path: 4 float4 = (d f / d theta)/f of the pending continuation
+                       // (written by a vertex that sends one on, read by the next vertex)
   uint32_t* rec_key;
-  float* rec_g;
+  float4* rec_a;
+  float* rec_b;
   float4* s_ga;        // per shadow slot: NEE gradient, params 0..3
   float* s_gb;         // per shadow slot: NEE gradient, param 4
   size_t n_records;

@@ -367,10 +367,11 @@ TRT_HD inline void shade(const SceneView& s, const Material* sampling_mats, cons
 }
 
 // Same vertex replayed for the adjoint: delta = dLoss/d(path radiance).
+template <int SEP = -1>
 TRT_HD inline void shade_adjoint(const SceneView& s, const Material* sampling_mats, const RenderParams& rp,
                                  const PathState& ps, const Hit& h, uint32_t depth, V3 delta, ShadeOut& out,
                                  AdjOut& adj) {
-  shade_impl<true>(s, sampling_mats, rp, ps, h, depth, out, delta, &adj);
+  shade_impl<true, SEP>(s, sampling_mats, rp, ps, h, depth, out, delta, &adj);
 }
 
 // Gradient of the BSDF-sampled continuation of a vertex once the radiance that
