@@ -83,3 +83,41 @@ def test_adjoint_of_an_instanced_scene(rend):
     ref = orc.backward(dldi)
     assert (np.abs(ref).max(axis=1) > 0).sum() >= 8  # most of the twelve palettes take part
     assert np.abs(g - ref).max() <= 1e-3 * np.abs(ref).max()
+
+
+def _node_bytes(rend):
+    rend.settings.width = rend.settings.height = 16
+    rend.settings.spp = 1
+    return rend.measure_traversal()["node_bytes"]
+
+
+@pytest.mark.parametrize("surrounding", [0.0, 3000.0], ids=["compact-nodes", "48-byte-nodes"])
+def test_both_node_layouts_match_brute_force(rend, surrounding):
+    """A soup, alone (its tree suits the 32-byte nodes) and as a small object far from the
+    centre of a large surrounding (its tree is too fine for their grid): hits and occlusion
+    equal a brute-force loop over random rays, rays parallel to an axis, unnormalised
+    directions and origins far away; and so does a rendered frame, path by path."""
+    sc = scenes.soup(n_tris=4000, seed=9, width=48, height=32, spp=4, max_depth=4)
+    if surrounding:
+        pos = sc["positions"].copy()
+        pos[0] = np.tile([-surrounding, -surrounding, -surrounding], 3) + [0, 0, 0, 1, 0, 0, 0, 1, 0]
+        pos[1] = np.tile([0.3 * surrounding, 0.2 * surrounding, 0.1 * surrounding], 3) + [0, 0, 0, 1, 0, 0, 0, 1, 0]
+        sc["positions"] = pos
+    rend.UpdateScene(sc)
+    assert _node_bytes(rend) == (48 if surrounding else 32)
+    rays = random_rays(6000, seed=3, toward=(0.0, 1.0))
+    rng = np.random.default_rng(4)
+    for k in range(3):  # parallel to an axis; the other components zero of either sign
+        rays[k * 500:(k + 1) * 500, 4:7] = 0.0
+        rays[k * 500:(k + 1) * 500, 4 + k] = rng.choice([-1.0, 1.0], 500)
+        rays[k * 500:k * 500 + 250, 4 + (k + 1) % 3] = -0.0
+    rays[2000:2500, 4:7] *= 1e-6
+    rays[2500:3000, 4:7] *= 1e6
+    rays[3000:3500, 0:3] = 0.5 - 1e4 * rays[3000:3500, 4:7]
+    hit = _check(rend, sc, rays)
+    assert hit.sum() > 1000
+    rend.SetSettings(rend.settings.from_dict(sc["render"]))
+    rend.RenderFrame()
+    got = rend.path_radiance()
+    want = _oracle(sc).render()["path_rgb"]
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))

@@ -98,6 +98,8 @@ struct trt_context {
   bool use_normals = false;
   bool two_level = false;
   int stack_cap = 1;
+  NodeSpace space{};                       // of the single-level tree or the top level
+  uint32_t node_bytes = sizeof(DevNode32);  // node layout of d_nodes and d_tlas
   trt_bvh_info info{};
   SkyParams sky{};  // disabled
 
@@ -330,10 +332,12 @@ trt_status ensure_frame(trt_context* ctx, uint32_t W, uint32_t H, uint32_t spp) 
 
 DevAccel accel_of(const trt_context* ctx) {
   DevAccel a;
-  a.nodes = ctx->d_nodes.as<DevNode48>();
+  a.nodes = ctx->d_nodes.p;
   a.tris = ctx->d_tris.as<float4>();
-  a.tlas = ctx->two_level ? ctx->d_tlas.as<DevNode48>() : nullptr;
-  a.inst = ctx->two_level ? ctx->d_inst_tlas.as<Instance>() : nullptr;
+  a.tlas = ctx->two_level ? ctx->d_tlas.p : nullptr;
+  a.inst = ctx->two_level ? ctx->d_inst_tlas.as<TlasInstance>() : nullptr;
+  a.space = ctx->space;
+  a.node_bytes = ctx->node_bytes;
   a.stack_cap = ctx->stack_cap;
   a.two_level = ctx->two_level ? 1 : 0;
   a.spill = ctx->d_spill.as<uint32_t>();
@@ -749,7 +753,9 @@ trt_status trt_build(trt_context* ctx, const trt_build_opts* opts) {
 
   std::vector<DevNode2> nodes;
   std::vector<float> tris;
-  std::vector<Instance> inst_orig, inst_tlas;
+  std::vector<Instance> inst_orig;
+  std::vector<uint32_t> tlas_order;    // instance of each top-level leaf slot
+  std::vector<uint32_t> blas_root;     // root node of each mesh's tree
   std::vector<DevNode2> tlas_nodes;
   ctx->two_level = !ctx->instances_in.empty();
   uint64_t n_nodes = 0, n_leaves = 0, n_refs = 0;
@@ -766,7 +772,7 @@ trt_status trt_build(trt_context* ctx, const trt_build_opts* opts) {
     sah = b.sah_cost;
     depth = b.depth;
   } else {
-    std::vector<uint32_t> blas_root(ctx->meshes.size());
+    blas_root.resize(ctx->meshes.size());
     std::vector<float> mesh_lo(ctx->meshes.size() * 3), mesh_hi(ctx->meshes.size() * 3);
     for (size_t mi = 0; mi < ctx->meshes.size(); ++mi) {
       const Mesh& m = ctx->meshes[mi];
@@ -796,7 +802,6 @@ trt_status trt_build(trt_context* ctx, const trt_build_opts* opts) {
       in.mesh = ti.mesh;
       in.tri_offset = ctx->meshes[ti.mesh].tri_offset;
       in.mat_offset = ti.material_offset;
-      in.blas_root = blas_root[ti.mesh] * kNodeBytes;  // byte offset, like every node reference
       in.id = i;
       const Mesh& m = ctx->meshes[ti.mesh];
       for (uint32_t k = 0; k < m.n_tris; ++k)
@@ -824,8 +829,7 @@ trt_status trt_build(trt_context* ctx, const trt_build_opts* opts) {
     }
     BuildResult tb = build_binned_sah(ibox.data(), ni, o.bins, o.max_leaf, threads, kTravCostInstances);
     tlas_nodes = to_device_layout(tb);
-    inst_tlas.resize(ni);
-    for (uint32_t k = 0; k < ni; ++k) inst_tlas[k] = inst_orig[tb.prim_order[k]];
+    tlas_order = tb.prim_order;
     tlas_depth = tb.depth;
     n_nodes += tb.nodes.size();
   }
@@ -855,24 +859,50 @@ trt_status trt_build(trt_context* ctx, const trt_build_opts* opts) {
   // child references are byte offsets below 2^31
   if (nodes.size() >= kMaxDeviceNodes || tlas_nodes.size() >= kMaxDeviceNodes)
     return fail(ctx, TRT_UNSUPPORTED, "BVH too large: more than 44M nodes in one tree array");
+  // Node layout: the compact one where every tree suits it (pack_nodes32), else 48-byte
+  // nodes throughout.
   std::vector<DevNode48> nodes48, tlas48;
-  if (!pack_nodes(nodes, nodes48) || !pack_nodes(tlas_nodes, tlas48))
+  std::vector<DevNode32> nodes32(nodes.size()), tlas32(tlas_nodes.size());
+  std::vector<NodeSpace> mesh_space(ctx->meshes.size());
+  bool compact = true;
+  if (!ctx->two_level) {
+    compact = pack_nodes32(nodes, 0, nodes.size(), ctx->space, nodes32.data());
+  } else {
+    for (size_t mi = 0; mi < ctx->meshes.size() && compact; ++mi) {
+      const size_t end = mi + 1 < ctx->meshes.size() ? blas_root[mi + 1] : nodes.size();
+      compact = pack_nodes32(nodes, blas_root[mi], end - blas_root[mi], mesh_space[mi], nodes32.data());
+    }
+    compact = compact && pack_nodes32(tlas_nodes, 0, tlas_nodes.size(), ctx->space, tlas32.data());
+  }
+  if (!compact && (!pack_nodes(nodes, nodes48) || !pack_nodes(tlas_nodes, tlas48)))
     return fail(ctx, TRT_UNSUPPORTED, "scene bounds too large for the node layout (infinite coordinates)");
+  ctx->node_bytes = compact ? sizeof(DevNode32) : sizeof(DevNode48);
+  const size_t node_bytes = nodes.size() * ctx->node_bytes, tlas_bytes = tlas_nodes.size() * ctx->node_bytes;
+  std::vector<TlasInstance> inst_tlas(tlas_order.size());
+  for (size_t k = 0; k < inst_tlas.size(); ++k) {
+    const Instance& in = inst_orig[tlas_order[k]];
+    TlasInstance& t = inst_tlas[k];
+    std::memset(&t, 0, sizeof(t));
+    std::memcpy(t.w2o, in.w2o, sizeof(t.w2o));
+    t.space = mesh_space[in.mesh];
+    t.blas_root = blas_root[in.mesh] * ctx->node_bytes;  // a byte offset, like every node reference
+    t.id = in.id;
+  }
 
   hipStream_t s = ctx->stream;
   HIPC(upload(ctx->d_pos, ctx->pos.data(), ctx->pos.size() * 4, s), "upload positions");
   if (ctx->use_normals) HIPC(upload(ctx->d_nrm, ctx->nrm.data(), ctx->nrm.size() * 4, s), "upload normals");
   HIPC(upload(ctx->d_mat_ids, ctx->mat_ids.data(), ctx->mat_ids.size() * 4, s), "upload material ids");
   HIPC(upload(ctx->d_materials, ctx->materials.data(), ctx->materials.size() * sizeof(Material), s), "upload materials");
-  HIPC(upload(ctx->d_nodes, nodes48.data(), nodes48.size() * sizeof(DevNode48), s), "upload nodes");
+  HIPC(upload(ctx->d_nodes, compact ? static_cast<const void*>(nodes32.data()) : nodes48.data(), node_bytes, s), "upload nodes");
   HIPC(upload(ctx->d_tris, tris.data(), tris.size() * 4, s), "upload triangles");
   HIPC(upload(ctx->d_lights, lt.lights.data(), lt.lights.size() * sizeof(LightTri), s), "upload lights");
   HIPC(upload(ctx->d_alias_p, lt.prob.data(), lt.prob.size() * 4, s), "upload alias");
   HIPC(upload(ctx->d_alias_i, lt.alias.data(), lt.alias.size() * 4, s), "upload alias");
   if (ctx->two_level) {
     HIPC(upload(ctx->d_inst, inst_orig.data(), inst_orig.size() * sizeof(Instance), s), "upload instances");
-    HIPC(upload(ctx->d_inst_tlas, inst_tlas.data(), inst_tlas.size() * sizeof(Instance), s), "upload instances");
-    HIPC(upload(ctx->d_tlas, tlas48.data(), tlas48.size() * sizeof(DevNode48), s), "upload tlas");
+    HIPC(upload(ctx->d_inst_tlas, inst_tlas.data(), inst_tlas.size() * sizeof(TlasInstance), s), "upload instances");
+    HIPC(upload(ctx->d_tlas, compact ? static_cast<const void*>(tlas32.data()) : tlas48.data(), tlas_bytes, s), "upload tlas");
   }
   HIPC(hipStreamSynchronize(s), "upload");
 
@@ -883,7 +913,7 @@ trt_status trt_build(trt_context* ctx, const trt_build_opts* opts) {
   // stack spill areas of the traversals: stack_cap entries per grid thread, twice (Extend
   // and the Shadow launch that runs beside it)
   ctx->spill_half = size_t(ctx->grid_trace) * 256 * size_t(ctx->stack_cap);
-  ctx->touch_node_words = uint32_t((nodes48.size() + 31) / 32);
+  ctx->touch_node_words = uint32_t((nodes.size() + 31) / 32);
   ctx->touch_tri_words = uint32_t((tris.size() / 12 + 31) / 32);
   HIPC(ctx->d_spill.ensure(2 * ctx->spill_half * 4), "alloc stack spill");
 
@@ -895,7 +925,7 @@ trt_status trt_build(trt_context* ctx, const trt_build_opts* opts) {
   ctx->info.stack_entries = uint32_t(cap);
   ctx->info.sah_cost = sah;
   ctx->info.build_ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
-  ctx->info.device_bytes = nodes48.size() * sizeof(DevNode48) + tris.size() * 4 + tlas48.size() * sizeof(DevNode48);
+  ctx->info.device_bytes = node_bytes + tris.size() * 4 + tlas_bytes;
   ctx->info.two_level = ctx->two_level ? 1 : 0;
   ctx->info.tlas_depth = uint32_t(tlas_depth);
   ctx->info.references = n_refs;
@@ -973,7 +1003,7 @@ trt_status trt_measure_traversal(trt_context* ctx, const trt_render_opts* o, trt
   out->closest_tris_per_ray = st.extend_rays ? double(c[1]) / st.extend_rays : 0.0;
   out->any_nodes_per_ray = st.shadow_rays ? double(c[2]) / st.shadow_rays : 0.0;
   out->any_tris_per_ray = st.shadow_rays ? double(c[3]) / st.shadow_rays : 0.0;
-  out->node_bytes = sizeof(DevNode48);
+  out->node_bytes = ctx->node_bytes;
   out->tri_bytes = 48;
   out->closest_spills = c[4];
   out->any_spills = c[5];

@@ -7,6 +7,7 @@
 // all three axes evaluated, leaves of at most `max_leaf` primitives, subtrees built
 // in parallel on host threads.
 #pragma once
+#include <stddef.h>
 #include <stdint.h>
 
 #include <vector>
@@ -106,6 +107,32 @@ constexpr double kHalfExtentMargin = 1.0 / 1024.0;
 // Converts nodes to the 48-byte layout. False for a non-finite bound, one that cannot
 // carry its byte, or kMaxDeviceNodes nodes or more.
 bool pack_nodes(const std::vector<DevNode2>& in, std::vector<DevNode48>& out);
+
+// Compact traversal layout: 32 bytes, each child box as fp16 centre c and half extent h per
+// axis on a grid of the tree, and the child reference in full:
+//   child k: w[4k + axis] = c | h << 16 (fp16 bits), w[4k + 3] = reference (internal: index x 32)
+// with box = org + scale (c -+ h), org the centre of the tree's bounds and scale a power of
+// two that puts their largest half side R into [2^13, 2^14) grid units, so c is within
+// 2^-12 R of the exact centre. The half extent covers the exact box from the stored centre,
+// is enlarged by 2^-10 of itself and by 2^-19 R (the traversal's slab distances lose up to
+// about 2^-23 R of position to cancellation) and rounded up, so every stored box contains
+// the exact one. The child of a leaf without triangles gets h = -inf, which no ray enters.
+struct NodeSpace {
+  float org[3];
+  float scale;
+};
+struct alignas(16) DevNode32 {
+  uint32_t w[8];
+};
+
+// Converts nodes [first, first + count) of one tree (indices relative to the whole array) to
+// the compact layout. False, with the output unusable, when the tree does not suit it: a
+// non-finite bound or one beyond the grid's range, or more than kCoarseShare of the boxes
+// grow by more than kCoarseGrowth (sum of half extents) because the tree's detail is too
+// fine for its extent (a small object in a large surrounding).
+constexpr double kCoarseGrowth = 1.25;
+constexpr double kCoarseShare = 1.0 / 16.0;
+bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, NodeSpace& space, DevNode32* out);
 
 // Converts a build tree into the device layout (depth-first order, node 0 = root).
 // Returns the device nodes; a root leaf is wrapped in a node with an empty second child.

@@ -35,15 +35,26 @@ struct ShadowQueue {
   float4* emit;     // emission list: rgb, path (bits); null where no Shade writes one
 };
 
+// An instance as the two-level traversal reads it, in the top level's leaf order.
+struct alignas(16) TlasInstance {
+  float w2o[12];
+  NodeSpace space;      // grid of the mesh's tree
+  uint32_t blas_root;   // byte offset of the mesh's root in the node array
+  uint32_t id;          // caller's instance index
+  uint32_t pad[2];
+};
+
 // Acceleration structure views.
 struct DevAccel {
-  const DevNode48* nodes;   // single-level BVH, or all BLAS nodes for two-level scenes
+  const void* nodes;        // single-level BVH, or all BLAS nodes for two-level scenes
   const float4* tris;       // reordered traversal triangles: 3 float4 per triangle (w of row 0 = prim id)
-  const DevNode48* tlas;    // top level over instances (nullptr for single-level)
-  const Instance* inst;     // instances (two-level)
+  const void* tlas;         // top level over instances (nullptr for single-level)
+  const TlasInstance* inst; // instances (two-level)
+  NodeSpace space;          // grid of the single-level tree or of the top level (32-byte nodes)
+  uint32_t node_bytes;      // layout of every node array: sizeof(DevNode32) or sizeof(DevNode48)
   int stack_cap;            // stack entries per lane (tree depth bound)
   int two_level;
-  uint32_t* spill;          // single-level kernels: per-lane stack spill area, stack_cap entries
+  uint32_t* spill;          // per-lane stack spill area, stack_cap entries
                             // per thread of the traversal grid (blockIdx.x * 256 + threadIdx.x)
   uint32_t* touch_nodes;    // counting kernels only (else null): one bit per (bottom-level) node
   uint32_t* touch_tris;     // and per triangle record, set when the launch reads it

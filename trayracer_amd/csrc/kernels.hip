@@ -170,67 +170,138 @@ __device__ __forceinline__ void touch(uint32_t* bits, uint32_t i) {
   if (bits) atomicOr(&bits[i >> 5], 1u << (i & 31u));
 }
 
-// Ray/box slab test of the device traversals (after Ize 2013's conservative form), on
-// boxes stored as centre c and half extent h per axis. With x = c - o and s = sign(inv)
-// (per ray, +-1), a slab's entry and exit are (x - s h) * inv and (x + s h) * inv, the
-// entry never above the exit; each is within a few ulp of itself plus u |x inv|. The
-// stored half extent exceeds the exact box by 2^-10 of itself, which covers the error
-// relative to h, and the far distance is widened by kBoxSlack, which covers the rest, so
-// no box the ray touches is culled and traversal equals a brute-force loop. inv = 1/d is
-// the IEEE reciprocal: for a zero direction component it is +-inf and the products give
-// the exact slab of a ray parallel to the axis: (-inf, +inf) when the origin lies inside
-// it, both +inf or both -inf (an empty interval) when outside, and NaN for an end whose
-// plane the origin lies on; the axes are combined with max / min that ignore NaN, so that
-// end limits nothing. Only FP32 subtracts, multiplies and adds, then three-operand max /
-// min: on gfx950 FP32 arithmetic issues at twice the rate of min / max, so this form is
-// cheaper than ordering each axis's two plane distances with min / max.
-struct RayBox {
-  V3 o;
-  V3 inv;  // 1 / d, infinite for a zero component
-  V3 sgn;  // +-1, the sign of inv
+// Ray/box slab tests of the device traversals (after Ize 2013's conservative form), on
+// boxes stored as centre c and half extent h per axis; one class per node layout. Both
+// are conservative: the far distance is widened by kBoxSlack, which covers errors
+// relative to the distances themselves, and the stored half extents carry margins for the
+// rest, so no box the ray touches is culled and traversal equals a brute-force loop. The
+// axes are combined with max / min that ignore NaN. A node is visited by its byte offset
+// from the (wave-uniform) array base: one 32-bit add per visit.
+struct NodeHits {
+  bool h0, h1;     // child boxes the ray enters in [tmin, tmax]
+  float t0, t1;    // where
+  int32_t c0, c1;  // child references
 };
 
-__device__ __forceinline__ RayBox ray_box_setup(V3 o, V3 d) {
-  RayBox b;
-  b.o = o;
-  b.inv = v3(1.f / d.x, 1.f / d.y, 1.f / d.z);
-  b.sgn = v3(__builtin_copysignf(1.f, b.inv.x), __builtin_copysignf(1.f, b.inv.y), __builtin_copysignf(1.f, b.inv.z));
-  return b;
-}
+// 48-byte nodes: fp32 boxes. With x = c - o and s = sign(inv) (per ray, +-1), a slab's
+// entry and exit are (x - s h) inv and (x + s h) inv, each within a few ulp of itself plus
+// u |x inv|. inv = 1/d is the IEEE reciprocal: for a zero direction component it is +-inf
+// and the products give the exact slab of a ray parallel to the axis.
+struct Nodes48 {
+  static constexpr uint32_t kBytes = kNodeBytes;
+  struct Ray {
+    V3 o;
+    V3 inv;  // 1 / d, infinite for a zero component
+    V3 sgn;  // +-1, the sign of inv
+  };
+  static __device__ __forceinline__ Ray setup(const NodeSpace&, V3 o, V3 d) {
+    Ray b;
+    b.o = o;
+    b.inv = v3(1.f / d.x, 1.f / d.y, 1.f / d.z);
+    b.sgn = v3(__builtin_copysignf(1.f, b.inv.x), __builtin_copysignf(1.f, b.inv.y), __builtin_copysignf(1.f, b.inv.z));
+    return b;
+  }
+  static __device__ __forceinline__ bool slab(float cx, float hx, float cy, float hy, float cz, float hz, const Ray& b,
+                                              float tmin, float tmax, float& tnear) {
+    const float xx = cx - b.o.x, sx = hx * b.sgn.x;
+    const float xy = cy - b.o.y, sy = hy * b.sgn.y;
+    const float xz = cz - b.o.z, sz = hz * b.sgn.z;
+    const float n = __builtin_fmaxf(__builtin_fmaxf((xx - sx) * b.inv.x, (xy - sy) * b.inv.y),
+                                    __builtin_fmaxf((xz - sz) * b.inv.z, tmin));
+    const float f = __builtin_fminf(__builtin_fminf((xx + sx) * b.inv.x, (xy + sy) * b.inv.y),
+                                    __builtin_fminf((xz + sz) * b.inv.z, tmax));
+    tnear = n;
+    return n <= f * kBoxSlack;
+  }
+  // Child reference from the low bytes of one node row (v_perm_b32 gathers two bytes per
+  // instruction).
+  static __device__ __forceinline__ int32_t child_ref(float4 r) {
+    const uint32_t lo = __builtin_amdgcn_perm(__float_as_uint(r.y), __float_as_uint(r.x), 0x0c0c0400u);
+    const uint32_t hi = __builtin_amdgcn_perm(__float_as_uint(r.w), __float_as_uint(r.z), 0x04000c0cu);
+    return static_cast<int32_t>(lo | hi);
+  }
+  static __device__ __forceinline__ NodeHits visit(const void* __restrict__ nodes, int32_t at, const Ray& b, float tmin,
+                                                   float tmax) {
+    const float4* p = reinterpret_cast<const float4*>(static_cast<const char*>(nodes) + static_cast<uint32_t>(at));
+    const float4 r0 = p[0], r1 = p[1], r2 = p[2];
+    NodeHits v;
+    v.h0 = slab(r0.x, r0.y, r0.z, r0.w, r2.x, r2.y, b, tmin, tmax, v.t0);
+    v.h1 = slab(r1.x, r1.y, r1.z, r1.w, r2.z, r2.w, b, tmin, tmax, v.t1);
+    v.c0 = child_ref(r0);
+    v.c1 = child_ref(r1);
+    return v;
+  }
+};
 
-__device__ __forceinline__ bool slab_ch(float cx, float hx, float cy, float hy, float cz, float hz,
-                                        const RayBox& b, float tmin, float tmax, float& tnear) {
-  const float xx = cx - b.o.x, sx = hx * b.sgn.x;
-  const float xy = cy - b.o.y, sy = hy * b.sgn.y;
-  const float xz = cz - b.o.z, sz = hz * b.sgn.z;
-  const float n = __builtin_fmaxf(__builtin_fmaxf((xx - sx) * b.inv.x, (xy - sy) * b.inv.y),
-                                  __builtin_fmaxf((xz - sz) * b.inv.z, tmin));
-  const float f = __builtin_fminf(__builtin_fminf((xx + sx) * b.inv.x, (xy + sy) * b.inv.y),
-                                  __builtin_fminf((xz + sz) * b.inv.z, tmax));
-  tnear = n;
-  return n <= f * kBoxSlack;
-}
-
-// Child reference from the low bytes of one node row (v_perm_b32 gathers two bytes per
-// instruction).
-__device__ __forceinline__ int32_t row_child_ref(float4 r) {
-  const uint32_t lo = __builtin_amdgcn_perm(__float_as_uint(r.y), __float_as_uint(r.x), 0x0c0c0400u);
-  const uint32_t hi = __builtin_amdgcn_perm(__float_as_uint(r.w), __float_as_uint(r.z), 0x04000c0cu);
-  return static_cast<int32_t>(lo | hi);
-}
-
-// One node at byte offset i (node references are byte offsets): three 16-byte loads,
-// child references from the x / y values' low bytes.
-__device__ __forceinline__ void load_node(const DevNode48* __restrict__ nodes, int32_t i, float4& r0, float4& r1,
-                                          float4& r2, int4& c) {
-  // a 32-bit offset from the (wave-uniform) array base: one add per visit and a load with
-  // a scalar base, instead of 64-bit address arithmetic
-  const float4* p = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(nodes) + static_cast<uint32_t>(i));
-  r0 = p[0];
-  r1 = p[1];
-  r2 = p[2];
-  c = make_int4(row_child_ref(r0), row_child_ref(r1), 0, 0);
-}
+// 32-byte nodes: fp16 boxes on the tree's grid (NodeSpace: world = org + scale * c). Two
+// 16-byte loads a visit instead of three (the load path bounds the traversal), and nothing
+// to decode: v_fma_mix_f32 takes an fp16 operand as it is, so per axis
+//   ct = fma(c, scale inv, (org - o) inv),  entry = ct - h |scale inv|,  exit = ct + h |scale inv|
+// are three instructions (six, plus six to gather the child references, with Nodes48).
+// The terms that cancel in ct have an error of up to 2u (|x| + R) |inv| (x the distance to
+// the box's centre, R the tree's half size): the part in |x| is relative to the distances,
+// and the half extents' margins (bvh_build.h) exceed the part in R. A direction component
+// below 2^-60 of the largest takes that magnitude, which moves no ray by more than the
+// margins; rays so extreme that a term could overflow take every box (NaN, which the axes'
+// max / min ignore): slow and still exact.
+struct Nodes32 {
+  static constexpr uint32_t kBytes = sizeof(DevNode32);
+  struct Ray {
+    V3 o;
+    V3 si;  // scale / d
+    V3 oi;  // (org - o) / d
+  };
+  static __device__ __forceinline__ Ray setup(const NodeSpace& g, V3 o, V3 d) {
+    Ray b;
+    b.o = o;
+    const float m = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(d.x), __builtin_fabsf(d.y)), __builtin_fabsf(d.z));
+    const float lim = m * 0x1p-60f;
+    const float ix = 1.f / (__builtin_fabsf(d.x) < lim ? __builtin_copysignf(lim, d.x) : d.x);
+    const float iy = 1.f / (__builtin_fabsf(d.y) < lim ? __builtin_copysignf(lim, d.y) : d.y);
+    const float iz = 1.f / (__builtin_fabsf(d.z) < lim ? __builtin_copysignf(lim, d.z) : d.z);
+    const V3 w = v3(g.org[0] - o.x, g.org[1] - o.y, g.org[2] - o.z);
+    b.si = v3(ix * g.scale, iy * g.scale, iz * g.scale);
+    b.oi = v3(w.x * ix, w.y * iy, w.z * iz);
+    // |si| in [2^-100, 2^100], |oi| < 2^126, |org - o| < 2^50 scale (2^36 R), all finite
+    const float s_hi = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(b.si.x), __builtin_fabsf(b.si.y)), __builtin_fabsf(b.si.z));
+    const float s_lo = __builtin_fminf(__builtin_fminf(__builtin_fabsf(b.si.x), __builtin_fabsf(b.si.y)), __builtin_fabsf(b.si.z));
+    const float o_hi = __builtin_fabsf(b.oi.x) + __builtin_fabsf(b.oi.y) + __builtin_fabsf(b.oi.z);
+    const float w_hi = __builtin_fabsf(w.x) + __builtin_fabsf(w.y) + __builtin_fabsf(w.z);
+    if (!(s_lo >= 0x1p-100f && s_hi <= 0x1p100f && o_hi < 0x1p126f && w_hi < 0x1p50f * g.scale)) {
+      b.si = v3(0.f);
+      b.oi = v3(__builtin_nanf(""));
+    }
+    return b;
+  }
+  // v: fp16 (c, h) pairs of the axes, then the child reference
+  static __device__ __forceinline__ bool slab(uint4 v, const Ray& b, float tmin, float tmax, float& tnear) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    const h2 x = __builtin_bit_cast(h2, v.x), y = __builtin_bit_cast(h2, v.y), z = __builtin_bit_cast(h2, v.z);
+    const float cx = __builtin_fmaf(static_cast<float>(x[0]), b.si.x, b.oi.x);
+    const float cy = __builtin_fmaf(static_cast<float>(y[0]), b.si.y, b.oi.y);
+    const float cz = __builtin_fmaf(static_cast<float>(z[0]), b.si.z, b.oi.z);
+    const float ax = __builtin_fabsf(b.si.x), ay = __builtin_fabsf(b.si.y), az = __builtin_fabsf(b.si.z);
+    const float n = __builtin_fmaxf(
+        __builtin_fmaxf(__builtin_fmaf(-static_cast<float>(x[1]), ax, cx), __builtin_fmaf(-static_cast<float>(y[1]), ay, cy)),
+        __builtin_fmaxf(__builtin_fmaf(-static_cast<float>(z[1]), az, cz), tmin));
+    const float f = __builtin_fminf(
+        __builtin_fminf(__builtin_fmaf(static_cast<float>(x[1]), ax, cx), __builtin_fmaf(static_cast<float>(y[1]), ay, cy)),
+        __builtin_fminf(__builtin_fmaf(static_cast<float>(z[1]), az, cz), tmax));
+    tnear = n;
+    return n <= f * kBoxSlack;
+  }
+  static __device__ __forceinline__ NodeHits visit(const void* __restrict__ nodes, int32_t at, const Ray& b, float tmin,
+                                                   float tmax) {
+    const uint4* p = reinterpret_cast<const uint4*>(static_cast<const char*>(nodes) + static_cast<uint32_t>(at));
+    const uint4 r0 = p[0], r1 = p[1];
+    NodeHits v;
+    v.h0 = slab(r0, b, tmin, tmax, v.t0);
+    v.h1 = slab(r1, b, tmin, tmax, v.t1);
+    v.c0 = static_cast<int32_t>(r0.w);
+    v.c1 = static_cast<int32_t>(r1.w);
+    return v;
+  }
+};
 
 // Sentinel of an exhausted traversal (never a leaf code: leaf first indices are < 2^28).
 constexpr int32_t kTravDone = static_cast<int32_t>(0x80000000u);
@@ -491,19 +562,19 @@ __device__ __forceinline__ bool leaf_phase(const LeafTasks& tk, const float4* __
 
 __device__ __forceinline__ int32_t pack_axes(const RayTri& t) { return t.kx | (t.ky << 2) | (t.kz << 4); }
 
-template <bool ANY, bool STATS, class Load, class Finish>
+template <class Nodes, bool ANY, bool STATS, class Load, class Finish>
 __device__ __forceinline__ void trace_queue(const DevAccel& acc, const SegIn& in, uint32_t* stk, uint32_t* tsk,
                                             uint32_t* overflow, TraceOut& stats, Load load, Finish finish) {
   const uint32_t lane = lane_id();
   const uint32_t n_seg = seg_counts(in), home = block_home();
   const int cap = acc.stack_cap;
-  const DevNode48* __restrict__ nodes = acc.nodes;
+  const void* __restrict__ nodes = acc.nodes;
   const float4* __restrict__ tris = acc.tris;
   uint64_t seg_done = seg_empty(n_seg, home, gridDim.x >= kSegs);
   bool drained = false;
   uint32_t slot = kNoHit;
   V3 o = v3(0.f), d = v3(0.f);
-  RayBox rb{};
+  typename Nodes::Ray rb{};
   float tmin = 0.f;
   int32_t kxyz = 0;        // ray_tri_setup's axis permutation, 2 bits per axis
   V3 shear = v3(0.f);      // and its shear constants
@@ -534,7 +605,7 @@ __device__ __forceinline__ void trace_queue(const DevAccel& acc, const SegIn& in
           const RayTri rt = ray_tri_setup(o, d);
           kxyz = pack_axes(rt);
           shear = v3(rt.sx, rt.sy, rt.sz);
-          rb = ray_box_setup(o, d);
+          rb = Nodes::setup(acc.space, o, d);
           r.t = tmax;
           r.prim = kNoHit;
           r.inst = kNoInstance;
@@ -550,28 +621,20 @@ __device__ __forceinline__ void trace_queue(const DevAccel& acc, const SegIn& in
     // inner nodes: a wave-uniform loop in which lanes without an inner node idle
     for (bool walks = node >= 0;;) {
       if (walks) {
-        float4 r0, r1, r2;
-        int4 c;
-        load_node(nodes, node, r0, r1, r2, c);
+        const NodeHits v = Nodes::visit(nodes, node, rb, tmin, r.t);
         if (STATS) {
           stats.nodes++;
-          touch(acc.touch_nodes, static_cast<uint32_t>(node) / kNodeBytes);
+          touch(acc.touch_nodes, static_cast<uint32_t>(node) / Nodes::kBytes);
         }
-        float t0, t1;
-        const bool h0 = slab_ch(r0.x, r0.y, r0.z, r0.w, r2.x, r2.y, rb, tmin, r.t, t0);
-        const bool h1 = slab_ch(r1.x, r1.y, r1.z, r1.w, r2.z, r2.w, rb, tmin, r.t, t1);
-        if (h0 && h1) {
-          int32_t nearc = c.x, farc = c.y;
-          if (t1 < t0) {
-            nearc = c.y;
-            farc = c.x;
-          }
+        if (v.h0 && v.h1) {
+          const bool swap = v.t1 < v.t0;
+          const int32_t farc = swap ? v.c0 : v.c1;
           stack_push<STATS>(st, static_cast<uint32_t>(farc), stats, [&] { atomicOr(overflow, 1u); });
-          node = nearc;
-        } else if (h0) {
-          node = c.x;
-        } else if (h1) {
-          node = c.y;
+          node = swap ? v.c1 : v.c0;
+        } else if (v.h0) {
+          node = v.c0;
+        } else if (v.h1) {
+          node = v.c1;
         } else {
           node = pop();
         }
@@ -629,20 +692,20 @@ __device__ __forceinline__ void trace_queue(const DevAccel& acc, const SegIn& in
 constexpr int32_t kTravExit = 0x7fffffff;                               // leave the instance (stack marker)
 constexpr int32_t kTravBlocked = static_cast<int32_t>(0x80000001u);     // waits at the marker with a parked leaf
 
-template <bool ANY, bool STATS, class Load, class Finish>
+template <class Nodes, bool ANY, bool STATS, class Load, class Finish>
 __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& in, uint32_t* stk, uint32_t* tsk,
                                              uint32_t* overflow, TraceOut& stats, Load load, Finish finish) {
   const uint32_t lane = lane_id();
   const uint32_t n_seg = seg_counts(in), home = wave_home();
   const int cap = acc.stack_cap;
-  const DevNode48* __restrict__ blas = acc.nodes;
-  const DevNode48* __restrict__ tlas = acc.tlas;
+  const void* __restrict__ blas = acc.nodes;
+  const void* __restrict__ tlas = acc.tlas;
   const float4* __restrict__ tris = acc.tris;
   uint64_t seg_done = seg_empty(n_seg);
   bool drained = false;
   uint32_t slot = kNoHit;
   V3 ow = v3(0.f), dw = v3(0.f);
-  RayBox rb{};  // in the current space (world outside instances)
+  typename Nodes::Ray rb{};  // in the current space (world outside instances)
   int32_t kxyz = 0;    // ray_tri_setup's axis permutation in the current instance, 2 bits per axis
   V3 shear = v3(0.f);  // and its shear constants
   float tmin = 0.f;
@@ -678,7 +741,7 @@ __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& i
         return kTravBlocked;
       }
       in_blas = false;
-      rb = ray_box_setup(ow, dw);  // back in world space (recomputed: fewer live registers)
+      rb = Nodes::setup(acc.space, ow, dw);  // back in world space (recomputed: fewer live registers)
     }
   };
   // Top-level leaf (instances [first, first + count)): enter the first instance.
@@ -687,10 +750,10 @@ __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& i
     const uint32_t first = c >> 3, cnt = c & 7u;
     if (cnt > 1u) push(~(((first + 1u) << 3) | (cnt - 1u)));  // the rest of the leaf
     push(static_cast<uint32_t>(kTravExit));
-    const Instance& ins = acc.inst[first];
+    const TlasInstance& ins = acc.inst[first];
     const V3 o = xform_point(ins.w2o, ow);
     const V3 d = xform_vector(ins.w2o, dw);
-    rb = ray_box_setup(o, d);
+    rb = Nodes::setup(ins.space, o, d);
     const RayTri rt = ray_tri_setup(o, d);
     kxyz = pack_axes(rt);
     shear = v3(rt.sx, rt.sy, rt.sz);
@@ -717,7 +780,7 @@ __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& i
           slot = base + rank;
           float tmax;
           load(slot, ow, dw, tmin, tmax);
-          rb = ray_box_setup(ow, dw);
+          rb = Nodes::setup(acc.space, ow, dw);
           in_blas = false;
           r.t = tmax;
           r.prim = kNoHit;
@@ -735,28 +798,19 @@ __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& i
       // inner nodes of either level (a while loop: the uniform form of the single-level
       // loop costs this kernel register spills)
       while (node >= 0) {
-        float4 r0, r1, r2;
-        int4 c;
-        load_node(in_blas ? blas : tlas, node, r0, r1, r2, c);
+        const NodeHits v = Nodes::visit(in_blas ? blas : tlas, node, rb, tmin, r.t);
         if (STATS) {
           stats.nodes++;
-          if (in_blas) touch(acc.touch_nodes, static_cast<uint32_t>(node) / kNodeBytes);
+          if (in_blas) touch(acc.touch_nodes, static_cast<uint32_t>(node) / Nodes::kBytes);
         }
-        float t0, t1;
-        const bool h0 = slab_ch(r0.x, r0.y, r0.z, r0.w, r2.x, r2.y, rb, tmin, r.t, t0);
-        const bool h1 = slab_ch(r1.x, r1.y, r1.z, r1.w, r2.z, r2.w, rb, tmin, r.t, t1);
-        if (h0 && h1) {
-          int32_t nearc = c.x, farc = c.y;
-          if (t1 < t0) {
-            nearc = c.y;
-            farc = c.x;
-          }
-          push(static_cast<uint32_t>(farc));
-          node = nearc;
-        } else if (h0) {
-          node = c.x;
-        } else if (h1) {
-          node = c.y;
+        if (v.h0 && v.h1) {
+          const bool swap = v.t1 < v.t0;
+          push(static_cast<uint32_t>(swap ? v.c0 : v.c1));
+          node = swap ? v.c1 : v.c0;
+        } else if (v.h0) {
+          node = v.c0;
+        } else if (v.h1) {
+          node = v.c1;
         } else {
           node = pop();
         }
@@ -936,14 +990,14 @@ struct RayLoad {
 // Single-level scenes: Extend and Shadow through trace_queue. Both are held to 72
 // VGPRs, 7 waves per SIMD (the allocator otherwise settles just above, at 6 waves,
 // which measured 5% slower).
-template <bool STATS>
+template <class Nodes, bool STATS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_extend_sl(DevAccel acc, RayQueue q, HitBuf h, SegIn in, uint32_t* ctr) {
   extern __shared__ uint32_t lds[];
   TraceOut st;
   st.nodes = 0;
   st.tests = 0;
   st.spills = 0;
-  trace_queue<false, STATS>(
+  trace_queue<Nodes, false, STATS>(
       acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st,
       RayLoad{q.o_tmin, q.d_tmax},
       [&](uint32_t slot, const TraceOut& r, bool) {
@@ -956,7 +1010,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
   }
 }
 
-template <bool STATS>
+template <class Nodes, bool STATS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_shadow_sl(DevAccel acc, ShadowQueue sq, float4* radiance, SegIn in,
                                                        uint32_t* ctr) {
   extern __shared__ uint32_t lds[];
@@ -964,7 +1018,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
   st.nodes = 0;
   st.tests = 0;
   st.spills = 0;
-  trace_queue<true, STATS>(
+  trace_queue<Nodes, true, STATS>(
       acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st,
       RayLoad{sq.o_tmin, sq.d_tmax},
       [&](uint32_t slot, const TraceOut&, bool occluded) {
@@ -987,14 +1041,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
 
 // Two-level scenes: Extend and Shadow through trace_queue2, held to 80 VGPRs, 6 waves
 // per SIMD (a few spilled dwords; 5 waves at the allocator's 86 measured 5% slower).
-template <bool STATS>
+template <class Nodes, bool STATS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_extend_tl(DevAccel acc, RayQueue q, HitBuf h, SegIn in, uint32_t* ctr) {
   extern __shared__ uint32_t lds[];
   TraceOut st;
   st.nodes = 0;
   st.tests = 0;
   st.spills = 0;
-  trace_queue2<false, STATS>(
+  trace_queue2<Nodes, false, STATS>(
       acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st,
       RayLoad{q.o_tmin, q.d_tmax},
       [&](uint32_t slot, const TraceOut& r, bool) {
@@ -1008,7 +1062,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
   }
 }
 
-template <bool STATS>
+template <class Nodes, bool STATS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_shadow_tl(DevAccel acc, ShadowQueue sq, float4* radiance, SegIn in,
                                                        uint32_t* ctr) {
   extern __shared__ uint32_t lds[];
@@ -1016,7 +1070,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
   st.nodes = 0;
   st.tests = 0;
   st.spills = 0;
-  trace_queue2<true, STATS>(
+  trace_queue2<Nodes, true, STATS>(
       acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st,
       RayLoad{sq.o_tmin, sq.d_tmax},
       [&](uint32_t slot, const TraceOut&, bool occluded) {
@@ -1398,20 +1452,22 @@ __device__ __forceinline__ void finish_shadow_adj(const ShadowQueue& sq, const A
   ab.rec_b[r] = gb;
 }
 
+template <class Nodes>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_shadow_adj_sl(
     DevAccel acc, ShadowQueue sq, AdjBuffers ab, SegIn in, uint32_t* ctr, uint32_t depth) {
   extern __shared__ uint32_t lds[];
   TraceOut st;
-  trace_queue<true, false>(
+  trace_queue<Nodes, true, false>(
       acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st, RayLoad{sq.o_tmin, sq.d_tmax},
       [&](uint32_t slot, const TraceOut&, bool occluded) { finish_shadow_adj(sq, ab, depth, slot, occluded); });
 }
 
+template <class Nodes>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_shadow_adj_tl(
     DevAccel acc, ShadowQueue sq, AdjBuffers ab, SegIn in, uint32_t* ctr, uint32_t depth) {
   extern __shared__ uint32_t lds[];
   TraceOut st;
-  trace_queue2<true, false>(
+  trace_queue2<Nodes, true, false>(
       acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st, RayLoad{sq.o_tmin, sq.d_tmax},
       [&](uint32_t slot, const TraceOut&, bool occluded) { finish_shadow_adj(sq, ab, depth, slot, occluded); });
 }
@@ -1511,36 +1567,48 @@ size_t trace_lds_bytes() { return ring_lds_bytes() + static_cast<size_t>(kTaskWo
 
 }  // namespace
 
-int trace_blocks_per_cu(const DevAccel& acc) {
-  int a = 0, b = 0;
-  hipError_t ea, eb;
-  if (acc.two_level) {
-    ea = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_extend_tl<false>, kBlock, trace_lds_bytes());
-    eb = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_shadow_tl<false>, kBlock, trace_lds_bytes());
-  } else {
-    ea = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_extend_sl<false>, kBlock, trace_lds_bytes());
-    eb = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_shadow_sl<false>, kBlock, trace_lds_bytes());
-  }
-  if (ea != hipSuccess) a = 4;
-  if (eb != hipSuccess) b = 4;
-  const int m = a < b ? a : b;
-  return m > 0 ? m : 1;
+// Calls f with the node layout of an acceleration structure.
+template <class F>
+auto with_nodes(const DevAccel& acc, F f) {
+  return acc.node_bytes == Nodes32::kBytes ? f(Nodes32{}) : f(Nodes48{});
 }
 
-bool traversal_lds_check() {
-  // The queue traversals address their LDS rings as 4 KiB-aligned blocks from LDS
-  // address 0: they must have no static LDS, which would move dynamic LDS up.
-  const void* ks[] = {reinterpret_cast<const void*>(k_extend_sl<false>), reinterpret_cast<const void*>(k_extend_sl<true>),
-                      reinterpret_cast<const void*>(k_shadow_sl<false>), reinterpret_cast<const void*>(k_shadow_sl<true>),
-                      reinterpret_cast<const void*>(k_extend_tl<false>), reinterpret_cast<const void*>(k_extend_tl<true>),
-                      reinterpret_cast<const void*>(k_shadow_tl<false>), reinterpret_cast<const void*>(k_shadow_tl<true>),
-                      reinterpret_cast<const void*>(k_shadow_adj_sl), reinterpret_cast<const void*>(k_shadow_adj_tl)};
+int trace_blocks_per_cu(const DevAccel& acc) {
+  return with_nodes(acc, [&](auto nodes) {
+    using N = decltype(nodes);
+    int a = 0, b = 0;
+    hipError_t ea, eb;
+    if (acc.two_level) {
+      ea = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_extend_tl<N, false>, kBlock, trace_lds_bytes());
+      eb = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_shadow_tl<N, false>, kBlock, trace_lds_bytes());
+    } else {
+      ea = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_extend_sl<N, false>, kBlock, trace_lds_bytes());
+      eb = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_shadow_sl<N, false>, kBlock, trace_lds_bytes());
+    }
+    if (ea != hipSuccess) a = 4;
+    if (eb != hipSuccess) b = 4;
+    const int m = a < b ? a : b;
+    return m > 0 ? m : 1;
+  });
+}
+
+// The queue traversals address their LDS rings as 4 KiB-aligned blocks from LDS
+// address 0: they must have no static LDS, which would move dynamic LDS up.
+template <class N>
+static bool no_static_lds() {
+  const void* ks[] = {reinterpret_cast<const void*>(k_extend_sl<N, false>), reinterpret_cast<const void*>(k_extend_sl<N, true>),
+                      reinterpret_cast<const void*>(k_shadow_sl<N, false>), reinterpret_cast<const void*>(k_shadow_sl<N, true>),
+                      reinterpret_cast<const void*>(k_extend_tl<N, false>), reinterpret_cast<const void*>(k_extend_tl<N, true>),
+                      reinterpret_cast<const void*>(k_shadow_tl<N, false>), reinterpret_cast<const void*>(k_shadow_tl<N, true>),
+                      reinterpret_cast<const void*>(k_shadow_adj_sl<N>), reinterpret_cast<const void*>(k_shadow_adj_tl<N>)};
   for (const void* k : ks) {
     hipFuncAttributes a{};
     if (hipFuncGetAttributes(&a, k) != hipSuccess || a.sharedSizeBytes != 0) return false;
   }
   return true;
 }
+
+bool traversal_lds_check() { return no_static_lds<Nodes32>() && no_static_lds<Nodes48>(); }
 
 void launch_zero_counters(uint32_t* ctr, hipStream_t stream) {
   hipLaunchKernelGGL(k_zero_counters, dim3((kNumCounters + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, ctr);
@@ -1569,18 +1637,12 @@ void launch_raygen(const RenderParams& rp, uint32_t n_paths, uint32_t cap, RayQu
 
 void launch_extend(const DevAccel& acc, RayQueue q, HitBuf h, SegIn in, uint32_t* ctr, int grid, bool stats,
                    hipStream_t stream) {
-  if (!acc.two_level) {
-    if (stats)
-      hipLaunchKernelGGL(k_extend_sl<true>, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, q, h, in, ctr);
-    else
-      hipLaunchKernelGGL(k_extend_sl<false>, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, q, h, in,
-                         ctr);
-    return;
-  }
-  if (stats)
-    hipLaunchKernelGGL(k_extend_tl<true>, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, q, h, in, ctr);
-  else
-    hipLaunchKernelGGL(k_extend_tl<false>, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, q, h, in, ctr);
+  with_nodes(acc, [&](auto nodes) {
+    using N = decltype(nodes);
+    const auto k = acc.two_level ? (stats ? k_extend_tl<N, true> : k_extend_tl<N, false>)
+                                 : (stats ? k_extend_sl<N, true> : k_extend_sl<N, false>);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, q, h, in, ctr);
+  });
 }
 
 void launch_shade(const SceneView& sv, const Material* sampling_mats, const RenderParams& rp, RayQueue q,
@@ -1606,21 +1668,12 @@ void launch_emit(const float4* emit, const uint32_t* emit_cnt, uint32_t cap, flo
 
 void launch_shadow(const DevAccel& acc, ShadowQueue sq, float4* radiance, SegIn in, uint32_t* ctr, int grid,
                    bool stats, hipStream_t stream) {
-  if (!acc.two_level) {
-    if (stats)
-      hipLaunchKernelGGL(k_shadow_sl<true>, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, sq, radiance,
-                         in, ctr);
-    else
-      hipLaunchKernelGGL(k_shadow_sl<false>, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, sq, radiance,
-                         in, ctr);
-    return;
-  }
-  if (stats)
-    hipLaunchKernelGGL(k_shadow_tl<true>, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, sq, radiance, in,
-                       ctr);
-  else
-    hipLaunchKernelGGL(k_shadow_tl<false>, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, sq, radiance, in,
-                       ctr);
+  with_nodes(acc, [&](auto nodes) {
+    using N = decltype(nodes);
+    const auto k = acc.two_level ? (stats ? k_shadow_tl<N, true> : k_shadow_tl<N, false>)
+                                 : (stats ? k_shadow_sl<N, true> : k_shadow_sl<N, false>);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, sq, radiance, in, ctr);
+  });
 }
 
 void launch_finalize(const RenderParams& rp, const float4* radiance, FrameBuffers fb, uint32_t reset,
@@ -1651,10 +1704,11 @@ void launch_shade_adj(const SceneView& sv, const Material* sampling_mats, const 
 
 void launch_shadow_adj(const DevAccel& acc, ShadowQueue sq, const AdjBuffers& ab, SegIn in, uint32_t* ctr,
                        uint32_t depth, int grid, hipStream_t stream) {
-  if (acc.two_level)
-    hipLaunchKernelGGL(k_shadow_adj_tl, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, sq, ab, in, ctr, depth);
-  else
-    hipLaunchKernelGGL(k_shadow_adj_sl, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, sq, ab, in, ctr, depth);
+  with_nodes(acc, [&](auto nodes) {
+    using N = decltype(nodes);
+    const auto k = acc.two_level ? k_shadow_adj_tl<N> : k_shadow_adj_sl<N>;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, sq, ab, in, ctr, depth);
+  });
 }
 
 void launch_grad_reduce(const AdjBuffers& ab, uint32_t mat_lo, uint32_t n_mat, float* partial, float* out,
