@@ -42,11 +42,15 @@ struct Ray32 {
   float si[3], oi[3];
 };
 static Ray32 setup(const NodeSpace& g, const float* o, const float* d) {
+  static int turn = 0;
+  ++turn;
   Ray32 b;
   const float m = std::max(std::max(std::fabs(d[0]), std::fabs(d[1])), std::fabs(d[2])), lim = m * 0x1p-60f;
   float s_hi = 0.f, s_lo = HUGE_VALF, o_hi = 0.f, w_hi = 0.f;
   for (int k = 0; k < 3; ++k) {
-    const float i = 1.f / (std::fabs(d[k]) < lim ? std::copysign(lim, d[k]) : d[k]), w = g.org[k] - o[k];
+    float i = 1.f / (std::fabs(d[k]) < lim ? std::copysign(lim, d[k]) : d[k]);
+    i = std::nextafter(i, k == turn % 3 ? 0.f : std::copysign(HUGE_VALF, i));  // v_rcp_f32 is within an ulp
+    const float w = g.org[k] - o[k];
     b.si[k] = i * g.scale;
     b.oi[k] = w * i;
     s_hi = std::max(s_hi, std::fabs(b.si[k]));

@@ -866,13 +866,13 @@ trt_status trt_build(trt_context* ctx, const trt_build_opts* opts) {
   std::vector<NodeSpace> mesh_space(ctx->meshes.size());
   bool compact = true;
   if (!ctx->two_level) {
-    compact = pack_nodes32(nodes, 0, nodes.size(), ctx->space, nodes32.data());
+    compact = pack_nodes32(nodes, 0, nodes.size(), ctx->space, nodes32.data(), threads);
   } else {
     for (size_t mi = 0; mi < ctx->meshes.size() && compact; ++mi) {
       const size_t end = mi + 1 < ctx->meshes.size() ? blas_root[mi + 1] : nodes.size();
-      compact = pack_nodes32(nodes, blas_root[mi], end - blas_root[mi], mesh_space[mi], nodes32.data());
+      compact = pack_nodes32(nodes, blas_root[mi], end - blas_root[mi], mesh_space[mi], nodes32.data(), threads);
     }
-    compact = compact && pack_nodes32(tlas_nodes, 0, tlas_nodes.size(), ctx->space, tlas32.data());
+    compact = compact && pack_nodes32(tlas_nodes, 0, tlas_nodes.size(), ctx->space, tlas32.data(), threads);
   }
   if (!compact && (!pack_nodes(nodes, nodes48) || !pack_nodes(tlas_nodes, tlas48)))
     return fail(ctx, TRT_UNSUPPORTED, "scene bounds too large for the node layout (infinite coordinates)");

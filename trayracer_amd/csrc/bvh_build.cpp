@@ -7,6 +7,7 @@
 #include <cstring>
 #include <future>
 #include <limits>
+#include <thread>
 
 namespace trt {
 namespace {
@@ -473,30 +474,39 @@ bool pack_nodes(const std::vector<DevNode2>& in, std::vector<DevNode48>& out) {
 
 namespace {
 
+// 2^e as a double, e in the normal range.
+double exp2_int(int e) {
+  const uint64_t u = uint64_t(e + 1023) << 52;
+  double d;
+  std::memcpy(&d, &u, 8);
+  return d;
+}
+
 // fp16 bits of v >= 0: to nearest (even), or upward. v < 2^16; below 2^-14 the spacing stays
 // that of the subnormals.
 uint32_t half_bits(double v, bool up) {
   if (!(v > 0.0)) return 0u;
-  int e = 0;
-  (void)std::frexp(v, &e);  // v in [2^(e-1), 2^e)
+  uint64_t u;
+  std::memcpy(&u, &v, 8);
+  const int e = int(u >> 52) - 1022;    // v in [2^(e-1), 2^e)
   const int q = std::max(e - 11, -24);  // exponent of the last place
-  const double m = std::ldexp(v, -q);
-  const double r = up ? std::ceil(m) : std::nearbyint(m);
+  const double m = v * exp2_int(-q);
   // r in [0, 2^11]: adding it below the exponent field carries into it where it must
+  const uint32_t r = uint32_t(up ? std::ceil(m) : std::nearbyint(m));
   const uint32_t expo = uint32_t(q + 24);
-  const uint32_t mant = uint32_t(r);
-  return expo == 0u ? mant : ((expo + 1u) << 10) + (mant - 1024u);
+  return expo == 0u ? r : ((expo + 1u) << 10) + (r - 1024u);
 }
 
 double half_value(uint32_t h) {
   const int e = int((h >> 10) & 31u);
   const double m = double(h & 1023u);
-  return e == 0 ? std::ldexp(m, -24) : std::ldexp(1024.0 + m, e - 25);
+  return e == 0 ? m * exp2_int(-24) : (1024.0 + m) * exp2_int(e - 25);
 }
 
 }  // namespace
 
-bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, NodeSpace& space, DevNode32* out) {
+bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, NodeSpace& space, DevNode32* out,
+                  int n_threads) {
   static_assert(sizeof(DevNode32) == 32, "node size");
   auto empty = [](int32_t c) { return c < 0 && (~uint32_t(c) & 7u) == 0u; };
   auto bounds = [](const DevNode2& n, int c, float lo[3], float hi[3]) {
@@ -525,38 +535,56 @@ bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, N
   if (!std::isfinite(R) || e < -60 || e > 60) return false;
   space.scale = float(std::ldexp(1.0, e - 14));
   const double S = space.scale, slack = R * std::ldexp(1.0, -19);
-  size_t boxes = 0, coarse = 0;
-  for (size_t i = first; i < first + count; ++i) {
-    const DevNode2& n = in[i];
-    DevNode32& d = out[i];
-    for (int c = 0; c < 2; ++c) {
-      const int32_t ref = n.c[c];
-      d.w[4 * c + 3] = uint32_t(ref >= 0 ? ref * int32_t(sizeof(DevNode32)) : ref);
-      if (empty(ref)) {
-        for (int k = 0; k < 3; ++k) d.w[4 * c + k] = 0xfc000000u;  // c = 0, h = -inf
-        continue;
+  std::atomic<size_t> boxes{0}, coarse{0};
+  std::atomic<bool> fits{true};
+  auto pack_range = [&](size_t begin, size_t end) {
+    size_t n_boxes = 0, n_coarse = 0;
+    for (size_t i = begin; i < end; ++i) {
+      const DevNode2& n = in[i];
+      DevNode32& d = out[i];
+      for (int c = 0; c < 2; ++c) {
+        const int32_t ref = n.c[c];
+        d.w[4 * c + 3] = uint32_t(ref >= 0 ? ref * int32_t(sizeof(DevNode32)) : ref);
+        if (empty(ref)) {
+          for (int k = 0; k < 3; ++k) d.w[4 * c + k] = 0xfc000000u;  // c = 0, h = -inf
+          continue;
+        }
+        float lo[3], hi[3];
+        bounds(n, c, lo, hi);
+        double exact = 0.0, stored = 0.0;
+        for (int k = 0; k < 3; ++k) {
+          const double mid = (0.5 * (double(lo[k]) + double(hi[k])) - space.org[k]) / S;
+          if (!(std::fabs(mid) < 32768.0)) {
+            fits = false;
+            return;
+          }
+          const uint32_t cb = half_bits(std::fabs(mid), false) | (mid < 0.0 ? 0x8000u : 0u);
+          const double cs = (mid < 0.0 ? -1.0 : 1.0) * half_value(cb & 0x7fffu) * S + space.org[k];
+          const double half = std::max(double(hi[k]) - cs, cs - double(lo[k]));
+          const double h = (half * (1.0 + kHalfExtentMargin) + slack) / S;
+          if (!(h < 65504.0)) {
+            fits = false;
+            return;
+          }
+          const uint32_t hb = half_bits(h, true);
+          d.w[4 * c + k] = cb | (hb << 16);
+          exact += 0.5 * (double(hi[k]) - double(lo[k]));
+          stored += half_value(hb) * S;
+        }
+        ++n_boxes;
+        n_coarse += stored > kCoarseGrowth * exact ? 1u : 0u;
       }
-      float lo[3], hi[3];
-      bounds(n, c, lo, hi);
-      double exact = 0.0, stored = 0.0;
-      for (int k = 0; k < 3; ++k) {
-        const double mid = (0.5 * (double(lo[k]) + double(hi[k])) - space.org[k]) / S;
-        if (!(std::fabs(mid) < 32768.0)) return false;
-        const uint32_t cb = half_bits(std::fabs(mid), false) | (mid < 0.0 ? 0x8000u : 0u);
-        const double cs = (mid < 0.0 ? -1.0 : 1.0) * half_value(cb & 0x7fffu) * S + space.org[k];
-        const double half = std::max(double(hi[k]) - cs, cs - double(lo[k]));
-        const double h = (half * (1.0 + kHalfExtentMargin) + slack) / S;
-        if (!(h < 65504.0)) return false;
-        const uint32_t hb = half_bits(h, true);
-        d.w[4 * c + k] = cb | (hb << 16);
-        exact += 0.5 * (double(hi[k]) - double(lo[k]));
-        stored += half_value(hb) * S;
-      }
-      ++boxes;
-      coarse += stored > kCoarseGrowth * exact ? 1u : 0u;
     }
-  }
-  return double(coarse) <= kCoarseShare * double(boxes);
+    boxes += n_boxes;
+    coarse += n_coarse;
+  };
+  const size_t n_parts = std::min<size_t>(size_t(std::max(1, n_threads)), count / 16384 + 1);
+  std::vector<std::thread> pool;
+  for (size_t t = 1; t < n_parts; ++t)
+    pool.emplace_back(pack_range, first + count * t / n_parts, first + count * (t + 1) / n_parts);
+  pack_range(first, first + count / n_parts);
+  for (std::thread& t : pool) t.join();
+  return fits && double(coarse) <= kCoarseShare * double(boxes);
 }
 
 std::vector<DevNode2> to_device_layout(const BuildResult& b) {

@@ -34,8 +34,8 @@ struct BuildResult {
 // primitives becomes a leaf when its cost (one per primitive) is no more than the
 // split's, trav_cost + the children's area-weighted primitive counts.
 //   kTravCostTriangles: triangle trees, whose leaf triangles the traversal tests
-//   spread over a whole wave (1.5 measured 2% faster than 1 on the 1M soup: leaves
-//   fill up, 43 instead of 46 node visits per ray for 9 instead of 6 triangle tests);
+//   spread over a whole wave (1.5 measured 2% faster than 1 and than 2 on the 1M soup:
+//   leaves fill up, 43 instead of 46 node visits per ray for 9 instead of 6 triangle tests);
 //   kTravCostInstances: the top level over instances, where a leaf primitive costs a
 //   whole bottom-level traversal (1.5 there cost 8%).
 constexpr double kTravCostTriangles = 1.5;
@@ -132,7 +132,8 @@ struct alignas(16) DevNode32 {
 // fine for its extent (a small object in a large surrounding).
 constexpr double kCoarseGrowth = 1.25;
 constexpr double kCoarseShare = 1.0 / 16.0;
-bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, NodeSpace& space, DevNode32* out);
+bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, NodeSpace& space, DevNode32* out,
+                  int n_threads = 1);
 
 // Converts a build tree into the device layout (depth-first order, node 0 = root).
 // Returns the device nodes; a root leaf is wrapped in a node with an empty second child.

@@ -45,6 +45,16 @@ __device__ __forceinline__ uint32_t prefix_count(uint64_t mask) {
   return __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
 }
 
+// This lane's bit of a (wave-uniform) lane mask: predicates combined as masks stay in scalar
+// registers, where combined bools would become vector integers.
+__device__ __forceinline__ bool lane_bit(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+
+__device__ __forceinline__ uint32_t mask_count(uint64_t m) {
+  // two 32-bit counts: a 64-bit compare of the count would be a vector instruction
+  return static_cast<uint32_t>(__builtin_popcount(static_cast<uint32_t>(m))) +
+         static_cast<uint32_t>(__builtin_popcount(static_cast<uint32_t>(m >> 32)));
+}
+
 __device__ __forceinline__ void wave_add_stat(unsigned long long* dst, uint32_t v) {
   // sum over the wave, one atomic
   uint32_t s = v;
@@ -178,10 +188,32 @@ __device__ __forceinline__ void touch(uint32_t* bits, uint32_t i) {
 // axes are combined with max / min that ignore NaN. A node is visited by its byte offset
 // from the (wave-uniform) array base: one 32-bit add per visit.
 struct NodeHits {
-  bool h0, h1;     // child boxes the ray enters in [tmin, tmax]
-  float t0, t1;    // where
-  int32_t c0, c1;  // child references
+  float n0, f0, n1, f1;  // per child: entry and (widened) exit; the ray meets the box when n <= f
+  int32_t c0, c1;        // child references
 };
+
+// max / min as the instructions have them: NaN operands are ignored without first being
+// made quiet (two more instructions per visit; no value here is a signalling NaN's).
+__device__ __forceinline__ float max3_ft(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+__device__ __forceinline__ float min3_ft(float a, float b, float c) {
+  float r;
+  asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+__device__ __forceinline__ float max_ft(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ float min_ft(float a, float b) {
+  float r;
+  asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
 
 // 48-byte nodes: fp32 boxes. With x = c - o and s = sign(inv) (per ray, +-1), a slab's
 // entry and exit are (x - s h) inv and (x + s h) inv, each within a few ulp of itself plus
@@ -201,17 +233,13 @@ struct Nodes48 {
     b.sgn = v3(__builtin_copysignf(1.f, b.inv.x), __builtin_copysignf(1.f, b.inv.y), __builtin_copysignf(1.f, b.inv.z));
     return b;
   }
-  static __device__ __forceinline__ bool slab(float cx, float hx, float cy, float hy, float cz, float hz, const Ray& b,
-                                              float tmin, float tmax, float& tnear) {
+  static __device__ __forceinline__ void slab(float cx, float hx, float cy, float hy, float cz, float hz, const Ray& b,
+                                              float tmin, float tmax, float& n, float& f) {
     const float xx = cx - b.o.x, sx = hx * b.sgn.x;
     const float xy = cy - b.o.y, sy = hy * b.sgn.y;
     const float xz = cz - b.o.z, sz = hz * b.sgn.z;
-    const float n = __builtin_fmaxf(__builtin_fmaxf((xx - sx) * b.inv.x, (xy - sy) * b.inv.y),
-                                    __builtin_fmaxf((xz - sz) * b.inv.z, tmin));
-    const float f = __builtin_fminf(__builtin_fminf((xx + sx) * b.inv.x, (xy + sy) * b.inv.y),
-                                    __builtin_fminf((xz + sz) * b.inv.z, tmax));
-    tnear = n;
-    return n <= f * kBoxSlack;
+    n = max_ft(max3_ft((xx - sx) * b.inv.x, (xy - sy) * b.inv.y, (xz - sz) * b.inv.z), tmin);
+    f = min_ft(min3_ft((xx + sx) * b.inv.x, (xy + sy) * b.inv.y, (xz + sz) * b.inv.z), tmax) * kBoxSlack;
   }
   // Child reference from the low bytes of one node row (v_perm_b32 gathers two bytes per
   // instruction).
@@ -225,8 +253,8 @@ struct Nodes48 {
     const float4* p = reinterpret_cast<const float4*>(static_cast<const char*>(nodes) + static_cast<uint32_t>(at));
     const float4 r0 = p[0], r1 = p[1], r2 = p[2];
     NodeHits v;
-    v.h0 = slab(r0.x, r0.y, r0.z, r0.w, r2.x, r2.y, b, tmin, tmax, v.t0);
-    v.h1 = slab(r1.x, r1.y, r1.z, r1.w, r2.z, r2.w, b, tmin, tmax, v.t1);
+    slab(r0.x, r0.y, r0.z, r0.w, r2.x, r2.y, b, tmin, tmax, v.n0, v.f0);
+    slab(r1.x, r1.y, r1.z, r1.w, r2.z, r2.w, b, tmin, tmax, v.n1, v.f1);
     v.c0 = child_ref(r0);
     v.c1 = child_ref(r1);
     return v;
@@ -241,7 +269,8 @@ struct Nodes48 {
 // The terms that cancel in ct have an error of up to 2u (|x| + R) |inv| (x the distance to
 // the box's centre, R the tree's half size): the part in |x| is relative to the distances,
 // and the half extents' margins (bvh_build.h) exceed the part in R. A direction component
-// below 2^-60 of the largest takes that magnitude, which moves no ray by more than the
+// below 2^-60 of the largest takes that magnitude (v_rcp_f32's ulp scales all of the
+// axis's distances alike), which moves no ray by more than the
 // margins; rays so extreme that a term could overflow take every box (NaN, which the axes'
 // max / min ignore): slow and still exact.
 struct Nodes32 {
@@ -256,9 +285,9 @@ struct Nodes32 {
     b.o = o;
     const float m = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(d.x), __builtin_fabsf(d.y)), __builtin_fabsf(d.z));
     const float lim = m * 0x1p-60f;
-    const float ix = 1.f / (__builtin_fabsf(d.x) < lim ? __builtin_copysignf(lim, d.x) : d.x);
-    const float iy = 1.f / (__builtin_fabsf(d.y) < lim ? __builtin_copysignf(lim, d.y) : d.y);
-    const float iz = 1.f / (__builtin_fabsf(d.z) < lim ? __builtin_copysignf(lim, d.z) : d.z);
+    const float ix = __builtin_amdgcn_rcpf(__builtin_fabsf(d.x) < lim ? __builtin_copysignf(lim, d.x) : d.x);
+    const float iy = __builtin_amdgcn_rcpf(__builtin_fabsf(d.y) < lim ? __builtin_copysignf(lim, d.y) : d.y);
+    const float iz = __builtin_amdgcn_rcpf(__builtin_fabsf(d.z) < lim ? __builtin_copysignf(lim, d.z) : d.z);
     const V3 w = v3(g.org[0] - o.x, g.org[1] - o.y, g.org[2] - o.z);
     b.si = v3(ix * g.scale, iy * g.scale, iz * g.scale);
     b.oi = v3(w.x * ix, w.y * iy, w.z * iz);
@@ -274,29 +303,28 @@ struct Nodes32 {
     return b;
   }
   // v: fp16 (c, h) pairs of the axes, then the child reference
-  static __device__ __forceinline__ bool slab(uint4 v, const Ray& b, float tmin, float tmax, float& tnear) {
+  static __device__ __forceinline__ void slab(uint4 v, const Ray& b, float tmin, float tmax, float& n, float& f) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
     const h2 x = __builtin_bit_cast(h2, v.x), y = __builtin_bit_cast(h2, v.y), z = __builtin_bit_cast(h2, v.z);
     const float cx = __builtin_fmaf(static_cast<float>(x[0]), b.si.x, b.oi.x);
     const float cy = __builtin_fmaf(static_cast<float>(y[0]), b.si.y, b.oi.y);
     const float cz = __builtin_fmaf(static_cast<float>(z[0]), b.si.z, b.oi.z);
     const float ax = __builtin_fabsf(b.si.x), ay = __builtin_fabsf(b.si.y), az = __builtin_fabsf(b.si.z);
-    const float n = __builtin_fmaxf(
-        __builtin_fmaxf(__builtin_fmaf(-static_cast<float>(x[1]), ax, cx), __builtin_fmaf(-static_cast<float>(y[1]), ay, cy)),
-        __builtin_fmaxf(__builtin_fmaf(-static_cast<float>(z[1]), az, cz), tmin));
-    const float f = __builtin_fminf(
-        __builtin_fminf(__builtin_fmaf(static_cast<float>(x[1]), ax, cx), __builtin_fmaf(static_cast<float>(y[1]), ay, cy)),
-        __builtin_fminf(__builtin_fmaf(static_cast<float>(z[1]), az, cz), tmax));
-    tnear = n;
-    return n <= f * kBoxSlack;
+    n = max_ft(max3_ft(__builtin_fmaf(-static_cast<float>(x[1]), ax, cx), __builtin_fmaf(-static_cast<float>(y[1]), ay, cy),
+                       __builtin_fmaf(-static_cast<float>(z[1]), az, cz)),
+               tmin);
+    f = min_ft(min3_ft(__builtin_fmaf(static_cast<float>(x[1]), ax, cx), __builtin_fmaf(static_cast<float>(y[1]), ay, cy),
+                       __builtin_fmaf(static_cast<float>(z[1]), az, cz)),
+               tmax) *
+        kBoxSlack;
   }
   static __device__ __forceinline__ NodeHits visit(const void* __restrict__ nodes, int32_t at, const Ray& b, float tmin,
                                                    float tmax) {
     const uint4* p = reinterpret_cast<const uint4*>(static_cast<const char*>(nodes) + static_cast<uint32_t>(at));
     const uint4 r0 = p[0], r1 = p[1];
     NodeHits v;
-    v.h0 = slab(r0, b, tmin, tmax, v.t0);
-    v.h1 = slab(r1, b, tmin, tmax, v.t1);
+    slab(r0, b, tmin, tmax, v.n0, v.f0);
+    slab(r1, b, tmin, tmax, v.n1, v.f1);
     v.c0 = static_cast<int32_t>(r0.w);
     v.c1 = static_cast<int32_t>(r1.w);
     return v;
@@ -310,28 +338,8 @@ constexpr int32_t kTravDone = static_cast<int32_t>(0x80000000u);
 // have no leaf parked, instead of none: the last few searching lanes would otherwise
 // hold the wave for a long tail of iterations in which most lanes idle. They keep their
 // state and go on walking in the next round. 16 measured best on the 1M-triangle soup
-// (8 -1.5%, 32 -6%; instanced: 8 -2%).
+// (Extend of a frame 7.97 ms; at 8 8.11, at 24 8.40) and as good as 8 on the instances.
 constexpr uint32_t kSearchBreakSpread = 16;
-
-// End of a queue traversal's node loop, evaluated by all lanes after each iteration as a
-// wave-uniform branch (two compares and scalar work): no lane has an inner node left
-// (walks), or at most kSearchBreakSpread of the lanes that walked in this iteration
-// (walked) hold no parked leaf.
-__device__ __forceinline__ bool walk_done(bool walked, bool walks, int32_t leaf) {
-  const uint64_t searching = __ballot(walked) & __ballot(leaf == 0);
-  // two 32-bit counts: a 64-bit compare of the count would be a vector instruction
-  const uint32_t n = static_cast<uint32_t>(__builtin_popcount(static_cast<uint32_t>(searching))) +
-                     static_cast<uint32_t>(__builtin_popcount(static_cast<uint32_t>(searching >> 32)));
-  return __ballot(walks) == 0 || n <= kSearchBreakSpread;
-}
-
-// Lanes of the wave (among the active ones) that hold no parked leaf.
-__device__ __forceinline__ uint32_t searching_lanes(int32_t leaf) {
-  const uint64_t m = __ballot(leaf == 0);
-  // two 32-bit counts: a 64-bit compare of the count would be a vector instruction
-  return static_cast<uint32_t>(__builtin_popcount(static_cast<uint32_t>(m))) +
-         static_cast<uint32_t>(__builtin_popcount(static_cast<uint32_t>(m >> 32)));
-}
 
 // Persistent single-level BVH2 traversal of a segmented ray queue, in rounds of the
 // "speculative while-while" form of Aila & Laine (2009, "Understanding the efficiency of
@@ -339,20 +347,28 @@ __device__ __forceinline__ uint32_t searching_lanes(int32_t leaf) {
 // holds a leaf (a lane that meets its first leaf parks it and keeps walking), then the
 // wave intersects leaves together. Before each round lanes whose ray has finished take new
 // rays from the queue ("dynamic fetch", same paper) once at least kRefill of them are
-// idle, so a few long rays do not hold the whole wave (40 of 64 measured best on MI355X
-// with the early end of the node loop and the spread leaf phase, 24 and 48 about 1-3%
-// slower). The result does not depend on the visiting order (closest hit under the
+// idle, so a few long rays do not hold the whole wave (40 of 64: a frame's Extend 7.97 ms
+// on the soup, at 32 8.04, at 24 8.12; a refill's queue atomic, loads and divisions cost
+// more lanes than they fill. Claiming 64 rays at a time and keeping them set up in
+// registers made refills cheap but scatters a CU's rays over more of the queue: 9.0 ms at
+// 24). The result does not depend on the visiting order (closest hit under the
 // (t, inst, prim) order, or any hit).
 // load(slot, o, d, tmin, tmax) reads a ray;
 // finish(slot, r, hit) consumes a result (hit: a hit was found).
 constexpr uint32_t kRefill = 40;
 
-// Traversal stack of the queue traversals: the top kRingEntries entries live in an
-// LDS ring (entry k in slot k % kRingEntries, lane-interleaved), older ones are moved
-// to the lane's area of a global spill buffer when the ring is full and brought back,
-// a ring at a time, when it runs empty. Deep traversals are rare, so the ring keeps
-// LDS small (4 KiB per wave, beside the 1.6 KiB leaf-task area) and occupancy bound by
-// registers, not by the tree depth.
+// Traversal stack of the queue traversals: the top entries live in an LDS ring of
+// kRingEntries slots (entry k in slot k % kRingEntries, lane-interleaved), older ones are
+// moved to the lane's area of a global spill buffer when the ring fills up and brought
+// back when it runs empty. Deep traversals are rare, so the ring keeps LDS small (4 KiB
+// per wave, beside the 1.6 KiB leaf-task area) and occupancy bound by registers, not by
+// the tree depth.
+//
+// Pushes and pops are free of branches: the two lowest entries are sentinels (popping one
+// ends the traversal, the second keeps the stack from looking empty then), every step
+// reads the top entry ahead and stores its far child above the top whether or not it is
+// pushed (one ring slot stays free for that), and stack_step moves the top. Only a ring
+// about to overflow or running empty takes a branch (stack_move).
 constexpr int kRingEntries = 16;
 
 // LDS word at a byte address (ds_read / ds_write with a 32-bit address formed by integer
@@ -374,21 +390,21 @@ __device__ __forceinline__ void lds_store(uint32_t a, uint32_t v) {
 // checked at start-up by traversal_lds_check), so the slot bits never meet the lane's base.
 constexpr uint32_t kSlotBytes = 64 * 4;
 constexpr uint32_t kRingMask = (kRingEntries - 1) * kSlotBytes;
+constexpr uint32_t kSentinels = 2;
+constexpr uint32_t kSpillStep = 4;  // entries moved at a time
 
 struct TwoTierStack {
   uint32_t ring;         // LDS byte address of the lane's first ring slot
   uint32_t* spill_wave;  // the wave's spill area; lane l's `cap` entries start at l * cap
-  uint32_t cap;          // capacity (entries)
-  uint32_t sp;           // entries on the stack, x kSlotBytes
-  uint32_t lo;           // entries [0, lo) are in the spill area, [lo, sp) in the ring (x kSlotBytes)
-  uint32_t lim;          // min(lo + kRingEntries, cap) x kSlotBytes: a push at sp == lim either moves
-                         // the ring's oldest entry out or, at the capacity, replaces the top entry
+  uint32_t cap;          // capacity of the spill area (entries)
+  uint32_t sp;           // entries on the stack, sentinels included, x kSlotBytes
+  uint32_t lo1;          // (lo + 1) x kSlotBytes: entries [0, lo) are in the spill area, the rest in the ring
 };
 
 __device__ __forceinline__ void stack_reset(TwoTierStack& s) {
-  s.sp = 0;
-  s.lo = 0;
-  s.lim = min(static_cast<uint32_t>(kRingEntries), s.cap) * kSlotBytes;
+  for (uint32_t k = 0; k < kSentinels; ++k) lds_store(s.ring | (k * kSlotBytes), static_cast<uint32_t>(kTravDone));
+  s.sp = kSentinels * kSlotBytes;
+  s.lo1 = kSlotBytes;
 }
 
 // The wave's spill area of the traversal grid (stack_cap entries per thread), taken
@@ -401,67 +417,96 @@ __device__ __forceinline__ uint32_t* wave_spill(uint32_t* spill, int cap) {
 
 __device__ __forceinline__ uint32_t* lane_spill(const TwoTierStack& s) { return s.spill_wave + lane_id() * s.cap; }
 
-// Pushes v. At the capacity (a tree deeper than the stack was sized for) v replaces the
-// top entry, which keeps every access in bounds, and on_full() reports the inexact
-// traversal.
+// Top entry (the stack always holds one) and the store of the entry above it.
+__device__ __forceinline__ int32_t stack_top(const TwoTierStack& s) {
+  return static_cast<int32_t>(lds_load(s.ring | ((s.sp - kSlotBytes) & kRingMask)));
+}
+__device__ __forceinline__ void stack_above(const TwoTierStack& s, int32_t v) {
+  lds_store(s.ring | (s.sp & kRingMask), static_cast<uint32_t>(v));
+}
+
+// Brings the ring back between its limits after sp moved: 1 to kRingEntries - 1 entries
+// (one slot stays free for stack_above). At the capacity (a tree deeper than the stack was
+// sized for) the top entry is dropped, which keeps every access in bounds, and on_full()
+// reports the inexact traversal.
 template <bool STATS, class OnFull>
-__device__ __forceinline__ void stack_push(TwoTierStack& s, uint32_t v, TraceOut& stats, OnFull on_full) {
-  if (s.sp == s.lim) {
-    if (s.sp == s.cap * kSlotBytes) {
-      on_full();
-      s.sp -= kSlotBytes;
-    } else {  // ring full: move its oldest entry out
-      lane_spill(s)[s.lo / kSlotBytes] = lds_load(s.ring | (s.lo & kRingMask));
-      s.lo += kSlotBytes;
-      s.lim = min(s.lo + kRingEntries * kSlotBytes, s.cap * kSlotBytes);
-      if (STATS) stats.spills++;
-    }
-  }
-  lds_store(s.ring | (s.sp & kRingMask), v);
-  s.sp += kSlotBytes;
-}
-
-__device__ __forceinline__ int32_t stack_pop(TwoTierStack& s) {
-  if (s.sp == s.lo) {
-    if (s.sp == 0) return kTravDone;
-    // ring empty: bring back up to a ring of spilled entries
-    const uint32_t lo = s.lo / kSlotBytes;
-    const uint32_t n = lo < kRingEntries ? lo : kRingEntries;
-    const uint32_t* sp = lane_spill(s);
+__device__ __forceinline__ void stack_move(TwoTierStack& s, TraceOut& stats, OnFull on_full) {
+  uint32_t* sp = lane_spill(s);
+  const uint32_t lo = s.lo1 / kSlotBytes - 1u;
+  if (s.sp < s.lo1) {  // ring empty: bring spilled entries back (lo > 0: the sentinels are below)
+    const uint32_t n = lo < kSpillStep ? lo : kSpillStep;
     for (uint32_t k = lo - n; k < lo; ++k) lds_store(s.ring | ((k * kSlotBytes) & kRingMask), sp[k]);
-    s.lo -= n * kSlotBytes;
-    s.lim = min(s.lo + kRingEntries * kSlotBytes, s.cap * kSlotBytes);
+    s.lo1 -= n * kSlotBytes;
+  } else if (lo + kSpillStep > s.cap) {
+    on_full();
+    s.sp -= kSlotBytes;
+  } else {  // ring full: move its oldest entries out
+    for (uint32_t k = lo; k < lo + kSpillStep; ++k) sp[k] = lds_load(s.ring | ((k * kSlotBytes) & kRingMask));
+    s.lo1 += kSpillStep * kSlotBytes;
+    if (STATS) stats.spills += kSpillStep;
   }
-  s.sp -= kSlotBytes;
-  return static_cast<int32_t>(lds_load(s.ring | (s.sp & kRingMask)));
 }
 
-// Leaf phase of the single-level loop, spread over the whole wave: every (ray, triangle)
+// One entry pushed (already stored by stack_above) or popped (already read by stack_top),
+// by the lanes of the masks.
+template <bool STATS, class OnFull>
+__device__ __forceinline__ void stack_step(TwoTierStack& s, uint64_t push, uint64_t pop, TraceOut& stats,
+                                           OnFull on_full) {
+  uint32_t by = lane_bit(push) ? kSlotBytes : 0u;
+  by = lane_bit(pop) ? 0u - kSlotBytes : by;
+  s.sp += by;
+  if (s.sp - s.lo1 > (kRingEntries - 3) * kSlotBytes)  // not 1 .. kRingEntries - 2 entries in the ring
+    stack_move<STATS>(s, stats, on_full);
+}
+
+// A ray's set-up of the watertight test (ray_tri_setup): axes packed 2 bits each, shear.
+struct RayShear {
+  int32_t kxyz;
+  V3 s;
+};
+__device__ __forceinline__ RayShear ray_shear(V3 d) {
+  const RayTri t = ray_tri_setup(v3(0.f), d);
+  return RayShear{t.kx | (t.ky << 2) | (t.kz << 4), v3(t.sx, t.sy, t.sz)};
+}
+
+// Leaf phase of the traversal loops, spread over the whole wave: every (ray, triangle)
 // pair of the leaves the lanes hold is a task, and the wave deals the tasks out 64 at a
 // time, each lane testing one with the owning lane's ray (read across lanes), instead of
 // each lane looping over its own leaves while most lanes wait (a round's leaves hold
-// ~120 triangles, which the per-lane loop tested at ~16 active lanes per iteration).
+// ~64 triangles, which a per-lane loop tests at ~16 active lanes per iteration).
+// A task finds its owner without a list: lanes that own tasks mark the place of their
+// first one, and a running maximum over the marks gives each place its owner (writing the
+// tasks out, up to 14 per lane, took a quarter of the phase's instructions).
 // An owner's closest hit is the minimum of a (t, prim) key over its tasks (LDS atomic
 // min; the lexicographic order of the closest-hit search), and the task that holds the
-// minimum writes the barycentrics. Per wave, in LDS: one window of kTaskWin task
-// triangles and owners per round, and a key and barycentrics per lane.
+// minimum writes the barycentrics. Per wave, in LDS: 64 marks, and a key and barycentrics
+// per lane. One window of kTaskWin tasks per round.
 constexpr uint32_t kTaskWin = 128;
-constexpr uint32_t kTaskWords = kTaskWin + kTaskWin / 4 + 64 * 2 + 64 * 2;
+constexpr uint32_t kTaskWords = 64 + 64 * 2 + 64 * 2;
 
 struct LeafTasks {
-  uint32_t* tri;            // [kTaskWin] triangle index
-  uint8_t* own;             // [kTaskWin] owning lane
+  uint32_t* mark;           // [64] 1 + owning lane at an owner's first task, else 0
   unsigned long long* key;  // [64] hit key per lane
   float2* bary;             // [64] barycentrics of the key's hit
 };
 
 __device__ __forceinline__ LeafTasks leaf_tasks(uint32_t* base) {
   LeafTasks t;
-  t.tri = base;
-  t.own = reinterpret_cast<uint8_t*>(base + kTaskWin);
-  t.key = reinterpret_cast<unsigned long long*>(base + kTaskWin + kTaskWin / 4);
-  t.bary = reinterpret_cast<float2*>(base + kTaskWin + kTaskWin / 4 + 128);
+  t.mark = base;
+  t.key = reinterpret_cast<unsigned long long*>(base + 64);
+  t.bary = reinterpret_cast<float2*>(base + 64 + 128);
   return t;
+}
+
+// Running maximum over the wave's lanes (all active), lane 0 first.
+__device__ __forceinline__ uint32_t wave_scan_max(uint32_t v) {
+  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x111, 0xf, 0xf, false)));  // row_shr 1
+  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x112, 0xf, 0xf, false)));  // row_shr 2
+  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x114, 0xf, 0xf, false)));  // row_shr 4
+  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x118, 0xf, 0xf, false)));  // row_shr 8
+  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x142, 0xa, 0xf, false)));  // row_bcast 15
+  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x143, 0xc, 0xf, false)));  // row_bcast 31
+  return v;
 }
 
 // Order-preserving (t, prim) key: t's bits mapped so that unsigned order is float
@@ -479,16 +524,15 @@ __device__ __forceinline__ float key_t(unsigned long long k) {
 }
 
 // One leaf phase: lane l contributes the tasks of ca triangles from fa and cb from fb,
-// tested with its ray (object-space origin o, ray_tri_setup's packed axes and shear,
-// tmin, tmax). A task hit counts if it beats the lane's best (t = tmax, prim0, and for
+// tested with its ray (object-space origin o, axes and shear of ray_shear, tmin, tmax). A task hit counts if it beats the lane's best (t = tmax, prim0, and for
 // TWO, instance inst0, with the lane's current instance cur). Returns whether the
 // lane's tasks were in this round's window (false: it keeps its leaves for the next
 // round); `better`: a task hit counted, the smallest (t, prim) key of those is kf, and
 // its barycentrics are in tk.bary[lane].
 template <bool STATS, bool TWO>
 __device__ __forceinline__ bool leaf_phase(const LeafTasks& tk, const float4* __restrict__ tris, uint32_t lane,
-                                           uint32_t fa, uint32_t ca, uint32_t fb, uint32_t cb, V3 o, int32_t kxyz,
-                                           V3 shear, float tmin, float tmax, uint32_t prim0, uint32_t inst0,
+                                           uint32_t fa, uint32_t ca, uint32_t fb, uint32_t cb, V3 o, const RayShear& rs,
+                                           float tmin, float tmax, uint32_t prim0, uint32_t inst0,
                                            uint32_t cur, bool& better, unsigned long long& kf, TraceOut& stats,
                                            uint32_t* touch_tris) {
   const uint32_t n_tasks = ca + cb;  // at most 14
@@ -509,26 +553,30 @@ __device__ __forceinline__ bool leaf_phase(const LeafTasks& tk, const float4* __
   // TWO: every hit up to tmax is a candidate, the owner's order is checked per hit
   const unsigned long long key0 = hit_key(tmax, TWO ? kNoHit : prim0);
   tk.key[lane] = key0;
-  if (fits) {
-    for (uint32_t k = 0; k < n_tasks; ++k) {
-      tk.tri[off + k] = k < ca ? fa + k : fb + (k - ca);
-      tk.own[off + k] = static_cast<uint8_t>(lane);
-    }
-  }
+  // triangle of place j: j + ta below ea, j + tb from there on
+  const uint32_t ea = off + ca, ta = fa - off, tb = fb - ea;
+  const bool owns = fits && n_tasks != 0;
+  uint32_t last = 0;  // owner mark of the last place dealt out
   for (uint32_t s0 = 0; s0 < m; s0 += 64) {
+    tk.mark[lane] = lane == 0 ? last : 0u;
+    if (owns && off - s0 < 64u) tk.mark[off - s0] = lane + 1u;
+    asm volatile("" ::: "memory");  // another lane may have marked this place
+    const uint32_t mark = wave_scan_max(tk.mark[lane]);
+    last = __builtin_amdgcn_readlane(mark, 63);
+    const int own = static_cast<int>(mark) - 1;
     const uint32_t j = s0 + lane;
     const bool act = j < m;
-    const uint32_t ti = act ? tk.tri[j] : 0u;
-    const int own = act ? static_cast<int>(tk.own[j]) : static_cast<int>(lane);
+    const uint32_t oea = __shfl(ea, own), ota = __shfl(ta, own), otb = __shfl(tb, own);
+    const uint32_t ti = j + (j < oea ? ota : otb);
     RayTri ort;
     ort.o = v3(__shfl(o.x, own), __shfl(o.y, own), __shfl(o.z, own));
-    const int kk = __shfl(kxyz, own);
+    const int kk = __shfl(rs.kxyz, own);
     ort.kx = kk & 3;
     ort.ky = (kk >> 2) & 3;
     ort.kz = kk >> 4;
-    ort.sx = __shfl(shear.x, own);
-    ort.sy = __shfl(shear.y, own);
-    ort.sz = __shfl(shear.z, own);
+    ort.sx = __shfl(rs.s.x, own);
+    ort.sy = __shfl(rs.s.y, own);
+    ort.sz = __shfl(rs.s.z, own);
     const float otmin = __shfl(tmin, own), otmax = __shfl(tmax, own);
     uint32_t oprim = 0, oinst = 0, ocur = 0;
     if (TWO) {
@@ -560,8 +608,6 @@ __device__ __forceinline__ bool leaf_phase(const LeafTasks& tk, const float4* __
   return fits;
 }
 
-__device__ __forceinline__ int32_t pack_axes(const RayTri& t) { return t.kx | (t.ky << 2) | (t.kz << 4); }
-
 template <class Nodes, bool ANY, bool STATS, class Load, class Finish>
 __device__ __forceinline__ void trace_queue(const DevAccel& acc, const SegIn& in, uint32_t* stk, uint32_t* tsk,
                                             uint32_t* overflow, TraceOut& stats, Load load, Finish finish) {
@@ -573,11 +619,9 @@ __device__ __forceinline__ void trace_queue(const DevAccel& acc, const SegIn& in
   uint64_t seg_done = seg_empty(n_seg, home, gridDim.x >= kSegs);
   bool drained = false;
   uint32_t slot = kNoHit;
-  V3 o = v3(0.f), d = v3(0.f);
   typename Nodes::Ray rb{};
   float tmin = 0.f;
-  int32_t kxyz = 0;        // ray_tri_setup's axis permutation, 2 bits per axis
-  V3 shear = v3(0.f);      // and its shear constants
+  RayShear rs{};
   TraceOut r;
   r.t = 0.f;
   r.b1 = r.b2 = 0.f;
@@ -589,22 +633,21 @@ __device__ __forceinline__ void trace_queue(const DevAccel& acc, const SegIn& in
   st.cap = static_cast<uint32_t>(cap);
   stack_reset(st);
   int32_t node = kTravDone, leaf = 0;
-  auto pop = [&]() -> int32_t { return stack_pop(st); };
+  const auto on_full = [&] { atomicOr(overflow, 1u); };
   const LeafTasks tk = leaf_tasks(tsk);
   for (;;) {
     const uint64_t idle = __ballot(slot == kNoHit);
-    const uint32_t n_idle = static_cast<uint32_t>(__popcll(idle));
+    const uint32_t n_idle = mask_count(idle);
     if (!drained && n_idle >= kRefill) {
       uint32_t base = 0, got = 0;
       if (seg_fetch_k(in, n_seg, home, seg_done, n_idle, base, got)) {
         const uint32_t rank = prefix_count(idle);
         if (slot == kNoHit && rank < got) {
           slot = base + rank;
+          V3 o, d;
           float tmax;
           load(slot, o, d, tmin, tmax);
-          const RayTri rt = ray_tri_setup(o, d);
-          kxyz = pack_axes(rt);
-          shear = v3(rt.sx, rt.sy, rt.sz);
+          rs = ray_shear(d);
           rb = Nodes::setup(acc.space, o, d);
           r.t = tmax;
           r.prim = kNoHit;
@@ -618,34 +661,37 @@ __device__ __forceinline__ void trace_queue(const DevAccel& acc, const SegIn& in
       }
     }
     if (!__any(slot != kNoHit)) break;  // drained and every lane idle
-    // inner nodes: a wave-uniform loop in which lanes without an inner node idle
-    for (bool walks = node >= 0;;) {
-      if (walks) {
-        const NodeHits v = Nodes::visit(nodes, node, rb, tmin, r.t);
-        if (STATS) {
+    // Inner nodes: a wave-uniform loop in which lanes without an inner node idle, and one
+    // straight line of predicated steps instead of a branch per outcome (both children,
+    // one, none, a leaf to park), each of which some lane takes on almost every iteration:
+    // the loop is bound by the instructions it issues. A popped leaf is parked by the next
+    // iteration (whose box test that lane wastes on the root) rather than by a second pop.
+    for (uint64_t walk = __ballot(node >= 0);;) {
+      if (lane_bit(walk)) {
+        const uint64_t inner = __ballot(node >= 0);  // the others hold a popped leaf
+        const int32_t top = stack_top(st);
+        const NodeHits v = Nodes::visit(nodes, max(node, 0), rb, tmin, r.t);
+        if (STATS && node >= 0) {
           stats.nodes++;
           touch(acc.touch_nodes, static_cast<uint32_t>(node) / Nodes::kBytes);
         }
-        if (v.h0 && v.h1) {
-          const bool swap = v.t1 < v.t0;
-          const int32_t farc = swap ? v.c0 : v.c1;
-          stack_push<STATS>(st, static_cast<uint32_t>(farc), stats, [&] { atomicOr(overflow, 1u); });
-          node = swap ? v.c1 : v.c0;
-        } else if (v.h0) {
-          node = v.c0;
-        } else if (v.h1) {
-          node = v.c1;
-        } else {
-          node = pop();
-        }
-        if (node < 0 && node != kTravDone && leaf == 0) {
-          leaf = node;
-          node = pop();
-        }
+        const uint64_t h0 = __ballot(v.n0 <= v.f0) | ~inner, h1 = __ballot(v.n1 <= v.f1) & inner;
+        const int32_t c0 = lane_bit(inner) ? v.c0 : node;
+        const uint64_t both = h0 & h1, first1 = (both & __ballot(v.n1 < v.n0)) | ~h0;
+        const int32_t nearc = lane_bit(first1) ? v.c1 : c0, farc = lane_bit(first1) ? c0 : v.c1;
+        const uint64_t park = (h0 | h1) & __ballot(nearc < 0) & __ballot(leaf == 0);
+        stack_above(st, farc);
+        leaf = lane_bit(park) ? nearc : leaf;
+        const uint64_t pop = ~(h0 | h1) | (park & ~both);
+        node = lane_bit(park) ? farc : nearc;
+        node = lane_bit(pop) ? top : node;
+        stack_step<STATS>(st, both & ~park, pop, stats, on_full);
       }
-      const bool walked = walks;
-      walks = node >= 0;
-      if (walk_done(walked, walks, leaf)) break;
+      // the loop ends (for the whole wave) once no lane walks, or at most
+      // kSearchBreakSpread of those that walked hold no parked leaf
+      const uint64_t no_leaf = __ballot(leaf == 0), searching = walk & no_leaf;
+      walk = __ballot(node >= 0) | (no_leaf & __ballot(node != kTravDone));
+      if (walk == 0 || mask_count(searching) <= kSearchBreakSpread) break;
     }
     // leaves (the parked one, and `node` when it is a leaf), spread over the wave
     bool hit = false;
@@ -655,7 +701,7 @@ __device__ __forceinline__ void trace_queue(const DevAccel& acc, const SegIn& in
     bool better;
     unsigned long long kf;
     if (leaf_phase<STATS, false>(tk, tris, lane, ~static_cast<uint32_t>(leaf) >> 3, ca, ~static_cast<uint32_t>(node) >> 3,
-                                 cb, rb.o, kxyz, shear, tmin, r.t, r.prim, kNoInstance, kNoInstance, better, kf,
+                                 cb, rb.o, rs, tmin, r.t, r.prim, kNoInstance, kNoInstance, better, kf,
                                  stats, acc.touch_tris) &&
         (leaf != 0 || node_leaf)) {  // not ca + cb != 0: an empty child's leaf holds no triangle
       if (better) {  // the barycentrics stay in tk.bary[lane] until the ray finishes
@@ -664,7 +710,10 @@ __device__ __forceinline__ void trace_queue(const DevAccel& acc, const SegIn& in
         hit = ANY;
       }
       leaf = 0;
-      if (node_leaf) node = pop();
+      if (node_leaf) {
+        node = stack_top(st);
+        stack_step<STATS>(st, 0ull, ~0ull, stats, on_full);
+      }
     }
     if (slot != kNoHit && (hit || (node == kTravDone && leaf == 0))) {
       r.b1 = r.b2 = 0.f;
@@ -681,16 +730,16 @@ __device__ __forceinline__ void trace_queue(const DevAccel& acc, const SegIn& in
   }
 }
 
-// Two-level counterpart of trace_queue (instanced scenes): the same speculative
-// while-while loop with lane refill, two-tier stack and wave-wide leaf phase, walking the
-// top-level tree over instance boxes and, inside an instance, its mesh's tree with the
-// ray in object space (leaf tasks use the owner's object-space ray).
-// Entering an instance pushes what is left of the top-level leaf and an exit marker;
-// popping the marker returns the ray to world space. A lane with a parked (not yet
-// intersected) leaf never leaves its instance: it waits at the marker until the leaf
-// is done, since the leaf's triangles are tested in that instance's space.
-constexpr int32_t kTravExit = 0x7fffffff;                               // leave the instance (stack marker)
-constexpr int32_t kTravBlocked = static_cast<int32_t>(0x80000001u);     // waits at the marker with a parked leaf
+// Two-level counterpart of trace_queue (instanced scenes): the same loop with lane refill,
+// two-tier stack and wave-wide leaf phase, walking the top-level tree over instance boxes
+// and, inside an instance, its mesh's tree with the ray in object space (leaf tasks use the
+// owner's object-space ray). A third phase of each round changes spaces: a lane that meets a
+// top-level leaf, or the marker pushed on entering an instance, waits for the round's end,
+// and all of those then leave and enter instances together (a transform and a ray set-up of
+// some 150 instructions, which inside the node loop ran for a lane or two at almost every
+// iteration). A lane with a parked leaf never leaves its instance: the leaf is tested in
+// that instance's space, before this phase.
+constexpr int32_t kTravExit = static_cast<int32_t>(0x80000001u);  // leave the instance (stack marker); below every leaf code
 
 template <class Nodes, bool ANY, bool STATS, class Load, class Finish>
 __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& in, uint32_t* stk, uint32_t* tsk,
@@ -706,8 +755,7 @@ __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& i
   uint32_t slot = kNoHit;
   V3 ow = v3(0.f), dw = v3(0.f);
   typename Nodes::Ray rb{};  // in the current space (world outside instances)
-  int32_t kxyz = 0;    // ray_tri_setup's axis permutation in the current instance, 2 bits per axis
-  V3 shear = v3(0.f);  // and its shear constants
+  RayShear rs{};  // in the current instance
   float tmin = 0.f;
   TraceOut r;
   r.t = 0.f;
@@ -722,56 +770,11 @@ __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& i
   st.cap = static_cast<uint32_t>(cap);
   stack_reset(st);
   int32_t node = kTravDone, leaf = 0;
-  bool ok = true;  // false after a stack overflow (reported once per lane)
-  auto push = [&](uint32_t v) {
-    stack_push<STATS>(st, v, stats, [&] {
-      if (ok) {
-        ok = false;
-        atomicOr(overflow, 1u);
-      }
-    });
-  };
-  // Pops the next node; leaves the instance at its marker unless a leaf is parked.
-  auto pop = [&]() -> int32_t {
-    for (;;) {
-      const int32_t e = stack_pop(st);
-      if (e != kTravExit) return e;
-      if (leaf != 0) {
-        stack_push<STATS>(st, static_cast<uint32_t>(kTravExit), stats, [] {});  // just popped: never full
-        return kTravBlocked;
-      }
-      in_blas = false;
-      rb = Nodes::setup(acc.space, ow, dw);  // back in world space (recomputed: fewer live registers)
-    }
-  };
-  // Top-level leaf (instances [first, first + count)): enter the first instance.
-  auto enter = [&](int32_t code) -> int32_t {
-    const uint32_t c = ~static_cast<uint32_t>(code);
-    const uint32_t first = c >> 3, cnt = c & 7u;
-    if (cnt > 1u) push(~(((first + 1u) << 3) | (cnt - 1u)));  // the rest of the leaf
-    push(static_cast<uint32_t>(kTravExit));
-    const TlasInstance& ins = acc.inst[first];
-    const V3 o = xform_point(ins.w2o, ow);
-    const V3 d = xform_vector(ins.w2o, dw);
-    rb = Nodes::setup(ins.space, o, d);
-    const RayTri rt = ray_tri_setup(o, d);
-    kxyz = pack_axes(rt);
-    shear = v3(rt.sx, rt.sy, rt.sz);
-    cur_id = ins.id;
-    in_blas = true;
-    if (STATS) stats.nodes++;
-    return static_cast<int32_t>(ins.blas_root);
-  };
-  // Resolves top-level leaves (entering instances) until node is an inner node, a
-  // mesh leaf, kTravBlocked or kTravDone.
-  auto settle = [&](int32_t n) -> int32_t {
-    while (!in_blas && n < 0 && n != kTravDone && n != kTravBlocked) n = enter(n);
-    return n;
-  };
+  const auto on_full = [&] { atomicOr(overflow, 1u); };
   const LeafTasks tk = leaf_tasks(tsk);
   for (;;) {
     const uint64_t idle = __ballot(slot == kNoHit);
-    const uint32_t n_idle = static_cast<uint32_t>(__popcll(idle));
+    const uint32_t n_idle = mask_count(idle);
     if (!drained && n_idle >= kRefill) {
       uint32_t base = 0, got = 0;
       if (seg_fetch_k(in, n_seg, home, seg_done, n_idle, base, got)) {
@@ -794,46 +797,44 @@ __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& i
       }
     }
     if (!__any(slot != kNoHit)) break;
-    if (slot != kNoHit) {
-      // inner nodes of either level (a while loop: the uniform form of the single-level
-      // loop costs this kernel register spills)
-      while (node >= 0) {
-        const NodeHits v = Nodes::visit(in_blas ? blas : tlas, node, rb, tmin, r.t);
-        if (STATS) {
+    // inner nodes of either level, as in trace_queue; only mesh leaves are parked
+    const uint64_t meshes = __ballot(in_blas);
+    for (uint64_t walk = __ballot(node >= 0);;) {
+      if (lane_bit(walk)) {
+        const uint64_t inner = __ballot(node >= 0);  // the others hold a popped mesh leaf
+        const int32_t top = stack_top(st);
+        const NodeHits v = Nodes::visit(in_blas ? blas : tlas, max(node, 0), rb, tmin, r.t);
+        if (STATS && node >= 0) {
           stats.nodes++;
           if (in_blas) touch(acc.touch_nodes, static_cast<uint32_t>(node) / Nodes::kBytes);
         }
-        if (v.h0 && v.h1) {
-          const bool swap = v.t1 < v.t0;
-          push(static_cast<uint32_t>(swap ? v.c0 : v.c1));
-          node = swap ? v.c1 : v.c0;
-        } else if (v.h0) {
-          node = v.c0;
-        } else if (v.h1) {
-          node = v.c1;
-        } else {
-          node = pop();
-        }
-        node = settle(node);
-        if (in_blas && node < 0 && node != kTravDone && node != kTravBlocked && leaf == 0) {
-          leaf = node;
-          node = settle(pop());
-        }
-        if (searching_lanes(leaf) <= kSearchBreakSpread) break;
+        const uint64_t h0 = __ballot(v.n0 <= v.f0) | ~inner, h1 = __ballot(v.n1 <= v.f1) & inner;
+        const int32_t c0 = lane_bit(inner) ? v.c0 : node;
+        const uint64_t both = h0 & h1, first1 = (both & __ballot(v.n1 < v.n0)) | ~h0;
+        const int32_t nearc = lane_bit(first1) ? v.c1 : c0, farc = lane_bit(first1) ? c0 : v.c1;
+        const uint64_t park = (h0 | h1) & __ballot(nearc < 0) & __ballot(leaf == 0) & meshes;
+        stack_above(st, farc);
+        leaf = lane_bit(park) ? nearc : leaf;
+        const uint64_t pop = ~(h0 | h1) | (park & ~both);
+        node = lane_bit(park) ? farc : nearc;
+        node = lane_bit(pop) ? top : node;
+        stack_step<STATS>(st, both & ~park, pop, stats, on_full);
       }
+      const uint64_t no_leaf = __ballot(leaf == 0), searching = walk & no_leaf;
+      walk = __ballot(node >= 0) | (no_leaf & meshes & __ballot(node > kTravExit));
+      if (walk == 0 || mask_count(searching) <= kSearchBreakSpread) break;
     }
     // mesh leaves (the parked one, and `node` when it is one; both in the current
-    // instance, which a lane with a parked leaf does not leave), spread over the wave.
-    // Task hits that beat the ray's best under the (t, inst, prim) order compete; the
-    // phase's (t, prim) minimum of those becomes the best.
+    // instance), spread over the wave. Task hits that beat the ray's best under the
+    // (t, inst, prim) order compete; the phase's (t, prim) minimum of those becomes the best.
     bool hit = false;
-    const bool node_leaf = in_blas && node < 0 && node != kTravDone && node != kTravBlocked;
+    const bool node_leaf = in_blas && node < 0 && node > kTravExit;
     const uint32_t ca = leaf != 0 ? (~static_cast<uint32_t>(leaf) & 7u) : 0u;
     const uint32_t cb = node_leaf ? (~static_cast<uint32_t>(node) & 7u) : 0u;
     bool better;
     unsigned long long kf;
     if (leaf_phase<STATS, true>(tk, tris, lane, ~static_cast<uint32_t>(leaf) >> 3, ca, ~static_cast<uint32_t>(node) >> 3,
-                                cb, rb.o, kxyz, shear, tmin, r.t, r.prim, r.inst, cur_id, better, kf, stats,
+                                cb, rb.o, rs, tmin, r.t, r.prim, r.inst, cur_id, better, kf, stats,
                                 acc.touch_tris) &&
         (leaf != 0 || node_leaf)) {
       if (better) {  // the barycentrics stay in tk.bary[lane] until the ray finishes
@@ -843,8 +844,43 @@ __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& i
         hit = ANY;
       }
       leaf = 0;
-      if (node_leaf) node = settle(pop());
-      if (node == kTravBlocked) node = settle(pop());  // the leaf is done: leave the instance
+      if (node_leaf) {
+        node = stack_top(st);
+        stack_step<STATS>(st, 0ull, ~0ull, stats, on_full);
+      }
+    }
+    // change of space: leave the instance at its marker, then enter the next one at a
+    // top-level leaf (the rest of the leaf and the marker go on the stack)
+    const bool leaves = leaf == 0 && node == kTravExit;
+    if (leaves) {
+      in_blas = false;
+      node = stack_top(st);
+      stack_step<STATS>(st, 0ull, ~0ull, stats, on_full);
+    }
+    const bool enters = !in_blas && node < 0 && node > kTravExit;
+    if (leaves || enters) {
+      V3 o = ow, d = dw;
+      NodeSpace space = acc.space;
+      if (enters) {
+        const uint32_t c = ~static_cast<uint32_t>(node);
+        const uint32_t first = c >> 3, cnt = c & 7u;
+        if (cnt > 1u) {
+          stack_above(st, static_cast<int32_t>(~(((first + 1u) << 3) | (cnt - 1u))));
+          stack_step<STATS>(st, ~0ull, 0ull, stats, on_full);
+        }
+        stack_above(st, kTravExit);
+        stack_step<STATS>(st, ~0ull, 0ull, stats, on_full);
+        const TlasInstance& ins = acc.inst[first];
+        o = xform_point(ins.w2o, ow);
+        d = xform_vector(ins.w2o, dw);
+        space = ins.space;
+        rs = ray_shear(d);
+        cur_id = ins.id;
+        in_blas = true;
+        node = static_cast<int32_t>(ins.blas_root);
+        if (STATS) stats.nodes++;
+      }
+      rb = Nodes::setup(space, o, d);
     }
     if (slot != kNoHit && (hit || (node == kTravDone && leaf == 0))) {
       r.b1 = r.b2 = 0.f;
@@ -987,9 +1023,10 @@ struct RayLoad {
   }
 };
 
-// Single-level scenes: Extend and Shadow through trace_queue. Both are held to 72
-// VGPRs, 7 waves per SIMD (the allocator otherwise settles just above, at 6 waves,
-// which measured 5% slower).
+// Single-level scenes: Extend and Shadow through trace_queue, held to 72 VGPRs, 7 waves per
+// SIMD. They are bound by throughput, not latency (the texture data path is 91 % busy and
+// VALU issue above its 4-cycle rate): 6 and 5 waves measured 11.98 and 12.01 ms a soup
+// frame against 11.82.
 template <class Nodes, bool STATS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_extend_sl(DevAccel acc, RayQueue q, HitBuf h, SegIn in, uint32_t* ctr) {
   extern __shared__ uint32_t lds[];
@@ -1039,10 +1076,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
   }
 }
 
-// Two-level scenes: Extend and Shadow through trace_queue2, held to 80 VGPRs, 6 waves
-// per SIMD (a few spilled dwords; 5 waves at the allocator's 86 measured 5% slower).
+// Two-level scenes: Extend and Shadow through trace_queue2, at 96 VGPRs, 5 waves per SIMD:
+// 11.8 ms per 4K frame of 1000 instances, against 12.5 at 6 waves and 13.2 at 7 (spilled
+// registers) and 11.9 at 4.
 template <class Nodes, bool STATS>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_extend_tl(DevAccel acc, RayQueue q, HitBuf h, SegIn in, uint32_t* ctr) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_extend_tl(DevAccel acc, RayQueue q, HitBuf h, SegIn in, uint32_t* ctr) {
   extern __shared__ uint32_t lds[];
   TraceOut st;
   st.nodes = 0;
@@ -1063,7 +1101,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
 }
 
 template <class Nodes, bool STATS>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_shadow_tl(DevAccel acc, ShadowQueue sq, float4* radiance, SegIn in,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_shadow_tl(DevAccel acc, ShadowQueue sq, float4* radiance, SegIn in,
                                                        uint32_t* ctr) {
   extern __shared__ uint32_t lds[];
   TraceOut st;
@@ -1463,7 +1501,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
 }
 
 template <class Nodes>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_shadow_adj_tl(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_shadow_adj_tl(
     DevAccel acc, ShadowQueue sq, AdjBuffers ab, SegIn in, uint32_t* ctr, uint32_t depth) {
   extern __shared__ uint32_t lds[];
   TraceOut st;
