@@ -223,12 +223,8 @@ hipError_t Unet::backward(const float* dout, int N, int H, int W, hipStream_t s)
                    float* gout) {
     const Conv& c = convs_[i];
     const size_t P = size_t(N) * h * w;
-    if (c.relu)
-      dn_relu_bwd(gin, act_[i], dz_, P * c.cout, s);
-    else
-      dn_to_bf16(gin, dz_, P * c.cout, s);
+    dn_relu_bias_bwd(gin, c.relu ? act_[i] : nullptr, dz_, P, c.cout, bpart_, g_ + c.boff, s);
     dn_wgrad(in, coarse, c1, dz_, wpart_, g_ + c.woff, N, h, w, c.cin, c.cout, kWgradTiles, s);
-    dn_bias_grad(dz_, P, c.cout, bpart_, g_ + c.boff, s);
     if (gout) dn_conv3x3(dz_, wd_ + c.woff, nullptr, gout, N, h, w, c.cout, c.cin, false, true, s);
   };
   layer(OUT, nullptr, 0, act_[D0B], H, W, dout, gA_);

@@ -42,8 +42,10 @@ bool dn_conv3x3(const uint16_t* X, const uint16_t* Wt, const float* bias, void* 
 int dn_wgrad_chunks(int N, int H, int W, int tiles_per_chunk);
 void dn_wgrad(const uint16_t* X, const uint16_t* coarse, int c1, const uint16_t* dZ, float* partial, float* dW, int N,
               int H, int W, int Cin, int Cout, int tiles_per_chunk, hipStream_t s);
-void dn_bias_grad(const uint16_t* dZ, size_t P, int C, float* partial, float* db, hipStream_t s);
-void dn_relu_bwd(const float* dY, const uint16_t* Y, uint16_t* dZ, size_t n, hipStream_t s);
+// dZ = bf16(dY masked by Y > 0; Y null: no mask) and its per-channel sums db (C <= 128,
+// C % 8 == 0; partial: kBiasBlocks x C)
+void dn_relu_bias_bwd(const float* dY, const uint16_t* Y, uint16_t* dZ, size_t P, int C, float* partial, float* db,
+                      hipStream_t s);
 void dn_to_bf16(const float* a, uint16_t* b, size_t n, hipStream_t s);
 void dn_pool_bwd(const float* dY, float* dX, int N, int H, int W, int C, bool accumulate, hipStream_t s);
 void dn_upcat_bwd(const float* dout, float* dcoarse, float* dskip, int N, int H, int W, int C1, int C2,

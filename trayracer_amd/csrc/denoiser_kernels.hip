@@ -29,7 +29,6 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
 
 constexpr int kTileH = 8, kTileW = 16;          // output pixels per workgroup
 constexpr int kPatchH = kTileH + 2, kPatchW = kTileW + 2;
-constexpr int kPatch = kPatchH * kPatchW;        // 180 staged input positions
 
 // ------------------------------------------------------------------------------------
 // 3x3 'same' convolution as an implicit GEMM (M = pixels, N = output channels,
@@ -439,108 +438,203 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
 // with M = co (32-block), N = ci (32-block), K = pixels. Each workgroup covers `tiles`
 // consecutive 8x16 pixel tiles of one image row band and writes its partial sums to
 // partial[chunk][co][tap][ci]; a fixed-order reduction over chunks follows.
-// Grid: (n_chunks, Cout/32 * ceil(Cin/32)); wave w handles taps w, w+4, w+8.
-__global__ __launch_bounds__(256) void k_wgrad(const uint16_t* __restrict__ X, const uint16_t* __restrict__ coarse,
-                                                int c1, const uint16_t* __restrict__ dZ, float* __restrict__ partial,
-                                                int N, int H, int W, int Cin, int Cout, int tiles_per_chunk) {
-  __shared__ uint16_t xs[32 * (kPatch + 8)];   // [ci][pos]
-  __shared__ uint16_t zs[32 * (kTileH * kTileW + 8)];  // [co][pix]
-  constexpr int XS = kPatch + 8, ZS = kTileH * kTileW + 8;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// Grid: (n_chunks, Cout/32 * ceil(Cin/32)); wave w handles the taps of kernel row w.
+//
+// The fragments hold eight consecutive pixels of one channel, while the tensors have the
+// channels together, so staging transposes: a thread loads 8 channels of four neighbouring
+// pixels (16 bytes each), exchanges halves in registers and writes eight 8-byte runs of
+// pixels to LDS as [channel][row][pixel]. A wave then reads one aligned run of ten pixels of
+// an input row and forms the three horizontally shifted fragments of its kernel row from it
+// in registers. The next tile's loads are issued before the current tile's MFMAs. (Element by
+// element staging took 220 us a layer on average at 8 x 128 x 128, 24 us now.)
+constexpr int kWgThreads = 192;
+constexpr int kWgRow = 24;                    // LDS pixels per staged input row (18 used)
+constexpr int kWgXs = kPatchH * kWgRow + 8;   // bf16 per channel: an odd number of 16-byte slots
+constexpr int kWgZs = kTileH * kTileW + 8;
+constexpr int kWgXItems = kPatchH * 5 * 4, kWgZItems = kTileH * 4 * 4;  // rows x pixel quads x channel octets
+constexpr int kWgItems = (kWgXItems + kWgZItems + kWgThreads - 1) / kWgThreads;
+
+__global__ __launch_bounds__(kWgThreads) void k_wgrad(const uint16_t* __restrict__ X, const uint16_t* __restrict__ coarse,
+                                                      int c1, const uint16_t* __restrict__ dZ, float* __restrict__ partial,
+                                                      int N, int H, int W, int Cin, int Cout, int tiles_per_chunk) {
+  __shared__ __align__(16) uint16_t xs[32 * kWgXs];  // [ci][row][pixel]
+  __shared__ __align__(16) uint16_t zs[32 * kWgZs];  // [co][row][pixel]
+  const int tid = threadIdx.x, lane = tid & 63, ky = tid >> 6;
   const int ci_blocks = (Cin + 31) / 32;
   const int cb = blockIdx.y / ci_blocks, ib = blockIdx.y - cb * ci_blocks;
   const int tiles_x = W / kTileW, tiles_y = (H + kTileH - 1) / kTileH;
   const int tiles_img = tiles_x * tiles_y;
-  const int total_tiles = tiles_img * N;
-  f32x16 acc[3];
-  for (int j = 0; j < 3; ++j)
-    for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
-  const int ntap = wave == 0 ? 3 : 2;  // taps {0,4,8}, {1,5}, {2,6}, {3,7}
-  const int khalf = (lane >> 5) * 8;
-  for (int t = 0; t < tiles_per_chunk; ++t) {
-    const int tile = blockIdx.x * tiles_per_chunk + t;
-    if (tile >= total_tiles) break;
+  const int first = blockIdx.x * tiles_per_chunk;
+  const int last = min(first + tiles_per_chunk, tiles_img * N);
+  const bool up = ib * 32 < c1;  // this input block comes from the upsampled coarse tensor
+  const int cx = Cin - c1;
+  // fixed per thread: which quad of pixels and octet of channels each item stages, and where
+  int iy[kWgItems], ix[kWgItems], ic[kWgItems], to[kWgItems];
+#pragma unroll
+  for (int k = 0; k < kWgItems; ++k) {
+    const int i = tid + k * kWgThreads, part = i & 3;
+    if (i < kWgXItems) {
+      const int g = i >> 2, row = g / 5, quad = g - row * 5;
+      iy[k] = row - 1;
+      ix[k] = quad * 4 - 1;
+      ic[k] = part * 8;
+      to[k] = part * 8 * kWgXs + row * kWgRow + quad * 4;
+    } else {
+      const int g = (i - kWgXItems) >> 2, row = g >> 2, quad = g & 3;
+      iy[k] = row;
+      ix[k] = quad * 4;
+      ic[k] = part * 8;
+      to[k] = part * 8 * kWgZs + row * kTileW + quad * 4;
+    }
+  }
+  u32x4 stage[kWgItems][4];
+  auto load_tile = [&](int tile) __attribute__((always_inline)) {
     const int n = tile / tiles_img, tr = tile - n * tiles_img;
-    const int ty = tr / tiles_x, tx = tr - ty * tiles_x;
-    const int y0 = ty * kTileH, x0 = tx * kTileW;
-    const size_t img = static_cast<size_t>(n) * H * W;
-    const size_t img_c = static_cast<size_t>(n) * (H >> 1) * (W >> 1);
-    const int cx = Cin - c1;
-    __syncthreads();
-    for (int i = threadIdx.x; i < 32 * kPatch; i += 256) {
-      const int ci = i / kPatch, pos = i - ci * kPatch;
-      const int py = pos / kPatchW, px = pos - py * kPatchW;
-      const int yy = y0 + py - 1, xx = x0 + px - 1, c = ib * 32 + ci;
-      uint16_t v = 0;
-      if (c < Cin && yy >= 0 && yy < H && xx >= 0 && xx < W)
-        v = c < c1 ? coarse[(img_c + static_cast<size_t>(yy >> 1) * (W >> 1) + (xx >> 1)) * c1 + c]
-                   : X[(img + static_cast<size_t>(yy) * W + xx) * cx + (c - c1)];
-      xs[ci * XS + pos] = v;
+    const int ty = tr / tiles_x, y0 = ty * kTileH, x0 = (tr - ty * tiles_x) * kTileW;
+#pragma unroll
+    for (int k = 0; k < kWgItems; ++k) {
+      const int i = tid + k * kWgThreads;
+      const bool is_x = i < kWgXItems;
+      const int yy = y0 + iy[k];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int xx = x0 + ix[k] + q;
+        stage[k][q] = u32x4{0u, 0u, 0u, 0u};
+        if (static_cast<unsigned>(yy) >= static_cast<unsigned>(H) || static_cast<unsigned>(xx) >= static_cast<unsigned>(W)) continue;
+        if (is_x) {
+          if (ix[k] + q > kTileW || ib * 32 + ic[k] >= Cin) continue;
+          const uint16_t* src =
+              up ? coarse + ((static_cast<size_t>(n) * (H >> 1) + (yy >> 1)) * (W >> 1) + (xx >> 1)) * c1 + ib * 32 + ic[k]
+                 : X + ((static_cast<size_t>(n) * H + yy) * W + xx) * cx + (ib * 32 - c1) + ic[k];
+          stage[k][q] = *reinterpret_cast<const u32x4*>(src);
+        } else if (i < kWgXItems + kWgZItems) {
+          stage[k][q] = *reinterpret_cast<const u32x4*>(dZ + ((static_cast<size_t>(n) * H + yy) * W + xx) * Cout + cb * 32 + ic[k]);
+        }
+      }
     }
-    for (int i = threadIdx.x; i < 32 * kTileH * kTileW; i += 256) {
-      const int co = i / (kTileH * kTileW), pix = i - co * (kTileH * kTileW);
-      const int yy = y0 + pix / kTileW, xx = x0 + (pix % kTileW);
-      uint16_t v = 0;
-      if (yy < H) v = dZ[(img + static_cast<size_t>(yy) * W + xx) * Cout + cb * 32 + co];
-      zs[co * ZS + pix] = v;
+  };
+  auto store_tile = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < kWgItems; ++k) {
+      const int i = tid + k * kWgThreads;
+      if (i >= kWgXItems + kWgZItems) continue;
+      uint16_t* dst = i < kWgXItems ? xs + to[k] : zs + to[k];
+      const int pitch = i < kWgXItems ? kWgXs : kWgZs;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {  // channels 2c, 2c + 1 in the halves of dword c
+        uint2 lo, hi;
+        lo.x = __builtin_amdgcn_perm(stage[k][1][c], stage[k][0][c], 0x05040100u);
+        lo.y = __builtin_amdgcn_perm(stage[k][3][c], stage[k][2][c], 0x05040100u);
+        hi.x = __builtin_amdgcn_perm(stage[k][1][c], stage[k][0][c], 0x07060302u);
+        hi.y = __builtin_amdgcn_perm(stage[k][3][c], stage[k][2][c], 0x07060302u);
+        *reinterpret_cast<uint2*>(dst + (2 * c) * pitch) = lo;
+        *reinterpret_cast<uint2*>(dst + (2 * c + 1) * pitch) = hi;
+      }
     }
+  };
+  f32x16 acc[3] = {f32x16{}, f32x16{}, f32x16{}};
+  const int khalf = (lane >> 5) * 8;
+  const uint16_t* zrow = zs + (lane & 31) * kWgZs + khalf;
+  const uint16_t* xrow = xs + (lane & 31) * kWgXs + ky * kWgRow + khalf;
+  if (first < last) load_tile(first);
+  for (int tile = first; tile < last; ++tile) {
     __syncthreads();
+    store_tile();
+    __syncthreads();
+    if (tile + 1 < last) load_tile(tile + 1);
+#pragma unroll
     for (int row = 0; row < kTileH; ++row) {  // K-step = 16 pixels of one tile row
-      bf16x8 a;
-      {
-        const uint16_t* src = zs + (lane & 31) * ZS + row * kTileW + khalf;
-        for (int v = 0; v < 8; ++v) a[v] = __builtin_bit_cast(__bf16, src[v]);
-      }
-      for (int j = 0; j < ntap; ++j) {
-        const int tap = wave + 4 * j;
-        const int ky = tap / 3, kx = tap - ky * 3;
-        bf16x8 bv;
-        const uint16_t* src = xs + (lane & 31) * XS + (row + ky) * kPatchW + kx + khalf;
-        for (int v = 0; v < 8; ++v) bv[v] = __builtin_bit_cast(__bf16, src[v]);
-        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bv, acc[j], 0, 0, 0);
-      }
+      const bf16x8 a = *reinterpret_cast<const bf16x8*>(zrow + row * kTileW);
+      const u32x4 x0 = *reinterpret_cast<const u32x4*>(xrow + row * kWgRow);
+      const uint32_t x4 = *reinterpret_cast<const uint32_t*>(xrow + row * kWgRow + 8);
+      const u32x4 x1 = {__builtin_amdgcn_alignbyte(x0[1], x0[0], 2), __builtin_amdgcn_alignbyte(x0[2], x0[1], 2),
+                        __builtin_amdgcn_alignbyte(x0[3], x0[2], 2), __builtin_amdgcn_alignbyte(x4, x0[3], 2)};
+      const u32x4 x2 = {x0[1], x0[2], x0[3], x4};
+      acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(bf16x8, x0), acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(bf16x8, x1), acc[1], 0, 0, 0);
+      acc[2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(bf16x8, x2), acc[2], 0, 0, 0);
     }
   }
   // write partial: rows = co (A rows), cols = ci (B cols)
   const size_t wsize = static_cast<size_t>(Cout) * 9 * Cin;
   float* out = partial + blockIdx.x * wsize;
-  for (int j = 0; j < ntap; ++j) {
-    const int tap = wave + 4 * j;
-    const int ci = ib * 32 + (lane & 31);
-    if (ci >= Cin) continue;
+  const int ci = ib * 32 + (lane & 31);
+  if (ci >= Cin) return;
+#pragma unroll
+  for (int kx = 0; kx < 3; ++kx)
+#pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int co = cb * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-      out[(static_cast<size_t>(co) * 9 + tap) * Cin + ci] = acc[j][r];
+      out[(static_cast<size_t>(co) * 9 + ky * 3 + kx) * Cin + ci] = acc[kx][r];
     }
+}
+
+// out[i] = sum over chunks c (in order) of partial[c][i]. A block takes 32 outputs: its 256
+// threads bring 128 chunks at a time into LDS with all loads in flight, then 32 threads add
+// them in order (one thread per output with its loads in a row was bound by their latency:
+// 36 us a layer on average at 8 x 128 x 128, 6.5 us now).
+constexpr int kReduceOuts = 32, kReduceChunks = 128;
+__global__ __launch_bounds__(256) void k_reduce_chunks(const float* __restrict__ partial, int n_chunks, size_t n,
+                                                       float* __restrict__ out) {
+  __shared__ float lds[kReduceChunks * kReduceOuts];
+  const int o = threadIdx.x & (kReduceOuts - 1), part = threadIdx.x / kReduceOuts;
+  const size_t i = static_cast<size_t>(blockIdx.x) * kReduceOuts + o;
+  float t = 0.f;
+  for (int c0 = 0; c0 < n_chunks; c0 += kReduceChunks) {
+    const int m = min(kReduceChunks, n_chunks - c0);
+    float v[kReduceChunks / 8];
+#pragma unroll
+    for (int k = 0; k < kReduceChunks / 8; ++k) {
+      const int c = part + 8 * k;
+      v[k] = c < m && i < n ? partial[static_cast<size_t>(c0 + c) * n + i] : 0.f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kReduceChunks / 8; ++k) lds[(part + 8 * k) * kReduceOuts + o] = v[k];
+    __syncthreads();
+    if (part == 0)
+      for (int c = 0; c < m; ++c) t += lds[c * kReduceOuts + o];
   }
+  if (part == 0 && i < n) out[i] = t;
 }
 
-// out[i] = sum over chunks c (in order) of partial[c][i]
-__global__ void k_reduce_chunks(const float* __restrict__ partial, int n_chunks, size_t n, float* __restrict__ out) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+// dZ = bf16(dY * (Y > 0)) (ReLU backward; Y is the post-activation output, null for a
+// linear layer) and the bias gradient's partial sums: block b takes pixels
+// [b*P/B, (b+1)*P/B), 64 at a time, stages their dZ in LDS and adds it per channel in pixel
+// order. Bound by its 8 bytes a value (as two kernels the sums re-read dZ with C threads a
+// block: 40 + 7 us a layer on average at 8 x 128 x 128, 9 us now).
+constexpr int kBiasPixels = 64, kBiasMaxChannels = 128;
+__global__ __launch_bounds__(256) void k_relu_bias(const float* __restrict__ dY, const uint16_t* __restrict__ Y,
+                                                   uint16_t* __restrict__ dZ, size_t P, int C,
+                                                   float* __restrict__ partial) {
+  __shared__ __align__(16) uint16_t lds[kBiasPixels * kBiasMaxChannels];
+  const size_t p0 = P * blockIdx.x / gridDim.x, p1 = P * (blockIdx.x + 1) / gridDim.x;
   float t = 0.f;
-  for (int c = 0; c < n_chunks; ++c) t += partial[static_cast<size_t>(c) * n + i];
-  out[i] = t;
-}
-
-// bias gradient partials: block b sums pixels [b*P/B, (b+1)*P/B) of dZ (bf16) per channel
-__global__ void k_bias_partial(const uint16_t* __restrict__ dZ, size_t P, int C, int n_blocks,
-                               float* __restrict__ partial) {
-  const int c = threadIdx.x;
-  if (c >= C) return;
-  const size_t p0 = P * blockIdx.x / n_blocks, p1 = P * (blockIdx.x + 1) / n_blocks;
-  float t = 0.f;
-  for (size_t p = p0; p < p1; ++p) t += bf2f(dZ[p * C + c]);
-  partial[static_cast<size_t>(blockIdx.x) * C + c] = t;
-}
-
-// dZ = bf16(dY * (Y > 0))  (ReLU backward; Y is the post-activation output)
-__global__ void k_relu_bwd(const float* __restrict__ dY, const uint16_t* __restrict__ Y, uint16_t* __restrict__ dZ,
-                           size_t n) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  dZ[i] = bf2f(Y[i]) > 0.f ? f2bf(dY[i]) : static_cast<uint16_t>(0);
+  for (size_t p = p0; p < p1; p += kBiasPixels) {
+    const int m = static_cast<int>(p1 - p < kBiasPixels ? p1 - p : kBiasPixels);
+    const int octets = m * C / 8;
+    __syncthreads();
+    for (int i = threadIdx.x; i < octets; i += 256) {
+      const size_t at = p * C + static_cast<size_t>(i) * 8;
+      const float4 g0 = *reinterpret_cast<const float4*>(dY + at), g1 = *reinterpret_cast<const float4*>(dY + at + 4);
+      const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+      u32x4 y = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};  // ones
+      if (Y) y = *reinterpret_cast<const u32x4*>(Y + at);
+      u32x4 z;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t lo = __uint_as_float(y[k] << 16) > 0.f ? f2bf(g[2 * k]) : 0u;
+        const uint32_t hi = __uint_as_float(y[k] & 0xffff0000u) > 0.f ? f2bf(g[2 * k + 1]) : 0u;
+        z[k] = lo | (hi << 16);
+      }
+      *reinterpret_cast<u32x4*>(dZ + at) = z;
+      *reinterpret_cast<u32x4*>(lds + i * 8) = z;
+    }
+    __syncthreads();
+    if (static_cast<int>(threadIdx.x) < C)
+      for (int q = 0; q < m; ++q) t += bf2f(lds[q * C + threadIdx.x]);
+  }
+  if (static_cast<int>(threadIdx.x) < C) partial[static_cast<size_t>(blockIdx.x) * C + threadIdx.x] = t;
 }
 
 __global__ void k_to_bf16(const float* __restrict__ a, uint16_t* __restrict__ b, size_t n) {
@@ -842,20 +936,17 @@ void dn_wgrad(const uint16_t* X, const uint16_t* coarse, int c1, const uint16_t*
               int H, int W, int Cin, int Cout, int tiles_per_chunk, hipStream_t s) {
   const int chunks = dn_wgrad_chunks(N, H, W, tiles_per_chunk);
   const dim3 grid(chunks, (Cout / 32) * ((Cin + 31) / 32));
-  hipLaunchKernelGGL(k_wgrad, grid, dim3(256), 0, s, X, coarse, c1, dZ, partial, N, H, W, Cin, Cout,
+  hipLaunchKernelGGL(k_wgrad, grid, dim3(kWgThreads), 0, s, X, coarse, c1, dZ, partial, N, H, W, Cin, Cout,
                      tiles_per_chunk);
   const size_t n = static_cast<size_t>(Cout) * 9 * Cin;
-  hipLaunchKernelGGL(k_reduce_chunks, dim3(blocks_for(n)), dim3(256), 0, s, partial, chunks, n, dW);
+  hipLaunchKernelGGL(k_reduce_chunks, dim3(blocks_for(n, kReduceOuts)), dim3(256), 0, s, partial, chunks, n, dW);
 }
 
-void dn_bias_grad(const uint16_t* dZ, size_t P, int C, float* partial, float* db, hipStream_t s) {
-  const int nb = kBiasBlocks;
-  hipLaunchKernelGGL(k_bias_partial, dim3(nb), dim3(256), 0, s, dZ, P, C, nb, partial);
-  hipLaunchKernelGGL(k_reduce_chunks, dim3(blocks_for(C)), dim3(256), 0, s, partial, nb, static_cast<size_t>(C), db);
-}
-
-void dn_relu_bwd(const float* dY, const uint16_t* Y, uint16_t* dZ, size_t n, hipStream_t s) {
-  hipLaunchKernelGGL(k_relu_bwd, dim3(blocks_for(n)), dim3(256), 0, s, dY, Y, dZ, n);
+void dn_relu_bias_bwd(const float* dY, const uint16_t* Y, uint16_t* dZ, size_t P, int C, float* partial, float* db,
+                      hipStream_t s) {
+  hipLaunchKernelGGL(k_relu_bias, dim3(kBiasBlocks), dim3(256), 0, s, dY, Y, dZ, P, C, partial);
+  hipLaunchKernelGGL(k_reduce_chunks, dim3(blocks_for(C, kReduceOuts)), dim3(256), 0, s, partial, kBiasBlocks,
+                     static_cast<size_t>(C), db);
 }
 void dn_to_bf16(const float* a, uint16_t* b, size_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_to_bf16, dim3(blocks_for(n)), dim3(256), 0, s, a, b, n);
