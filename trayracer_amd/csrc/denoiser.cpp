@@ -12,7 +12,6 @@ namespace trt {
 namespace {
 // conv index -> role
 enum { E0A, E0B, E1A, E1B, E2A, E2B, E3A, E3B, D2A, D2B, D1A, D1B, D0A, D0B, OUT, NCONV };
-constexpr int kWgradTiles = 8;
 }  // namespace
 
 Unet::Unet() {
@@ -32,6 +31,11 @@ Unet::Unet() {
     convs_.push_back(cv);
   }
   n_params_ = off;
+  for (size_t li = 1; li < convs_.size(); ++li) {  // the first layer needs no input gradient
+    table_.off[table_.n] = int(convs_[li].woff);
+    table_.cin[table_.n] = convs_[li].cin;
+    table_.cout[table_.n++] = convs_[li].cout;
+  }
   act_.assign(NCONV, nullptr);
 }
 
@@ -78,9 +82,7 @@ hipError_t Unet::set_params(const float* host, hipStream_t s) {
   if ((e = hipMemcpyAsync(w_, host, n_params_ * 4, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
   if ((e = hipMemsetAsync(m_, 0, n_params_ * 4, s)) != hipSuccess) return e;
   if ((e = hipMemsetAsync(v_, 0, n_params_ * 4, s)) != hipSuccess) return e;
-  dn_to_bf16(w_, wb_, n_params_, s);
-  for (size_t li = 1; li < convs_.size(); ++li)
-    dn_flip_weights(wb_ + convs_[li].woff, wd_ + convs_[li].woff, convs_[li].cin, convs_[li].cout, s);
+  dn_weights_bf16(w_, wb_, wd_, table_, n_params_, s);
   t_ = 0;
   return hipStreamSynchronize(s);
 }
@@ -97,7 +99,7 @@ hipError_t Unet::get_grads(float* host, hipStream_t s) {
   return hipStreamSynchronize(s);
 }
 
-hipError_t Unet::ensure(int N, int H, int W) {
+hipError_t Unet::ensure(int N, int H, int W, hipStream_t s) {
   if (N == N_ && H == H_ && W == W_) return hipSuccess;
   free_acts();
   auto alloc = [&](size_t bytes, void** p) {
@@ -115,20 +117,22 @@ hipError_t Unet::ensure(int N, int H, int W) {
   if ((e = alloc(P2 * 64 * 2, reinterpret_cast<void**>(&p1_))) != hipSuccess) return e;
   if ((e = alloc(P3 * 96 * 2, reinterpret_cast<void**>(&p2_))) != hipSuccess) return e;
   if ((e = alloc(P0 * 32 * 4, reinterpret_cast<void**>(&out_))) != hipSuccess) return e;
-  // backward scratch: the largest per-pixel gradient tensor is 96 ch at full resolution
-  const size_t gmax = P0 * 96;
+  // backward scratch: gradients of the three concatenated inputs (kept until their skip
+  // shares are used), two others of at most 32 channels at full resolution, and bf16 dZ
+  const size_t gmax = P0 * 32;
   if ((e = alloc(gmax * 4, reinterpret_cast<void**>(&gA_))) != hipSuccess) return e;
   if ((e = alloc(gmax * 4, reinterpret_cast<void**>(&gB_))) != hipSuccess) return e;
-  if ((e = alloc(P0 * 32 * 4, reinterpret_cast<void**>(&gs0_))) != hipSuccess) return e;
-  if ((e = alloc(P1 * 64 * 4, reinterpret_cast<void**>(&gs1_))) != hipSuccess) return e;
-  if ((e = alloc(P2 * 96 * 4, reinterpret_cast<void**>(&gs2_))) != hipSuccess) return e;
+  if ((e = alloc(P0 * 96 * 4, reinterpret_cast<void**>(&gu0_))) != hipSuccess) return e;
+  if ((e = alloc(P1 * 160 * 4, reinterpret_cast<void**>(&gu1_))) != hipSuccess) return e;
+  if ((e = alloc(P2 * 224 * 4, reinterpret_cast<void**>(&gu2_))) != hipSuccess) return e;
   if ((e = alloc(P0 * 32 * 4, reinterpret_cast<void**>(&dout_))) != hipSuccess) return e;
+  if ((e = hipMemsetAsync(dout_, 0, P0 * 32 * 4, s)) != hipSuccess) return e;  // its padding channels stay zero
   if ((e = alloc(gmax * 2, reinterpret_cast<void**>(&dz_))) != hipSuccess) return e;
   size_t wp = 0;
   for (int i = 0; i < NCONV; ++i) {
     const int hh = (i <= E0B || i >= D0A) ? H : (i <= E1B || i >= D1A) ? H / 2 : (i <= E2B || i >= D2A) ? H / 4 : H / 8;
     const int ww = W * hh / H;
-    const size_t chunks = size_t(dn_wgrad_chunks(N, hh, ww, kWgradTiles));
+    const size_t chunks = size_t(dn_wgrad_chunks(N, hh, ww));
     const size_t need = chunks * convs_[i].cout * 9 * convs_[i].cin;
     if (need > wp) wp = need;
   }
@@ -152,7 +156,7 @@ size_t Unet::activation_elems(int i) const {
 
 hipError_t Unet::forward(const uint16_t* x, int N, int H, int W, hipStream_t s, float4* radiance) {
   if (!w_ || !shape_ok(H, W)) return hipErrorInvalidValue;
-  hipError_t e = ensure(N, H, W);
+  hipError_t e = ensure(N, H, W, s);
   if (e != hipSuccess) return e;
   x_ = x;
   have_output_ = false;
@@ -219,35 +223,33 @@ hipError_t Unet::backward(const float* dout, int N, int H, int W, hipStream_t s)
   if (N != N_ || H != H_ || W != W_ || !x_ || !have_output_) return hipErrorInvalidValue;
   const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4, H3 = H / 8, W3 = W / 8;
   // one conv layer: gradient in (fp32, post-activation) -> dW, db, gradient out (fp32)
-  auto layer = [&](int i, const uint16_t* coarse, int c1, const uint16_t* in, int h, int w, const float* gin,
+  auto layer = [&](int i, const uint16_t* coarse, int c1, const uint16_t* in, int h, int w, const DnGrad& gin,
                    float* gout) {
     const Conv& c = convs_[i];
-    const size_t P = size_t(N) * h * w;
-    dn_relu_bias_bwd(gin, c.relu ? act_[i] : nullptr, dz_, P, c.cout, bpart_, g_ + c.boff, s);
-    dn_wgrad(in, coarse, c1, dz_, wpart_, g_ + c.woff, N, h, w, c.cin, c.cout, kWgradTiles, s);
+    dn_layer_bwd(gin, c.relu ? act_[i] : nullptr, in, coarse, c1, dz_, N, h, w, c.cin, c.cout, wpart_, bpart_,
+                 g_ + c.woff, g_ + c.boff, s);
     if (gout) dn_conv3x3(dz_, wd_ + c.woff, nullptr, gout, N, h, w, c.cout, c.cin, false, true, s);
   };
-  layer(OUT, nullptr, 0, act_[D0B], H, W, dout, gA_);
-  layer(D0B, nullptr, 0, act_[D0A], H, W, gA_, gB_);
-  layer(D0A, act_[D1B], 64, act_[E0B], H, W, gB_, gA_);  // gA = d u0 (96 ch @H)
-  dn_upcat_bwd(gA_, gB_, gs0_, N, H, W, 64, 32, false, s);  // gB = d d1b (64 @H1), gs0 = d e0b (skip part)
-  layer(D1B, nullptr, 0, act_[D1A], H1, W1, gB_, gA_);
-  layer(D1A, act_[D2B], 96, act_[E1B], H1, W1, gA_, gB_);  // gB = d u1 (160 @H1)
-  dn_upcat_bwd(gB_, gA_, gs1_, N, H1, W1, 96, 64, false, s);  // gA = d d2b (96 @H2), gs1 = d e1b
-  layer(D2B, nullptr, 0, act_[D2A], H2, W2, gA_, gB_);
-  layer(D2A, act_[E3B], 128, act_[E2B], H2, W2, gB_, gA_);  // gA = d u2 (224 @H2)
-  dn_upcat_bwd(gA_, gB_, gs2_, N, H2, W2, 128, 96, false, s);  // gB = d e3b (128 @H3), gs2 = d e2b
-  layer(E3B, nullptr, 0, act_[E3A], H3, W3, gB_, gA_);
-  layer(E3A, nullptr, 0, p2_, H3, W3, gA_, gB_);  // gB = d p2 (96 @H3)
-  dn_pool_bwd(gB_, gs2_, N, H2, W2, 96, true, s);  // gs2 += pool backward
-  layer(E2B, nullptr, 0, act_[E2A], H2, W2, gs2_, gA_);
-  layer(E2A, nullptr, 0, p1_, H2, W2, gA_, gB_);  // gB = d p1 (64 @H2)
-  dn_pool_bwd(gB_, gs1_, N, H1, W1, 64, true, s);
-  layer(E1B, nullptr, 0, act_[E1A], H1, W1, gs1_, gA_);
-  layer(E1A, nullptr, 0, p0_, H1, W1, gA_, gB_);  // gB = d p0 (32 @H1)
-  dn_pool_bwd(gB_, gs0_, N, H, W, 32, true, s);
-  layer(E0B, nullptr, 0, act_[E0A], H, W, gs0_, gA_);
-  layer(E0A, nullptr, 0, x_, H, W, gA_, nullptr);  // the input gradient of the network is not needed
+  const auto plain = [](const float* g) { return DnGrad{kGradPlain, g}; };
+  // the coarse and the skip share of a concatenated input's gradient (the skip tensor was
+  // pooled as well)
+  const auto up = [](const float* g, int gc) { return DnGrad{kGradUp, g, gc, 0}; };
+  const auto skip = [](const float* g, int gc, int c0, const float* pooled) { return DnGrad{kGradSkip, g, gc, c0, pooled}; };
+  layer(OUT, nullptr, 0, act_[D0B], H, W, plain(dout), gA_);
+  layer(D0B, nullptr, 0, act_[D0A], H, W, plain(gA_), gB_);
+  layer(D0A, act_[D1B], 64, act_[E0B], H, W, plain(gB_), gu0_);  // d [up d1b (64) | e0b (32)]
+  layer(D1B, nullptr, 0, act_[D1A], H1, W1, up(gu0_, 96), gA_);
+  layer(D1A, act_[D2B], 96, act_[E1B], H1, W1, plain(gA_), gu1_);  // d [up d2b (96) | e1b (64)]
+  layer(D2B, nullptr, 0, act_[D2A], H2, W2, up(gu1_, 160), gA_);
+  layer(D2A, act_[E3B], 128, act_[E2B], H2, W2, plain(gA_), gu2_);  // d [up e3b (128) | e2b (96)]
+  layer(E3B, nullptr, 0, act_[E3A], H3, W3, up(gu2_, 224), gA_);
+  layer(E3A, nullptr, 0, p2_, H3, W3, plain(gA_), gB_);  // gB = d p2 (96 @H3)
+  layer(E2B, nullptr, 0, act_[E2A], H2, W2, skip(gu2_, 224, 128, gB_), gA_);
+  layer(E2A, nullptr, 0, p1_, H2, W2, plain(gA_), gB_);  // gB = d p1 (64 @H2)
+  layer(E1B, nullptr, 0, act_[E1A], H1, W1, skip(gu1_, 160, 96, gB_), gA_);
+  layer(E1A, nullptr, 0, p0_, H1, W1, plain(gA_), gB_);  // gB = d p0 (32 @H1)
+  layer(E0B, nullptr, 0, act_[E0A], H, W, skip(gu0_, 96, 64, gB_), gA_);
+  layer(E0A, nullptr, 0, x_, H, W, plain(gA_), nullptr);  // the input gradient of the network is not needed
   return hipGetLastError();
 }
 
@@ -262,9 +264,7 @@ hipError_t Unet::train_step(const uint16_t* x, const float* target, int N, int H
   ++t_;
   const float b1 = 0.9f, b2 = 0.999f;
   const float c1 = 1.f - std::pow(b1, float(t_)), c2 = 1.f - std::pow(b2, float(t_));
-  dn_adam(w_, m_, v_, g_, wb_, nullptr, n_params_, lr, b1, b2, c1, c2, 1e-8f, s);
-  for (size_t li = 1; li < convs_.size(); ++li)
-    dn_flip_weights(wb_ + convs_[li].woff, wd_ + convs_[li].woff, convs_[li].cin, convs_[li].cout, s);
+  dn_adam(w_, m_, v_, g_, wb_, wd_, table_, n_params_, lr, b1, b2, c1, c2, 1e-8f, s);
   std::vector<float> lp(static_cast<size_t>(nb));
   if ((e = hipMemcpyAsync(lp.data(), lpart_, size_t(nb) * 4, hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
   if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;

@@ -39,17 +39,24 @@ struct DnConv {
 bool dn_conv(const DnConv& c, hipStream_t s);
 bool dn_conv3x3(const uint16_t* X, const uint16_t* Wt, const float* bias, void* Y, int N, int H, int W, int Cin,
                 int Cout, bool relu, bool out_f32, hipStream_t s);
-int dn_wgrad_chunks(int N, int H, int W, int tiles_per_chunk);
-void dn_wgrad(const uint16_t* X, const uint16_t* coarse, int c1, const uint16_t* dZ, float* partial, float* dW, int N,
-              int H, int W, int Cin, int Cout, int tiles_per_chunk, hipStream_t s);
-// dZ = bf16(dY masked by Y > 0; Y null: no mask) and its per-channel sums db (C <= 128,
-// C % 8 == 0; partial: kBiasBlocks x C)
-void dn_relu_bias_bwd(const float* dY, const uint16_t* Y, uint16_t* dZ, size_t P, int C, float* partial, float* db,
-                      hipStream_t s);
-void dn_to_bf16(const float* a, uint16_t* b, size_t n, hipStream_t s);
-void dn_pool_bwd(const float* dY, float* dX, int N, int H, int W, int C, bool accumulate, hipStream_t s);
-void dn_upcat_bwd(const float* dout, float* dcoarse, float* dskip, int N, int H, int W, int C1, int C2,
-                  bool accumulate_skip, hipStream_t s);
+// 8x16 pixel tiles per partial sum of the weight gradient (fixes the order of its additions)
+constexpr int kWgradTiles = 8;
+int dn_wgrad_chunks(int N, int H, int W);
+// Where a layer's output gradient comes from (k_relu_bias).
+enum DnGradKind { kGradPlain = 0, kGradUp = 1, kGradSkip = 2 };
+struct DnGrad {
+  int kind;
+  const float* g;
+  int gc = 0, c0 = 0;             // kGradUp, kGradSkip: channels of g, first of this tensor's share
+  const float* pooled = nullptr;  // kGradSkip
+};
+// One layer's backward but for the input gradient: dZ = bf16(gradient masked by Y > 0; Y
+// null: no mask), the bias gradient db = its per-channel sums, the weight gradient dW.
+// Cout <= 128, a multiple of 32; wpartial: dn_wgrad_chunks x Cout x 9 x Cin; bpartial:
+// kBiasBlocks x Cout.
+void dn_layer_bwd(const DnGrad& grad, const uint16_t* Y, const uint16_t* X, const uint16_t* coarse, int c1, uint16_t* dZ,
+                  int N, int H, int W, int Cin, int Cout, float* wpartial, float* bpartial, float* dW, float* db,
+                  hipStream_t s);
 void dn_features(const float4* color, const float4* albedo, const float4* normal, uint16_t* out, size_t P,
                  hipStream_t s);
 void dn_target(const float4* color, float* out, size_t P, hipStream_t s);
@@ -58,9 +65,14 @@ void dn_blend(float4* den, const float4* color, float b, size_t P, hipStream_t s
 void dn_gather_crop(const uint16_t* feat, const float* tgt, int Hs, int Ws, const int4* crops, int B, int S,
                     uint16_t* fo, float* to, hipStream_t s);
 int dn_loss(const float* Y, const uint16_t* X, const float* T, size_t P, float* dY, float* partial, hipStream_t s);
-void dn_adam(float* w, float* m, float* v, const float* g, uint16_t* wb, const uint8_t* mask, size_t n, float lr,
-             float b1, float b2, float c1, float c2, float eps, hipStream_t s);
-void dn_flip_weights(const uint16_t* w, uint16_t* wd, int cin, int cout, hipStream_t s);
+// The layers that have a flipped weight copy: parameter offset and channels.
+struct WeightTable {
+  int n;
+  int off[16], cin[16], cout[16];
+};
+void dn_adam(float* w, float* m, float* v, const float* g, uint16_t* wb, uint16_t* wd, const WeightTable& table, size_t n,
+             float lr, float b1, float b2, float c1, float c2, float eps, hipStream_t s);
+void dn_weights_bf16(const float* w, uint16_t* wb, uint16_t* wd, const WeightTable& table, size_t n, hipStream_t s);
 
 // Network: 4-level U-Net, 32/64/96/128 channels, 3x3 convolutions with ReLU, 2x2
 // average pooling, nearest upsampling + skip concatenation, a final 3x3 convolution to
@@ -101,9 +113,10 @@ class Unet {
   uint32_t adam_steps() const { return t_; }
 
  private:
-  hipError_t ensure(int N, int H, int W);
+  hipError_t ensure(int N, int H, int W, hipStream_t s);
   void free_acts();
   std::vector<Conv> convs_;
+  WeightTable table_{};
   size_t n_params_ = 0;
   float *w_ = nullptr, *m_ = nullptr, *v_ = nullptr, *g_ = nullptr;  // fp32 master, Adam moments, grads
   uint16_t *wb_ = nullptr, *wd_ = nullptr;                              // bf16 weights, flipped for dgrad
@@ -114,7 +127,7 @@ class Unet {
   bool have_output_ = false;  // out_ holds the last forward's output
   const uint16_t* x_ = nullptr;  // input of the last forward (read by the first layer's wgrad)
   // backward scratch
-  float *gA_ = nullptr, *gB_ = nullptr, *gs0_ = nullptr, *gs1_ = nullptr, *gs2_ = nullptr, *dout_ = nullptr;
+  float *gA_ = nullptr, *gB_ = nullptr, *gu0_ = nullptr, *gu1_ = nullptr, *gu2_ = nullptr, *dout_ = nullptr;
   uint16_t* dz_ = nullptr;
   float *wpart_ = nullptr, *bpart_ = nullptr, *lpart_ = nullptr;
   size_t wpart_elems_ = 0;

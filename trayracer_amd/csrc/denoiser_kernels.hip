@@ -435,8 +435,8 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
 // ------------------------------------------------------------------------------------
 // Weight gradient: dW[co][tap][ci] = sum_p dZ[p][co] X[p + s(tap)][ci] (X optionally
 // [upsample(coarse) | X] as in the forward convolution), as an MFMA GEMM
-// with M = co (32-block), N = ci (32-block), K = pixels. Each workgroup covers `tiles`
-// consecutive 8x16 pixel tiles of one image row band and writes its partial sums to
+// with M = co (32-block), N = ci (32-block), K = pixels. Each workgroup covers kWgradTiles
+// consecutive 8x16 pixel tiles and writes its partial sums to
 // partial[chunk][co][tap][ci]; a fixed-order reduction over chunks follows.
 // Grid: (n_chunks, Cout/32 * ceil(Cin/32)); wave w handles the taps of kernel row w.
 //
@@ -445,18 +445,21 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
 // pixels (16 bytes each), exchanges halves in registers and writes eight 8-byte runs of
 // pixels to LDS as [channel][row][pixel]. A wave then reads one aligned run of ten pixels of
 // an input row and forms the three horizontally shifted fragments of its kernel row from it
-// in registers. The next tile's loads are issued before the current tile's MFMAs. (Element by
-// element staging took 220 us a layer on average at 8 x 128 x 128, 24 us now.)
+// in registers. The loads of the next kWgAhead tiles are in flight while a tile is
+// multiplied: training crops leave at most a block per CU, so a chunk's time is its tiles'
+// load latency. (Element by element staging took 220 us a layer on average at 8 x 128 x 128;
+// one tile ahead, through loads in branches, 24 us; now 16 us.)
 constexpr int kWgThreads = 192;
+constexpr int kWgAhead = 3;                   // tiles whose loads are in flight
 constexpr int kWgRow = 24;                    // LDS pixels per staged input row (18 used)
 constexpr int kWgXs = kPatchH * kWgRow + 8;   // bf16 per channel: an odd number of 16-byte slots
 constexpr int kWgZs = kTileH * kTileW + 8;
-constexpr int kWgXItems = kPatchH * 5 * 4, kWgZItems = kTileH * 4 * 4;  // rows x pixel quads x channel octets
-constexpr int kWgItems = (kWgXItems + kWgZItems + kWgThreads - 1) / kWgThreads;
+constexpr int kWgXItems = kPatchH * 5 * 4;    // rows x pixel quads x channel octets (dZ: 8 x 4 x 4 = 128)
+constexpr int kWgItems = 2;                   // per thread
 
 __global__ __launch_bounds__(kWgThreads) void k_wgrad(const uint16_t* __restrict__ X, const uint16_t* __restrict__ coarse,
                                                       int c1, const uint16_t* __restrict__ dZ, float* __restrict__ partial,
-                                                      int N, int H, int W, int Cin, int Cout, int tiles_per_chunk) {
+                                                      int N, int H, int W, int Cin, int Cout) {
   __shared__ __align__(16) uint16_t xs[32 * kWgXs];  // [ci][row][pixel]
   __shared__ __align__(16) uint16_t zs[32 * kWgZs];  // [co][row][pixel]
   const int tid = threadIdx.x, lane = tid & 63, ky = tid >> 6;
@@ -464,62 +467,71 @@ __global__ __launch_bounds__(kWgThreads) void k_wgrad(const uint16_t* __restrict
   const int cb = blockIdx.y / ci_blocks, ib = blockIdx.y - cb * ci_blocks;
   const int tiles_x = W / kTileW, tiles_y = (H + kTileH - 1) / kTileH;
   const int tiles_img = tiles_x * tiles_y;
-  const int first = blockIdx.x * tiles_per_chunk;
-  const int last = min(first + tiles_per_chunk, tiles_img * N);
+  const int first = blockIdx.x * kWgradTiles;
+  const int last = min(first + kWgradTiles, tiles_img * N);
   const bool up = ib * 32 < c1;  // this input block comes from the upsampled coarse tensor
   const int cx = Cin - c1;
-  // fixed per thread: which quad of pixels and octet of channels each item stages, and where
-  int iy[kWgItems], ix[kWgItems], ic[kWgItems], to[kWgItems];
+  // Two items per thread (a quad of pixels, an octet of channels): item 0 of the input patch,
+  // item 1 of dZ (waves 0 and 1) or the rest of the patch (wave 2). Every thread issues the
+  // same eight buffer loads on every tile, padding and idle ones past the buffer's end (they
+  // return zero): with loads in branches the wait before a tile's stores could not tell how
+  // many later ones are in flight and drained them all.
+  constexpr int kOOB = 0x7fffffff;
+  int py[kWgItems], px[kWgItems], rel[kWgItems][4], to[kWgItems];  // first pixel, byte offsets from the tile's corner, place in LDS
+  const bool z1 = __builtin_amdgcn_readfirstlane(ky) < 2;          // item 1 is one of dZ
+  bool have[kWgItems];
 #pragma unroll
   for (int k = 0; k < kWgItems; ++k) {
-    const int i = tid + k * kWgThreads, part = i & 3;
-    if (i < kWgXItems) {
-      const int g = i >> 2, row = g / 5, quad = g - row * 5;
-      iy[k] = row - 1;
-      ix[k] = quad * 4 - 1;
-      ic[k] = part * 8;
-      to[k] = part * 8 * kWgXs + row * kWgRow + quad * 4;
-    } else {
-      const int g = (i - kWgXItems) >> 2, row = g >> 2, quad = g & 3;
-      iy[k] = row;
-      ix[k] = quad * 4;
-      ic[k] = part * 8;
-      to[k] = part * 8 * kWgZs + row * kTileW + quad * 4;
+    const bool z = k == 1 && z1;
+    const int i = k == 0 || z ? tid : kWgThreads + tid - 128;  // of the patch or of dZ
+    const int part = i & 3, g = i >> 2, quads = z ? 4 : 5;
+    const int row = g / quads, quad = g - row * quads;
+    have[k] = z ? true : i < kWgXItems && ib * 32 + part * 8 < Cin;
+    py[k] = z ? row : row - 1;
+    px[k] = z ? quad * 4 : quad * 4 - 1;
+    to[k] = i < kWgXItems ? part * 8 * (z ? kWgZs : kWgXs) + row * (z ? kTileW : kWgRow) + quad * 4 : -1;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int y = py[k], x = px[k] + q;
+      rel[k][q] = z    ? (y * W + x) * Cout * 2 + part * 16
+                  : up ? ((y >> 1) * (W >> 1) + (x >> 1)) * c1 * 2 + part * 16
+                       : (y * W + x) * cx * 2 + part * 16;
     }
   }
-  u32x4 stage[kWgItems][4];
-  auto load_tile = [&](int tile) __attribute__((always_inline)) {
+  const int x_bytes = up ? (H >> 1) * (W >> 1) * c1 * 2 : H * W * cx * 2, z_bytes = H * W * Cout * 2;
+  u32x4 stage[kWgAhead][kWgItems][4];
+  auto load_tile = [&](u32x4(&stage)[kWgItems][4], int tile) __attribute__((always_inline)) {
     const int n = tile / tiles_img, tr = tile - n * tiles_img;
     const int ty = tr / tiles_x, y0 = ty * kTileH, x0 = (tr - ty * tiles_x) * kTileW;
+    const uint16_t* xb = up ? coarse + static_cast<size_t>(n) * (H >> 1) * (W >> 1) * c1 + ib * 32
+                            : X + static_cast<size_t>(n) * H * W * cx + (ib * 32 - c1);
+    const __amdgpu_buffer_rsrc_t rx =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(xb), static_cast<short>(0), x_bytes, kBufFlags);
+    const __amdgpu_buffer_rsrc_t rz = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(dZ) + static_cast<size_t>(n) * H * W * Cout + cb * 32, static_cast<short>(0), z_bytes, kBufFlags);
+    const int xc = up ? ((y0 >> 1) * (W >> 1) + (x0 >> 1)) * c1 * 2 : (y0 * W + x0) * cx * 2;
+    const int zc = (y0 * W + x0) * Cout * 2;
 #pragma unroll
     for (int k = 0; k < kWgItems; ++k) {
-      const int i = tid + k * kWgThreads;
-      const bool is_x = i < kWgXItems;
-      const int yy = y0 + iy[k];
+      const bool row_ok = have[k] && static_cast<unsigned>(y0 + py[k]) < static_cast<unsigned>(H);
+      const int corner = k == 1 && z1 ? zc : xc;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int xx = x0 + ix[k] + q;
-        stage[k][q] = u32x4{0u, 0u, 0u, 0u};
-        if (static_cast<unsigned>(yy) >= static_cast<unsigned>(H) || static_cast<unsigned>(xx) >= static_cast<unsigned>(W)) continue;
-        if (is_x) {
-          if (ix[k] + q > kTileW || ib * 32 + ic[k] >= Cin) continue;
-          const uint16_t* src =
-              up ? coarse + ((static_cast<size_t>(n) * (H >> 1) + (yy >> 1)) * (W >> 1) + (xx >> 1)) * c1 + ib * 32 + ic[k]
-                 : X + ((static_cast<size_t>(n) * H + yy) * W + xx) * cx + (ib * 32 - c1) + ic[k];
-          stage[k][q] = *reinterpret_cast<const u32x4*>(src);
-        } else if (i < kWgXItems + kWgZItems) {
-          stage[k][q] = *reinterpret_cast<const u32x4*>(dZ + ((static_cast<size_t>(n) * H + yy) * W + xx) * Cout + cb * 32 + ic[k]);
-        }
+        const int x = px[k] + q;
+        const bool ok = row_ok && x <= kTileW && static_cast<unsigned>(x0 + x) < static_cast<unsigned>(W);
+        const int off = ok ? corner + rel[k][q] : kOOB;
+        stage[k][q] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(k == 1 && z1 ? rz : rx, off, 0, 0));
       }
     }
   };
-  auto store_tile = [&]() __attribute__((always_inline)) {
+  auto store_tile = [&](const u32x4(&stage)[kWgItems][4]) __attribute__((always_inline)) {
 #pragma unroll
     for (int k = 0; k < kWgItems; ++k) {
-      const int i = tid + k * kWgThreads;
-      if (i >= kWgXItems + kWgZItems) continue;
-      uint16_t* dst = i < kWgXItems ? xs + to[k] : zs + to[k];
-      const int pitch = i < kWgXItems ? kWgXs : kWgZs;
+      const bool z = k == 1 && z1;
+      if (to[k] < 0) continue;
+      uint16_t* dst = (z ? zs : xs) + to[k];
+      const int pitch = z ? kWgZs : kWgXs;
 #pragma unroll
       for (int c = 0; c < 4; ++c) {  // channels 2c, 2c + 1 in the halves of dword c
         uint2 lo, hi;
@@ -536,12 +548,16 @@ __global__ __launch_bounds__(kWgThreads) void k_wgrad(const uint16_t* __restrict
   const int khalf = (lane >> 5) * 8;
   const uint16_t* zrow = zs + (lane & 31) * kWgZs + khalf;
   const uint16_t* xrow = xs + (lane & 31) * kWgXs + ky * kWgRow + khalf;
-  if (first < last) load_tile(first);
-  for (int tile = first; tile < last; ++tile) {
+#pragma unroll
+  for (int t = 0; t < kWgAhead; ++t)
+    if (first + t < last) load_tile(stage[t], first + t);
+#pragma unroll
+  for (int t = 0; t < kWgradTiles; ++t) {
+    if (first + t >= last) break;
     __syncthreads();
-    store_tile();
+    store_tile(stage[t % kWgAhead]);
     __syncthreads();
-    if (tile + 1 < last) load_tile(tile + 1);
+    if (t + kWgAhead < kWgradTiles && first + t + kWgAhead < last) load_tile(stage[t % kWgAhead], first + t + kWgAhead);
 #pragma unroll
     for (int row = 0; row < kTileH; ++row) {  // K-step = 16 pixels of one tile row
       const bf16x8 a = *reinterpret_cast<const bf16x8*>(zrow + row * kTileW);
@@ -573,51 +589,103 @@ __global__ __launch_bounds__(kWgThreads) void k_wgrad(const uint16_t* __restrict
 // threads bring 128 chunks at a time into LDS with all loads in flight, then 32 threads add
 // them in order (one thread per output with its loads in a row was bound by their latency:
 // 36 us a layer on average at 8 x 128 x 128, 6.5 us now).
+// Two sums in one launch: blocks below `blocks_a` reduce the first.
 constexpr int kReduceOuts = 32, kReduceChunks = 128;
-__global__ __launch_bounds__(256) void k_reduce_chunks(const float* __restrict__ partial, int n_chunks, size_t n,
-                                                       float* __restrict__ out) {
+struct ChunkSum {
+  const float* partial;
+  int n_chunks;
+  size_t n;
+  float* out;
+};
+__global__ __launch_bounds__(256) void k_reduce_chunks(ChunkSum sa, ChunkSum sb, unsigned blocks_a) {
   __shared__ float lds[kReduceChunks * kReduceOuts];
+  const ChunkSum r = blockIdx.x < blocks_a ? sa : sb;
+  const unsigned block = blockIdx.x < blocks_a ? blockIdx.x : blockIdx.x - blocks_a;
   const int o = threadIdx.x & (kReduceOuts - 1), part = threadIdx.x / kReduceOuts;
-  const size_t i = static_cast<size_t>(blockIdx.x) * kReduceOuts + o;
+  const size_t i = static_cast<size_t>(block) * kReduceOuts + o;
   float t = 0.f;
-  for (int c0 = 0; c0 < n_chunks; c0 += kReduceChunks) {
-    const int m = min(kReduceChunks, n_chunks - c0);
+  for (int c0 = 0; c0 < r.n_chunks; c0 += kReduceChunks) {
+    const int m = min(kReduceChunks, r.n_chunks - c0);
     float v[kReduceChunks / 8];
 #pragma unroll
     for (int k = 0; k < kReduceChunks / 8; ++k) {
       const int c = part + 8 * k;
-      v[k] = c < m && i < n ? partial[static_cast<size_t>(c0 + c) * n + i] : 0.f;
+      v[k] = c < m && i < r.n ? r.partial[static_cast<size_t>(c0 + c) * r.n + i] : 0.f;
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kReduceChunks / 8; ++k) lds[(part + 8 * k) * kReduceOuts + o] = v[k];
     __syncthreads();
-    if (part == 0)
-      for (int c = 0; c < m; ++c) t += lds[c * kReduceOuts + o];
+    if (part == 0) {
+      int c = 0;
+      for (; c + 8 <= m; c += 8) {
+        float u[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) u[k] = lds[(c + k) * kReduceOuts + o];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) t += u[k];
+      }
+      for (; c < m; ++c) t += lds[c * kReduceOuts + o];
+    }
   }
-  if (part == 0 && i < n) out[i] = t;
+  if (part == 0 && i < r.n) r.out[i] = t;
 }
 
 // dZ = bf16(dY * (Y > 0)) (ReLU backward; Y is the post-activation output, null for a
 // linear layer) and the bias gradient's partial sums: block b takes pixels
-// [b*P/B, (b+1)*P/B), 64 at a time, stages their dZ in LDS and adds it per channel in pixel
-// order. Bound by its 8 bytes a value (as two kernels the sums re-read dZ with C threads a
-// block: 40 + 7 us a layer on average at 8 x 128 x 128, 9 us now).
-constexpr int kBiasPixels = 64, kBiasMaxChannels = 128;
-__global__ __launch_bounds__(256) void k_relu_bias(const float* __restrict__ dY, const uint16_t* __restrict__ Y,
+// [b*P/B, (b+1)*P/B), stages their dZ in LDS and adds it per channel in pixel order. Bound by
+// its 8 bytes a value. (As two kernels the sums re-read dZ with C threads a block: 40 + 7 us
+// a layer on average at 8 x 128 x 128, plus 6 launches that wrote the gathered gradients; now
+// 11 us and none.)
+// dY is formed on the way from what the layers above left:
+//   kGradPlain  gradient of this tensor
+//   kGradUp     gradient g of [upsample(this) | skip] at twice the side: the 2x2 sum
+//   kGradSkip   this tensor's skip share of such a gradient g, plus a quarter of the
+//               gradient `pooled` of its 2x2 pooling
+constexpr int kBiasElems = 16384;  // bf16 staged at a time
+struct GradSrc {
+  const float* g;
+  const float* pooled;  // kGradSkip
+  int kind;
+  int H, W;    // of this tensor
+  int gc, c0;  // channels of g, first channel of this tensor's share
+};
+__device__ __forceinline__ float4 add4(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
+// p: pixel over all images (below 2^31: a gradient tensor of that many would not fit the GPU)
+__device__ __forceinline__ float4 grad4(const GradSrc& s, int C, unsigned p, int c) {
+  if (s.kind == kGradPlain) return *reinterpret_cast<const float4*>(s.g + static_cast<size_t>(p) * C + c);
+  const unsigned W = static_cast<unsigned>(s.W);
+  const size_t row = p / W;  // over all images
+  const unsigned x = p % W;
+  if (s.kind == kGradUp) {
+    const float* q = s.g + (2 * row * 2 * W + 2 * x) * s.gc + c;
+    const size_t down = static_cast<size_t>(2 * W) * s.gc;
+    return add4(add4(*reinterpret_cast<const float4*>(q), *reinterpret_cast<const float4*>(q + s.gc)),
+                add4(*reinterpret_cast<const float4*>(q + down), *reinterpret_cast<const float4*>(q + down + s.gc)));
+  }
+  const float4 k = *reinterpret_cast<const float4*>(s.g + static_cast<size_t>(p) * s.gc + s.c0 + c);
+  // H is even: the rows of an image pair up
+  const float4 h = *reinterpret_cast<const float4*>(s.pooled + ((row >> 1) * (W >> 1) + (x >> 1)) * C + c);
+  return make_float4(k.x + 0.25f * h.x, k.y + 0.25f * h.y, k.z + 0.25f * h.z, k.w + 0.25f * h.w);
+}
+
+__global__ __launch_bounds__(256) void k_relu_bias(GradSrc src, const uint16_t* __restrict__ Y,
                                                    uint16_t* __restrict__ dZ, size_t P, int C,
                                                    float* __restrict__ partial) {
-  __shared__ __align__(16) uint16_t lds[kBiasPixels * kBiasMaxChannels];
+  __shared__ __align__(16) uint16_t lds[kBiasElems];
   const size_t p0 = P * blockIdx.x / gridDim.x, p1 = P * (blockIdx.x + 1) / gridDim.x;
+  const int pixels = kBiasElems / C, octets = C / 8;
   float t = 0.f;
-  for (size_t p = p0; p < p1; p += kBiasPixels) {
-    const int m = static_cast<int>(p1 - p < kBiasPixels ? p1 - p : kBiasPixels);
-    const int octets = m * C / 8;
+  for (size_t p = p0; p < p1; p += pixels) {
+    const int m = static_cast<int>(p1 - p < static_cast<size_t>(pixels) ? p1 - p : pixels);
     __syncthreads();
-    for (int i = threadIdx.x; i < octets; i += 256) {
-      const size_t at = p * C + static_cast<size_t>(i) * 8;
-      const float4 g0 = *reinterpret_cast<const float4*>(dY + at), g1 = *reinterpret_cast<const float4*>(dY + at + 4);
+#pragma unroll 4
+    for (int i = threadIdx.x; i < m * octets; i += 256) {
+      const int q = static_cast<int>(static_cast<unsigned>(i) / static_cast<unsigned>(octets)), c = (i - q * octets) * 8;
+      const unsigned pq = static_cast<unsigned>(p) + static_cast<unsigned>(q);
+      const float4 g0 = grad4(src, C, pq, c), g1 = grad4(src, C, pq, c + 4);
       const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+      const size_t at = (p + q) * C + c;
       u32x4 y = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};  // ones
       if (Y) y = *reinterpret_cast<const u32x4*>(Y + at);
       u32x4 z;
@@ -631,60 +699,19 @@ __global__ __launch_bounds__(256) void k_relu_bias(const float* __restrict__ dY,
       *reinterpret_cast<u32x4*>(lds + i * 8) = z;
     }
     __syncthreads();
-    if (static_cast<int>(threadIdx.x) < C)
-      for (int q = 0; q < m; ++q) t += bf2f(lds[q * C + threadIdx.x]);
+    if (static_cast<int>(threadIdx.x) < C) {
+      int q = 0;
+      for (; q + 16 <= m; q += 16) {
+        float u[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) u[k] = bf2f(lds[(q + k) * C + threadIdx.x]);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) t += u[k];
+      }
+      for (; q < m; ++q) t += bf2f(lds[q * C + threadIdx.x]);
+    }
   }
   if (static_cast<int>(threadIdx.x) < C) partial[static_cast<size_t>(blockIdx.x) * C + threadIdx.x] = t;
-}
-
-__global__ void k_to_bf16(const float* __restrict__ a, uint16_t* __restrict__ b, size_t n) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) b[i] = f2bf(a[i]);
-}
-
-// dX (fine, fp32) (+)= dY(coarse)/4 broadcast; accumulate selects += vs =
-__global__ void k_pool_bwd(const float* __restrict__ dY, float* __restrict__ dX, int N, int H, int W, int C,
-                           int accumulate) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const size_t total = static_cast<size_t>(N) * H * W * C;
-  if (i >= total) return;
-  const int c = static_cast<int>(i % C);
-  size_t r = i / C;
-  const int x = static_cast<int>(r % W);
-  r /= W;
-  const int y = static_cast<int>(r % H);
-  const int n = static_cast<int>(r / H);
-  const float g = 0.25f * dY[((static_cast<size_t>(n) * (H / 2) + y / 2) * (W / 2) + x / 2) * C + c];
-  dX[i] = accumulate ? dX[i] + g : g;
-}
-
-// coarse gradient: d_coarse[n][y][x][c] = sum of the 2x2 fine gradients of channel c < C1
-__global__ void k_upcat_bwd_coarse(const float* __restrict__ dout, float* __restrict__ dcoarse, int N, int Hc,
-                                   int Wc, int C1, int C2) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const size_t total = static_cast<size_t>(N) * Hc * Wc * C1;
-  if (i >= total) return;
-  const int C = C1 + C2;
-  const int c = static_cast<int>(i % C1);
-  size_t r = i / C1;
-  const int x = static_cast<int>(r % Wc);
-  r /= Wc;
-  const int y = static_cast<int>(r % Hc);
-  const int n = static_cast<int>(r / Hc);
-  const int W = 2 * Wc;
-  const size_t b = ((static_cast<size_t>(n) * 2 * Hc + 2 * y) * W + 2 * x) * C + c;
-  dcoarse[i] = (dout[b] + dout[b + C]) + (dout[b + static_cast<size_t>(W) * C] + dout[b + static_cast<size_t>(W) * C + C]);
-}
-
-// skip gradient: dskip (+)= dout[..][C1 + c]
-__global__ void k_upcat_bwd_skip(const float* __restrict__ dout, float* __restrict__ dskip, size_t P, int C1, int C2,
-                                 int accumulate) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= P * C2) return;
-  const size_t p = i / C2;
-  const int c = static_cast<int>(i % C2);
-  const float g = dout[p * (C1 + C2) + C1 + c];
-  dskip[i] = accumulate ? dskip[i] + g : g;
 }
 
 // Input features (16 channels, 10 used): log(1+radiance) rgb, albedo rgb (clamped to
@@ -755,7 +782,8 @@ __global__ void k_gather_crop(const uint16_t* __restrict__ feat, const float* __
 // L1 loss in log space. The network predicts a correction added to the noisy input
 // (feature channels 0..2 = log(1 + radiance)): prediction = x + y over the first 3 of
 // 32 output channels. Partial sums of |x + y - t| per block and dOut = sign(x + y - t) /
-// (3 P) (zero on padding channels). L1 keeps the firefly pixels of many-emitter scenes
+// (3 P); the padding channels of dOut stay zero as allocated (writing them too was most of
+// the kernel's traffic). L1 keeps the firefly pixels of many-emitter scenes
 // from dominating the gradient (with an L2 loss the network trained on the soup and the
 // instanced scene reached relMSE 0.0125 at 8 spp on a held-out soup view; with L1,
 // 0.0085).
@@ -766,15 +794,13 @@ __global__ void k_loss(const float* __restrict__ Y, const uint16_t* __restrict__
   float l = 0.f;
   if (p < P) {
     const float inv = 1.f / (3.f * static_cast<float>(P));
-    for (int c = 0; c < 32; ++c) {
-      float g = 0.f;
-      if (c < 3) {
-        const float d = (bf2f(X[p * 16 + c]) + Y[p * 32 + c]) - T[p * 3 + c];
-        l += fabsf(d);
-        g = (d > 0.f ? inv : (d < 0.f ? -inv : 0.f));
-      }
-      dY[p * 32 + c] = g;
+    float g[3];
+    for (int c = 0; c < 3; ++c) {
+      const float d = (bf2f(X[p * 16 + c]) + Y[p * 32 + c]) - T[p * 3 + c];
+      l += fabsf(d);
+      g[c] = (d > 0.f ? inv : (d < 0.f ? -inv : 0.f));
     }
+    *reinterpret_cast<float4*>(dY + p * 32) = make_float4(g[0], g[1], g[2], 0.f);
   }
   red[threadIdx.x] = l;
   __syncthreads();
@@ -785,14 +811,26 @@ __global__ void k_loss(const float* __restrict__ Y, const uint16_t* __restrict__
   if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-// Adam (Kingma & Ba 2015) on fp32 master weights; bf16 copy refreshed; `mask` zeroes
-// updates of padding entries (nullable)
+// The data-gradient convolution is a 3x3 convolution of dZ with the spatially flipped,
+// channel-transposed kernel Wd[ci][tap][co] = W[co][8 - tap][ci]: where parameter i of the
+// network goes in the flipped copy (-1: a bias, or a layer without one).
+__device__ __forceinline__ int flipped_index(const WeightTable& t, int i) {
+  for (int l = 0; l < t.n; ++l) {
+    const int r = i - t.off[l], k = 9 * t.cin[l];
+    if (r < 0 || r >= k * t.cout[l]) continue;
+    const int co = r / k, tap = (r - co * k) / t.cin[l], ci = r - co * k - tap * t.cin[l];
+    return t.off[l] + (ci * 9 + (8 - tap)) * t.cout[l] + co;
+  }
+  return -1;
+}
+
+// Adam (Kingma & Ba 2015) on fp32 master weights; the bf16 copy and the flipped bf16 copy
+// are refreshed in the same pass (a launch per layer for the flips cost 3 us each).
 __global__ void k_adam(float* __restrict__ w, float* __restrict__ m, float* __restrict__ v, const float* __restrict__ g,
-                       uint16_t* __restrict__ wb, const uint8_t* __restrict__ mask, size_t n, float lr, float b1,
-                       float b2, float c1, float c2, float eps) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+                       uint16_t* __restrict__ wb, uint16_t* __restrict__ wd, WeightTable table, int n, float lr,
+                       float b1, float b2, float c1, float c2, float eps) {
+  const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
   if (i >= n) return;
-  if (mask && !mask[i]) return;
   const float gi = g[i];
   const float mi = b1 * m[i] + (1.f - b1) * gi;
   const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
@@ -800,19 +838,21 @@ __global__ void k_adam(float* __restrict__ w, float* __restrict__ m, float* __re
   v[i] = vi;
   const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
   w[i] = wi;
-  if (wb) wb[i] = f2bf(wi);
+  const uint16_t h = f2bf(wi);
+  wb[i] = h;
+  const int f = flipped_index(table, i);
+  if (f >= 0) wd[f] = h;
 }
 
-// Wd[ci][tap][co] = W[co][8 - tap][ci]: the data-gradient convolution is a 3x3
-// convolution of dZ with the spatially flipped, channel-transposed kernel
-__global__ void k_flip(const uint16_t* __restrict__ w, uint16_t* __restrict__ wd, int cin, int cout) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const size_t n = static_cast<size_t>(cin) * 9 * cout;
+// bf16 copies of the weights (plain and flipped) without an update
+__global__ void k_weights_bf16(const float* __restrict__ w, uint16_t* __restrict__ wb, uint16_t* __restrict__ wd,
+                               WeightTable table, int n) {
+  const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
   if (i >= n) return;
-  const int ci = static_cast<int>(i / (9 * cout));
-  const int r = static_cast<int>(i % (9 * cout));
-  const int tap = r / cout, co = r % cout;
-  wd[i] = w[(static_cast<size_t>(co) * 9 + (8 - tap)) * cin + ci];
+  const uint16_t h = f2bf(w[i]);
+  wb[i] = h;
+  const int f = flipped_index(table, i);
+  if (f >= 0) wd[f] = h;
 }
 
 inline unsigned blocks_for(size_t n, unsigned b = 256) { return static_cast<unsigned>((n + b - 1) / b); }
@@ -927,41 +967,25 @@ bool dn_conv3x3(const uint16_t* X, const uint16_t* Wt, const float* bias, void* 
   return dn_conv(c, s);
 }
 
-int dn_wgrad_chunks(int N, int H, int W, int tiles_per_chunk) {
+int dn_wgrad_chunks(int N, int H, int W) {
   const int tiles = (W / kTileW) * ((H + kTileH - 1) / kTileH) * N;
-  return (tiles + tiles_per_chunk - 1) / tiles_per_chunk;
+  return (tiles + kWgradTiles - 1) / kWgradTiles;
 }
 
-void dn_wgrad(const uint16_t* X, const uint16_t* coarse, int c1, const uint16_t* dZ, float* partial, float* dW, int N,
-              int H, int W, int Cin, int Cout, int tiles_per_chunk, hipStream_t s) {
-  const int chunks = dn_wgrad_chunks(N, H, W, tiles_per_chunk);
+void dn_layer_bwd(const DnGrad& grad, const uint16_t* Y, const uint16_t* X, const uint16_t* coarse, int c1, uint16_t* dZ,
+                  int N, int H, int W, int Cin, int Cout, float* wpartial, float* bpartial, float* dW, float* db,
+                  hipStream_t s) {
+  const GradSrc src{grad.g, grad.pooled, grad.kind, H, W, grad.gc, grad.c0};
+  hipLaunchKernelGGL(k_relu_bias, dim3(kBiasBlocks), dim3(256), 0, s, src, Y, dZ, static_cast<size_t>(N) * H * W, Cout,
+                     bpartial);
+  const int chunks = dn_wgrad_chunks(N, H, W);
   const dim3 grid(chunks, (Cout / 32) * ((Cin + 31) / 32));
-  hipLaunchKernelGGL(k_wgrad, grid, dim3(kWgThreads), 0, s, X, coarse, c1, dZ, partial, N, H, W, Cin, Cout,
-                     tiles_per_chunk);
+  hipLaunchKernelGGL(k_wgrad, grid, dim3(kWgThreads), 0, s, X, coarse, c1, dZ, wpartial, N, H, W, Cin, Cout);
   const size_t n = static_cast<size_t>(Cout) * 9 * Cin;
-  hipLaunchKernelGGL(k_reduce_chunks, dim3(blocks_for(n, kReduceOuts)), dim3(256), 0, s, partial, chunks, n, dW);
-}
-
-void dn_relu_bias_bwd(const float* dY, const uint16_t* Y, uint16_t* dZ, size_t P, int C, float* partial, float* db,
-                      hipStream_t s) {
-  hipLaunchKernelGGL(k_relu_bias, dim3(kBiasBlocks), dim3(256), 0, s, dY, Y, dZ, P, C, partial);
-  hipLaunchKernelGGL(k_reduce_chunks, dim3(blocks_for(C, kReduceOuts)), dim3(256), 0, s, partial, kBiasBlocks,
-                     static_cast<size_t>(C), db);
-}
-void dn_to_bf16(const float* a, uint16_t* b, size_t n, hipStream_t s) {
-  hipLaunchKernelGGL(k_to_bf16, dim3(blocks_for(n)), dim3(256), 0, s, a, b, n);
-}
-void dn_pool_bwd(const float* dY, float* dX, int N, int H, int W, int C, bool accumulate, hipStream_t s) {
-  hipLaunchKernelGGL(k_pool_bwd, dim3(blocks_for(static_cast<size_t>(N) * H * W * C)), dim3(256), 0, s, dY, dX, N, H,
-                     W, C, accumulate ? 1 : 0);
-}
-void dn_upcat_bwd(const float* dout, float* dcoarse, float* dskip, int N, int H, int W, int C1, int C2,
-                  bool accumulate_skip, hipStream_t s) {
-  hipLaunchKernelGGL(k_upcat_bwd_coarse, dim3(blocks_for(static_cast<size_t>(N) * (H / 2) * (W / 2) * C1)),
-                     dim3(256), 0, s, dout, dcoarse, N, H / 2, W / 2, C1, C2);
-  const size_t P = static_cast<size_t>(N) * H * W;
-  hipLaunchKernelGGL(k_upcat_bwd_skip, dim3(blocks_for(P * C2)), dim3(256), 0, s, dout, dskip, P, C1, C2,
-                     accumulate_skip ? 1 : 0);
+  const unsigned blocks = blocks_for(n, kReduceOuts);
+  hipLaunchKernelGGL(k_reduce_chunks, dim3(blocks + blocks_for(Cout, kReduceOuts)), dim3(256), 0, s,
+                     ChunkSum{wpartial, chunks, n, dW}, ChunkSum{bpartial, kBiasBlocks, static_cast<size_t>(Cout), db},
+                     blocks);
 }
 void dn_features(const float4* color, const float4* albedo, const float4* normal, uint16_t* out, size_t P,
                  hipStream_t s) {
@@ -983,13 +1007,14 @@ int dn_loss(const float* Y, const uint16_t* X, const float* T, size_t P, float* 
   hipLaunchKernelGGL(k_loss, dim3(nb), dim3(256), 0, s, Y, X, T, P, dY, partial);
   return static_cast<int>(nb);
 }
-void dn_adam(float* w, float* m, float* v, const float* g, uint16_t* wb, const uint8_t* mask, size_t n, float lr,
-             float b1, float b2, float c1, float c2, float eps, hipStream_t s) {
-  hipLaunchKernelGGL(k_adam, dim3(blocks_for(n)), dim3(256), 0, s, w, m, v, g, wb, mask, n, lr, b1, b2, c1, c2, eps);
+void dn_adam(float* w, float* m, float* v, const float* g, uint16_t* wb, uint16_t* wd, const WeightTable& table, size_t n,
+             float lr, float b1, float b2, float c1, float c2, float eps, hipStream_t s) {
+  hipLaunchKernelGGL(k_adam, dim3(blocks_for(n)), dim3(256), 0, s, w, m, v, g, wb, wd, table, static_cast<int>(n), lr, b1,
+                     b2, c1, c2, eps);
 }
 
-void dn_flip_weights(const uint16_t* w, uint16_t* wd, int cin, int cout, hipStream_t s) {
-  hipLaunchKernelGGL(k_flip, dim3(blocks_for(static_cast<size_t>(cin) * 9 * cout)), dim3(256), 0, s, w, wd, cin, cout);
+void dn_weights_bf16(const float* w, uint16_t* wb, uint16_t* wd, const WeightTable& table, size_t n, hipStream_t s) {
+  hipLaunchKernelGGL(k_weights_bf16, dim3(blocks_for(n)), dim3(256), 0, s, w, wb, wd, table, static_cast<int>(n));
 }
 
 }  // namespace trt
