@@ -121,3 +121,29 @@ def test_both_node_layouts_match_brute_force(rend, surrounding):
     got = rend.path_radiance()
     want = _oracle(sc).render()["path_rgb"]
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 4096, 4097, 70_001])
+@pytest.mark.parametrize("levels", ["single", "two-level"])
+def test_ray_query_sizes(rend, n, levels):
+    """Ray queries at the edges of their paths (one checking block, pinned exchange, copies):
+    hits, instances and occlusion equal the oracle's; an invalid last ray is named, and one
+    whose only fault is a negative tmin is told apart."""
+    from trayracer_amd._lib import TrtError
+    sc = _tiny(36) if levels == "single" else _instanced_view()
+    rend.UpdateScene(sc)
+    rays = random_rays(n, seed=n, lo=-0.2, hi=1.2 if levels == "single" else 5.0, tmin=1e-4)
+    orc = _oracle(sc)
+    hg, ig = rend.trace_closest(rays)
+    hb, ib = orc.trace_closest(rays)
+    hit = prim_of(hb) != 0xFFFFFFFF
+    assert np.array_equal(prim_of(hg), prim_of(hb)) and np.array_equal(ig, ib)
+    assert np.array_equal(hg[hit].view(np.uint32), hb[hit].view(np.uint32))
+    assert np.array_equal(rend.trace_any(rays), orc.trace_any(rays))
+    for col, val, what in ((6, np.nan, "non-finite"), (3, -1.0, "negative tmin"), (7, np.nan, "NaN bound")):
+        bad = rays.copy()
+        bad[n - 1, col] = val
+        for query in (rend.trace_closest, rend.trace_any):
+            with pytest.raises(TrtError, match=f"ray {n - 1} .*{what}"):
+                query(bad)
+    assert np.array_equal(rend.trace_any(rays), orc.trace_any(rays))  # usable afterwards

@@ -68,6 +68,11 @@ struct Mesh {
   uint32_t tri_offset, n_tris;
 };
 
+// Ray queries of up to this many rays exchange records and results through pinned host
+// memory; per ray: 32 B record, 16 B hit, 4 B instance, 1 B occlusion.
+constexpr uint32_t kSmallQuery = 4096;
+constexpr size_t kSmallQueryBytes = 32 + 16 + 4 + 1;
+
 }  // namespace
 
 struct trt_context {
@@ -124,6 +129,7 @@ struct trt_context {
   DevBuf tonemapped;  // RGBA8 display image
   DevBuf counters;
   DevBuf scratch_rays, scratch_hits, scratch_inst, scratch_occ;
+  void* small_query = nullptr;  // pinned host block of small ray queries
   uint64_t path_capacity = 0;
   uint64_t queue_slots = 0;  // kSegs * seg_cap slots allocated per queue
   uint32_t seg_cap = 0;      // slots per queue segment for the current frame size
@@ -388,6 +394,14 @@ RenderParams params_of_opts(const trt_context* ctx, const trt_render_opts& o) {
   return rp;
 }
 
+// Grid of a persistent kernel over at most n queue items: every resident slot, but no more
+// than a wave per 64 items (idle waves cost launch time and failed queue fetches: 0.37 ->
+// 0.35 ms for a 640 x 360 frame; half as many waves again were slower) and at least a
+// block per queue segment.
+int grid_for(int resident, uint64_t n) {
+  return int(std::min<uint64_t>(uint64_t(resident), std::max<uint64_t>(kSegs, (n + 255) / 256)));
+}
+
 // Launches one frame on ctx->stream. stats = counting traversal kernels (no timing use).
 trt_status run_frame(trt_context* ctx, const trt_render_opts& o, bool stats, bool accumulate, trt_stats* st) {
   trt_status s = ensure_frame(ctx, o.width, o.height, o.spp);
@@ -427,6 +441,7 @@ trt_status run_frame(trt_context* ctx, const trt_render_opts& o, bool stats, boo
                                                         o.mode == kModeAmbientOcclusionShading) ? 2u : 1u);
 
   const uint32_t cap = ctx->seg_cap;
+  const int grid_trace = grid_for(ctx->grid_trace, n), grid_shade = grid_for(ctx->grid_shade, n);
   // the concurrent Shadow launches use the second spill area
   DevAccel acc = acc0;
   DevAccel acc_sh = acc;
@@ -459,7 +474,7 @@ trt_status run_frame(trt_context* ctx, const trt_render_opts& o, bool stats, boo
     const int cur = int(d & 1u), nxt = cur ^ 1;
     const int di = int(d);
     launch_extend(acc, q[cur], hb, SegIn{ctr + seg_ctr(kSegExt, di), ctr + seg_ctr(kSegWorkExt, di), cap}, ctr,
-                  ctx->grid_trace, stats, stm);
+                  grid_trace, stats, stm);
     if (stats) {
       launch_touch_count(acc.touch_nodes, ctx->touch_node_words, ctr64 + 6, stm);
       launch_touch_count(acc.touch_tris, ctx->touch_tri_words, ctr64 + 7, stm);
@@ -473,7 +488,7 @@ trt_status run_frame(trt_context* ctx, const trt_render_opts& o, bool stats, boo
     launch_shade(sv, sampling_mats(ctx), rp, q[cur], hb, q[nxt], sq[cur], fb,
                  SegIn{ctr + seg_ctr(kSegExt, di), ctr + seg_ctr(kSegWorkShade, di), cap},
                  ctr + seg_ctr(kSegExt, di + 1), ctr + seg_ctr(kSegShadow, di), ctr + seg_ctr(kSegEmit, di), ctr, d,
-                 ctx->grid_shade, stm);
+                 grid_shade, stm);
     HIPC(hipEventRecord(ev[4 + 4 * d + 1], stm), "event");
     HIPC(hipStreamWaitEvent(stm2, ev[4 + 4 * d + 1], 0), "wait");
     if (timing) HIPC(hipEventRecord(ev2[2 * d], stm2), "event");
@@ -481,7 +496,7 @@ trt_status run_frame(trt_context* ctx, const trt_render_opts& o, bool stats, boo
     // found at bounce d after the shadow rays of bounce d - 1, before those of bounce d
     launch_emit(sq[cur].emit, ctr + seg_ctr(kSegEmit, di), cap, fb.radiance, stm2);
     launch_shadow(acc_sh, sq[cur], fb.radiance,
-                  SegIn{ctr + seg_ctr(kSegShadow, di), ctr + seg_ctr(kSegWorkShadow, di), cap}, ctr, ctx->grid_trace,
+                  SegIn{ctr + seg_ctr(kSegShadow, di), ctr + seg_ctr(kSegWorkShadow, di), cap}, ctr, grid_trace,
                   stats, stm2);
     if (stats) {
       launch_touch_count(acc_sh.touch_nodes, ctx->touch_node_words, ctr64 + 8, stm2);
@@ -607,6 +622,7 @@ void trt_destroy(trt_context* ctx) {
     if (e) (void)hipEventDestroy(e);
   for (auto& e : ctx->ev2)
     if (e) (void)hipEventDestroy(e);
+  if (ctx->small_query) (void)hipHostFree(ctx->small_query);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   if (ctx->stream2) (void)hipStreamDestroy(ctx->stream2);
   delete ctx;
@@ -1095,84 +1111,76 @@ trt_status trt_read_path_radiance(trt_context* ctx, float* rgb, uint64_t n_paths
   return TRT_OK;
 }
 
-// Test hook of the traversal: the rays go through the render's own Extend (closest) or
-// Shadow (any) kernels, as one depth-0 queue whose slot i is ray i (kSegs segments of
-// ceil(n / kSegs) slots). Occlusion comes back through Shadow's own result path: each
-// ray carries a unit contribution to its own radiance slot, added when unoccluded.
+// Ray queries: the caller's records go to the GPU as they are, are checked there by the
+// kernel that makes them a queue, and are traced by the render's own traversal (closest hit:
+// its Extend kernels). Up to kSmallQuery rays the kernels read the records from and write
+// the results to one pinned host block, so a query is three launches and a wait, without
+// copies; larger ones copy to and from the caller's memory. (The records were checked and
+// rearranged on the host and any-hit results came as 16 bytes a ray.)
 static trt_status trace_common(trt_context* ctx, const float* rays, uint32_t n, float* hits, uint32_t* inst,
                                uint8_t* occ, bool any) {
   if (!ctx || (n && !rays)) return TRT_INVALID_ARG;
   if (!ctx->built) return fail(ctx, TRT_NOT_BUILT, "scene not built");
   if (n == 0) return TRT_OK;
   HIPC(hipSetDevice(ctx->device), "hipSetDevice");
+  hipStream_t s = ctx->stream;
+  const bool small = n <= kSmallQuery, want_inst = !any && inst && ctx->two_level;
   HIPC(ctx->scratch_rays.ensure(size_t(n) * 32), "alloc rays");
-  HIPC(ctx->scratch_hits.ensure(size_t(n) * 16), "alloc hits");
-  HIPC(ctx->scratch_inst.ensure(size_t(n) * 4), "alloc hits");
-  HIPC(ctx->scratch_occ.ensure(size_t(n) * 16), "alloc hits");
-  // (o, tmin) rows first, then (d, tmax) rows
-  std::vector<float> soa(size_t(n) * 8);
-  for (uint32_t i = 0; i < n; ++i) {
-    const float* r = &rays[size_t(i) * 8];
-    // origins and directions finite, interval bounds not NaN (tmax may be +inf), tmin >= 0
-    // (the traversal's box test widens far distances relatively, which is conservative
-    // only for boxes at non-negative distances)
-    if (!finite_all(r, 3) || !finite_all(r + 4, 3) || r[3] != r[3] || r[7] != r[7])
-      return fail(ctx, TRT_INVALID_ARG, "ray " + std::to_string(i) + " has a non-finite origin or direction or a NaN bound");
-    if (!(r[3] >= 0.f)) return fail(ctx, TRT_INVALID_ARG, "ray " + std::to_string(i) + " has a negative tmin");
-    std::memcpy(&soa[size_t(i) * 4], &rays[size_t(i) * 8], 16);
-    std::memcpy(&soa[(size_t(n) + i) * 4], &rays[size_t(i) * 8 + 4], 16);
+  if (!ctx->small_query) HIPC(hipHostMalloc(&ctx->small_query, size_t(kSmallQuery) * kSmallQueryBytes + 16), "alloc rays");
+  if (!small && any) {
+    HIPC(ctx->scratch_occ.ensure(n), "alloc hits");
+  } else if (!small) {
+    HIPC(ctx->scratch_hits.ensure(size_t(n) * 16), "alloc hits");
+    HIPC(ctx->scratch_inst.ensure(size_t(n) * 4), "alloc hits");
   }
-  float4* o_tmin = ctx->scratch_rays.as<float4>();
-  float4* d_tmax = o_tmin + n;
-  HIPC(hipMemcpyAsync(o_tmin, soa.data(), size_t(n) * 32, hipMemcpyHostToDevice, ctx->stream), "upload rays");
+  uint8_t* const block = static_cast<uint8_t*>(ctx->small_query);  // records, hits, instances, occlusion, status
+  float4* const rec = ctx->scratch_rays.as<float4>();
+  const float4* src = rec;
+  float4* d_hits = ctx->scratch_hits.as<float4>();
+  uint32_t* d_inst = ctx->scratch_inst.as<uint32_t>();
+  uint8_t* d_occ = ctx->scratch_occ.as<uint8_t>();
+  if (small) {
+    std::memcpy(block, rays, size_t(n) * 32);
+    src = reinterpret_cast<const float4*>(block);
+    d_hits = reinterpret_cast<float4*>(block + size_t(kSmallQuery) * 32);
+    d_inst = reinterpret_cast<uint32_t*>(block + size_t(kSmallQuery) * 48);
+    d_occ = block + size_t(kSmallQuery) * 52;
+  } else {
+    HIPC(hipMemcpyAsync(rec, rays, size_t(n) * 32, hipMemcpyHostToDevice, s), "upload rays");
+  }
   uint32_t* ctr = ctx->counters.as<uint32_t>();
-  launch_zero_counters(ctr, ctx->stream);
-  const uint32_t per = (n + kSegs - 1) / kSegs;
-  std::vector<uint32_t> cnt(size_t(kSegs) * kLine, 0u);
-  for (uint32_t sgm = 0; sgm < kSegs; ++sgm) {
-    const uint64_t first = uint64_t(sgm) * per;
-    cnt[size_t(sgm) * kLine] = first >= n ? 0u : uint32_t(std::min<uint64_t>(per, n - first));
-  }
-  const int kind = any ? kSegShadow : kSegExt, work = any ? kSegWorkShadow : kSegWorkExt;
-  HIPC(hipMemcpyAsync(ctr + seg_ctr(kind, 0), cnt.data(), cnt.size() * 4, hipMemcpyHostToDevice, ctx->stream),
-       "upload queue counts");
-  const SegIn in{ctr + seg_ctr(kind, 0), ctr + seg_ctr(work, 0), per};
+  const uint32_t per = uint32_t((uint64_t(n) + kSegs - 1) / kSegs);
+  launch_ray_queue(src, rec, n, per, ctr, s);
+  const SegIn in{ctr + seg_ctr(kSegExt, 0), ctr + seg_ctr(kSegWorkExt, 0), per};
   const DevAccel acc = accel_of(ctx);
-  if (any) {
-    std::vector<float> unit(size_t(n) * 4);
-    for (uint32_t i = 0; i < n; ++i) {
-      unit[size_t(i) * 4 + 0] = unit[size_t(i) * 4 + 1] = unit[size_t(i) * 4 + 2] = 1.f;
-      std::memcpy(&unit[size_t(i) * 4 + 3], &i, 4);
-    }
-    float4* contrib = ctx->scratch_hits.as<float4>();
-    float4* result = ctx->scratch_occ.as<float4>();
-    HIPC(hipMemcpyAsync(contrib, unit.data(), size_t(n) * 16, hipMemcpyHostToDevice, ctx->stream), "upload contrib");
-    HIPC(hipMemsetAsync(result, 0, size_t(n) * 16, ctx->stream), "clear result");
-    launch_shadow(acc, ShadowQueue{o_tmin, d_tmax, contrib}, result, in, ctr, ctx->grid_trace, false, ctx->stream);
-  } else {
-    launch_extend(acc, RayQueue{o_tmin, d_tmax, nullptr, nullptr},
-                  HitBuf{ctx->scratch_hits.as<float4>(), ctx->scratch_inst.as<uint32_t>()}, in, ctr, ctx->grid_trace,
-                  false, ctx->stream);
-  }
+  const RayQueue q{rec, rec + 1, nullptr, nullptr, 2};
+  const int grid = grid_for(ctx->grid_trace, n);
+  if (any)
+    launch_occluded(acc, q, d_occ, in, ctr, grid, s);
+  else
+    launch_extend(acc, q, HitBuf{d_hits, d_inst}, in, ctr, grid, false, s);
   HIPC(hipGetLastError(), "trace launch");
-  HIPC(hipStreamSynchronize(ctx->stream), "trace");
-  uint32_t overflow = 0;
-  HIPC(hipMemcpy(&overflow, ctr + kCtrOverflow, 4, hipMemcpyDeviceToHost), "read overflow");
-  if (overflow) return fail(ctx, TRT_DEVICE, "traversal stack overflow");
-  if (any) {
-    std::vector<float> r(size_t(n) * 4);
-    HIPC(hipMemcpy(r.data(), ctx->scratch_occ.p, size_t(n) * 16, hipMemcpyDeviceToHost), "read occlusion");
-    for (uint32_t i = 0; i < n; ++i) occ[i] = r[size_t(i) * 4] == 0.f ? 1u : 0u;
+  uint32_t* const status = reinterpret_cast<uint32_t*>(block + size_t(kSmallQuery) * kSmallQueryBytes);  // overflow, -, first invalid ray
+  HIPC(hipMemcpyAsync(status, ctr + kCtrOverflow, 16, hipMemcpyDeviceToHost, s), "read status");
+  HIPC(hipStreamSynchronize(s), "trace");
+  uint64_t bad;
+  std::memcpy(&bad, status + (kCtrBadRay - kCtrOverflow), 8);
+  if (bad != ~uint64_t(0))
+    return fail(ctx, TRT_INVALID_ARG,
+                "ray " + std::to_string(bad >> 1) +
+                    (bad & 1u ? " has a negative tmin" : " has a non-finite origin or direction or a NaN bound"));
+  if (status[0]) return fail(ctx, TRT_DEVICE, "traversal stack overflow");
+  if (small) {
+    if (any) std::memcpy(occ, d_occ, n);
+    else std::memcpy(hits, d_hits, size_t(n) * 16);
+    if (want_inst) std::memcpy(inst, d_inst, size_t(n) * 4);
   } else {
-    HIPC(hipMemcpy(hits, ctx->scratch_hits.p, size_t(n) * 16, hipMemcpyDeviceToHost), "read hits");
-    if (inst) {
-      if (ctx->two_level) {
-        HIPC(hipMemcpy(inst, ctx->scratch_inst.p, size_t(n) * 4, hipMemcpyDeviceToHost), "read hits");
-      } else {
-        for (uint32_t i = 0; i < n; ++i) inst[i] = kNoInstance;
-      }
-    }
+    if (any) HIPC(hipMemcpyAsync(occ, d_occ, n, hipMemcpyDeviceToHost, s), "read occlusion");
+    else HIPC(hipMemcpyAsync(hits, d_hits, size_t(n) * 16, hipMemcpyDeviceToHost, s), "read hits");
+    if (want_inst) HIPC(hipMemcpyAsync(inst, d_inst, size_t(n) * 4, hipMemcpyDeviceToHost, s), "read hits");
+    HIPC(hipStreamSynchronize(s), "read hits");
   }
+  if (!any && inst && !want_inst) std::memset(inst, 0xff, size_t(n) * 4);  // kNoInstance
   return TRT_OK;
 }
 
@@ -1392,6 +1400,7 @@ trt_status trt_backward(trt_context* ctx, const trt_render_opts* o, const float*
   // As in the forward frame, Shadow of bounce d runs on the second stream beside Extend of
   // bounce d + 1 (it has the second spill area; they share no buffer); Shade of bounce
   // d + 1 needs the radiance that Shadow took off its paths, so it waits.
+  const int grid_trace = grid_for(ctx->grid_trace, n), grid_shade = grid_for(ctx->grid_shade, n);
   DevAccel acc_sh = acc;
   acc_sh.spill = acc.spill + ctx->spill_half;
   hipStream_t stm2 = ctx->stream2;
@@ -1401,15 +1410,15 @@ trt_status trt_backward(trt_context* ctx, const trt_render_opts* o, const float*
     const int cur = int(d & 1u), nxt = cur ^ 1;
     const int di = int(d);
     launch_extend(acc, q[cur], hb, SegIn{ctr + seg_ctr(kSegExt, di), ctr + seg_ctr(kSegWorkExt, di), cap}, ctr,
-                  ctx->grid_trace, false, stm);
+                  grid_trace, false, stm);
     if (d > 0) HIPC(hipStreamWaitEvent(stm, ctx->ev2[2 * (d - 1) + 1], 0), "wait");
     launch_shade_adj(sv, sampling_mats(ctx), rp, q[cur], hb, q[nxt], sq, ab,
                      SegIn{ctr + seg_ctr(kSegExt, di), ctr + seg_ctr(kSegWorkShade, di), cap},
-                     ctr + seg_ctr(kSegExt, di + 1), ctr + seg_ctr(kSegShadow, di), ctr, d, ctx->grid_shade, stm);
+                     ctr + seg_ctr(kSegExt, di + 1), ctr + seg_ctr(kSegShadow, di), ctr, d, grid_shade, stm);
     HIPC(hipEventRecord(ctx->ev[4 + 4 * d + 1], stm), "event");
     HIPC(hipStreamWaitEvent(stm2, ctx->ev[4 + 4 * d + 1], 0), "wait");
     launch_shadow_adj(acc_sh, sq, ab, SegIn{ctr + seg_ctr(kSegShadow, di), ctr + seg_ctr(kSegWorkShadow, di), cap},
-                      ctr, d, ctx->grid_trace, stm2);
+                      ctr, d, grid_trace, stm2);
     HIPC(hipEventRecord(ctx->ev2[2 * d + 1], stm2), "event");
   }
   HIPC(hipStreamWaitEvent(stm, ctx->ev2[2 * (D - 1) + 1], 0), "wait");

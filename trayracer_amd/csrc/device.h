@@ -18,6 +18,7 @@ struct RayQueue {
   float4* d_tmax;   // direction, tmax
   float4* t_pdf;    // throughput rgb, pdf of the sampled direction
   uint32_t* meta;   // path << 2 | flags
+  uint32_t stride = 1;  // slot s's ray at o_tmin[s * stride], d_tmax[s * stride] (2: a caller's ray records)
 };
 
 // Closest-hit results, indexed like the ray queue slot that produced them.
@@ -77,13 +78,16 @@ constexpr uint32_t kLine = 32;  // uint32 words per 128-byte line
 //   [kCtrShadow + d] total shadow rays emitted at depth d; both written at the end of a
 //                    frame by k_sum_counts from the per-segment counters
 //   [kCtrOverflow]   bit 0: traversal stack overflow; bit 1: queue append failed
+//   [kCtrBadRay]     64 bits, ray queries: 2 x the first invalid ray's index + 1 when its only
+//                    fault is a negative tmin; all ones when every ray is valid
 //   [kCtrStats + k]  traversal statistics (node visits, triangle tests, stack entries moved
 //                    from the LDS ring to the spill area: 64-bit pairs)
 //   [seg_ctr(kind, d) + s * kLine] per-segment counters, kinds below
 constexpr int kMaxDepth = 32;
 constexpr int kCtrExt = 0;
 constexpr int kCtrShadow = 32;
-constexpr int kCtrOverflow = 161;
+constexpr int kCtrOverflow = 160;
+constexpr int kCtrBadRay = 162;
 constexpr int kCtrStats = 164;  // 10 x uint64: closest nodes, closest tris, any nodes, any tris,
                                 // closest stack spills, any stack spills, then the distinct
                                 // nodes and triangle records read (summed over launches) by
@@ -169,6 +173,14 @@ void launch_shade(const SceneView& sv, const Material* sampling_mats, const Rend
 void launch_emit(const float4* emit, const uint32_t* emit_cnt, uint32_t cap, float4* radiance, hipStream_t stream);
 void launch_shadow(const DevAccel& acc, ShadowQueue sq, float4* radiance, SegIn in, uint32_t* ctr, int grid,
                    bool stats, hipStream_t stream);
+// Ray queries on n caller's records (8 floats: origin, tmin, direction, tmax). launch_ray_queue
+// makes them a depth-0 queue of kind kSegExt whose slot i is ray i (kSegs segments of `per`
+// slots), copying the records from `src` (which the GPU may read from host memory) to `rec`
+// unless they are the same, and checks them: kCtrBadRay tells of the first invalid one, and
+// invalid rays get an empty interval. launch_occluded: any hit, one byte per ray.
+void launch_ray_queue(const float4* src, float4* rec, uint32_t n, uint32_t per, uint32_t* ctr, hipStream_t stream);
+void launch_occluded(const DevAccel& acc, RayQueue q, uint8_t* occluded, SegIn in, uint32_t* ctr, int grid,
+                     hipStream_t stream);
 void launch_sum_counts(uint32_t* ctr, uint32_t cap, hipStream_t stream);
 // Adds the set bits of a touch bitmap (`words` 32-bit words) to *out and clears it.
 void launch_touch_count(uint32_t* bits, uint32_t words, unsigned long long* out, hipStream_t stream);

@@ -27,6 +27,8 @@
 //    bounce's shadow launch.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "device.h"
 #include "trt/tonemap.h"
 
@@ -1013,9 +1015,10 @@ __device__ __forceinline__ uint32_t* wave_tasks(uint32_t* lds) {
 struct RayLoad {
   const float4* o_tmin;
   const float4* d_tmax;
+  uint32_t stride;
   __device__ __forceinline__ void operator()(uint32_t slot, V3& o, V3& d, float& tmin, float& tmax) const {
-    const float4 a = o_tmin[slot];
-    const float4 b = d_tmax[slot];
+    const float4 a = o_tmin[static_cast<size_t>(slot) * stride];
+    const float4 b = d_tmax[static_cast<size_t>(slot) * stride];
     o = v3(a.x, a.y, a.z);
     d = v3(b.x, b.y, b.z);
     tmin = a.w;
@@ -1036,7 +1039,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
   st.spills = 0;
   trace_queue<Nodes, false, STATS>(
       acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st,
-      RayLoad{q.o_tmin, q.d_tmax},
+      RayLoad{q.o_tmin, q.d_tmax, q.stride},
       [&](uint32_t slot, const TraceOut& r, bool) {
         h.thit[slot] = make_float4(r.t, r.b1, r.b2, __uint_as_float(r.prim));
       });
@@ -1057,7 +1060,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
   st.spills = 0;
   trace_queue<Nodes, true, STATS>(
       acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st,
-      RayLoad{sq.o_tmin, sq.d_tmax},
+      RayLoad{sq.o_tmin, sq.d_tmax, 1u},
       [&](uint32_t slot, const TraceOut&, bool occluded) {
         if (!occluded) {
           const float4 c = sq.contrib[slot];
@@ -1088,7 +1091,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
   st.spills = 0;
   trace_queue2<Nodes, false, STATS>(
       acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st,
-      RayLoad{q.o_tmin, q.d_tmax},
+      RayLoad{q.o_tmin, q.d_tmax, q.stride},
       [&](uint32_t slot, const TraceOut& r, bool) {
         h.thit[slot] = make_float4(r.t, r.b1, r.b2, __uint_as_float(r.prim));
         h.inst[slot] = r.inst;
@@ -1110,7 +1113,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
   st.spills = 0;
   trace_queue2<Nodes, true, STATS>(
       acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st,
-      RayLoad{sq.o_tmin, sq.d_tmax},
+      RayLoad{sq.o_tmin, sq.d_tmax, 1u},
       [&](uint32_t slot, const TraceOut&, bool occluded) {
         if (!occluded) {
           const float4 c = sq.contrib[slot];
@@ -1129,6 +1132,70 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
   }
 }
 
+
+// Any-hit ray queries: one byte per ray.
+template <class Nodes>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_occluded_sl(
+    DevAccel acc, RayQueue q, uint8_t* occluded, SegIn in, uint32_t* ctr) {
+  extern __shared__ uint32_t lds[];
+  TraceOut st;
+  trace_queue<Nodes, true, false>(
+      acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st, RayLoad{q.o_tmin, q.d_tmax, q.stride},
+      [&](uint32_t slot, const TraceOut&, bool hit) { occluded[slot] = hit ? 1 : 0; });
+}
+
+template <class Nodes>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_occluded_tl(
+    DevAccel acc, RayQueue q, uint8_t* occluded, SegIn in, uint32_t* ctr) {
+  extern __shared__ uint32_t lds[];
+  TraceOut st;
+  trace_queue2<Nodes, true, false>(
+      acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st, RayLoad{q.o_tmin, q.d_tmax, q.stride},
+      [&](uint32_t slot, const TraceOut&, bool hit) { occluded[slot] = hit ? 1 : 0; });
+}
+
+// A caller's ray records as a depth-0 queue: checks them (origin and direction finite,
+// bounds not NaN, tmin not negative: the traversal's box tests are conservative for those),
+// gives an invalid ray an empty interval and reports the first. The counters the query uses
+// are reset first: by the block itself when it is the only one, else by k_ray_reset.
+__device__ __forceinline__ void ray_reset(uint32_t t, uint32_t n, uint32_t per, uint32_t* ctr) {
+  if (t < kSegs) {
+    const uint64_t first = static_cast<uint64_t>(t) * per;
+    ctr[seg_ctr(kSegExt, 0) + t * kLine] = first >= n ? 0u : (n - first < per ? static_cast<uint32_t>(n - first) : per);
+    ctr[seg_ctr(kSegWorkExt, 0) + t * kLine] = 0u;
+  }
+  if (t == kSegs) {
+    ctr[kCtrOverflow] = 0u;
+    ctr[kCtrBadRay] = ctr[kCtrBadRay + 1] = 0xffffffffu;
+  }
+}
+__global__ __launch_bounds__(64) void k_ray_reset(uint32_t n, uint32_t per, uint32_t* ctr) {
+  ray_reset(threadIdx.x, n, per, ctr);
+}
+__global__ __launch_bounds__(kBlock) void k_ray_check(const float4* src, float4* rec, uint32_t n, uint32_t per, uint32_t* ctr) {
+  if (gridDim.x == 1) {
+    ray_reset(threadIdx.x, n, per, ctr);
+    __syncthreads();
+  }
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
+  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; i < n; i += stride) {
+    const float4 a = src[2 * i];
+    float4 b = src[2 * i + 1];
+    const float inf = __builtin_huge_valf();
+    const bool finite = __builtin_fabsf(a.x) < inf && __builtin_fabsf(a.y) < inf && __builtin_fabsf(a.z) < inf &&
+                        __builtin_fabsf(b.x) < inf && __builtin_fabsf(b.y) < inf && __builtin_fabsf(b.z) < inf &&
+                        a.w == a.w && b.w == b.w;
+    const bool bad = !finite || !(a.w >= 0.f);
+    if (bad) {
+      atomicMin(reinterpret_cast<unsigned long long*>(ctr + kCtrBadRay), 2ull * i + (finite ? 1ull : 0ull));
+      b = make_float4(0.f, 0.f, 1.f, -1.f);
+    }
+    if (src != rec || bad) {
+      rec[2 * i] = bad ? make_float4(0.f, 0.f, 0.f, 0.f) : a;
+      rec[2 * i + 1] = b;
+    }
+  }
+}
 
 // Per-wave LDS list of Shade's pending work: queue slots whose ray needs shading, with
 // the ray's (direction, tmax) and hit records already read when the slot was fetched.
@@ -1496,7 +1563,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
   extern __shared__ uint32_t lds[];
   TraceOut st;
   trace_queue<Nodes, true, false>(
-      acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st, RayLoad{sq.o_tmin, sq.d_tmax},
+      acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st, RayLoad{sq.o_tmin, sq.d_tmax, 1u},
       [&](uint32_t slot, const TraceOut&, bool occluded) { finish_shadow_adj(sq, ab, depth, slot, occluded); });
 }
 
@@ -1506,7 +1573,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
   extern __shared__ uint32_t lds[];
   TraceOut st;
   trace_queue2<Nodes, true, false>(
-      acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st, RayLoad{sq.o_tmin, sq.d_tmax},
+      acc, in, wave_ring(lds), wave_tasks(lds), &ctr[kCtrOverflow], st, RayLoad{sq.o_tmin, sq.d_tmax, 1u},
       [&](uint32_t slot, const TraceOut&, bool occluded) { finish_shadow_adj(sq, ab, depth, slot, occluded); });
 }
 
@@ -1638,7 +1705,8 @@ static bool no_static_lds() {
                       reinterpret_cast<const void*>(k_shadow_sl<N, false>), reinterpret_cast<const void*>(k_shadow_sl<N, true>),
                       reinterpret_cast<const void*>(k_extend_tl<N, false>), reinterpret_cast<const void*>(k_extend_tl<N, true>),
                       reinterpret_cast<const void*>(k_shadow_tl<N, false>), reinterpret_cast<const void*>(k_shadow_tl<N, true>),
-                      reinterpret_cast<const void*>(k_shadow_adj_sl<N>), reinterpret_cast<const void*>(k_shadow_adj_tl<N>)};
+                      reinterpret_cast<const void*>(k_shadow_adj_sl<N>), reinterpret_cast<const void*>(k_shadow_adj_tl<N>),
+                      reinterpret_cast<const void*>(k_occluded_sl<N>), reinterpret_cast<const void*>(k_occluded_tl<N>)};
   for (const void* k : ks) {
     hipFuncAttributes a{};
     if (hipFuncGetAttributes(&a, k) != hipSuccess || a.sharedSizeBytes != 0) return false;
@@ -1680,6 +1748,23 @@ void launch_extend(const DevAccel& acc, RayQueue q, HitBuf h, SegIn in, uint32_t
     const auto k = acc.two_level ? (stats ? k_extend_tl<N, true> : k_extend_tl<N, false>)
                                  : (stats ? k_extend_sl<N, true> : k_extend_sl<N, false>);
     hipLaunchKernelGGL(k, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, q, h, in, ctr);
+  });
+}
+
+void launch_ray_queue(const float4* src, float4* rec, uint32_t n, uint32_t per, uint32_t* ctr, hipStream_t stream) {
+  // one block takes up to four rays a thread (one launch less: 8 us of a query of 64 rays);
+  // beyond that a block per 256 rays, up to a grid that covers the device several times
+  const uint32_t blocks = n <= 4 * kBlock ? 1u : std::min<uint32_t>((n + 0ull + kBlock - 1) / kBlock, 1u << 16);
+  if (blocks > 1) hipLaunchKernelGGL(k_ray_reset, dim3(1), dim3(64), 0, stream, n, per, ctr);
+  hipLaunchKernelGGL(k_ray_check, dim3(blocks), dim3(kBlock), 0, stream, src, rec, n, per, ctr);
+}
+
+void launch_occluded(const DevAccel& acc, RayQueue q, uint8_t* occluded, SegIn in, uint32_t* ctr, int grid,
+                     hipStream_t stream) {
+  with_nodes(acc, [&](auto nodes) {
+    using N = decltype(nodes);
+    const auto k = acc.two_level ? k_occluded_tl<N> : k_occluded_sl<N>;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, q, occluded, in, ctr);
   });
 }
 
