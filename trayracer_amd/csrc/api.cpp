@@ -146,6 +146,7 @@ struct trt_context {
 
   // differentiable rendering
   std::vector<Material> sampling_materials;  // empty = same as materials
+  bool sampling_same = false;  // not empty, and holds the same bytes as materials
   DevBuf d_mat_sampling;
   DevBuf d_sky;  // `sky` as the kernels read it (SceneView::sky)
   bool has_frame = false;      // the last frame's per-path radiance matches the current scene
@@ -390,7 +391,7 @@ RenderParams params_of_opts(const trt_context* ctx, const trt_render_opts& o) {
   rp.mode_flags = o.mode_flags;
   rp.ao_dist = o.ao_dist;
   rp.zdepth_max = o.zdepth_max;
-  rp.separate_sampling = ctx->sampling_materials.empty() ? 0u : 1u;
+  rp.separate_sampling = ctx->sampling_materials.empty() ? 0u : ctx->sampling_same ? 2u : 1u;
   return rp;
 }
 
@@ -1327,6 +1328,8 @@ trt_status trt_set_material_params(trt_context* ctx, const float* params, uint32
   };
   if (which & 1) apply(ctx->materials);
   if (which & 2) apply(ctx->sampling_materials);
+  ctx->sampling_same =
+      std::memcmp(ctx->materials.data(), ctx->sampling_materials.data(), ctx->materials.size() * sizeof(Material)) == 0;
   HIPC(upload(ctx->d_materials, ctx->materials.data(), ctx->materials.size() * sizeof(Material), ctx->stream),
        "upload materials");
   HIPC(upload(ctx->d_mat_sampling, ctx->sampling_materials.data(), ctx->sampling_materials.size() * sizeof(Material),
@@ -1385,6 +1388,7 @@ trt_status trt_backward(trt_context* ctx, const trt_render_opts* o, const float*
   ab.s_ga = ctx->a_sga.as<float4>();
   ab.s_gb = ctx->a_sgb.as<float>();
   ab.n_records = R;
+  ab.n_paths = n;
   ab.depth = D;
   RayQueue q[2];
   for (int i = 0; i < 2; ++i) {

@@ -129,23 +129,24 @@ struct FrameBuffers {
   float4* aov_sum_n;
 };
 
-// Adjoint (path replay) state. Records: one per (path, depth) slot r = path*depth + d,
+// Adjoint (path replay) state. Records: one per (depth, path) slot r = d * n_paths + path,
 // key = material id of the vertex (0xffffffff = none), gradient of parameters 0..3 in
 // rec_a[r] and of parameter 4 in rec_b[r] (valid where the key is). A vertex's record is
 // written whole by one kernel and read whole by the next, at an address that its queue
 // neighbours do not share, so the five parameters sit in two arrays (two lines per
-// record), not five.
+// record), not five; a depth's records lie together, as its launches touch them (neighbouring
+// rays are neighbouring pixels).
 struct AdjBuffers {
   const float* dldi;   // dLoss/dImage, 3 floats per pixel
   float4* lrem;        // per path: radiance not yet attributed to earlier vertices
-  float4* pend;        // per path: 4 float4 = (d f / d theta)/f of the pending continuation
+  float4* pend;        // 4 arrays of a float4 per path: (d f / d theta)/f of the pending continuation
                        // (written by a vertex that sends one on, read by the next vertex)
   uint32_t* rec_key;
   float4* rec_a;
   float* rec_b;
   float4* s_ga;        // per shadow slot: NEE gradient, params 0..3
   float* s_gb;         // per shadow slot: NEE gradient, param 4
-  size_t n_records;
+  size_t n_records, n_paths;
   uint32_t depth;
 };
 constexpr int kGradBlocks = 1024;       // fixed: the reduction order is device independent

@@ -1214,8 +1214,8 @@ struct ShadeList {
 // per-slot loop left idle through the whole shading step. Held to 3 waves per SIMD (150
 // VGPRs with one material set; the allocator could otherwise take more than 170, 2 waves;
 // 4 waves spill 20 bytes per lane and measured 1% slower).
-// SEP: the sampling materials are a set of their own (1) or the evaluation materials (0),
-// fixed per launch from RenderParams::separate_sampling.
+// SEP: the material-set mode of shade_impl (0, 1 or 2), fixed per launch from
+// RenderParams::separate_sampling.
 template <bool DEBUG, int SEP>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_shade(SceneView sv, const Material* sampling_mats, RenderParams rp,
                                                    RayQueue q, HitBuf h, RayQueue qn, ShadowQueue sq,
@@ -1409,7 +1409,7 @@ __global__ __launch_bounds__(kBlock) void k_tonemap(const float4* src, uint32_t 
 
 // ------------------------------------------------------------------------------------
 // Adjoint (path-replay backpropagation). Gradient records live in fixed slots
-// r = path * D + depth, so their values never depend on queue order; the reduction
+// r = depth * paths + path, so their values never depend on queue order; the reduction
 // below sums them in slot order.
 __global__ __launch_bounds__(kBlock) void k_raygen_adj(RenderParams rp, uint32_t n_paths, uint32_t per, uint32_t cap,
                                                         RayQueue q, const float4* radiance, AdjBuffers ab,
@@ -1421,13 +1421,17 @@ __global__ __launch_bounds__(kBlock) void k_raygen_adj(RenderParams rp, uint32_t
     PathState ps;
     const bool alive = raygen(rp, p, ps);
     ab.lrem[p] = radiance[p];
-    for (uint32_t d = 0; d < ab.depth; ++d) ab.rec_key[static_cast<size_t>(p) * ab.depth + d] = kNoHit;
+    for (uint32_t d = 0; d < ab.depth; ++d) ab.rec_key[static_cast<size_t>(d) * ab.n_paths + p] = kNoHit;
     store_primary(q, primary_slot(t, per, cap), p, ps, alive, rp.eps);
   }
 }
 
+
+// The adjoint's Shade. Held to 168 VGPRs, 3 waves per SIMD: it moves ~400 bytes a vertex
+// through gathers (queue, hit, records, pending derivatives), 2.5 TB/s, and waits on them
+// (512 x 512 x 64 spp step: 21.6 ms at 3 waves, 22.5 at 2).
 template <int SEP>
-__global__ __launch_bounds__(kBlock) void k_shade_adj(SceneView sv, const Material* sampling_mats, RenderParams rp,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_shade_adj(SceneView sv, const Material* sampling_mats, RenderParams rp,
                                                        RayQueue q, HitBuf h, RayQueue qn, ShadowQueue sq,
                                                        AdjBuffers ab, SegIn in, uint32_t* next_cnt,
                                                        uint32_t* shadow_cnt, uint32_t* ctr, uint32_t depth,
@@ -1466,8 +1470,9 @@ __global__ __launch_bounds__(kBlock) void k_shade_adj(SceneView sv, const Materi
       // continuation gradient of the previous vertex (which had a record and sent this
       // ray on): the radiance still unaccounted for arrived through its sampled direction
       if (depth > 0) {
-        const float4* pp = ab.pend + static_cast<size_t>(path) * 4;
-        const float4 p0 = pp[0], p1 = pp[1], p2 = pp[2], p3 = pp[3];
+        const float4* pp = ab.pend + path;
+        const size_t np = ab.n_paths;
+        const float4 p0 = pp[0], p1 = pp[np], p2 = pp[2 * np], p3 = pp[3 * np];
         AdjOut prev;
         prev.r[0][0] = p0.x; prev.r[0][1] = p0.y; prev.r[0][2] = p0.z;
         prev.r[1][0] = p0.w; prev.r[1][1] = p1.x; prev.r[1][2] = p1.y;
@@ -1476,7 +1481,7 @@ __global__ __launch_bounds__(kBlock) void k_shade_adj(SceneView sv, const Materi
         prev.r[4][0] = p3.x; prev.r[4][1] = p3.y; prev.r[4][2] = p3.z;
         float g[kNumParams];
         continuation_grad(prev, delta, v3(lr.x, lr.y, lr.z), g);
-        const size_t r = static_cast<size_t>(path) * ab.depth + (depth - 1);
+        const size_t r = static_cast<size_t>(depth - 1) * ab.n_paths + path;
         const float4 a4 = ab.rec_a[r];
         ab.rec_a[r] = make_float4(a4.x + g[0], a4.y + g[1], a4.z + g[2], a4.w + g[3]);
         ab.rec_b[r] += g[4];
@@ -1487,7 +1492,7 @@ __global__ __launch_bounds__(kBlock) void k_shade_adj(SceneView sv, const Materi
       hit.b2 = hh.z;
       hit.prim = __float_as_uint(hh.w);
       hit.inst = two_level ? h.inst[slot] : kNoInstance;
-      shade_adjoint<SEP>(sv, sampling_mats, rp, ps, hit, depth, delta, out, adj);
+      shade_adjoint<SEP, 2>(sv, sampling_mats, rp, ps, hit, depth, delta, out, adj);
       if (!is_black(out.L)) {
         lr.x -= out.L.x;
         lr.y -= out.L.y;
@@ -1495,7 +1500,7 @@ __global__ __launch_bounds__(kBlock) void k_shade_adj(SceneView sv, const Materi
         ab.lrem[path] = lr;
       }
       if (adj.mat != kNoHit) {
-        const size_t r = static_cast<size_t>(path) * ab.depth + depth;
+        const size_t r = static_cast<size_t>(depth) * ab.n_paths + path;
         ab.rec_key[r] = adj.mat;
         if (!out.has_shadow) {  // else the vertex's shadow ray writes the record
           ab.rec_a[r] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1503,11 +1508,12 @@ __global__ __launch_bounds__(kBlock) void k_shade_adj(SceneView sv, const Materi
         }
       }
       if (out.has_ext) {
-        float4* pp = ab.pend + static_cast<size_t>(path) * 4;
+        float4* pp = ab.pend + path;
+        const size_t np = ab.n_paths;
         pp[0] = make_float4(adj.r[0][0], adj.r[0][1], adj.r[0][2], adj.r[1][0]);
-        pp[1] = make_float4(adj.r[1][1], adj.r[1][2], adj.r[2][0], adj.r[2][1]);
-        pp[2] = make_float4(adj.r[2][2], adj.r[3][0], adj.r[3][1], adj.r[3][2]);
-        pp[3] = make_float4(adj.r[4][0], adj.r[4][1], adj.r[4][2], 0.f);
+        pp[np] = make_float4(adj.r[1][1], adj.r[1][2], adj.r[2][0], adj.r[2][1]);
+        pp[2 * np] = make_float4(adj.r[2][2], adj.r[3][0], adj.r[3][1], adj.r[3][2]);
+        pp[3 * np] = make_float4(adj.r[4][0], adj.r[4][1], adj.r[4][2], 0.f);
       }
     }
     const bool ext = out.has_ext != 0;
@@ -1552,7 +1558,7 @@ __device__ __forceinline__ void finish_shadow_adj(const ShadowQueue& sq, const A
     ga = ab.s_ga[slot];
     gb = ab.s_gb[slot];
   }
-  const size_t r = static_cast<size_t>(path) * ab.depth + depth;
+  const size_t r = static_cast<size_t>(depth) * ab.n_paths + path;
   ab.rec_a[r] = ga;
   ab.rec_b[r] = gb;
 }
@@ -1772,15 +1778,12 @@ void launch_shade(const SceneView& sv, const Material* sampling_mats, const Rend
                   HitBuf h, RayQueue qn, ShadowQueue sq, FrameBuffers fb, SegIn in, uint32_t* next_cnt,
                   uint32_t* shadow_cnt, uint32_t* emit_cnt, uint32_t* ctr, uint32_t depth, int grid,
                   hipStream_t stream) {
-  if (rp.mode != kModePathTracing)
-    hipLaunchKernelGGL((k_shade<true, -1>), dim3(grid), dim3(kBlock), 0, stream, sv, sampling_mats, rp, q, h, qn, sq,
-                       fb, in, next_cnt, shadow_cnt, emit_cnt, ctr, depth, sv.instances ? 1u : 0u, sv.sky);
-  else if (rp.separate_sampling)
-    hipLaunchKernelGGL((k_shade<false, 1>), dim3(grid), dim3(kBlock), 0, stream, sv, sampling_mats, rp, q, h, qn, sq,
-                       fb, in, next_cnt, shadow_cnt, emit_cnt, ctr, depth, sv.instances ? 1u : 0u, sv.sky);
-  else
-    hipLaunchKernelGGL((k_shade<false, 0>), dim3(grid), dim3(kBlock), 0, stream, sv, sampling_mats, rp, q, h, qn, sq,
-                       fb, in, next_cnt, shadow_cnt, emit_cnt, ctr, depth, sv.instances ? 1u : 0u, sv.sky);
+  const auto k = rp.mode != kModePathTracing     ? k_shade<true, -1>
+                 : rp.separate_sampling == 0u ? k_shade<false, 0>
+                 : rp.separate_sampling == 1u ? k_shade<false, 1>
+                                              : k_shade<false, 2>;
+  hipLaunchKernelGGL(k, dim3(grid), dim3(kBlock), 0, stream, sv, sampling_mats, rp, q, h, qn, sq, fb, in, next_cnt,
+                     shadow_cnt, emit_cnt, ctr, depth, sv.instances ? 1u : 0u, sv.sky);
 }
 
 void launch_emit(const float4* emit, const uint32_t* emit_cnt, uint32_t cap, float4* radiance, hipStream_t stream) {
@@ -1817,12 +1820,9 @@ void launch_raygen_adj(const RenderParams& rp, uint32_t n_paths, uint32_t cap, R
 void launch_shade_adj(const SceneView& sv, const Material* sampling_mats, const RenderParams& rp, RayQueue q,
                       HitBuf h, RayQueue qn, ShadowQueue sq, const AdjBuffers& ab, SegIn in, uint32_t* next_cnt,
                       uint32_t* shadow_cnt, uint32_t* ctr, uint32_t depth, int grid, hipStream_t stream) {
-  if (rp.separate_sampling)
-    hipLaunchKernelGGL(k_shade_adj<1>, dim3(grid), dim3(kBlock), 0, stream, sv, sampling_mats, rp, q, h, qn, sq, ab, in,
-                       next_cnt, shadow_cnt, ctr, depth, sv.instances ? 1u : 0u, sv.sky);
-  else
-    hipLaunchKernelGGL(k_shade_adj<0>, dim3(grid), dim3(kBlock), 0, stream, sv, sampling_mats, rp, q, h, qn, sq, ab, in,
-                       next_cnt, shadow_cnt, ctr, depth, sv.instances ? 1u : 0u, sv.sky);
+  const auto k = rp.separate_sampling == 0u ? k_shade_adj<0> : rp.separate_sampling == 1u ? k_shade_adj<1> : k_shade_adj<2>;
+  hipLaunchKernelGGL(k, dim3(grid), dim3(kBlock), 0, stream, sv, sampling_mats, rp, q, h, qn, sq, ab, in, next_cnt,
+                     shadow_cnt, ctr, depth, sv.instances ? 1u : 0u, sv.sky);
 }
 
 void launch_shadow_adj(const DevAccel& acc, ShadowQueue sq, const AdjBuffers& ab, SegIn in, uint32_t* ctr,

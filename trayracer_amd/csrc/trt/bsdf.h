@@ -185,6 +185,82 @@ TRT_HD T3<S> bsdf_f(const BsdfParams<S>& p, V3 wo, V3 wi) {
   return out;
 }
 
+// Derivatives of bsdf_f with respect to (base r, g, b, roughness, metallic):
+// g[k][c] = d f_c / d theta_k. With
+//   f_c = base_c kd + s_c ks + F_c q + clearcoat,   F_c = c0_c + (1 - c0_c) FH,
+// kd and q = D G / (4 cl cv) depend on the roughness, kd, ks and c0 on the metallic
+// parameter, and the base colour enters directly and through the tint; written out so that
+// each intermediate carries only the derivatives it has (bsdf_f on five-component dual
+// numbers carries all five through every operation, about eight times the arithmetic).
+TRT_HD inline void bsdf_grad(const BsdfParams<float>& p, V3 wo, V3 wi, float g[5][3]) {
+  for (int k = 0; k < 5; ++k) g[k][0] = g[k][1] = g[k][2] = 0.f;
+  if (wo.z <= 0.f || wi.z <= 0.f) return;
+  if (p.model == kModelLambert) {
+    for (int c = 0; c < 3; ++c) g[c][c] = kInvPi;
+    return;
+  }
+  const V3 h = normalize(wo + wi);
+  const float cl = wi.z, cv = wo.z, cd = dot(wi, h);
+  const float FL = schlick_weight(cl), FV = schlick_weight(cv), FH = schlick_weight(cd);
+  const float one_m_metal = 1.f - p.metallic;
+  const float base[3] = {p.base.x, p.base.y, p.base.z};
+  const float wlum[3] = {0.2126729f, 0.7151522f, 0.0721750f};
+  const float lum = lum3(p.base);
+  const float ilum = lum > 0.f ? 1.f / lum : 0.f;
+  float tint[3];
+  for (int c = 0; c < 3; ++c) tint[c] = lum > 0.f ? base[c] * ilum : 1.f;
+
+  // diffuse weight and its roughness derivative
+  const float cd2 = cd * cd, rcd2 = p.roughness * cd2;
+  const float fd1 = (0.5f + 2.f * rcd2) - 1.f;
+  const float A = 1.f + fd1 * FL, B = 1.f + fd1 * FV;
+  float dw = A * B, dw_r = 2.f * cd2 * (FL * B + FV * A);
+  if (p.subsurface > 0.f) {
+    const float As = 1.f + (rcd2 - 1.f) * FL, Bs = 1.f + (rcd2 - 1.f) * FV;
+    const float k = 1.f / (cl + cv) - 0.5f;
+    const float ss = 1.25f * (As * Bs * k + 0.5f), ss_r = 1.25f * k * cd2 * (FL * Bs + FV * As);
+    dw = (1.f - p.subsurface) * dw + p.subsurface * ss;
+    dw_r = (1.f - p.subsurface) * dw_r + p.subsurface * ss_r;
+  }
+  const float kd = dw * kInvPi * one_m_metal, kd_r = dw_r * kInvPi * one_m_metal;
+
+  // specular weight q = D G / (4 cl cv) and its roughness derivative
+  const float aspect = sqrt(1.f - 0.9f * p.anisotropic);
+  const float r2 = p.roughness * p.roughness;
+  const float ux = r2 / aspect, uy = r2 * aspect;
+  const float ax = fmax(ux, 1e-3f), ay = fmax(uy, 1e-3f);
+  const float ax_r = ux > 1e-3f ? 2.f * p.roughness / aspect : 0.f;  // the clamp holds the rest constant
+  const float ay_r = uy > 1e-3f ? 2.f * p.roughness * aspect : 0.f;
+  const float iax = 1.f / ax, iay = 1.f / ay;
+  const float hx2 = (h.x * iax) * (h.x * iax), hy2 = (h.y * iay) * (h.y * iay);
+  const float t = hx2 + hy2 + h.z * h.z;
+  const float lx = ax_r * iax, ly = ay_r * iay;  // d ln ax, d ln ay
+  const float D = 1.f / (kPi * ax * ay * t * t);
+  const float dlnD = 4.f * (hx2 * lx + hy2 * ly) / t - (lx + ly);
+  const float io2 = 1.f / (wo.z * wo.z), ii2 = 1.f / (wi.z * wi.z);
+  const float ox = ax * wo.x, oy = ay * wo.y, ix = ax * wi.x, iy = ay * wi.y;
+  const float so = sqrt(1.f + (ox * ox + oy * oy) * io2), si = sqrt(1.f + (ix * ix + iy * iy) * ii2);
+  const float G = 1.f / (1.f + (so - 1.f) * 0.5f + (si - 1.f) * 0.5f);
+  const float dL = 0.5f * ((ox * ox * lx + oy * oy * ly) * io2 / so + (ix * ix * lx + iy * iy * ly) * ii2 / si);
+  const float q = D * G / (4.f * cl * cv);
+  const float q_r = q * (dlnD - G * dL);
+
+  const float sp = p.specular * 0.08f, stt = p.specular_tint;
+  const float sheen = FH * p.sheen, st = p.sheen_tint;
+  const float one_m_FH = 1.f - FH;
+  // base colour: on its own channel, and through the tint's luminance on every channel
+  const float own = kd + q * one_m_FH * p.metallic;
+  const float via = (one_m_metal * (sheen * st + q * one_m_FH * sp * stt)) * ilum;
+  for (int c = 0; c < 3; ++c) {
+    const float spec_c = sp * ((1.f - stt) + stt * tint[c]);
+    const float c0 = p.metallic * base[c] + one_m_metal * spec_c;
+    const float F = c0 + (1.f - c0) * FH;
+    for (int k = 0; k < 3; ++k) g[k][c] = (k == c ? own + via : 0.f) - via * tint[c] * wlum[k];
+    g[3][c] = base[c] * kd_r + F * q_r;
+    g[4][c] = q * one_m_FH * (base[c] - spec_c) - base[c] * (dw * kInvPi) - ((1.f - st) + st * tint[c]) * sheen;
+  }
+}
+
 // Lobe selection probabilities (diffuse, specular, clearcoat) for sampling.
 TRT_FI void lobe_probs(const BsdfParams<float>& p, float cos_o, float& pd, float& ps, float& pc) {
   const float FV = schlick_weight(cos_o);

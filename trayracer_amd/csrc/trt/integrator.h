@@ -39,7 +39,8 @@ struct alignas(16) RenderParams {
   uint32_t mode;    // render mode (render_modes.h); 0 = path tracing
   uint32_t mode_flags;  // material property shown by the material-property mode
   uint32_t separate_sampling;  // 1: the sampling materials are a set of their own
-                               // (differentiable renders), see the Russian roulette
+                               // (differentiable renders), see the Russian roulette;
+                               // 2: and hold the same values as the evaluation materials
   uint32_t strategy;  // emitter estimators: 0 = both, MIS-weighted (the renderer always);
                       // 1 = light sampling only, 2 = BSDF sampling only (each alone is
                       // unbiased too: the oracle's tests compare the three means)
@@ -118,13 +119,34 @@ struct AdjOut {
   float r[kNumParams][3];       // (d f_c / d theta_k) / f_c at the sampled extension
 };
 
-// SEP: whether the sampling materials are a set of their own, -1 = as rp.separate_sampling
-// says (the device kernels fix it at compile time, so that with one set the material is
-// read once and the separate-set code is left out).
-template <bool ADJ, int SEP = -1>
+// (d f_c / d theta_k) at (wo, wi): dual numbers (ADJ 1, parameters bd) or bsdf_grad (ADJ 2).
+template <int ADJ>
+TRT_FI void bsdf_gradient(const BsdfParams<float>& bp, const BsdfParams<Dual<kNumParams>>& bd, V3 wo, V3 wi,
+                          float g[kNumParams][3]) {
+  if (ADJ == 2) {
+    bsdf_grad(bp, wo, wi, g);
+  } else {
+    const T3<Dual<kNumParams>> fd = bsdf_f(bd, wo, wi);
+    for (int k = 0; k < kNumParams; ++k) {
+      g[k][0] = fd.x.d[k];
+      g[k][1] = fd.y.d[k];
+      g[k][2] = fd.z.d[k];
+    }
+  }
+}
+
+// SEP: the sampling materials are 0 the evaluation materials, 1 a set of their own, 2 a set
+// of their own that holds the same values (the usual step of an optimisation), -1 as
+// rp.separate_sampling says, taking 2 as 1. The device kernels fix it at compile time: with
+// 0 and 2 the material is read once and evaluated in one pass per direction. 2 differs from
+// 0 in the Russian roulette only, which follows the sampling set's rule.
+// ADJ: 0 the plain step; the adjoint extras with BSDF derivatives 1 from dual numbers (the
+// oracle), 2 from bsdf_grad (the device).
+template <int ADJ, int SEP = -1>
 TRT_HD inline void shade_impl(const SceneView& s, const Material* sampling_mats, const RenderParams& rp,
                               const PathState& ps, const Hit& h, uint32_t depth, ShadeOut& out, V3 delta,
                               AdjOut* adj) {
+  const bool own_rr = SEP < 0 ? rp.separate_sampling != 0u : SEP != 0;
   const bool sep = SEP < 0 ? rp.separate_sampling != 0u : SEP == 1;
   out.L = v3(0.f);
   out.has_shadow = 0;
@@ -216,6 +238,8 @@ TRT_HD inline void shade_impl(const SceneView& s, const Material* sampling_mats,
     adj->mat = sp.mat;
     for (int k = 0; k < kNumParams; ++k) adj->nee_g[k] = 0.f;
     for (int k = 0; k < kNumParams; ++k) adj->r[k][0] = adj->r[k][1] = adj->r[k][2] = 0.f;
+  }
+  if (ADJ == 1) {
     bd.base = t3(dvar<kNumParams>(m.base[0], 0), dvar<kNumParams>(m.base[1], 1), dvar<kNumParams>(m.base[2], 2));
     bd.roughness = dvar<kNumParams>(m.roughness, 3);
     bd.metallic = dvar<kNumParams>(m.metallic, 4);
@@ -284,11 +308,12 @@ TRT_HD inline void shade_impl(const SceneView& s, const Material* sampling_mats,
           out.s_tmax = s_tmax;
           out.s_contrib = clamp_contrib(c, rp.clamp);
           if (ADJ) {
-            const T3<Dual<kNumParams>> fd = bsdf_f(bd, wo, wi);
+            float fg[kNumParams][3];
+            bsdf_gradient<ADJ>(bp, bd, wo, wi, fg);
             const float kx = delta.x * ps.T.x * lrad.x * k, ky = delta.y * ps.T.y * lrad.y * k,
                         kz = delta.z * ps.T.z * lrad.z * k;
             for (int j = 0; j < kNumParams; ++j)
-              adj->nee_g[j] = (kx * fd.x.d[j] + ky * fd.y.d[j]) + kz * fd.z.d[j];
+              adj->nee_g[j] = (kx * fg[j][0] + ky * fg[j][1]) + kz * fg[j][2];
           }
         }
       }
@@ -326,8 +351,8 @@ TRT_HD inline void shade_impl(const SceneView& s, const Material* sampling_mats,
           // carries earlier vertices' evaluation parameters), which the adjoint holds
           // fixed, so the continuation's derivative stays (df/dtheta) / f
           float q;
-          if (sep) {
-            const T3<float> fs = bsdf_f(bs, wo, smp.wi);
+          if (own_rr) {
+            const T3<float> fs = sep ? bsdf_f(bs, wo, smp.wi) : f1;
             q = fmin(1.f, fmax(fmax(fs.x, fs.y), fs.z) * k);
           } else {
             q = fmin(1.f, max3(Tn));
@@ -344,11 +369,12 @@ TRT_HD inline void shade_impl(const SceneView& s, const Material* sampling_mats,
           out.next.flags = 0u;
           out.next.path = ps.path;
           if (ADJ) {
-            const T3<Dual<kNumParams>> fd = bsdf_f(bd, wo, smp.wi);
+            float fg[kNumParams][3];
+            bsdf_gradient<ADJ>(bp, bd, wo, smp.wi, fg);
             for (int j = 0; j < kNumParams; ++j) {
-              adj->r[j][0] = f.x != 0.f ? fd.x.d[j] / f.x : 0.f;
-              adj->r[j][1] = f.y != 0.f ? fd.y.d[j] / f.y : 0.f;
-              adj->r[j][2] = f.z != 0.f ? fd.z.d[j] / f.z : 0.f;
+              adj->r[j][0] = f.x != 0.f ? fg[j][0] / f.x : 0.f;
+              adj->r[j][1] = f.y != 0.f ? fg[j][1] / f.y : 0.f;
+              adj->r[j][2] = f.z != 0.f ? fg[j][2] / f.z : 0.f;
             }
           }
         }
@@ -363,15 +389,15 @@ TRT_HD inline void shade_impl(const SceneView& s, const Material* sampling_mats,
 template <int SEP = -1>
 TRT_HD inline void shade(const SceneView& s, const Material* sampling_mats, const RenderParams& rp,
                          const PathState& ps, const Hit& h, uint32_t depth, ShadeOut& out) {
-  shade_impl<false, SEP>(s, sampling_mats, rp, ps, h, depth, out, v3(0.f), nullptr);
+  shade_impl<0, SEP>(s, sampling_mats, rp, ps, h, depth, out, v3(0.f), nullptr);
 }
 
 // Same vertex replayed for the adjoint: delta = dLoss/d(path radiance).
-template <int SEP = -1>
+template <int SEP = -1, int ADJ = 1>
 TRT_HD inline void shade_adjoint(const SceneView& s, const Material* sampling_mats, const RenderParams& rp,
                                  const PathState& ps, const Hit& h, uint32_t depth, V3 delta, ShadeOut& out,
                                  AdjOut& adj) {
-  shade_impl<true, SEP>(s, sampling_mats, rp, ps, h, depth, out, delta, &adj);
+  shade_impl<ADJ, SEP>(s, sampling_mats, rp, ps, h, depth, out, delta, &adj);
 }
 
 // Gradient of the BSDF-sampled continuation of a vertex once the radiance that
