@@ -92,7 +92,7 @@ struct trt_context {
   bool built = false;
 
   // device scene
-  DevBuf d_pos, d_nrm, d_mat_ids, d_materials, d_inst, d_inst_tlas, d_lights, d_alias_p, d_alias_i;
+  DevBuf d_tri_rec, d_nrm, d_materials, d_inst, d_inst_tlas, d_lights, d_alias;
   DevBuf d_nodes, d_tris, d_tlas;
   DevBuf d_spill;  // traversal stack spill areas
   DevBuf d_touch;  // counting frames: touch bitmaps of Extend (nodes, triangles), then Shadow's
@@ -356,14 +356,12 @@ DevAccel accel_of(const trt_context* ctx) {
 
 SceneView view_of(const trt_context* ctx) {
   SceneView s{};
-  s.tri_pos = ctx->d_pos.as<float>();
+  s.tri_rec = ctx->d_tri_rec.as<TriRec>();
   s.tri_nrm = ctx->use_normals ? ctx->d_nrm.as<float>() : nullptr;
-  s.tri_mat = ctx->d_mat_ids.as<uint32_t>();
   s.materials = ctx->d_materials.as<Material>();
   s.instances = ctx->two_level ? ctx->d_inst.as<Instance>() : nullptr;
   s.lights = ctx->d_lights.as<LightTri>();
-  s.alias_prob = ctx->d_alias_p.as<float>();
-  s.alias_idx = ctx->d_alias_i.as<uint32_t>();
+  s.alias = ctx->d_alias.as<AliasEntry>();
   s.n_lights = ctx->n_lights;
   s.total_power = ctx->total_power;
   s.n_tris = uint32_t(ctx->mat_ids.size());
@@ -909,15 +907,25 @@ trt_status trt_build(trt_context* ctx, const trt_build_opts* opts) {
   }
 
   hipStream_t s = ctx->stream;
-  HIPC(upload(ctx->d_pos, ctx->pos.data(), ctx->pos.size() * 4, s), "upload positions");
+  std::vector<TriRec> recs(n_tris);
+  for (uint32_t i = 0; i < n_tris; ++i) {
+    const float* p = &ctx->pos[size_t(i) * 9];
+    TriRec& r = recs[i];
+    std::memcpy(r.p0, p, 12);
+    std::memcpy(r.p1, p + 3, 12);
+    std::memcpy(r.p2, p + 6, 12);
+    r.mat = ctx->mat_ids[i];
+    r.pad1 = r.pad2 = 0u;
+  }
+  std::vector<AliasEntry> alias(lt.prob.size());
+  for (size_t i = 0; i < alias.size(); ++i) alias[i] = AliasEntry{lt.prob[i], lt.alias[i]};
+  HIPC(upload(ctx->d_tri_rec, recs.data(), recs.size() * sizeof(TriRec), s), "upload triangles");
   if (ctx->use_normals) HIPC(upload(ctx->d_nrm, ctx->nrm.data(), ctx->nrm.size() * 4, s), "upload normals");
-  HIPC(upload(ctx->d_mat_ids, ctx->mat_ids.data(), ctx->mat_ids.size() * 4, s), "upload material ids");
   HIPC(upload(ctx->d_materials, ctx->materials.data(), ctx->materials.size() * sizeof(Material), s), "upload materials");
   HIPC(upload(ctx->d_nodes, compact ? static_cast<const void*>(nodes32.data()) : nodes48.data(), node_bytes, s), "upload nodes");
   HIPC(upload(ctx->d_tris, tris.data(), tris.size() * 4, s), "upload triangles");
   HIPC(upload(ctx->d_lights, lt.lights.data(), lt.lights.size() * sizeof(LightTri), s), "upload lights");
-  HIPC(upload(ctx->d_alias_p, lt.prob.data(), lt.prob.size() * 4, s), "upload alias");
-  HIPC(upload(ctx->d_alias_i, lt.alias.data(), lt.alias.size() * 4, s), "upload alias");
+  HIPC(upload(ctx->d_alias, alias.data(), alias.size() * sizeof(AliasEntry), s), "upload alias");
   if (ctx->two_level) {
     HIPC(upload(ctx->d_inst, inst_orig.data(), inst_orig.size() * sizeof(Instance), s), "upload instances");
     HIPC(upload(ctx->d_inst_tlas, inst_tlas.data(), inst_tlas.size() * sizeof(TlasInstance), s), "upload instances");

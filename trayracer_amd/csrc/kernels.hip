@@ -1226,6 +1226,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
   // sv.sky again, as a restrict kernel argument: nothing the kernel writes can alias it, so
   // its fields are read with scalar loads where they are used
   sv.sky = sky;
+  __builtin_assume(sv.tri_rec != nullptr && sv.alias != nullptr);
   __shared__ ShadeList lists[kWavesPerBlock];
   ShadeList& L = lists[threadIdx.x >> 6];
   const uint32_t lane = lane_id();
@@ -1437,6 +1438,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
                                                        uint32_t* shadow_cnt, uint32_t* ctr, uint32_t depth,
                                                        uint32_t two_level, const SkyParams* __restrict__ sky) {
   sv.sky = sky;  // scalar loads of the sky's fields, as in k_shade
+  __builtin_assume(sv.tri_rec != nullptr && sv.alias != nullptr);
   const uint32_t lane = lane_id();
   const uint32_t npix = rp.width * rp.height;
   const float inv_spp = 1.f / static_cast<float>(rp.spp);

@@ -107,6 +107,14 @@ TRT_FI float light_pdf_hit(V3 le, float area, float cos_l, float t, float total)
 // Selection weight of the sun disc in next-event estimation (0 when it is not a light).
 TRT_FI float sun_weight(const SceneView& s) { return s.sky->sun_nee ? s.sky->sun_power : 0.f; }
 
+// Light chosen by power: column from u0, coin from u1 (alias_sample).
+TRT_FI uint32_t sample_light(const SceneView& s, float u0, float u1) {
+  if (!s.alias) return alias_sample(s.alias_prob, s.alias_idx, s.n_lights, u0, u1);
+  const uint32_t i = alias_column(s.n_lights, u0);
+  const AliasEntry e = s.alias[i];
+  return u1 < e.prob ? i : e.alias;
+}
+
 // Adjoint extras of one vertex (path-replay backpropagation, Vicini et al. 2021):
 // derivatives of the vertex's terms with respect to its material's differentiable
 // parameters theta = (baseColor r, g, b, roughness, metallic). Sampling decisions and
@@ -198,7 +206,7 @@ TRT_HD inline void shade_impl(const SceneView& s, const Material* sampling_mats,
       pick_sun = u0 < ps_sun;
       u0 = fmin((u0 - ps_sun) / (1.f - ps_sun), 0x1.fffffep-1f);
     }
-    if (!pick_sun) L = s.lights[alias_sample(s.alias_prob, s.alias_idx, s.n_lights, u0, u[1])];
+    if (!pick_sun) L = s.lights[sample_light(s, u0, u[1])];
   }
 
   const SurfacePoint sp = surface_at(s, h, ps.o, ps.d);

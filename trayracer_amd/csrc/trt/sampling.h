@@ -72,9 +72,12 @@ TRT_FI void sample_triangle(float u0, float u1, float& b1, float& b2) {
 }
 
 // Vose alias table lookup: column from u0, coin from u1.
+TRT_FI uint32_t alias_column(uint32_t n, float u0) {
+  const uint32_t i = static_cast<uint32_t>(u0 * static_cast<float>(n));
+  return i >= n ? n - 1 : i;
+}
 TRT_FI uint32_t alias_sample(const float* prob, const uint32_t* alias, uint32_t n, float u0, float u1) {
-  uint32_t i = static_cast<uint32_t>(u0 * static_cast<float>(n));
-  if (i >= n) i = n - 1;
+  const uint32_t i = alias_column(n, u0);
   return u1 < prob[i] ? i : alias[i];
 }
 
