@@ -147,3 +147,29 @@ def test_ray_query_sizes(rend, n, levels):
             with pytest.raises(TrtError, match=f"ray {n - 1} .*{what}"):
                 query(bad)
     assert np.array_equal(rend.trace_any(rays), orc.trace_any(rays))  # usable afterwards
+
+
+@pytest.mark.parametrize("sky", [False, True])
+def test_small_frames_after_large_ones(rend, sky):
+    """A frame's counters are reset by RayGen's own threads, of which a small frame has few:
+    1, 63 and 300 paths after a large frame, with emitter hits or a sky in the emission lists,
+    give the oracle's paths, and the counting frame (no accumulation) the same rays."""
+    sc = scenes.cornell(width=96, height=64, spp=3, max_depth=5, seed=31)
+    if sky:
+        sc["sky"] = dict(enabled=True, draw_sun=True, dir=(0.3, 0.8, -0.5), angular_diameter=32.0,
+                         intensity=1000.0, turbidity=4.0, sun_nee=True)
+    rend.UpdateScene(sc)
+    orc = _oracle(sc)
+    for size in (dict(width=96, height=64, spp=3), dict(width=1, height=1, spp=1), dict(width=9, height=7, spp=1),
+                 dict(width=96, height=64, spp=3), dict(width=10, height=6, spp=5)):
+        for k, v in size.items():
+            setattr(rend.settings, k, v)
+        rend.Reset()
+        st = rend.RenderFrame()
+        ref = orc.render(render=size)
+        assert st["paths"] == st["primary_rays"] == size["width"] * size["height"] * size["spp"]
+        assert np.array_equal(rend.path_radiance().view(np.uint32), ref["path_rgb"].view(np.uint32)), size
+        assert (st["extend_rays"], st["shadow_rays"]) == tuple(ref["counts"].sum(axis=1)), size
+        rend.Reset()  # the same samples again
+        m = rend.measure_traversal()
+        assert (m["closest_rays"], m["any_rays"]) == (st["extend_rays"], st["shadow_rays"]), size

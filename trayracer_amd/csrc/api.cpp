@@ -129,6 +129,7 @@ struct trt_context {
   DevBuf tonemapped;  // RGBA8 display image
   DevBuf counters;
   DevBuf scratch_rays, scratch_hits, scratch_inst, scratch_occ;
+  void* frame_report = nullptr;  // pinned: a frame's counters, written by its last kernel
   void* small_query = nullptr;  // pinned host block of small ray queries
   void* read_stage = nullptr;   // pinned buffers of read_back's threads
   uint64_t path_capacity = 0;
@@ -410,6 +411,9 @@ trt_status run_frame(trt_context* ctx, const trt_render_opts& o, bool stats, boo
   const uint32_t n = o.width * o.height * o.spp;
   const DevAccel acc0 = accel_of(ctx);
   const SceneView sv = view_of(ctx);
+  if (!ctx->frame_report)
+    HIPC(hipHostMalloc(&ctx->frame_report, size_t(kCtrSegBase) * 4), "alloc frame report");
+  uint32_t* const hc = static_cast<uint32_t*>(ctx->frame_report);
   uint32_t* ctr = ctx->counters.as<uint32_t>();
   FrameBuffers fb;
   fb.radiance = ctx->radiance.as<float4>();
@@ -466,7 +470,6 @@ trt_status run_frame(trt_context* ctx, const trt_render_opts& o, bool stats, boo
   // event recorded between two kernels of a stream delays the second by a few
   // microseconds, so those are left out when phase timing is off.
   const bool timing = ctx->phase_timing;
-  launch_zero_counters(ctr, stm);
   HIPC(hipEventRecord(ev[0], stm), "event");
   launch_raygen(rp, n, cap, q[0], fb, ctr, stm);
   if (timing) HIPC(hipEventRecord(ev[1], stm), "event");
@@ -493,11 +496,10 @@ trt_status run_frame(trt_context* ctx, const trt_render_opts& o, bool stats, boo
     HIPC(hipStreamWaitEvent(stm2, ev[4 + 4 * d + 1], 0), "wait");
     if (timing) HIPC(hipEventRecord(ev2[2 * d], stm2), "event");
     // all path radiance is added on this stream, in vertex order: the emission Shade
-    // found at bounce d after the shadow rays of bounce d - 1, before those of bounce d
-    launch_emit(sq[cur].emit, ctr + seg_ctr(kSegEmit, di), cap, fb.radiance, stm2);
+    // found at bounce d after the shadow rays of bounce d - 1, with those of bounce d
     launch_shadow(acc_sh, sq[cur], fb.radiance,
-                  SegIn{ctr + seg_ctr(kSegShadow, di), ctr + seg_ctr(kSegWorkShadow, di), cap}, ctr, grid_trace,
-                  stats, stm2);
+                  SegIn{ctr + seg_ctr(kSegShadow, di), ctr + seg_ctr(kSegWorkShadow, di), cap},
+                  ctr + seg_ctr(kSegEmit, di), ctr, grid_trace, stats, stm2);
     if (stats) {
       launch_touch_count(acc_sh.touch_nodes, ctx->touch_node_words, ctr64 + 8, stm2);
       launch_touch_count(acc_sh.touch_tris, ctx->touch_tri_words, ctr64 + 9, stm2);
@@ -508,14 +510,13 @@ trt_status run_frame(trt_context* ctx, const trt_render_opts& o, bool stats, boo
   if (timing) HIPC(hipEventRecord(ev[3], stm), "event");
   if (accumulate)
     launch_finalize(rp, fb.radiance, fb, ctx->sample_count == 0 ? 1u : 0u, ctx->aov_count == 0 ? 1u : 0u,
-                    ctx->aov_count + o.spp, stm);
+                    ctx->aov_count + o.spp, ctr, cap, hc, stm);
+  else
+    launch_report_counters(ctr, cap, hc, stm);
   HIPC(hipEventRecord(ev[2], stm), "event");
-  launch_sum_counts(ctr, cap, stm);
   HIPC(hipGetLastError(), "kernel launch");
   HIPC(hipStreamSynchronize(stm), "frame");
 
-  uint32_t hc[kCtrSegBase];
-  HIPC(hipMemcpy(hc, ctr, sizeof(hc), hipMemcpyDeviceToHost), "read counters");
   ctx->last_paths = n;
   ctx->has_frame = true;
   ++ctx->frame_id;
@@ -622,6 +623,7 @@ void trt_destroy(trt_context* ctx) {
     if (e) (void)hipEventDestroy(e);
   for (auto& e : ctx->ev2)
     if (e) (void)hipEventDestroy(e);
+  if (ctx->frame_report) (void)hipHostFree(ctx->frame_report);
   if (ctx->small_query) (void)hipHostFree(ctx->small_query);
   if (ctx->read_stage) (void)hipHostFree(ctx->read_stage);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -1481,7 +1483,6 @@ trt_status trt_backward(trt_context* ctx, const trt_render_opts* o, const float*
   DevAccel acc_sh = acc;
   acc_sh.spill = acc.spill + ctx->spill_half;
   hipStream_t stm2 = ctx->stream2;
-  launch_zero_counters(ctr, stm);
   launch_raygen_adj(rp, uint32_t(n), cap, q[0], ctx->radiance.as<float4>(), ab, ctr, stm);
   for (uint32_t d = 0; d < D; ++d) {
     const int cur = int(d & 1u), nxt = cur ^ 1;

@@ -72,11 +72,11 @@ struct DevAccel {
 constexpr uint32_t kSegs = 32;
 constexpr uint32_t kLine = 32;  // uint32 words per 128-byte line
 
-// Counters in device memory; zeroed at the start of every frame by a kernel.
+// Counters in device memory; zeroed at the start of every frame by RayGen.
 // Layout (uint32 indices):
 //   [kCtrExt + d]    total rays in the extension queue of depth d (d = 0: primary rays),
-//   [kCtrShadow + d] total shadow rays emitted at depth d; both written at the end of a
-//                    frame by k_sum_counts from the per-segment counters
+//   [kCtrShadow + d] total shadow rays emitted at depth d; both only in the
+//                    report made at the end of a frame, from the per-segment counters
 //   [kCtrOverflow]   bit 0: traversal stack overflow; bit 1: queue append failed
 //   [kCtrBadRay]     64 bits, ray queries: 2 x the first invalid ray's index + 1 when its only
 //                    fault is a negative tmin; all ones when every ray is valid
@@ -164,16 +164,16 @@ void launch_raygen(const RenderParams& rp, uint32_t n_paths, uint32_t cap, RayQu
 void launch_extend(const DevAccel& acc, RayQueue q, HitBuf h, SegIn in, uint32_t* ctr, int grid, bool stats,
                    hipStream_t stream);
 // Shade writes no path radiance: what a vertex emits goes to the emission list sq.emit
-// (segmented, counters emit_cnt), which launch_emit adds to the paths.
+// (segmented, counters emit_cnt), which the bounce's launch_shadow adds to the paths.
 void launch_shade(const SceneView& sv, const Material* sampling_mats, const RenderParams& rp, RayQueue q,
                   HitBuf h, RayQueue qn, ShadowQueue sq, FrameBuffers fb, SegIn in, uint32_t* next_cnt,
                   uint32_t* shadow_cnt, uint32_t* emit_cnt, uint32_t* ctr, uint32_t depth, int grid,
                   hipStream_t stream);
-// Adds an emission list (kSegs segments of `cap` slots, counters emit_cnt) to the path
-// radiance; every path is listed at most once, so entries need no atomics.
-void launch_emit(const float4* emit, const uint32_t* emit_cnt, uint32_t cap, float4* radiance, hipStream_t stream);
-void launch_shadow(const DevAccel& acc, ShadowQueue sq, float4* radiance, SegIn in, uint32_t* ctr, int grid,
-                   bool stats, hipStream_t stream);
+// Adds the bounce's emission list (sq.emit, counters emit_cnt; every path is listed at most
+// once and has no shadow ray in the same bounce, so no atomics) and the unoccluded shadow
+// rays' contributions to the path radiance.
+void launch_shadow(const DevAccel& acc, ShadowQueue sq, float4* radiance, SegIn in, const uint32_t* emit_cnt,
+                   uint32_t* ctr, int grid, bool stats, hipStream_t stream);
 // Ray queries on n caller's records (8 floats: origin, tmin, direction, tmax). launch_ray_queue
 // makes them a depth-0 queue of kind kSegExt whose slot i is ray i (kSegs segments of `per`
 // slots), copying the records from `src` (which the GPU may read from host memory) to `rec`
@@ -182,14 +182,17 @@ void launch_shadow(const DevAccel& acc, ShadowQueue sq, float4* radiance, SegIn 
 void launch_ray_queue(const float4* src, float4* rec, uint32_t n, uint32_t per, uint32_t* ctr, hipStream_t stream);
 void launch_occluded(const DevAccel& acc, RayQueue q, uint8_t* occluded, SegIn in, uint32_t* ctr, int grid,
                      hipStream_t stream);
-void launch_sum_counts(uint32_t* ctr, uint32_t cap, hipStream_t stream);
+// The counters' first kCtrSegBase words, with the totals per depth, to `report` (host memory
+// the GPU can write); launch_finalize does the same.
+void launch_report_counters(const uint32_t* ctr, uint32_t cap, uint32_t* report, hipStream_t stream);
 // Adds the set bits of a touch bitmap (`words` 32-bit words) to *out and clears it.
 void launch_touch_count(uint32_t* bits, uint32_t words, unsigned long long* out, hipStream_t stream);
 void launch_tonemap(const float4* src, uint32_t n, const TonemapParams& tp, uchar4* dst, hipStream_t stream);
 // reset: restart the accumulator; aov_reset: restart the AOV sums; aov_count: samples in
 // the AOV sums after this frame.
 void launch_finalize(const RenderParams& rp, const float4* radiance, FrameBuffers fb, uint32_t reset,
-                     uint32_t aov_reset, uint32_t aov_count, hipStream_t stream);
+                     uint32_t aov_reset, uint32_t aov_count, const uint32_t* ctr, uint32_t cap, uint32_t* report,
+                     hipStream_t stream);
 void launch_raygen_adj(const RenderParams& rp, uint32_t n_paths, uint32_t cap, RayQueue q, const float4* radiance,
                        const AdjBuffers& ab, uint32_t* ctr, hipStream_t stream);
 void launch_shade_adj(const SceneView& sv, const Material* sampling_mats, const RenderParams& rp, RayQueue q,

@@ -905,18 +905,35 @@ __global__ __launch_bounds__(kBlock) void k_zero_counters(uint32_t* ctr) {
   if (i < static_cast<uint32_t>(kNumCounters)) ctr[i] = 0u;
 }
 
-// Totals per depth of the extension and shadow queues (lane = depth, two waves).
-__global__ __launch_bounds__(64) void k_sum_counts(uint32_t* ctr, uint32_t cap) {
-  const uint32_t t = threadIdx.x;
-  if (t >= 2u * kMaxDepth) return;
-  const uint32_t kind = t < kMaxDepth ? kSegExt : kSegShadow, d = t % kMaxDepth;
-  const uint32_t* c = ctr + seg_ctr(static_cast<int>(kind), static_cast<int>(d));
-  uint32_t total = 0;
-  for (uint32_t sgm = 0; sgm < kSegs; ++sgm) {
-    const uint32_t v = c[sgm * kLine];
-    total += v < cap ? v : cap;
+// A frame's counters before their first use, by RayGen's threads: the plain words and one
+// word per segment line, but for the primary queue's, which primary_counts writes.
+__device__ __forceinline__ void reset_counters(uint32_t* ctr) {
+  constexpr uint32_t kWords = kCtrSegBase + (kNumCounters - kCtrSegBase) / kLine;
+  constexpr uint32_t kPrimary = seg_ctr(kSegExt, 0);
+  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < kWords; i += gridDim.x * kBlock) {
+    const uint32_t w = i < static_cast<uint32_t>(kCtrSegBase) ? i : kCtrSegBase + (i - kCtrSegBase) * kLine;
+    if (w < kPrimary || w >= kPrimary + kSegs * kLine) ctr[w] = 0u;
   }
-  ctr[(kind == kSegExt ? kCtrExt : kCtrShadow) + d] = total;
+}
+
+// The plain counter words as the host reads them after a frame, with the totals per depth of
+// the extension and shadow queues, into (pinned host) memory. One block.
+__device__ __forceinline__ void report_counters(const uint32_t* ctr, uint32_t cap, uint32_t* out) {
+  static_assert(kCtrSegBase == kBlock && kCtrExt == 0 && kCtrShadow == kMaxDepth, "a word per thread");
+  const uint32_t t = threadIdx.x;
+  uint32_t v = ctr[t];
+  if (t < 2u * kMaxDepth) {
+    const uint32_t* c = ctr + seg_ctr(t < kMaxDepth ? kSegExt : kSegShadow, static_cast<int>(t % kMaxDepth));
+    v = 0u;
+    for (uint32_t sgm = 0; sgm < kSegs; ++sgm) {
+      const uint32_t n = c[sgm * kLine];
+      v += n < cap ? n : cap;
+    }
+  }
+  out[t] = v;
+}
+__global__ __launch_bounds__(kBlock) void k_report_counters(const uint32_t* ctr, uint32_t cap, uint32_t* out) {
+  report_counters(ctr, cap, out);
 }
 
 // Distinct items a launch read: set bits of its touch bitmap, which is cleared for the
@@ -987,6 +1004,7 @@ __device__ __forceinline__ uint32_t tiled_path(uint32_t t, uint32_t W, uint32_t 
 __global__ __launch_bounds__(kBlock) void k_raygen(RenderParams rp, uint32_t n_paths, uint32_t per, uint32_t cap,
                                                     RayQueue q, FrameBuffers fb, uint32_t* ctr) {
   const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+  reset_counters(ctr);
   primary_counts(n_paths, per, ctr + seg_ctr(kSegExt, 0));
   if (t < n_paths) {
     const uint32_t p = tiled_path(t, rp.width, rp.height);
@@ -1026,6 +1044,38 @@ struct RayLoad {
   }
 };
 
+// A bounce's emission list into the path radiance, before the block's share of the bounce's
+// shadow rays: a path ends where it emits, so no path of the list has a shadow ray of this
+// bounce, and the radiance of every path is summed in vertex order. The blocks of a grid
+// deal the segments out; the next entry is read while the last one is added. A launch of
+// its own had waited, on the second stream, for CUs that Extend of the next bounce already
+// filled (37 us a bounce of a 256 x 256 x 16 frame). With the counters reset in RayGen and
+// reported by Finalize, six launches and a copy fewer: 0.517 -> 0.484 ms a 640 x 360 frame
+// of four bounces, 0.80 -> 0.77 ms a 256 x 256 x 16 one.
+__device__ __forceinline__ void add_emission(const float4* __restrict__ emit, const uint32_t* __restrict__ cnt,
+                                             uint32_t cap, float4* radiance) {
+  for (uint32_t sgm = blockIdx.x % kSegs; sgm < kSegs; sgm += gridDim.x) {
+    const uint32_t c = cnt[sgm * kLine];
+    const uint32_t n = c < cap ? c : cap;
+    const uint32_t first = blockIdx.x / kSegs * kBlock, step = (gridDim.x - sgm + kSegs - 1) / kSegs * kBlock;
+    const float4* seg = emit + static_cast<size_t>(sgm) * cap;
+    uint32_t i = first + threadIdx.x;
+    float4 e = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i < n) e = seg[i];
+    while (i < n) {
+      const float4 cur = e;
+      i += step;
+      if (i < n) e = seg[i];
+      const uint32_t path = __float_as_uint(cur.w);
+      float4 L = radiance[path];
+      L.x += cur.x;
+      L.y += cur.y;
+      L.z += cur.z;
+      radiance[path] = L;
+    }
+  }
+}
+
 // Single-level scenes: Extend and Shadow through trace_queue, held to 72 VGPRs, 7 waves per
 // SIMD. They are bound by throughput, not latency (the texture data path is 91 % busy and
 // VALU issue above its 4-cycle rate): 6 and 5 waves measured 11.98 and 12.01 ms a soup
@@ -1052,8 +1102,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
 
 template <class Nodes, bool STATS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_shadow_sl(DevAccel acc, ShadowQueue sq, float4* radiance, SegIn in,
-                                                       uint32_t* ctr) {
+                                                       const uint32_t* emit_cnt, uint32_t* ctr) {
   extern __shared__ uint32_t lds[];
+  add_emission(sq.emit, emit_cnt, in.cap, radiance);
   TraceOut st;
   st.nodes = 0;
   st.tests = 0;
@@ -1105,8 +1156,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
 
 template <class Nodes, bool STATS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_shadow_tl(DevAccel acc, ShadowQueue sq, float4* radiance, SegIn in,
-                                                       uint32_t* ctr) {
+                                                       const uint32_t* emit_cnt, uint32_t* ctr) {
   extern __shared__ uint32_t lds[];
+  add_emission(sq.emit, emit_cnt, in.cap, radiance);
   TraceOut st;
   st.nodes = 0;
   st.tests = 0;
@@ -1337,26 +1389,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
   }
 }
 
-// A bounce's emission list into the path radiance. It runs on the shadow stream after
-// the previous bounce's shadow rays and before this bounce's, so every path's radiance
-// is summed in vertex order: emission at vertex d, then the next-event estimate of d.
-// Block (x, y) takes every gridDim.x-th group of kBlock entries of segment y.
-__global__ __launch_bounds__(kBlock) void k_emit(const float4* __restrict__ emit, const uint32_t* __restrict__ cnt,
-                                                 uint32_t cap, float4* radiance) {
-  const uint32_t sgm = blockIdx.y;
-  const uint32_t c = cnt[sgm * kLine];
-  const uint32_t n = c < cap ? c : cap;
-  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-    const float4 e = emit[size_t(sgm) * cap + i];
-    const uint32_t path = __float_as_uint(e.w);
-    float4 L = radiance[path];
-    L.x += e.x;
-    L.y += e.y;
-    L.z += e.z;
-    radiance[path] = L;
-  }
-}
-
 __device__ __forceinline__ float4 add4(float4 a, float4 b) {
   return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
 }
@@ -1364,8 +1396,14 @@ __device__ __forceinline__ float4 add4(float4 a, float4 b) {
 // Per pixel, in sample order: the frame's radiance into the accumulator (mean colour),
 // and its first-hit AOVs into their sums (means over the accumulated samples: the
 // denoiser's guide images, anti-aliased like the colour).
+// The grid's last block reports the frame's counters instead.
 __global__ __launch_bounds__(kBlock) void k_finalize(RenderParams rp, const float4* radiance, FrameBuffers fb,
-                                                      uint32_t reset, uint32_t aov_reset, uint32_t aov_count) {
+                                                      uint32_t reset, uint32_t aov_reset, uint32_t aov_count,
+                                                      const uint32_t* ctr, uint32_t cap, uint32_t* report) {
+  if (blockIdx.x == gridDim.x - 1) {
+    report_counters(ctr, cap, report);
+    return;
+  }
   const uint32_t pix = blockIdx.x * kBlock + threadIdx.x;
   const uint32_t npix = rp.width * rp.height;
   if (pix >= npix) return;
@@ -1416,6 +1454,7 @@ __global__ __launch_bounds__(kBlock) void k_raygen_adj(RenderParams rp, uint32_t
                                                         RayQueue q, const float4* radiance, AdjBuffers ab,
                                                         uint32_t* ctr) {
   const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+  reset_counters(ctr);
   primary_counts(n_paths, per, ctr + seg_ctr(kSegExt, 0));
   if (t < n_paths) {
     const uint32_t p = tiled_path(t, rp.width, rp.height);
@@ -1732,8 +1771,8 @@ void launch_tonemap(const float4* src, uint32_t n, const TonemapParams& tp, ucha
   hipLaunchKernelGGL(k_tonemap, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, src, n, tp, dst);
 }
 
-void launch_sum_counts(uint32_t* ctr, uint32_t cap, hipStream_t stream) {
-  hipLaunchKernelGGL(k_sum_counts, dim3(1), dim3(64), 0, stream, ctr, cap);
+void launch_report_counters(const uint32_t* ctr, uint32_t cap, uint32_t* report, hipStream_t stream) {
+  hipLaunchKernelGGL(k_report_counters, dim3(1), dim3(kBlock), 0, stream, ctr, cap, report);
 }
 
 void launch_touch_count(uint32_t* bits, uint32_t words, unsigned long long* out, hipStream_t stream) {
@@ -1788,27 +1827,22 @@ void launch_shade(const SceneView& sv, const Material* sampling_mats, const Rend
                      shadow_cnt, emit_cnt, ctr, depth, sv.instances ? 1u : 0u, sv.sky);
 }
 
-void launch_emit(const float4* emit, const uint32_t* emit_cnt, uint32_t cap, float4* radiance, hipStream_t stream) {
-  // 16 blocks per segment: most lists are short (emitter hits); sky scenes list a third
-  // of the paths
-  hipLaunchKernelGGL(k_emit, dim3(16, kSegs), dim3(kBlock), 0, stream, emit, emit_cnt, cap, radiance);
-}
-
-void launch_shadow(const DevAccel& acc, ShadowQueue sq, float4* radiance, SegIn in, uint32_t* ctr, int grid,
-                   bool stats, hipStream_t stream) {
+void launch_shadow(const DevAccel& acc, ShadowQueue sq, float4* radiance, SegIn in, const uint32_t* emit_cnt,
+                   uint32_t* ctr, int grid, bool stats, hipStream_t stream) {
   with_nodes(acc, [&](auto nodes) {
     using N = decltype(nodes);
     const auto k = acc.two_level ? (stats ? k_shadow_tl<N, true> : k_shadow_tl<N, false>)
                                  : (stats ? k_shadow_sl<N, true> : k_shadow_sl<N, false>);
-    hipLaunchKernelGGL(k, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, sq, radiance, in, ctr);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(kBlock), trace_lds_bytes(), stream, acc, sq, radiance, in, emit_cnt, ctr);
   });
 }
 
 void launch_finalize(const RenderParams& rp, const float4* radiance, FrameBuffers fb, uint32_t reset,
-                     uint32_t aov_reset, uint32_t aov_count, hipStream_t stream) {
+                     uint32_t aov_reset, uint32_t aov_count, const uint32_t* ctr, uint32_t cap, uint32_t* report,
+                     hipStream_t stream) {
   const uint32_t npix = rp.width * rp.height;
-  hipLaunchKernelGGL(k_finalize, dim3((npix + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, rp, radiance, fb,
-                     reset, aov_reset, aov_count);
+  hipLaunchKernelGGL(k_finalize, dim3((npix + kBlock - 1) / kBlock + 1), dim3(kBlock), 0, stream, rp, radiance, fb,
+                     reset, aov_reset, aov_count, ctr, cap, report);
 }
 
 
