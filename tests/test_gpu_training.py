@@ -42,3 +42,39 @@ def test_backward_at_ragged_levels(N, H, W):
             a, b = g[at:at + n], gr[at:at + n]
             at += n
             assert np.linalg.norm(a - b) <= 1e-2 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("N,H,W", [(4, 256, 256), (2, 128, 128), (3, 88, 128)],
+                         ids=["16-row-tiles", "32-chunks", "33-chunks"])
+def test_batch_gradient_is_the_sum_over_its_images(N, H, W):
+    """Gradients of a batch against the sum of its images' own, which take other routes: the
+    batch of 262144 pixels convolves 16-row tiles in launches of their own and its images
+    8-row tiles beside the weight gradient; 32 partial sums are added in registers, 33 in LDS.
+    The terms are the same bits (the forward outputs are checked to be), only the order of
+    their fp32 additions differs: chains of at most 2^14 additions of terms of either sign
+    round by about sqrt(2^14) 2^-24 = 7.6e-6 of a sum; 1e-4 in relative norm per parameter
+    block."""
+    from oracle import unet_ref as U
+    rng = np.random.default_rng(N * H)
+    rend = Renderer(0)
+    try:
+        rend.denoiser_set_params(U.init_params(17))
+        feats = np.zeros((N, H, W, 16), np.float32)
+        feats[..., :10] = rng.normal(0.5, 0.5, (N, H, W, 10))
+        dout = rng.normal(size=(N, H, W, 32)).astype(np.float32)
+        dout[..., 3:] = 0
+        out = rend.denoiser_forward(feats)
+        g = rend.denoiser_backward(dout).astype(np.float64)
+        total = np.zeros_like(g)
+        for n in range(N):
+            one = rend.denoiser_forward(feats[n:n + 1])
+            assert np.array_equal(np.asarray(one)[0].view(np.uint32), np.asarray(out)[n].view(np.uint32))
+            total += rend.denoiser_backward(dout[n:n + 1])
+    finally:
+        rend.close()
+    at = 0
+    for ci, co, _ in U.SPEC:
+        for n in (co * 9 * ci, co):
+            a, b = g[at:at + n], total[at:at + n]
+            at += n
+            assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b)

@@ -138,7 +138,8 @@ hipError_t Unet::ensure(int N, int H, int W, hipStream_t s) {
   }
   wpart_elems_ = wp;
   if ((e = alloc(wp * 4, reinterpret_cast<void**>(&wpart_))) != hipSuccess) return e;
-  if ((e = alloc(size_t(kBiasBlocks) * 256 * 4, reinterpret_cast<void**>(&bpart_))) != hipSuccess) return e;
+  for (float*& b : bpart_)
+    if ((e = alloc(size_t(kBiasBlocks) * 256 * 4, reinterpret_cast<void**>(&b))) != hipSuccess) return e;
   if ((e = alloc((P0 / 256 + 2) * 4, reinterpret_cast<void**>(&lpart_))) != hipSuccess) return e;
   N_ = N;
   H_ = H;
@@ -222,13 +223,17 @@ hipError_t Unet::forward(const uint16_t* x, int N, int H, int W, hipStream_t s, 
 hipError_t Unet::backward(const float* dout, int N, int H, int W, hipStream_t s) {
   if (N != N_ || H != H_ || W != W_ || !x_ || !have_output_) return hipErrorInvalidValue;
   const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4, H3 = H / 8, W3 = W / 8;
-  // one conv layer: gradient in (fp32, post-activation) -> dW, db, gradient out (fp32)
+  // one conv layer: gradient in (fp32, post-activation) -> dW, db (summed with the next layer),
+  // gradient out (fp32)
+  DnSums sums;
+  int turn = 0;
   auto layer = [&](int i, const uint16_t* coarse, int c1, const uint16_t* in, int h, int w, const DnGrad& gin,
                    float* gout) {
     const Conv& c = convs_[i];
-    dn_layer_bwd(gin, c.relu ? act_[i] : nullptr, in, coarse, c1, dz_, N, h, w, c.cin, c.cout, wpart_, bpart_,
-                 g_ + c.woff, g_ + c.boff, s);
-    if (gout) dn_conv3x3(dz_, wd_ + c.woff, nullptr, gout, N, h, w, c.cout, c.cin, false, true, s);
+    float* const bpart = bpart_[turn ^= 1];
+    dn_relu_bias(gin, c.relu ? act_[i] : nullptr, dz_, N, h, w, c.cout, bpart, sums, s);
+    dn_conv_wgrad(in, coarse, c1, dz_, N, h, w, c.cin, c.cout, wpart_, wd_ + c.woff, gout, s);
+    sums = DnSums{wpart_, dn_wgrad_chunks(N, h, w), size_t(c.cout) * 9 * c.cin, g_ + c.woff, bpart, c.cout, g_ + c.boff};
   };
   const auto plain = [](const float* g) { return DnGrad{kGradPlain, g}; };
   // the coarse and the skip share of a concatenated input's gradient (the skip tensor was
@@ -250,6 +255,7 @@ hipError_t Unet::backward(const float* dout, int N, int H, int W, hipStream_t s)
   layer(E1A, nullptr, 0, p0_, H1, W1, plain(gA_), gB_);  // gB = d p0 (32 @H1)
   layer(E0B, nullptr, 0, act_[E0A], H, W, skip(gu0_, 96, 64, gB_), gA_);
   layer(E0A, nullptr, 0, x_, H, W, plain(gA_), nullptr);  // the input gradient of the network is not needed
+  dn_sums(sums, s);
   return hipGetLastError();
 }
 

@@ -50,13 +50,26 @@ struct DnGrad {
   int gc = 0, c0 = 0;             // kGradUp, kGradSkip: channels of g, first of this tensor's share
   const float* pooled = nullptr;  // kGradSkip
 };
-// One layer's backward but for the input gradient: dZ = bf16(gradient masked by Y > 0; Y
-// null: no mask), the bias gradient db = its per-channel sums, the weight gradient dW.
-// Cout <= 128, a multiple of 32; wpartial: dn_wgrad_chunks x Cout x 9 x Cin; bpartial:
-// kBiasBlocks x Cout.
-void dn_layer_bwd(const DnGrad& grad, const uint16_t* Y, const uint16_t* X, const uint16_t* coarse, int c1, uint16_t* dZ,
-                  int N, int H, int W, int Cin, int Cout, float* wpartial, float* bpartial, float* dW, float* db,
-                  hipStream_t s);
+// Partial sums of a layer's parameter gradients and where they go (wpartial null: none).
+struct DnSums {
+  const float* wpartial = nullptr;  // chunks x n_weights
+  int chunks = 0;
+  size_t n_weights = 0;
+  float* dW = nullptr;
+  const float* bpartial = nullptr;  // kBiasBlocks x cout
+  int cout = 0;
+  float* db = nullptr;
+};
+// One layer's backward, Cout <= 128, a multiple of 32. dn_relu_bias: dZ = bf16(gradient
+// masked by Y > 0; Y null: no mask), its sums per channel and block in bpartial, and the
+// layer above's sums. dn_conv_wgrad: the weight gradient's partial sums (dn_wgrad_chunks x
+// Cout x 9 x Cin) and the input gradient gout (fp32; null: not needed) from the flipped
+// weights Wd. dn_sums: a layer's sums alone.
+void dn_relu_bias(const DnGrad& grad, const uint16_t* Y, uint16_t* dZ, int N, int H, int W, int Cout, float* bpartial,
+                  const DnSums& above, hipStream_t s);
+bool dn_conv_wgrad(const uint16_t* X, const uint16_t* coarse, int c1, const uint16_t* dZ, int N, int H, int W, int Cin,
+                   int Cout, float* wpartial, const uint16_t* Wd, float* gout, hipStream_t s);
+void dn_sums(const DnSums& p, hipStream_t s);
 void dn_features(const float4* color, const float4* albedo, const float4* normal, uint16_t* out, size_t P,
                  hipStream_t s);
 void dn_target(const float4* color, float* out, size_t P, hipStream_t s);
@@ -129,7 +142,8 @@ class Unet {
   // backward scratch
   float *gA_ = nullptr, *gB_ = nullptr, *gu0_ = nullptr, *gu1_ = nullptr, *gu2_ = nullptr, *dout_ = nullptr;
   uint16_t* dz_ = nullptr;
-  float *wpart_ = nullptr, *bpart_ = nullptr, *lpart_ = nullptr;
+  float *wpart_ = nullptr, *lpart_ = nullptr;
+  float* bpart_[2] = {};  // by turns: a layer's is summed while the next layer's is written
   size_t wpart_elems_ = 0;
   int N_ = 0, H_ = 0, W_ = 0;
   uint32_t t_ = 0;

@@ -80,21 +80,31 @@ constexpr int kPosStride = 40;           // bf16 per staged position (32 + 8 pad
 constexpr int kRowPitch = 112 * 8;       // bf16 per staged patch row (18 positions + padding)
 constexpr int kWStride = 9 * 32 + 8;     // bf16 per staged output channel
 
+// LDS of a k_conv workgroup; one spare 16-byte slot at the end of patch and wl takes the
+// stores of idle threads.
+template <int MB, int NB, int EPI>
+struct ConvLds {
+  static constexpr int TH = 8 * MB, PH = TH + 2, PW = kTileW + 2;
+  static constexpr int OS = 32 * NB + 8;                             // bf16 per pixel in the output staging
+  static constexpr int OWAVE = (EPI == kEpiF32 ? 8 : MB * 32 * OS);  // output staging per wave (bf16)
+  alignas(16) uint16_t patch[PH * kRowPitch + 8];
+  alignas(16) uint16_t wl[32 * NB * kWStride + 8];
+  alignas(16) uint16_t ob[4 * OWAVE];
+  alignas(16) float bl[32 * NB];
+};
+
+// The workgroup `block` of `blocks` (a multiple of 8).
 template <int MB, int NB, int EPI, bool SC, bool C16>
-__global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
-  constexpr int TH = 8 * MB, PH = TH + 2, PW = kTileW + 2, NPOS = PH * PW;
+__device__ __forceinline__ void conv_block(const ConvArgs& a, unsigned block, unsigned blocks, ConvLds<MB, NB, EPI>& lds) {
+  using L = ConvLds<MB, NB, EPI>;
+  constexpr int TH = L::TH, PH = L::PH, PW = L::PW, NPOS = PH * PW, OS = L::OS, OWAVE = L::OWAVE;
   constexpr int PLOADS = (NPOS * 4 + 255) / 256;
   constexpr int WLOADS = (32 * NB * 9 * 4 + 255) / 256;
-  constexpr int OS = 32 * NB + 8;                                 // bf16 per pixel in the output staging
-  constexpr int OWAVE = (EPI == kEpiF32 ? 8 : MB * 32 * OS);      // output staging per wave (bf16)
   constexpr int PARTS = 4 * NB;                                   // 16-byte parts per staged pixel
   constexpr int FLUSH = (MB * 32 * PARTS) / 64;                   // 16-byte stores per lane per tile
   constexpr int kOOB = 0x7fffffff;                                // buffer offset past every range
-  // one spare 16-byte slot at the end of patch and wl takes the stores of idle threads
-  __shared__ __align__(16) uint16_t patch[PH * kRowPitch + 8];
-  __shared__ __align__(16) uint16_t wl[32 * NB * kWStride + 8];
-  __shared__ __align__(16) uint16_t ob[4 * OWAVE];
-  __shared__ __align__(16) float bl[32 * NB];
+  uint16_t *const patch = lds.patch, *const wl = lds.wl, *const ob = lds.ob;
+  float* const bl = lds.bl;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int H = a.H, W = a.W, Cin = a.c1 + a.cx, Cout = a.cout;
   constexpr int gs = C16 ? 1 : 2;    // log2 of 16-byte groups per staged position
@@ -105,15 +115,15 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
   const int tiles_x = W / kTileW, tiles_y = (H + TH - 1) / TH;
   const int total = tiles_x * tiles_y * a.N * a.groups;
   // Persistent workgroups. Workgroups are dealt round-robin over the 8 XCDs, so XCD
-  // x = blockIdx % 8 gets one contiguous range of items (neighbouring tiles share
+  // x = block % 8 gets one contiguous range of items (neighbouring tiles share
   // their halo rows in that XCD's L2); its workgroups stride through the range by
   // `per`, a multiple of the group count, so one workgroup keeps one channel group.
   // Item order: channel group fastest, then tile column, tile row, image.
-  const int per = static_cast<int>(gridDim.x) >> 3, xcd = static_cast<int>(blockIdx.x) & 7;
+  const int per = static_cast<int>(blocks) >> 3, xcd = static_cast<int>(block) & 7;
   const int q = total >> 3, rem = total & 7;
   const int begin = xcd * q + (xcd < rem ? xcd : rem);
   const int end = begin + q + (xcd < rem ? 1 : 0);
-  const int first = begin + (static_cast<int>(blockIdx.x) >> 3);
+  const int first = begin + (static_cast<int>(block) >> 3);
   if (first >= end) return;
   struct Step {
     int it, ch;  // item, input-channel chunk
@@ -432,13 +442,19 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
   if (pend) flush(pend_step);
 }
 
+template <int MB, int NB, int EPI, bool SC, bool C16>
+__global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
+  __shared__ ConvLds<MB, NB, EPI> lds;
+  conv_block<MB, NB, EPI, SC, C16>(a, blockIdx.x, gridDim.x, lds);
+}
+
 // ------------------------------------------------------------------------------------
 // Weight gradient: dW[co][tap][ci] = sum_p dZ[p][co] X[p + s(tap)][ci] (X optionally
 // [upsample(coarse) | X] as in the forward convolution), as an MFMA GEMM
 // with M = co (32-block), N = ci (32-block), K = pixels. Each workgroup covers kWgradTiles
 // consecutive 8x16 pixel tiles and writes its partial sums to
 // partial[chunk][co][tap][ci]; a fixed-order reduction over chunks follows.
-// Grid: (n_chunks, Cout/32 * ceil(Cin/32)); wave w handles the taps of kernel row w.
+// Blocks: n_chunks x (Cout/32 * ceil(Cin/32)); wave w handles the taps of kernel row w.
 //
 // The fragments hold eight consecutive pixels of one channel, while the tensors have the
 // channels together, so staging transposes: a thread loads 8 channels of four neighbouring
@@ -448,26 +464,35 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
 // in registers. The loads of the next kWgAhead tiles are in flight while a tile is
 // multiplied: training crops leave at most a block per CU, so a chunk's time is its tiles'
 // load latency. (Element by element staging took 220 us a layer on average at 8 x 128 x 128;
-// one tile ahead, through loads in branches, 24 us; now 16 us.)
+// one tile ahead, through loads in branches, 24 us; now 16 us, with two tiles ahead as with
+// three.)
 constexpr int kWgThreads = 192;
-constexpr int kWgAhead = 3;                   // tiles whose loads are in flight
+constexpr int kWgAhead = 2;                   // tiles whose loads are in flight
 constexpr int kWgRow = 24;                    // LDS pixels per staged input row (18 used)
 constexpr int kWgXs = kPatchH * kWgRow + 8;   // bf16 per channel: an odd number of 16-byte slots
 constexpr int kWgZs = kTileH * kTileW + 8;
 constexpr int kWgXItems = kPatchH * 5 * 4;    // rows x pixel quads x channel octets (dZ: 8 x 4 x 4 = 128)
 constexpr int kWgItems = 2;                   // per thread
 
-__global__ __launch_bounds__(kWgThreads) void k_wgrad(const uint16_t* __restrict__ X, const uint16_t* __restrict__ coarse,
-                                                      int c1, const uint16_t* __restrict__ dZ, float* __restrict__ partial,
-                                                      int N, int H, int W, int Cin, int Cout) {
-  __shared__ __align__(16) uint16_t xs[32 * kWgXs];  // [ci][row][pixel]
-  __shared__ __align__(16) uint16_t zs[32 * kWgZs];  // [co][row][pixel]
+struct WgradArgs {
+  const uint16_t *x, *coarse, *dz;
+  float* partial;
+  int c1, N, H, W, cin, cout, chunks;
+};
+struct WgradLds {
+  alignas(16) uint16_t xs[32 * kWgXs];  // [ci][row][pixel]
+  alignas(16) uint16_t zs[32 * kWgZs];  // [co][row][pixel]
+};
+__device__ __forceinline__ void wgrad_block(const WgradArgs& a, int chunk, int channels, WgradLds& lds) {
+  uint16_t *const xs = lds.xs, *const zs = lds.zs;
+  const uint16_t *const X = a.x, *const coarse = a.coarse, *const dZ = a.dz;
+  const int c1 = a.c1, N = a.N, H = a.H, W = a.W, Cin = a.cin, Cout = a.cout;
   const int tid = threadIdx.x, lane = tid & 63, ky = tid >> 6;
   const int ci_blocks = (Cin + 31) / 32;
-  const int cb = blockIdx.y / ci_blocks, ib = blockIdx.y - cb * ci_blocks;
+  const int cb = channels / ci_blocks, ib = channels - cb * ci_blocks;
   const int tiles_x = W / kTileW, tiles_y = (H + kTileH - 1) / kTileH;
   const int tiles_img = tiles_x * tiles_y;
-  const int first = blockIdx.x * kWgradTiles;
+  const int first = chunk * kWgradTiles;
   const int last = min(first + kWgradTiles, tiles_img * N);
   const bool up = ib * 32 < c1;  // this input block comes from the upsampled coarse tensor
   const int cx = Cin - c1;
@@ -573,7 +598,7 @@ __global__ __launch_bounds__(kWgThreads) void k_wgrad(const uint16_t* __restrict
   }
   // write partial: rows = co (A rows), cols = ci (B cols)
   const size_t wsize = static_cast<size_t>(Cout) * 9 * Cin;
-  float* out = partial + blockIdx.x * wsize;
+  float* out = a.partial + chunk * wsize;
   const int ci = ib * 32 + (lane & 31);
   if (ci >= Cin) return;
 #pragma unroll
@@ -584,37 +609,88 @@ __global__ __launch_bounds__(kWgThreads) void k_wgrad(const uint16_t* __restrict
       out[(static_cast<size_t>(co) * 9 + ky * 3 + kx) * Cin + ci] = acc[kx][r];
     }
 }
+__global__ __launch_bounds__(kWgThreads) void k_wgrad(WgradArgs a) {
+  __shared__ WgradLds lds;
+  wgrad_block(a, blockIdx.x, blockIdx.y, lds);
+}
 
-// out[i] = sum over chunks c (in order) of partial[c][i]. A block takes 32 outputs: its 256
-// threads bring 128 chunks at a time into LDS with all loads in flight, then 32 threads add
-// them in order (one thread per output with its loads in a row was bound by their latency:
-// 36 us a layer on average at 8 x 128 x 128, 6.5 us now).
-// Two sums in one launch: blocks below `blocks_a` reduce the first.
-constexpr int kReduceOuts = 32, kReduceChunks = 128;
+// A layer's input gradient (a convolution of dZ) and its weight gradient in one launch: they
+// are independent and, at the sizes of training crops, each is a chain of load latencies
+// that leaves most of the chip idle (8 x 128 x 128: 12 and 16 us a layer on average one after
+// the other, 20 us together). The last conv_blocks workgroups convolve; the wave that the
+// weight gradient has no use for ends. Held to 168 VGPRs, 3 waves per SIMD, which two tiles
+// ahead in the weight gradient allow (a step at 8 x 128 x 128: 0.79 ms; with three tiles
+// ahead at 2 waves 0.82; convolution first 0.80).
+template <int MB, int NB, bool SC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_conv_wgrad(ConvArgs c, unsigned conv_blocks,
+                                                                                           WgradArgs w) {
+  __shared__ union {
+    ConvLds<MB, NB, kEpiF32> conv;
+    WgradLds wgrad;
+  } lds;
+  const unsigned wgrad_blocks = gridDim.x - conv_blocks;
+  if (blockIdx.x >= wgrad_blocks) {
+    conv_block<MB, NB, kEpiF32, SC, false>(c, blockIdx.x - wgrad_blocks, conv_blocks, lds.conv);
+  } else if (threadIdx.x < kWgThreads) {
+    const int b = static_cast<int>(blockIdx.x);
+    wgrad_block(w, b % w.chunks, b / w.chunks, lds.wgrad);
+  }
+}
+
+// out[i] = sum over chunks c (in order) of partial[c][i], all loads in flight (one after the
+// other they were bound by their latency: 36 us a layer on average at 8 x 128 x 128).
+// Up to kReduceDirect chunks a thread adds one output's in registers. Beyond, a block takes
+// kReduceOuts outputs: its threads bring 128 chunks at a time into LDS and kReduceOuts of
+// them add them in order.
+// A layer's two sums share a launch: the first blocks reduce the biases' (256 chunks, the
+// longest chain), the others the weights'.
+constexpr int kReduceOuts = 32, kReduceChunks = 128, kReduceDirect = 32;
 struct ChunkSum {
   const float* partial;
   int n_chunks;
   size_t n;
   float* out;
 };
-__global__ __launch_bounds__(256) void k_reduce_chunks(ChunkSum sa, ChunkSum sb, unsigned blocks_a) {
-  __shared__ float lds[kReduceChunks * kReduceOuts];
-  const ChunkSum r = blockIdx.x < blocks_a ? sa : sb;
-  const unsigned block = blockIdx.x < blocks_a ? blockIdx.x : blockIdx.x - blocks_a;
+struct LayerSums {
+  ChunkSum weights, biases;
+  unsigned first, blocks;
+};
+struct ReduceLds {
+  float v[kReduceChunks * kReduceOuts];
+};
+template <int kThreads>
+__device__ __forceinline__ void reduce_block(const LayerSums& sums, unsigned block, ReduceLds& l) {
+  float* const lds = l.v;
+  const ChunkSum r = block < sums.first ? sums.biases : sums.weights;
+  if (block >= sums.first) block -= sums.first;
+  if (r.n_chunks <= kReduceDirect) {
+    const size_t i = static_cast<size_t>(block) * kThreads + threadIdx.x;
+    if (i >= r.n) return;
+    float v[kReduceDirect];
+#pragma unroll
+    for (int c = 0; c < kReduceDirect; ++c) v[c] = c < r.n_chunks ? r.partial[static_cast<size_t>(c) * r.n + i] : 0.f;
+    float t = 0.f;
+#pragma unroll
+    for (int c = 0; c < kReduceDirect; ++c)
+      if (c < r.n_chunks) t += v[c];
+    r.out[i] = t;
+    return;
+  }
+  constexpr int kParts = kThreads / kReduceOuts, kEach = kReduceChunks / kParts;
   const int o = threadIdx.x & (kReduceOuts - 1), part = threadIdx.x / kReduceOuts;
   const size_t i = static_cast<size_t>(block) * kReduceOuts + o;
   float t = 0.f;
   for (int c0 = 0; c0 < r.n_chunks; c0 += kReduceChunks) {
     const int m = min(kReduceChunks, r.n_chunks - c0);
-    float v[kReduceChunks / 8];
+    float v[kEach];
 #pragma unroll
-    for (int k = 0; k < kReduceChunks / 8; ++k) {
-      const int c = part + 8 * k;
+    for (int k = 0; k < kEach; ++k) {
+      const int c = part + kParts * k;
       v[k] = c < m && i < r.n ? r.partial[static_cast<size_t>(c0 + c) * r.n + i] : 0.f;
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < kReduceChunks / 8; ++k) lds[(part + 8 * k) * kReduceOuts + o] = v[k];
+    for (int k = 0; k < kEach; ++k) lds[(part + kParts * k) * kReduceOuts + o] = v[k];
     __syncthreads();
     if (part == 0) {
       int c = 0;
@@ -630,13 +706,18 @@ __global__ __launch_bounds__(256) void k_reduce_chunks(ChunkSum sa, ChunkSum sb,
   }
   if (part == 0 && i < r.n) r.out[i] = t;
 }
+__global__ __launch_bounds__(256) void k_reduce_chunks(LayerSums sums) {
+  __shared__ ReduceLds lds;
+  reduce_block<256>(sums, blockIdx.x, lds);
+}
 
 // dZ = bf16(dY * (Y > 0)) (ReLU backward; Y is the post-activation output, null for a
 // linear layer) and the bias gradient's partial sums: block b takes pixels
 // [b*P/B, (b+1)*P/B), stages their dZ in LDS and adds it per channel in pixel order. Bound by
-// its 8 bytes a value. (As two kernels the sums re-read dZ with C threads a block: 40 + 7 us
-// a layer on average at 8 x 128 x 128, plus 6 launches that wrote the gathered gradients; now
-// 11 us and none.)
+// its 8 bytes a value and, at training crops, by the latency of one block per CU. (As two
+// kernels the sums re-read dZ with C threads a block: 40 + 7 us a layer on average at
+// 8 x 128 x 128, plus 6 launches that wrote the gathered gradients; as one of 256 threads
+// 10 us and 6.5 for the sums of the layer above in a launch of their own; now 11 for both.)
 // dY is formed on the way from what the layers above left:
 //   kGradPlain  gradient of this tensor
 //   kGradUp     gradient g of [upsample(this) | skip] at twice the side: the 2x2 sum
@@ -669,18 +750,29 @@ __device__ __forceinline__ float4 grad4(const GradSrc& s, int C, unsigned p, int
   return make_float4(k.x + 0.25f * h.x, k.y + 0.25f * h.y, k.z + 0.25f * h.z, k.w + 0.25f * h.w);
 }
 
-__global__ __launch_bounds__(256) void k_relu_bias(GradSrc src, const uint16_t* __restrict__ Y,
+// The blocks from kBiasBlocks on add up the parameter gradients of the layer above, whose
+// partial sums the previous launch left.
+constexpr int kBiasThreads = 512;
+__global__ __launch_bounds__(kBiasThreads) void k_relu_bias(GradSrc src, const uint16_t* __restrict__ Y,
                                                    uint16_t* __restrict__ dZ, size_t P, int C,
-                                                   float* __restrict__ partial) {
-  __shared__ __align__(16) uint16_t lds[kBiasElems];
-  const size_t p0 = P * blockIdx.x / gridDim.x, p1 = P * (blockIdx.x + 1) / gridDim.x;
+                                                   float* __restrict__ partial, LayerSums above) {
+  __shared__ union {
+    alignas(16) uint16_t z[kBiasElems];
+    ReduceLds reduce;
+  } u;
+  if (blockIdx.x >= kBiasBlocks) {
+    reduce_block<kBiasThreads>(above, blockIdx.x - kBiasBlocks, u.reduce);
+    return;
+  }
+  uint16_t* const lds = u.z;
+  const size_t p0 = P * blockIdx.x / kBiasBlocks, p1 = P * (blockIdx.x + 1) / kBiasBlocks;
   const int pixels = kBiasElems / C, octets = C / 8;
   float t = 0.f;
   for (size_t p = p0; p < p1; p += pixels) {
     const int m = static_cast<int>(p1 - p < static_cast<size_t>(pixels) ? p1 - p : pixels);
     __syncthreads();
 #pragma unroll 4
-    for (int i = threadIdx.x; i < m * octets; i += 256) {
+    for (int i = threadIdx.x; i < m * octets; i += kBiasThreads) {
       const int q = static_cast<int>(static_cast<unsigned>(i) / static_cast<unsigned>(octets)), c = (i - q * octets) * 8;
       const unsigned pq = static_cast<unsigned>(p) + static_cast<unsigned>(q);
       const float4 g0 = grad4(src, C, pq, c), g1 = grad4(src, C, pq, c + 4);
@@ -863,9 +955,10 @@ using namespace dn;
 
 // Persistent grid: as many workgroups as fit on the device at once (occupancy of the
 // instantiation x CUs), a multiple of 8 (one share per XCD) whose per-XCD share is a
-// multiple of the channel-group count, so a workgroup keeps one group's weights.
+// multiple of the channel-group count, so a workgroup keeps one group's weights. `beside`:
+// workgroups of other work in the same launch, which get up to half of the room.
 template <typename K>
-static unsigned persistent_blocks(K kernel, long items, int groups) {
+static unsigned persistent_blocks(K kernel, long items, int groups, long beside = 0) {
   static thread_local int cus = 0, dev = -1;
   int d = 0;
   (void)hipGetDevice(&d);
@@ -875,7 +968,8 @@ static unsigned persistent_blocks(K kernel, long items, int groups) {
   }
   int occ = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, 256, 0) != hipSuccess || occ <= 0) occ = 1;
-  long per = long(cus) * occ / 8;
+  const long fit = long(cus) * occ;
+  long per = (fit - beside > fit / 2 ? fit - beside : fit / 2) / 8;
   per = per / groups * groups;
   if (per < groups) per = groups;
   const long need = (items + 7) / 8;
@@ -910,7 +1004,12 @@ static void launch_conv(const ConvArgs& a, int epi, long items, hipStream_t s) {
 
 // Tile shape per layer: 16-row tiles (MB = 2) unless that leaves < 1024 tiles, then
 // 8-row tiles with 64-channel groups (NB = 2) when Cout is a multiple of 64.
-bool dn_conv(const DnConv& c, hipStream_t s) {
+struct ConvPlan {
+  ConvArgs a;
+  int MB, NB;
+  long items;
+};
+static bool plan_conv(const DnConv& c, ConvPlan& p) {
   const int Cin = c.c1 + c.cx;
   const bool shape_ok = (Cin == 16 && c.c1 == 0) || (c.c1 % 32 == 0 && c.cx % 32 == 0 && Cin > 0);
   if (!shape_ok || c.cout % 32 || c.W % kTileW || c.H <= 0 || c.N <= 0) return false;
@@ -922,10 +1021,10 @@ bool dn_conv(const DnConv& c, hipStream_t s) {
   if (long(c.H) * c.W * widest >= (1L << 31)) return false;
   if (c.epi == kEpiRadiance && Cin > 32) return false;  // feature prefetch assumes one chunk
   const long tiles16 = long(c.W / kTileW) * ((c.H + 15) / 16) * c.N;
-  const int MB = tiles16 >= 1024 ? 2 : 1;
+  const int MB = p.MB = tiles16 >= 1024 ? 2 : 1;
   const long tiles = long(c.W / kTileW) * ((c.H + 8 * MB - 1) / (8 * MB)) * c.N;
-  const int NB = MB == 1 && c.cout % 64 == 0 ? 2 : 1;  // MB = NB = 2 would need > 100 KB of LDS
-  ConvArgs a;
+  const int NB = p.NB = MB == 1 && c.cout % 64 == 0 ? 2 : 1;  // MB = NB = 2 would need > 100 KB of LDS
+  ConvArgs& a = p.a;
   a.x = c.x;
   a.coarse = c.coarse;
   a.c1 = c.c1;
@@ -941,11 +1040,17 @@ bool dn_conv(const DnConv& c, hipStream_t s) {
   a.H = c.H;
   a.W = c.W;
   a.groups = c.cout / (32 * NB);
-  const long items = tiles * a.groups;
-  if (MB == 2) {
-    launch_conv<2, 1>(a, c.epi, items, s);
+  p.items = tiles * a.groups;
+  return true;
+}
+
+bool dn_conv(const DnConv& c, hipStream_t s) {
+  ConvPlan p;
+  if (!plan_conv(c, p)) return false;
+  if (p.MB == 2) {
+    launch_conv<2, 1>(p.a, c.epi, p.items, s);
   } else {
-    if (NB == 2) launch_conv<1, 2>(a, c.epi, items, s); else launch_conv<1, 1>(a, c.epi, items, s);
+    if (p.NB == 2) launch_conv<1, 2>(p.a, c.epi, p.items, s); else launch_conv<1, 1>(p.a, c.epi, p.items, s);
   }
   return true;
 }
@@ -972,20 +1077,64 @@ int dn_wgrad_chunks(int N, int H, int W) {
   return (tiles + kWgradTiles - 1) / kWgradTiles;
 }
 
-void dn_layer_bwd(const DnGrad& grad, const uint16_t* Y, const uint16_t* X, const uint16_t* coarse, int c1, uint16_t* dZ,
-                  int N, int H, int W, int Cin, int Cout, float* wpartial, float* bpartial, float* dW, float* db,
-                  hipStream_t s) {
+static LayerSums layer_sums(const DnSums& p, int threads) {
+  if (!p.wpartial) return LayerSums{};
+  const auto blocks = [&](int chunks, size_t n) {
+    return blocks_for(n, static_cast<unsigned>(chunks <= kReduceDirect ? threads : kReduceOuts));
+  };
+  const unsigned first = blocks(kBiasBlocks, p.cout);
+  return LayerSums{ChunkSum{p.wpartial, p.chunks, p.n_weights, p.dW},
+                   ChunkSum{p.bpartial, kBiasBlocks, static_cast<size_t>(p.cout), p.db}, first,
+                   first + blocks(p.chunks, p.n_weights)};
+}
+
+void dn_relu_bias(const DnGrad& grad, const uint16_t* Y, uint16_t* dZ, int N, int H, int W, int Cout, float* bpartial,
+                  const DnSums& above, hipStream_t s) {
   const GradSrc src{grad.g, grad.pooled, grad.kind, H, W, grad.gc, grad.c0};
-  hipLaunchKernelGGL(k_relu_bias, dim3(kBiasBlocks), dim3(256), 0, s, src, Y, dZ, static_cast<size_t>(N) * H * W, Cout,
-                     bpartial);
-  const int chunks = dn_wgrad_chunks(N, H, W);
-  const dim3 grid(chunks, (Cout / 32) * ((Cin + 31) / 32));
-  hipLaunchKernelGGL(k_wgrad, grid, dim3(kWgThreads), 0, s, X, coarse, c1, dZ, wpartial, N, H, W, Cin, Cout);
-  const size_t n = static_cast<size_t>(Cout) * 9 * Cin;
-  const unsigned blocks = blocks_for(n, kReduceOuts);
-  hipLaunchKernelGGL(k_reduce_chunks, dim3(blocks + blocks_for(Cout, kReduceOuts)), dim3(256), 0, s,
-                     ChunkSum{wpartial, chunks, n, dW}, ChunkSum{bpartial, kBiasBlocks, static_cast<size_t>(Cout), db},
-                     blocks);
+  const LayerSums sums = layer_sums(above, kBiasThreads);
+  hipLaunchKernelGGL(k_relu_bias, dim3(kBiasBlocks + sums.blocks), dim3(kBiasThreads), 0, s, src, Y, dZ,
+                     static_cast<size_t>(N) * H * W, Cout, bpartial, sums);
+}
+
+void dn_sums(const DnSums& p, hipStream_t s) {
+  const LayerSums sums = layer_sums(p, 256);
+  if (sums.blocks) hipLaunchKernelGGL(k_reduce_chunks, dim3(sums.blocks), dim3(256), 0, s, sums);
+}
+
+template <int MB, int NB, bool SC>
+static void launch_conv_wgrad(const ConvPlan& p, const WgradArgs& w, unsigned wblocks, hipStream_t s) {
+  const unsigned blocks = persistent_blocks(k_conv_wgrad<MB, NB, SC>, p.items, p.a.groups, wblocks);
+  hipLaunchKernelGGL((k_conv_wgrad<MB, NB, SC>), dim3(blocks + wblocks), dim3(256), 0, s, p.a, blocks, w);
+}
+
+// One launch for the two where the convolution has 8-row tiles, which is where either leaves
+// compute units idle; each alone, with its own registers and occupancy, above.
+bool dn_conv_wgrad(const uint16_t* X, const uint16_t* coarse, int c1, const uint16_t* dZ, int N, int H, int W, int Cin,
+                   int Cout, float* wpartial, const uint16_t* Wd, float* gout, hipStream_t s) {
+  const WgradArgs w{X, coarse, dZ, wpartial, c1, N, H, W, Cin, Cout, dn_wgrad_chunks(N, H, W)};
+  const unsigned channels = (Cout / 32) * ((Cin + 31) / 32), wblocks = w.chunks * channels;
+  DnConv c;
+  ConvPlan p;
+  if (gout) {
+    c.x = dZ;
+    c.cx = Cout;
+    c.w = Wd;
+    c.y = gout;
+    c.cout = Cin;
+    c.N = N;
+    c.H = H;
+    c.W = W;
+    c.epi = kEpiF32;
+    if (!plan_conv(c, p)) return false;
+    if (p.MB == 1) {
+      if (p.NB == 2) launch_conv_wgrad<1, 2, false>(p, w, wblocks, s);
+      else if (Cout == 32) launch_conv_wgrad<1, 1, true>(p, w, wblocks, s);
+      else launch_conv_wgrad<1, 1, false>(p, w, wblocks, s);
+      return true;
+    }
+  }
+  hipLaunchKernelGGL(k_wgrad, dim3(w.chunks, channels), dim3(kWgThreads), 0, s, w);
+  return !gout || dn_conv(c, s);
 }
 void dn_features(const float4* color, const float4* albedo, const float4* normal, uint16_t* out, size_t P,
                  hipStream_t s) {
