@@ -156,7 +156,7 @@ struct trt_context {
   uint64_t frame_id = 0;       // frames rendered by this context
   trt_render_opts last_opts{};
   uint32_t last_sample_offset = 0;
-  DevBuf a_lrem, a_pend, a_key, a_ga, a_gb, a_sga, a_sgb, a_dldi, a_partial, a_out;
+  DevBuf a_lrem, a_pend, a_key, a_ga, a_gb, a_contrib, a_spath, a_dldi, a_partial, a_out;
 
   // denoiser
   std::unique_ptr<Unet> unet;
@@ -1441,8 +1441,8 @@ trt_status trt_backward(trt_context* ctx, const trt_render_opts* o, const float*
   HIPC(ctx->a_key.ensure(R * 4), "alloc adjoint");
   HIPC(ctx->a_ga.ensure(R * 16), "alloc adjoint");
   HIPC(ctx->a_gb.ensure(R * 4), "alloc adjoint");
-  HIPC(ctx->a_sga.ensure(ctx->queue_slots * 16), "alloc adjoint");  // per shadow-queue slot
-  HIPC(ctx->a_sgb.ensure(ctx->queue_slots * 4), "alloc adjoint");
+  HIPC(ctx->a_contrib.ensure(n * 16), "alloc adjoint");
+  HIPC(ctx->a_spath.ensure(ctx->queue_slots * 4), "alloc adjoint");  // per shadow-queue slot
   HIPC(ctx->a_dldi.ensure(uint64_t(W) * H * 12), "alloc adjoint");
   HIPC(ctx->a_partial.ensure(size_t(kGradBlocks) * kGradMatsPerPass * kNumParams * 4), "alloc adjoint");
   HIPC(ctx->a_out.ensure(size_t(nm) * kNumParams * 4 + 16), "alloc adjoint");
@@ -1455,13 +1455,14 @@ trt_status trt_backward(trt_context* ctx, const trt_render_opts* o, const float*
   uint32_t* ctr = ctx->counters.as<uint32_t>();
   AdjBuffers ab;
   ab.dldi = ctx->a_dldi.as<float>();
+  ab.radiance = ctx->radiance.as<float4>();
   ab.lrem = ctx->a_lrem.as<float4>();
+  ab.contrib = ctx->a_contrib.as<float4>();
   ab.pend = ctx->a_pend.as<float4>();
   ab.rec_key = ctx->a_key.as<uint32_t>();
   ab.rec_a = ctx->a_ga.as<float4>();
   ab.rec_b = ctx->a_gb.as<float>();
-  ab.s_ga = ctx->a_sga.as<float4>();
-  ab.s_gb = ctx->a_sgb.as<float>();
+  ab.s_path = ctx->a_spath.as<uint32_t>();
   ab.n_records = R;
   ab.n_paths = n;
   ab.depth = D;
@@ -1483,7 +1484,7 @@ trt_status trt_backward(trt_context* ctx, const trt_render_opts* o, const float*
   DevAccel acc_sh = acc;
   acc_sh.spill = acc.spill + ctx->spill_half;
   hipStream_t stm2 = ctx->stream2;
-  launch_raygen_adj(rp, uint32_t(n), cap, q[0], ctx->radiance.as<float4>(), ab, ctr, stm);
+  launch_raygen_adj(rp, uint32_t(n), cap, q[0], ab, ctr, stm);
   for (uint32_t d = 0; d < D; ++d) {
     const int cur = int(d & 1u), nxt = cur ^ 1;
     const int di = int(d);

@@ -131,24 +131,27 @@ struct FrameBuffers {
 
 // Adjoint (path replay) state. Records: one per (depth, path) slot r = d * n_paths + path,
 // key = material id of the vertex (0xffffffff = none), gradient of parameters 0..3 in
-// rec_a[r] and of parameter 4 in rec_b[r] (valid where the key is). A vertex's record is
-// written whole by one kernel and read whole by the next, at an address that its queue
+// rec_a[r] and of parameter 4 in rec_b[r] (valid where the key is, without kRecUnlit). A
+// vertex's record is written whole by its Shade and read whole by the next vertex's, at an address that its queue
 // neighbours do not share, so the five parameters sit in two arrays (two lines per
 // record), not five; a depth's records lie together, as its launches touch them (neighbouring
 // rays are neighbouring pixels).
 struct AdjBuffers {
   const float* dldi;   // dLoss/dImage, 3 floats per pixel
+  const float4* radiance;  // per path, of the frame
   float4* lrem;        // per path: radiance not yet attributed to earlier vertices
+  float4* contrib;     // per path: next-event contribution of the last vertex, if light reached it
   float4* pend;        // 4 arrays of a float4 per path: (d f / d theta)/f of the pending continuation
                        // (written by a vertex that sends one on, read by the next vertex)
-  uint32_t* rec_key;
+  uint32_t* rec_key;   // material of the record's vertex, | kRecUnlit while it holds no gradient (its
+                       // next-event estimate is zero); kNoHit: no record
   float4* rec_a;
   float* rec_b;
-  float4* s_ga;        // per shadow slot: NEE gradient, params 0..3
-  float* s_gb;         // per shadow slot: NEE gradient, param 4
+  uint32_t* s_path;    // per shadow slot: its path
   size_t n_records, n_paths;
   uint32_t depth;
 };
+constexpr uint32_t kRecUnlit = 1u << 31;
 constexpr int kGradBlocks = 1024;       // fixed: the reduction order is device independent
 constexpr uint32_t kGradMatsPerPass = 512;
 
@@ -193,8 +196,8 @@ void launch_tonemap(const float4* src, uint32_t n, const TonemapParams& tp, ucha
 void launch_finalize(const RenderParams& rp, const float4* radiance, FrameBuffers fb, uint32_t reset,
                      uint32_t aov_reset, uint32_t aov_count, const uint32_t* ctr, uint32_t cap, uint32_t* report,
                      hipStream_t stream);
-void launch_raygen_adj(const RenderParams& rp, uint32_t n_paths, uint32_t cap, RayQueue q, const float4* radiance,
-                       const AdjBuffers& ab, uint32_t* ctr, hipStream_t stream);
+void launch_raygen_adj(const RenderParams& rp, uint32_t n_paths, uint32_t cap, RayQueue q, const AdjBuffers& ab,
+                       uint32_t* ctr, hipStream_t stream);
 void launch_shade_adj(const SceneView& sv, const Material* sampling_mats, const RenderParams& rp, RayQueue q,
                       HitBuf h, RayQueue qn, ShadowQueue sq, const AdjBuffers& ab, SegIn in, uint32_t* next_cnt,
                       uint32_t* shadow_cnt, uint32_t* ctr, uint32_t depth, int grid, hipStream_t stream);
