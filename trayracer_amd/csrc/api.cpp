@@ -1437,7 +1437,7 @@ trt_status trt_backward(trt_context* ctx, const trt_render_opts* o, const float*
   const uint64_t R = n * D;
   const uint32_t nm = uint32_t(ctx->materials.size());
   HIPC(ctx->a_lrem.ensure(n * 16), "alloc adjoint");
-  HIPC(ctx->a_pend.ensure(n * 64), "alloc adjoint");
+  HIPC(ctx->a_pend.ensure(n * 48), "alloc adjoint");
   HIPC(ctx->a_key.ensure(R * 4), "alloc adjoint");
   HIPC(ctx->a_ga.ensure(R * 16), "alloc adjoint");
   HIPC(ctx->a_gb.ensure(R * 4), "alloc adjoint");

@@ -141,7 +141,7 @@ struct AdjBuffers {
   const float4* radiance;  // per path, of the frame
   float4* lrem;        // per path: radiance not yet attributed to earlier vertices
   float4* contrib;     // per path: next-event contribution of the last vertex, if light reached it
-  float4* pend;        // 4 arrays of a float4 per path: (d f / d theta)/f of the pending continuation
+  float4* pend;        // 3 arrays of a float4 per path: (d f / d theta)/f of the pending continuation
                        // (written by a vertex that sends one on, read by the next vertex)
   uint32_t* rec_key;   // material of the record's vertex, | kRecUnlit while it holds no gradient (its
                        // next-event estimate is zero); kNoHit: no record

@@ -1465,9 +1465,10 @@ __global__ __launch_bounds__(kBlock) void k_raygen_adj(RenderParams rp, uint32_t
 }
 
 
-// The adjoint's Shade. Held to 168 VGPRs, 3 waves per SIMD: it moves ~400 bytes a vertex
-// through gathers (queue, hit, records, pending derivatives), 2.5 TB/s, and waits on them
-// (512 x 512 x 64 spp step: 21.6 ms at 3 waves, 22.5 at 2).
+// The adjoint's Shade. Held to 168 VGPRs, 3 waves per SIMD (2 waves: 4 % slower step). VALU
+// issue fills four fifths of its time, gathers by path (records, remaining radiance, pending
+// derivatives: ~250 bytes a vertex) the rest: 1.29 ms a bounce of 512 x 512 x 64 paths, 1.40
+// before a vertex's derivatives shared their terms and came as twelve numbers of fifteen.
 template <int SEP>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_shade_adj(SceneView sv, const Material* sampling_mats, RenderParams rp,
                                                        RayQueue q, HitBuf h, RayQueue qn, ShadowQueue sq,
@@ -1515,7 +1516,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
         float a1 = ab.rec_b[r];
         const float4 c = ab.contrib[path];
         const float4* pp = ab.pend + path;
-        const float4 p0 = pp[0], p1 = pp[np], p2 = pp[2 * np], p3 = pp[3 * np];
+        const float4 p0 = pp[0], p1 = pp[np], p2 = pp[2 * np];
         if (key & kRecUnlit) {  // no light reached it: the record holds nothing yet
           ab.rec_key[r] = key ^ kRecUnlit;
           a4 = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1525,12 +1526,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
           lr.y -= c.y;
           lr.z -= c.z;
         }
-        AdjOut prev;
-        prev.r[0][0] = p0.x; prev.r[0][1] = p0.y; prev.r[0][2] = p0.z;
-        prev.r[1][0] = p0.w; prev.r[1][1] = p1.x; prev.r[1][2] = p1.y;
-        prev.r[2][0] = p1.z; prev.r[2][1] = p1.w; prev.r[2][2] = p2.x;
-        prev.r[3][0] = p2.y; prev.r[3][1] = p2.z; prev.r[3][2] = p2.w;
-        prev.r[4][0] = p3.x; prev.r[4][1] = p3.y; prev.r[4][2] = p3.z;
+        const BsdfGrad prev = {{p0.x, p0.y, p0.z}, {p0.w, p1.x, p1.y}, {p1.z, p1.w, p2.x}, {p2.y, p2.z, p2.w}};
         float g[kNumParams];
         continuation_grad(prev, delta, v3(lr.x, lr.y, lr.z), g);
         ab.rec_a[r] = make_float4(a4.x + g[0], a4.y + g[1], a4.z + g[2], a4.w + g[3]);
@@ -1556,10 +1552,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
         if (out.has_shadow) ab.contrib[path] = make_float4(out.s_contrib.x, out.s_contrib.y, out.s_contrib.z, 0.f);
         float4* pp = ab.pend + path;
         const size_t np = ab.n_paths;
-        pp[0] = make_float4(adj.r[0][0], adj.r[0][1], adj.r[0][2], adj.r[1][0]);
-        pp[np] = make_float4(adj.r[1][1], adj.r[1][2], adj.r[2][0], adj.r[2][1]);
-        pp[2 * np] = make_float4(adj.r[2][2], adj.r[3][0], adj.r[3][1], adj.r[3][2]);
-        pp[3 * np] = make_float4(adj.r[4][0], adj.r[4][1], adj.r[4][2], 0.f);
+        const BsdfGrad& e = adj.rel;
+        pp[0] = make_float4(e.own[0], e.own[1], e.own[2], e.tint[0]);
+        pp[np] = make_float4(e.tint[1], e.tint[2], e.rough[0], e.rough[1]);
+        pp[2 * np] = make_float4(e.rough[2], e.metal[0], e.metal[1], e.metal[2]);
       }
     }
     const bool ext = out.has_ext != 0;

@@ -192,11 +192,56 @@ TRT_HD T3<S> bsdf_f(const BsdfParams<S>& p, V3 wo, V3 wi) {
 // parameter, and the base colour enters directly and through the tint; written out so that
 // each intermediate carries only the derivatives it has (bsdf_f on five-component dual
 // numbers carries all five through every operation, about eight times the arithmetic).
-TRT_HD inline void bsdf_grad(const BsdfParams<float>& p, V3 wo, V3 wi, float g[5][3]) {
-  for (int k = 0; k < 5; ++k) g[k][0] = g[k][1] = g[k][2] = 0.f;
+// The base colour's nine are a diagonal less the tint's luminance weights times one vector:
+//   g[k][c] = (k == c) own[c] - w[k] tint[c],
+// so twelve numbers hold all fifteen (and as many a path carries to its next vertex).
+struct BsdfGrad {
+  float own[3], tint[3], rough[3], metal[3];
+};
+// w[k] above: the weights of lum3
+TRT_FI float lum_weight(int k) { return k == 0 ? 0.2126729f : k == 1 ? 0.7151522f : 0.0721750f; }
+
+// out[k] = sum_c g[k][c] x[c]
+TRT_FI void bsdf_grad_dot(const BsdfGrad& g, V3 x, float out[5]) {
+  const float t = (g.tint[0] * x.x + g.tint[1] * x.y) + g.tint[2] * x.z;
+  out[0] = g.own[0] * x.x - lum_weight(0) * t;
+  out[1] = g.own[1] * x.y - lum_weight(1) * t;
+  out[2] = g.own[2] * x.z - lum_weight(2) * t;
+  out[3] = (g.rough[0] * x.x + g.rough[1] * x.y) + g.rough[2] * x.z;
+  out[4] = (g.metal[0] * x.x + g.metal[1] * x.y) + g.metal[2] * x.z;
+}
+
+// What the derivatives at every wi share (Disney model, wo.z > 0): 1 / luminance, the GGX
+// alphas, their reciprocals and d ln alpha / d roughness, and sqrt(1 + tan^2) of Lambda(wo)
+// with its derivative.
+struct BsdfGradPre {
+  float ilum, ax, ay, iax, iay, lx, ly, so, so_r;
+};
+TRT_HD inline BsdfGradPre bsdf_grad_pre(const BsdfParams<float>& p, V3 wo) {
+  BsdfGradPre q{};
+  if (p.model == kModelLambert || !(wo.z > 0.f)) return q;
+  const float lum = lum3(p.base);
+  q.ilum = lum > 0.f ? 1.f / lum : 0.f;
+  const float aspect = sqrt(1.f - 0.9f * p.anisotropic);
+  const float r2 = p.roughness * p.roughness;
+  const float ux = r2 / aspect, uy = r2 * aspect;
+  q.ax = fmax(ux, 1e-3f);
+  q.ay = fmax(uy, 1e-3f);
+  q.iax = 1.f / q.ax;
+  q.iay = 1.f / q.ay;
+  q.lx = (ux > 1e-3f ? 2.f * p.roughness / aspect : 0.f) * q.iax;  // the clamp holds the rest constant
+  q.ly = (uy > 1e-3f ? 2.f * p.roughness * aspect : 0.f) * q.iay;
+  const float io2 = 1.f / (wo.z * wo.z), ox = q.ax * wo.x, oy = q.ay * wo.y;
+  q.so = sqrt(1.f + (ox * ox + oy * oy) * io2);
+  q.so_r = (ox * ox * q.lx + oy * oy * q.ly) * io2 / q.so;
+  return q;
+}
+
+TRT_HD inline void bsdf_grad_at(const BsdfParams<float>& p, const BsdfGradPre& pre, V3 wo, V3 wi, BsdfGrad& g) {
+  for (int c = 0; c < 3; ++c) g.own[c] = g.tint[c] = g.rough[c] = g.metal[c] = 0.f;
   if (wo.z <= 0.f || wi.z <= 0.f) return;
   if (p.model == kModelLambert) {
-    for (int c = 0; c < 3; ++c) g[c][c] = kInvPi;
+    for (int c = 0; c < 3; ++c) g.own[c] = kInvPi;
     return;
   }
   const V3 h = normalize(wo + wi);
@@ -204,11 +249,6 @@ TRT_HD inline void bsdf_grad(const BsdfParams<float>& p, V3 wo, V3 wi, float g[5
   const float FL = schlick_weight(cl), FV = schlick_weight(cv), FH = schlick_weight(cd);
   const float one_m_metal = 1.f - p.metallic;
   const float base[3] = {p.base.x, p.base.y, p.base.z};
-  const float wlum[3] = {0.2126729f, 0.7151522f, 0.0721750f};
-  const float lum = lum3(p.base);
-  const float ilum = lum > 0.f ? 1.f / lum : 0.f;
-  float tint[3];
-  for (int c = 0; c < 3; ++c) tint[c] = lum > 0.f ? base[c] * ilum : 1.f;
 
   // diffuse weight and its roughness derivative
   const float cd2 = cd * cd, rcd2 = p.roughness * cd2;
@@ -225,23 +265,15 @@ TRT_HD inline void bsdf_grad(const BsdfParams<float>& p, V3 wo, V3 wi, float g[5
   const float kd = dw * kInvPi * one_m_metal, kd_r = dw_r * kInvPi * one_m_metal;
 
   // specular weight q = D G / (4 cl cv) and its roughness derivative
-  const float aspect = sqrt(1.f - 0.9f * p.anisotropic);
-  const float r2 = p.roughness * p.roughness;
-  const float ux = r2 / aspect, uy = r2 * aspect;
-  const float ax = fmax(ux, 1e-3f), ay = fmax(uy, 1e-3f);
-  const float ax_r = ux > 1e-3f ? 2.f * p.roughness / aspect : 0.f;  // the clamp holds the rest constant
-  const float ay_r = uy > 1e-3f ? 2.f * p.roughness * aspect : 0.f;
-  const float iax = 1.f / ax, iay = 1.f / ay;
-  const float hx2 = (h.x * iax) * (h.x * iax), hy2 = (h.y * iay) * (h.y * iay);
+  const float hx2 = (h.x * pre.iax) * (h.x * pre.iax), hy2 = (h.y * pre.iay) * (h.y * pre.iay);
   const float t = hx2 + hy2 + h.z * h.z;
-  const float lx = ax_r * iax, ly = ay_r * iay;  // d ln ax, d ln ay
-  const float D = 1.f / (kPi * ax * ay * t * t);
-  const float dlnD = 4.f * (hx2 * lx + hy2 * ly) / t - (lx + ly);
-  const float io2 = 1.f / (wo.z * wo.z), ii2 = 1.f / (wi.z * wi.z);
-  const float ox = ax * wo.x, oy = ay * wo.y, ix = ax * wi.x, iy = ay * wi.y;
-  const float so = sqrt(1.f + (ox * ox + oy * oy) * io2), si = sqrt(1.f + (ix * ix + iy * iy) * ii2);
-  const float G = 1.f / (1.f + (so - 1.f) * 0.5f + (si - 1.f) * 0.5f);
-  const float dL = 0.5f * ((ox * ox * lx + oy * oy * ly) * io2 / so + (ix * ix * lx + iy * iy * ly) * ii2 / si);
+  const float D = 1.f / (kPi * pre.ax * pre.ay * t * t);
+  const float dlnD = 4.f * (hx2 * pre.lx + hy2 * pre.ly) / t - (pre.lx + pre.ly);
+  const float ii2 = 1.f / (wi.z * wi.z);
+  const float ix = pre.ax * wi.x, iy = pre.ay * wi.y;
+  const float si = sqrt(1.f + (ix * ix + iy * iy) * ii2);
+  const float G = 1.f / (1.f + (pre.so - 1.f) * 0.5f + (si - 1.f) * 0.5f);
+  const float dL = 0.5f * (pre.so_r + (ix * ix * pre.lx + iy * iy * pre.ly) * ii2 / si);
   const float q = D * G / (4.f * cl * cv);
   const float q_r = q * (dlnD - G * dL);
 
@@ -250,14 +282,27 @@ TRT_HD inline void bsdf_grad(const BsdfParams<float>& p, V3 wo, V3 wi, float g[5
   const float one_m_FH = 1.f - FH;
   // base colour: on its own channel, and through the tint's luminance on every channel
   const float own = kd + q * one_m_FH * p.metallic;
-  const float via = (one_m_metal * (sheen * st + q * one_m_FH * sp * stt)) * ilum;
+  const float via = (one_m_metal * (sheen * st + q * one_m_FH * sp * stt)) * pre.ilum;
   for (int c = 0; c < 3; ++c) {
-    const float spec_c = sp * ((1.f - stt) + stt * tint[c]);
+    const float tint = pre.ilum > 0.f ? base[c] * pre.ilum : 1.f;
+    const float spec_c = sp * ((1.f - stt) + stt * tint);
     const float c0 = p.metallic * base[c] + one_m_metal * spec_c;
     const float F = c0 + (1.f - c0) * FH;
-    for (int k = 0; k < 3; ++k) g[k][c] = (k == c ? own + via : 0.f) - via * tint[c] * wlum[k];
-    g[3][c] = base[c] * kd_r + F * q_r;
-    g[4][c] = q * one_m_FH * (base[c] - spec_c) - base[c] * (dw * kInvPi) - ((1.f - st) + st * tint[c]) * sheen;
+    g.own[c] = own + via;
+    g.tint[c] = via * tint;
+    g.rough[c] = base[c] * kd_r + F * q_r;
+    g.metal[c] = q * one_m_FH * (base[c] - spec_c) - base[c] * (dw * kInvPi) - ((1.f - st) + st * tint) * sheen;
+  }
+}
+
+// All fifteen.
+TRT_HD inline void bsdf_grad(const BsdfParams<float>& p, V3 wo, V3 wi, float g[5][3]) {
+  BsdfGrad b;
+  bsdf_grad_at(p, bsdf_grad_pre(p, wo), wo, wi, b);
+  for (int c = 0; c < 3; ++c) {
+    for (int k = 0; k < 3; ++k) g[k][c] = (k == c ? b.own[c] : 0.f) - lum_weight(k) * b.tint[c];
+    g[3][c] = b.rough[c];
+    g[4][c] = b.metal[c];
   }
 }
 

@@ -124,22 +124,17 @@ constexpr int kNumParams = 5;
 struct AdjOut {
   uint32_t mat;                 // material of the vertex (kNoHit when none)
   float nee_g[kNumParams];      // sum_c delta_c d(NEE contribution_c)/d theta_k
-  float r[kNumParams][3];       // (d f_c / d theta_k) / f_c at the sampled extension
+  float r[kNumParams][3];       // (d f_c / d theta_k) / f_c at the sampled extension (ADJ 1)
+  BsdfGrad rel;                 // the same, each term over its channel's f_c (ADJ 2)
 };
 
-// (d f_c / d theta_k) at (wo, wi): dual numbers (ADJ 1, parameters bd) or bsdf_grad (ADJ 2).
-template <int ADJ>
-TRT_FI void bsdf_gradient(const BsdfParams<float>& bp, const BsdfParams<Dual<kNumParams>>& bd, V3 wo, V3 wi,
-                          float g[kNumParams][3]) {
-  if (ADJ == 2) {
-    bsdf_grad(bp, wo, wi, g);
-  } else {
-    const T3<Dual<kNumParams>> fd = bsdf_f(bd, wo, wi);
-    for (int k = 0; k < kNumParams; ++k) {
-      g[k][0] = fd.x.d[k];
-      g[k][1] = fd.y.d[k];
-      g[k][2] = fd.z.d[k];
-    }
+// (d f_c / d theta_k) at (wo, wi) from dual numbers.
+TRT_FI void bsdf_gradient_dual(const BsdfParams<Dual<kNumParams>>& bd, V3 wo, V3 wi, float g[kNumParams][3]) {
+  const T3<Dual<kNumParams>> fd = bsdf_f(bd, wo, wi);
+  for (int k = 0; k < kNumParams; ++k) {
+    g[k][0] = fd.x.d[k];
+    g[k][1] = fd.y.d[k];
+    g[k][2] = fd.z.d[k];
   }
 }
 
@@ -149,7 +144,7 @@ TRT_FI void bsdf_gradient(const BsdfParams<float>& bp, const BsdfParams<Dual<kNu
 // 0 and 2 the material is read once and evaluated in one pass per direction. 2 differs from
 // 0 in the Russian roulette only, which follows the sampling set's rule.
 // ADJ: 0 the plain step; the adjoint extras with BSDF derivatives 1 from dual numbers (the
-// oracle), 2 from bsdf_grad (the device).
+// oracle), 2 from bsdf_grad_at (the device).
 template <int ADJ, int SEP = -1>
 TRT_HD inline void shade_impl(const SceneView& s, const Material* sampling_mats, const RenderParams& rp,
                               const PathState& ps, const Hit& h, uint32_t depth, ShadeOut& out, V3 delta,
@@ -242,12 +237,17 @@ TRT_HD inline void shade_impl(const SceneView& s, const Material* sampling_mats,
   BsdfPre pre{};
   if (!sep) pre = bsdf_pre(bp, wo);
   BsdfParams<Dual<kNumParams>> bd;
+  BsdfGradPre gpre{};
   if (ADJ) {
     adj->mat = sp.mat;
     for (int k = 0; k < kNumParams; ++k) adj->nee_g[k] = 0.f;
-    for (int k = 0; k < kNumParams; ++k) adj->r[k][0] = adj->r[k][1] = adj->r[k][2] = 0.f;
+  }
+  if (ADJ == 2) {
+    adj->rel = BsdfGrad{};
+    gpre = bsdf_grad_pre(bp, wo);
   }
   if (ADJ == 1) {
+    for (int k = 0; k < kNumParams; ++k) adj->r[k][0] = adj->r[k][1] = adj->r[k][2] = 0.f;
     bd.base = t3(dvar<kNumParams>(m.base[0], 0), dvar<kNumParams>(m.base[1], 1), dvar<kNumParams>(m.base[2], 2));
     bd.roughness = dvar<kNumParams>(m.roughness, 3);
     bd.metallic = dvar<kNumParams>(m.metallic, 4);
@@ -316,12 +316,18 @@ TRT_HD inline void shade_impl(const SceneView& s, const Material* sampling_mats,
           out.s_tmax = s_tmax;
           out.s_contrib = clamp_contrib(c, rp.clamp);
           if (ADJ) {
-            float fg[kNumParams][3];
-            bsdf_gradient<ADJ>(bp, bd, wo, wi, fg);
             const float kx = delta.x * ps.T.x * lrad.x * k, ky = delta.y * ps.T.y * lrad.y * k,
                         kz = delta.z * ps.T.z * lrad.z * k;
-            for (int j = 0; j < kNumParams; ++j)
-              adj->nee_g[j] = (kx * fg[j][0] + ky * fg[j][1]) + kz * fg[j][2];
+            if (ADJ == 2) {
+              BsdfGrad fg;
+              bsdf_grad_at(bp, gpre, wo, wi, fg);
+              bsdf_grad_dot(fg, v3(kx, ky, kz), adj->nee_g);
+            } else {
+              float fg[kNumParams][3];
+              bsdf_gradient_dual(bd, wo, wi, fg);
+              for (int j = 0; j < kNumParams; ++j)
+                adj->nee_g[j] = (kx * fg[j][0] + ky * fg[j][1]) + kz * fg[j][2];
+            }
           }
         }
       }
@@ -376,9 +382,21 @@ TRT_HD inline void shade_impl(const SceneView& s, const Material* sampling_mats,
           out.next.pdf = smp.pdf;
           out.next.flags = 0u;
           out.next.path = ps.path;
-          if (ADJ) {
+          if (ADJ == 2) {
+            BsdfGrad fg;
+            bsdf_grad_at(bp, gpre, wo, smp.wi, fg);
+            const float fc[3] = {f.x, f.y, f.z};
+            for (int c = 0; c < 3; ++c) {
+              const bool on = fc[c] != 0.f;
+              adj->rel.own[c] = on ? fg.own[c] / fc[c] : 0.f;
+              adj->rel.tint[c] = on ? fg.tint[c] / fc[c] : 0.f;
+              adj->rel.rough[c] = on ? fg.rough[c] / fc[c] : 0.f;
+              adj->rel.metal[c] = on ? fg.metal[c] / fc[c] : 0.f;
+            }
+          }
+          if (ADJ == 1) {
             float fg[kNumParams][3];
-            bsdf_gradient<ADJ>(bp, bd, wo, smp.wi, fg);
+            bsdf_gradient_dual(bd, wo, smp.wi, fg);
             for (int j = 0; j < kNumParams; ++j) {
               adj->r[j][0] = f.x != 0.f ? fg[j][0] / f.x : 0.f;
               adj->r[j][1] = f.y != 0.f ? fg[j][1] / f.y : 0.f;
@@ -413,6 +431,10 @@ TRT_HD inline void shade_adjoint(const SceneView& s, const Material* sampling_ma
 TRT_FI void continuation_grad(const AdjOut& a, V3 delta, V3 l_after, float* g) {
   const float x = delta.x * l_after.x, y = delta.y * l_after.y, z = delta.z * l_after.z;
   for (int k = 0; k < kNumParams; ++k) g[k] = (a.r[k][0] * x + a.r[k][1] * y) + a.r[k][2] * z;
+}
+
+TRT_FI void continuation_grad(const BsdfGrad& rel, V3 delta, V3 l_after, float* g) {
+  bsdf_grad_dot(rel, v3(delta.x * l_after.x, delta.y * l_after.y, delta.z * l_after.z), g);
 }
 
 }  // namespace trt
