@@ -29,3 +29,21 @@ def test_pixels_round_trip(width, height):
         assert img.shape == (height, width, 4) and (img[..., 3] == 255).all()
     finally:
         r.close()
+
+
+def test_bytes_round_trip():
+    """4 MiB + 5 occlusion bytes (a last part whose length is no multiple of 16) against the
+    same rays asked in two calls below the threaded reads."""
+    from tests.gpu_util import random_rays
+    n = (4 << 20) + 5
+    rays = random_rays(n, seed=3, lo=0.02, hi=0.98)
+    rays[:, 7] = 0.6
+    r = Renderer(0)
+    try:
+        r.UpdateScene(scenes.cornell(width=16, height=16, spp=1))
+        whole = r.trace_any(rays)
+        parts = np.concatenate([r.trace_any(rays[:n // 2]), r.trace_any(rays[n // 2:])])
+    finally:
+        r.close()
+    assert 0.1 < parts.mean() < 0.9
+    assert np.array_equal(whole, parts)

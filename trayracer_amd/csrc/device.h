@@ -190,6 +190,8 @@ void launch_occluded(const DevAccel& acc, RayQueue q, uint8_t* occluded, SegIn i
 void launch_report_counters(const uint32_t* ctr, uint32_t cap, uint32_t* report, hipStream_t stream);
 // Adds the set bits of a touch bitmap (`words` 32-bit words) to *out and clears it.
 void launch_touch_count(uint32_t* bits, uint32_t words, unsigned long long* out, hipStream_t stream);
+// Copies `bytes` from device to pinned host memory, both 16-byte aligned.
+void launch_copy_out(const void* src, void* dst, uint32_t bytes, hipStream_t stream);
 void launch_tonemap(const float4* src, uint32_t n, const TonemapParams& tp, uchar4* dst, hipStream_t stream);
 // reset: restart the accumulator; aov_reset: restart the AOV sums; aov_count: samples in
 // the AOV sums after this frame.

@@ -936,6 +936,16 @@ __global__ __launch_bounds__(kBlock) void k_report_counters(const uint32_t* ctr,
   report_counters(ctr, cap, out);
 }
 
+// Device to pinned host memory, both 16-byte aligned. Bound by the host link, which few waves
+// fill: 32, 64 and 128 blocks bring a 33 MB image over in the same time.
+constexpr uint32_t kCopyBlocks = 64;
+__global__ __launch_bounds__(kBlock) void k_copy_out(const uint4* __restrict__ src, uint4* __restrict__ dst, uint32_t bytes) {
+  const uint32_t n = bytes / 16;
+  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) dst[i] = src[i];
+  const uint32_t t = n * 16 + threadIdx.x;
+  if (blockIdx.x == 0 && t < bytes) reinterpret_cast<uint8_t*>(dst)[t] = reinterpret_cast<const uint8_t*>(src)[t];
+}
+
 // Distinct items a launch read: set bits of its touch bitmap, which is cleared for the
 // next launch.
 __global__ __launch_bounds__(kBlock) void k_touch_count(uint32_t* bits, uint32_t words, unsigned long long* out) {
@@ -1750,6 +1760,12 @@ bool traversal_lds_check() { return no_static_lds<Nodes32>() && no_static_lds<No
 
 void launch_zero_counters(uint32_t* ctr, hipStream_t stream) {
   hipLaunchKernelGGL(k_zero_counters, dim3((kNumCounters + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, ctr);
+}
+
+void launch_copy_out(const void* src, void* dst, uint32_t bytes, hipStream_t stream) {
+  const uint32_t blocks = std::min<uint32_t>((bytes / 16 + kBlock - 1) / kBlock, kCopyBlocks);
+  hipLaunchKernelGGL(k_copy_out, dim3(blocks ? blocks : 1), dim3(kBlock), 0, stream, static_cast<const uint4*>(src),
+                     static_cast<uint4*>(dst), bytes);
 }
 
 void launch_tonemap(const float4* src, uint32_t n, const TonemapParams& tp, uchar4* dst, hipStream_t stream) {
