@@ -271,12 +271,12 @@ def extend_roofline(tc, info, ext_rays, ext_ms, launches, workload):
     """Two ceilings for the closest-hit traversal (Extend), per launch, from HIP-event
     launch times:
     * HBM: the bytes a launch must move at least, its rays' records (32 B ray in, 16 B hit
-      out) plus every distinct node and triangle record it reads once (48 B each; counted
-      by the counting pass's touch bitmaps), against the 8 TB/s peak; `traffic` is the
+      out) plus every distinct node (32 or 48 B) and triangle record (48 B) it reads once
+      (counted by the counting pass's touch bitmaps), against the 8 TB/s peak; `traffic` is the
       rocprofv3 measurement of the same kernel (FETCH_SIZE + WRITE_SIZE, copy-calibrated),
       null when the profile was taken from other kernel sources;
-    * vector memory: the bytes every ray loads (ray and hit records, node visits x 48 B,
-      triangle tests x 48 B) against the rate of independent random 48-byte gathers from
+    * vector memory: the bytes every ray loads (ray and hit records, node visits x the
+      node's bytes, triangle tests x 48 B) against the rate of independent random 48-byte gathers from
       an L1-resident buffer (trt_measure_gather), the fastest such loads go through the
       CUs' load path (Extend's node loads mostly hit L1 and L2)."""
     n = max(1, launches)
@@ -305,10 +305,11 @@ def extend_roofline(tc, info, ext_rays, ext_ms, launches, workload):
         "traffic_stale": stale,
         "dram_gbs": round(traffic / avg_s / 1e9, 1) if traffic else None,
         "dram_frac": round(traffic / avg_s / 1e9 / HBM_PEAK_GBS, 4) if traffic else None,
-        "kernel": "k_extend_tl<false>" if info["two_level"] else "k_extend_sl<false>",
+        "kernel": ("k_extend_tl" if info["two_level"] else "k_extend_sl") + f"<Nodes{tc['node_bytes']}, false>",
         "avg_launch_ms": round(ext_ms / n, 4), "rays_per_launch": round(rays_per_launch),
         "algorithmic_bytes_per_launch": round(compulsory),
-        "algorithmic_bytes": "48 B per ray (ray in, hit out) + 48 B per distinct node and triangle record read",
+        "algorithmic_bytes": "48 B per ray (ray in, hit out) + 32 B per distinct node (48 B where the "
+                             "compact nodes do not fit) + 48 B per distinct triangle record read",
         "vector_memory": {"achieved": round(loaded, 1), "peak": vm_peak, "unit": "GB/s",
                           "frac": round(loaded / vm_peak, 4) if vm_peak else None,
                           "bytes_per_ray": round(per_ray, 1), "nodes_per_ray": round(tc["closest_nodes_per_ray"], 2),

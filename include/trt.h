@@ -380,8 +380,8 @@ typedef struct trt_trace_counts {
 trt_status trt_measure_traversal(trt_context* ctx, const trt_render_opts* opts, trt_trace_counts* out);
 
 /* Measurement hook (no counterpart in the reference): the vector-memory ceiling of the
- * traversal's loads. Lanes read 48-byte records (a node or a triangle record, three
- * 16-byte loads) at pseudo-random indices of a device buffer of `buffer_bytes`, `iters`
+ * traversal's loads. Lanes read 48-byte records (as triangles are kept; three 16-byte
+ * loads) at pseudo-random indices of a device buffer of `buffer_bytes`, `iters`
  * records per lane, with independent loads; *gbs = bytes read per second (GB/s, best of
  * three timed launches). Over a buffer that fits the L2 this is the highest rate such
  * gathers reach on the device. No context: it runs on `device` with its own buffers. */

@@ -1075,13 +1075,15 @@ static void populate_pages(void* p, size_t bytes) {
 // the runtime, 1.11 with its copies into two threads' chunks, 0.87 with the kernel, 0.82 with
 // four threads; 133 MB: 12.8, 5.8, 5.8, 3.9; 7.6 MB after training: 1.07 by the runtime, 0.26.
 // 512 KB chunks are slower, 2 MB ones no faster. From kReadLarge bytes on, below which threads
-// cost more than they save. Returns when the copy is done.
+// cost more than they save. Returns when the copy is done. idle: nothing is queued on the
+// context's stream (a small copy then needs no stream: 39 us instead of 43 for 655 KB).
 constexpr size_t kReadLarge = size_t(4) << 20, kReadChunk = size_t(1) << 20;
 constexpr int kReadThreads = 4;
-static hipError_t read_back(trt_context* ctx, void* out, const void* src, size_t bytes) {
+static hipError_t read_back(trt_context* ctx, void* out, const void* src, size_t bytes, bool idle = false) {
   hipStream_t s = ctx->stream;
   const size_t parts = std::min<size_t>({size_t(kReadThreads), size_t(std::max(1, default_build_threads())), bytes / kReadChunk});
   if (bytes < kReadLarge || parts < 2 || (reinterpret_cast<uintptr_t>(src) & 15)) {
+    if (idle) return hipMemcpy(out, src, bytes, hipMemcpyDeviceToHost);
     const hipError_t e = hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, s);
     return e == hipSuccess ? hipStreamSynchronize(s) : e;
   }
@@ -1139,7 +1141,7 @@ static trt_status read_pixels(trt_context* ctx, DevBuf& b, float* out) {
   if (!ctx || !out) return TRT_INVALID_ARG;
   if (ctx->width == 0) return fail(ctx, TRT_NOT_BUILT, "nothing rendered yet");
   HIPC(hipSetDevice(ctx->device), "hipSetDevice");
-  HIPC(read_back(ctx, out, b.p, size_t(ctx->width) * ctx->height * 16), "read pixels");
+  HIPC(read_back(ctx, out, b.p, size_t(ctx->width) * ctx->height * 16, true), "read pixels");
   return TRT_OK;
 }
 trt_status trt_read_accum(trt_context* ctx, float* rgba) { return ctx ? read_pixels(ctx, ctx->accum, rgba) : TRT_INVALID_ARG; }
