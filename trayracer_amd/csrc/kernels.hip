@@ -1692,14 +1692,23 @@ __global__ __launch_bounds__(kBlock) void k_grad_reduce(const uint32_t* __restri
 
 // Sum of the blocks' partial gradients, in a fixed order: a block takes 16 parameters,
 // sixteen threads each (thread t of a parameter the partials t, t + 16, ..., so that 16
-// neighbouring parameters are read together), then adds the sixteen sums pairwise.
+// neighbouring parameters are read together), then adds the sixteen sums pairwise. A thread's
+// loads go sixteen at a time (one after the other: 21 us for 512 materials; now 6).
 __global__ __launch_bounds__(kBlock) void k_grad_final(const float* __restrict__ partial, uint32_t n_blocks, uint32_t P,
                                                         float* out) {
   __shared__ float sum[kBlock];
   const uint32_t i = blockIdx.x * 16u + (threadIdx.x & 15u), part = threadIdx.x >> 4;
   float t = 0.f;
-  if (i < P)
-    for (uint32_t b = part; b < n_blocks; b += 16u) t += partial[static_cast<size_t>(b) * P + i];
+  for (uint32_t b0 = 0; b0 < n_blocks; b0 += 256u) {
+    float v[16];
+#pragma unroll
+    for (uint32_t k = 0; k < 16u; ++k) {
+      const uint32_t b = b0 + part + 16u * k;
+      v[k] = i < P && b < n_blocks ? partial[static_cast<size_t>(b) * P + i] : 0.f;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 16u; ++k) t += v[k];
+  }
   sum[threadIdx.x] = t;
   for (uint32_t s = 128u; s >= 16u; s >>= 1) {
     __syncthreads();
