@@ -30,6 +30,7 @@
 #include <algorithm>
 
 #include "device.h"
+#include "trt/slab32.h"
 #include "trt/tonemap.h"
 
 namespace trt {
@@ -270,11 +271,8 @@ struct Nodes48 {
 // are three instructions (six, plus six to gather the child references, with Nodes48).
 // The terms that cancel in ct have an error of up to 2u (|x| + R) |inv| (x the distance to
 // the box's centre, R the tree's half size): the part in |x| is relative to the distances,
-// and the half extents' margins (bvh_build.h) exceed the part in R. A direction component
-// below 2^-60 of the largest takes that magnitude (v_rcp_f32's ulp scales all of the
-// axis's distances alike), which moves no ray by more than the
-// margins; rays so extreme that a term could overflow take every box (NaN, which the axes'
-// max / min ignore): slow and still exact.
+// and the half extents' margins (bvh_build.h) exceed the part in R. The per-ray
+// terms, and what they do with tiny direction components and extreme rays: slab32_ray.
 struct Nodes32 {
   static constexpr uint32_t kBytes = sizeof(DevNode32);
   struct Ray {
@@ -285,23 +283,7 @@ struct Nodes32 {
   static __device__ __forceinline__ Ray setup(const NodeSpace& g, V3 o, V3 d) {
     Ray b;
     b.o = o;
-    const float m = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(d.x), __builtin_fabsf(d.y)), __builtin_fabsf(d.z));
-    const float lim = m * 0x1p-60f;
-    const float ix = __builtin_amdgcn_rcpf(__builtin_fabsf(d.x) < lim ? __builtin_copysignf(lim, d.x) : d.x);
-    const float iy = __builtin_amdgcn_rcpf(__builtin_fabsf(d.y) < lim ? __builtin_copysignf(lim, d.y) : d.y);
-    const float iz = __builtin_amdgcn_rcpf(__builtin_fabsf(d.z) < lim ? __builtin_copysignf(lim, d.z) : d.z);
-    const V3 w = v3(g.org[0] - o.x, g.org[1] - o.y, g.org[2] - o.z);
-    b.si = v3(ix * g.scale, iy * g.scale, iz * g.scale);
-    b.oi = v3(w.x * ix, w.y * iy, w.z * iz);
-    // |si| in [2^-100, 2^100], |oi| < 2^126, |org - o| < 2^50 scale (2^36 R), all finite
-    const float s_hi = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(b.si.x), __builtin_fabsf(b.si.y)), __builtin_fabsf(b.si.z));
-    const float s_lo = __builtin_fminf(__builtin_fminf(__builtin_fabsf(b.si.x), __builtin_fabsf(b.si.y)), __builtin_fabsf(b.si.z));
-    const float o_hi = __builtin_fabsf(b.oi.x) + __builtin_fabsf(b.oi.y) + __builtin_fabsf(b.oi.z);
-    const float w_hi = __builtin_fabsf(w.x) + __builtin_fabsf(w.y) + __builtin_fabsf(w.z);
-    if (!(s_lo >= 0x1p-100f && s_hi <= 0x1p100f && o_hi < 0x1p126f && w_hi < 0x1p50f * g.scale)) {
-      b.si = v3(0.f);
-      b.oi = v3(__builtin_nanf(""));
-    }
+    slab32_ray(g.org, g.scale, o, d, [](float x) { return __builtin_amdgcn_rcpf(x); }, b.si, b.oi);
     return b;
   }
   // v: fp16 (c, h) pairs of the axes, then the child reference
