@@ -53,7 +53,7 @@ int main() {
         const V3 o = v3(half * u(rng), half * u(rng), half * u(rng));
         const float tmax = r % 2 ? 0.f : (r % 3 ? 1e30f : HUGE_VALF);  // 0: an all-zero record
         V3 si, oi;
-        slab32_ray(g.org, g.scale, o, d, [](float x) { return 1.f / x; }, si, oi);
+        slab32_ray(g.org, g.step, o, d, [](float x) { return 1.f / x; }, si, oi);
         std::vector<int32_t> stack = {0};
         size_t visits = 0;
         while (!stack.empty()) {

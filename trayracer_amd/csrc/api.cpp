@@ -346,7 +346,7 @@ DevAccel accel_of(const trt_context* ctx) {
   a.tris = ctx->d_tris.as<float4>();
   a.tlas = ctx->two_level ? ctx->d_tlas.p : nullptr;
   a.inst = ctx->two_level ? ctx->d_inst_tlas.as<TlasInstance>() : nullptr;
-  a.space = ctx->space;
+  a.space = grid_of(ctx->space);
   a.node_bytes = ctx->node_bytes;
   a.stack_cap = ctx->stack_cap;
   a.two_level = ctx->two_level ? 1 : 0;
@@ -904,7 +904,7 @@ trt_status trt_build(trt_context* ctx, const trt_build_opts* opts) {
     TlasInstance& t = inst_tlas[k];
     std::memset(&t, 0, sizeof(t));
     std::memcpy(t.w2o, in.w2o, sizeof(t.w2o));
-    t.space = mesh_space[in.mesh];
+    t.space = grid_of(mesh_space[in.mesh]);
     t.blas_root = blas_root[in.mesh] * ctx->node_bytes;  // a byte offset, like every node reference
     t.id = in.id;
   }

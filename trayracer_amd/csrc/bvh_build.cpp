@@ -503,57 +503,117 @@ double half_value(uint32_t h) {
   return e == 0 ? m * exp2_int(-24) : (1024.0 + m) * exp2_int(e - 25);
 }
 
+bool empty_child(int32_t c) { return c < 0 && (~uint32_t(c) & 7u) == 0u; }
+
+void child_bounds(const DevNode2& n, int c, float lo[3], float hi[3]) {
+  const float* xy = c ? n.r1 : n.r0;
+  lo[0] = xy[0]; hi[0] = xy[1]; lo[1] = xy[2]; hi[1] = xy[3];
+  lo[2] = n.r2[2 * c]; hi[2] = n.r2[2 * c + 1];
+}
+
+// The up to two coordinates at which the most leaf boxes of a tree, and at least kPlaneBoxes,
+// are flat on an axis, of up to kPlaneNodes of its nodes taken evenly.
+constexpr size_t kPlaneNodes = 16384, kPlaneBoxes = 32;
+int flat_planes(const std::vector<DevNode2>& in, size_t first, size_t count, int axis, double at[2]) {
+  std::vector<float> v;
+  const size_t step = (count + kPlaneNodes - 1) / kPlaneNodes;
+  for (size_t i = 0; i < count; i += step)
+    for (int c = 0; c < 2; ++c) {
+      const DevNode2& n = in[first + i];
+      if (n.c[c] >= 0 || empty_child(n.c[c])) continue;
+      float lo[3], hi[3];
+      child_bounds(n, c, lo, hi);
+      if (lo[axis] == hi[axis]) v.push_back(lo[axis]);
+    }
+  std::sort(v.begin(), v.end());
+  size_t boxes[2] = {kPlaneBoxes - 1, kPlaneBoxes - 1};
+  int found = 0;
+  for (size_t a = 0, b; a < v.size(); a = b) {
+    for (b = a + 1; b < v.size() && v[b] == v[a];) ++b;
+    if (b - a <= boxes[1]) continue;
+    const int place = b - a > boxes[0] ? 0 : 1;
+    if (place == 0) {
+      boxes[1] = boxes[0];
+      at[1] = at[0];
+    }
+    boxes[place] = b - a;
+    at[place] = v[a];
+    found = std::min(2, found + 1);
+  }
+  return found;
+}
+
 }  // namespace
 
 bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, NodeSpace& space, DevNode32* out,
                   int n_threads) {
   static_assert(sizeof(DevNode32) == 32, "node size");
-  auto empty = [](int32_t c) { return c < 0 && (~uint32_t(c) & 7u) == 0u; };
-  auto bounds = [](const DevNode2& n, int c, float lo[3], float hi[3]) {
-    const float* xy = c ? n.r1 : n.r0;
-    lo[0] = xy[0]; hi[0] = xy[1]; lo[1] = xy[2]; hi[1] = xy[3];
-    lo[2] = n.r2[2 * c]; hi[2] = n.r2[2 * c + 1];
-  };
   double blo[3] = {HUGE_VAL, HUGE_VAL, HUGE_VAL}, bhi[3] = {-HUGE_VAL, -HUGE_VAL, -HUGE_VAL};
   for (int c = 0; c < 2; ++c) {  // the root's children bound the tree
-    if (empty(in[first].c[c])) continue;
+    if (empty_child(in[first].c[c])) continue;
     float lo[3], hi[3];
-    bounds(in[first], c, lo, hi);
+    child_bounds(in[first], c, lo, hi);
     for (int k = 0; k < 3; ++k) {
       blo[k] = std::min(blo[k], double(lo[k]));
       bhi[k] = std::max(bhi[k], double(hi[k]));
     }
   }
-  double R = 0.0;
+  double Rk[3], R = 0.0;  // the tree's half sides, and the largest
   for (int k = 0; k < 3; ++k) {
     space.org[k] = blo[k] <= bhi[k] ? float(0.5 * (blo[k] + bhi[k])) : 0.f;
     if (!std::isfinite(space.org[k])) return false;
-    if (blo[k] <= bhi[k]) R = std::max(R, std::max(bhi[k] - space.org[k], space.org[k] - blo[k]));
+    Rk[k] = blo[k] <= bhi[k] ? std::max(bhi[k] - space.org[k], space.org[k] - blo[k]) : 0.0;
+    R = std::max(R, Rk[k]);
   }
   int e = 0;
   if (R > 0.0) (void)std::frexp(R, &e);
   if (!std::isfinite(R) || e < -60 || e > 60) return false;
   space.scale = float(std::ldexp(1.0, e - 14));
-  const double S = space.scale, slack = R * std::ldexp(1.0, -19);
+  // the two planes with the most flat boxes on each axis are put on the grid
+  for (int k = 0; k < 3; ++k) {
+    space.step[k] = space.scale;
+    double at[2], c[2];
+    const int n = flat_planes(in, first, count, k, at);
+    for (int i = 0; i < n; ++i) {
+      const double mid = (at[i] - space.org[k]) / space.scale;
+      c[i] = half_value(half_bits(std::fabs(mid), false)) * (mid < 0.0 ? -1.0 : 1.0);
+    }
+    if (n == 2 && c[0] != c[1]) {
+      const double step = (at[1] - at[0]) / (c[1] - c[0]);
+      if (std::fabs(step - space.scale) < kMaxStretch * space.scale) space.step[k] = float(step);
+    }
+    if (n) space.org[k] = float(at[0] - c[0] * space.step[k]);
+  }
+  double slack[3];
+  for (int k = 0; k < 3; ++k) slack[k] = Rk[k] * std::ldexp(1.0, -19);
   std::atomic<size_t> boxes{0}, coarse{0};
   std::atomic<bool> fits{true};
+  // leaf boxes that are flat and yet thick, by axis and stored centre
+  std::vector<std::atomic<uint32_t>> flat(2 * count > kMaxThickFlat ? size_t(3) << 16 : 0);
   auto pack_range = [&](size_t begin, size_t end) {
     size_t n_boxes = 0, n_coarse = 0;
+    size_t flat_at[3] = {};
+    uint32_t flat_run[3] = {};  // boxes at flat_at[axis] not yet counted in `flat`
+    auto count_flat = [&](int k, size_t at) {
+      if (at != flat_at[k] && flat_run[k]) flat[flat_at[k]] += flat_run[k];
+      flat_run[k] = at == flat_at[k] ? flat_run[k] + 1u : 1u;
+      flat_at[k] = at;
+    };
     for (size_t i = begin; i < end; ++i) {
       const DevNode2& n = in[i];
       DevNode32& d = out[i];
       for (int c = 0; c < 2; ++c) {
         const int32_t ref = n.c[c];
         d.w[4 * c + 3] = uint32_t(ref >= 0 ? ref * int32_t(sizeof(DevNode32)) : ref);
-        if (empty(ref)) {
+        if (empty_child(ref)) {
           for (int k = 0; k < 3; ++k) d.w[4 * c + k] = 0xfc000000u;  // c = 0, h = -inf
           continue;
         }
         float lo[3], hi[3];
-        bounds(n, c, lo, hi);
+        child_bounds(n, c, lo, hi);
         double exact = 0.0, stored = 0.0;
         for (int k = 0; k < 3; ++k) {
-          const double mid = (0.5 * (double(lo[k]) + double(hi[k])) - space.org[k]) / S;
+          const double S = space.step[k], mid = (0.5 * (double(lo[k]) + double(hi[k])) - space.org[k]) / S;
           if (!(std::fabs(mid) < 32768.0)) {
             fits = false;
             return;
@@ -561,13 +621,14 @@ bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, N
           const uint32_t cb = half_bits(std::fabs(mid), false) | (mid < 0.0 ? 0x8000u : 0u);
           const double cs = (mid < 0.0 ? -1.0 : 1.0) * half_value(cb & 0x7fffu) * S + space.org[k];
           const double half = std::max(double(hi[k]) - cs, cs - double(lo[k]));
-          const double h = (half * (1.0 + kHalfExtentMargin) + slack) / S;
+          const double h = (half * (1.0 + kHalfExtentMargin) + slack[k]) / S;
           if (!(h < 65504.0)) {
             fits = false;
             return;
           }
           const uint32_t hb = half_bits(h, true);
           d.w[4 * c + k] = cb | (hb << 16);
+          if (!flat.empty() && ref < 0 && lo[k] == hi[k] && half_value(hb) * S > kThinHalf * Rk[k]) count_flat(k, (size_t(k) << 16) + cb);
           exact += 0.5 * (double(hi[k]) - double(lo[k]));
           stored += half_value(hb) * S;
         }
@@ -577,6 +638,8 @@ bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, N
     }
     boxes += n_boxes;
     coarse += n_coarse;
+    for (int k = 0; k < 3; ++k)
+      if (flat_run[k]) flat[flat_at[k]] += flat_run[k];
   };
   const size_t n_parts = std::min<size_t>(size_t(std::max(1, n_threads)), count / 16384 + 1);
   std::vector<std::thread> pool;
@@ -584,7 +647,9 @@ bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, N
     pool.emplace_back(pack_range, first + count * t / n_parts, first + count * (t + 1) / n_parts);
   pack_range(first, first + count / n_parts);
   for (std::thread& t : pool) t.join();
-  return fits && double(coarse) <= kCoarseShare * double(boxes);
+  size_t coplanar = 0;
+  for (const std::atomic<uint32_t>& n : flat) coplanar += n >= kThickPlane ? n.load() : 0u;
+  return fits && coplanar <= kMaxThickFlat && double(coarse) <= kCoarseShare * double(boxes);
 }
 
 std::vector<DevNode2> to_device_layout(const BuildResult& b) {

@@ -36,13 +36,20 @@ struct ShadowQueue {
   float4* emit;     // emission list: rgb, path (bits); null where no Shade writes one
 };
 
+// A tree's grid (NodeSpace) as the traversal reads it.
+struct NodeGrid {
+  float org[3], step[3];
+};
+inline NodeGrid grid_of(const NodeSpace& s) {
+  return NodeGrid{{s.org[0], s.org[1], s.org[2]}, {s.step[0], s.step[1], s.step[2]}};
+}
+
 // An instance as the two-level traversal reads it, in the top level's leaf order.
 struct alignas(16) TlasInstance {
   float w2o[12];
-  NodeSpace space;      // grid of the mesh's tree
+  NodeGrid space;       // of the mesh's tree
   uint32_t blas_root;   // byte offset of the mesh's root in the node array
   uint32_t id;          // caller's instance index
-  uint32_t pad[2];
 };
 
 // Acceleration structure views.
@@ -51,7 +58,7 @@ struct DevAccel {
   const float4* tris;       // reordered traversal triangles: 3 float4 per triangle (w of row 0 = prim id)
   const void* tlas;         // top level over instances (nullptr for single-level)
   const TlasInstance* inst; // instances (two-level)
-  NodeSpace space;          // grid of the single-level tree or of the top level (32-byte nodes)
+  NodeGrid space;           // of the single-level tree or of the top level (32-byte nodes)
   uint32_t node_bytes;      // layout of every node array: sizeof(DevNode32) or sizeof(DevNode48)
   int stack_cap;            // stack entries per lane (tree depth bound)
   int two_level;

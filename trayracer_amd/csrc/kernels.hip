@@ -229,7 +229,7 @@ struct Nodes48 {
     V3 inv;  // 1 / d, infinite for a zero component
     V3 sgn;  // +-1, the sign of inv
   };
-  static __device__ __forceinline__ Ray setup(const NodeSpace&, V3 o, V3 d) {
+  static __device__ __forceinline__ Ray setup(const NodeGrid&, V3 o, V3 d) {
     Ray b;
     b.o = o;
     b.inv = v3(1.f / d.x, 1.f / d.y, 1.f / d.z);
@@ -264,10 +264,10 @@ struct Nodes48 {
   }
 };
 
-// 32-byte nodes: fp16 boxes on the tree's grid (NodeSpace: world = org + scale * c). Two
+// 32-byte nodes: fp16 boxes on the tree's grid (NodeSpace: world = org + step * c). Two
 // 16-byte loads a visit instead of three (the load path bounds the traversal), and nothing
 // to decode: v_fma_mix_f32 takes an fp16 operand as it is, so per axis
-//   ct = fma(c, scale inv, (org - o) inv),  entry = ct - h |scale inv|,  exit = ct + h |scale inv|
+//   ct = fma(c, step inv, (org - o) inv),  entry = ct - h |step inv|,  exit = ct + h |step inv|
 // are three instructions (six, plus six to gather the child references, with Nodes48).
 // The terms that cancel in ct have an error of up to 2u (|x| + R) |inv| (x the distance to
 // the box's centre, R the tree's half size): the part in |x| is relative to the distances,
@@ -277,13 +277,13 @@ struct Nodes32 {
   static constexpr uint32_t kBytes = sizeof(DevNode32);
   struct Ray {
     V3 o;
-    V3 si;  // scale / d
+    V3 si;  // step / d
     V3 oi;  // (org - o) / d
   };
-  static __device__ __forceinline__ Ray setup(const NodeSpace& g, V3 o, V3 d) {
+  static __device__ __forceinline__ Ray setup(const NodeGrid& g, V3 o, V3 d) {
     Ray b;
     b.o = o;
-    slab32_ray(g.org, g.scale, o, d, [](float x) { return __builtin_amdgcn_rcpf(x); }, b.si, b.oi);
+    slab32_ray(g.org, g.step, o, d, [](float x) { return __builtin_amdgcn_rcpf(x); }, b.si, b.oi);
     return b;
   }
   // v: fp16 (c, h) pairs of the axes, then the child reference
@@ -844,7 +844,7 @@ __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& i
     const bool enters = !in_blas && node < 0 && node > kTravExit;
     if (leaves || enters) {
       V3 o = ow, d = dw;
-      NodeSpace space = acc.space;
+      NodeGrid space = acc.space;
       if (enters) {
         const uint32_t c = ~static_cast<uint32_t>(node);
         const uint32_t first = c >> 3, cnt = c & 7u;
