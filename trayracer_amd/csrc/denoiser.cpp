@@ -227,12 +227,14 @@ hipError_t Unet::backward(const float* dout, int N, int H, int W, hipStream_t s)
   // gradient out (fp32)
   DnSums sums;
   int turn = 0;
+  bool ok = true;
   auto layer = [&](int i, const uint16_t* coarse, int c1, const uint16_t* in, int h, int w, const DnGrad& gin,
                    float* gout) {
+    if (!ok) return;
     const Conv& c = convs_[i];
     float* const bpart = bpart_[turn ^= 1];
     dn_relu_bias(gin, c.relu ? act_[i] : nullptr, dz_, N, h, w, c.cout, bpart, sums, s);
-    dn_conv_wgrad(in, coarse, c1, dz_, N, h, w, c.cin, c.cout, wpart_, wd_ + c.woff, gout, s);
+    ok = dn_conv_wgrad(in, coarse, c1, dz_, N, h, w, c.cin, c.cout, wpart_, wd_ + c.woff, gout, s);
     sums = DnSums{wpart_, dn_wgrad_chunks(N, h, w), size_t(c.cout) * 9 * c.cin, g_ + c.woff, bpart, c.cout, g_ + c.boff};
   };
   const auto plain = [](const float* g) { return DnGrad{kGradPlain, g}; };
@@ -255,6 +257,7 @@ hipError_t Unet::backward(const float* dout, int N, int H, int W, hipStream_t s)
   layer(E1A, nullptr, 0, p0_, H1, W1, plain(gA_), gB_);  // gB = d p0 (32 @H1)
   layer(E0B, nullptr, 0, act_[E0A], H, W, skip(gu0_, 96, 64, gB_), gA_);
   layer(E0A, nullptr, 0, x_, H, W, plain(gA_), nullptr);  // the input gradient of the network is not needed
+  if (!ok) return hipErrorInvalidValue;
   dn_sums(sums, s);
   return hipGetLastError();
 }

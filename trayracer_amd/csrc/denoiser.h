@@ -64,7 +64,8 @@ struct DnSums {
 // masked by Y > 0; Y null: no mask), its sums per channel and block in bpartial, and the
 // layer above's sums. dn_conv_wgrad: the weight gradient's partial sums (dn_wgrad_chunks x
 // Cout x 9 x Cin) and the input gradient gout (fp32; null: not needed) from the flipped
-// weights Wd. dn_sums: a layer's sums alone.
+// weights Wd; false, with nothing launched, for a shape that the kernels cannot address (none
+// that the forward pass accepts). dn_sums: a layer's sums alone.
 void dn_relu_bias(const DnGrad& grad, const uint16_t* Y, uint16_t* dZ, int N, int H, int W, int Cout, float* bpartial,
                   const DnSums& above, hipStream_t s);
 bool dn_conv_wgrad(const uint16_t* X, const uint16_t* coarse, int c1, const uint16_t* dZ, int N, int H, int W, int Cin,

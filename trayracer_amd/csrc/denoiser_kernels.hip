@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include "denoiser.h"
+#include "dn_limits.h"
 
 namespace trt {
 namespace dn {
@@ -61,6 +62,7 @@ struct ConvArgs {
 typedef unsigned v4u32_t __attribute__((ext_vector_type(4)));
 // third dword of a raw buffer resource on gfx9 parts (32-bit data format, no swizzle)
 constexpr int kBufFlags = 0x00020000;
+constexpr int kOOB = static_cast<int>(kBufOutside);  // buffer offset past every range
 
 // two floats -> packed bf16 (round to nearest even), low half first
 __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
@@ -102,7 +104,6 @@ __device__ __forceinline__ void conv_block(const ConvArgs& a, unsigned block, un
   constexpr int WLOADS = (32 * NB * 9 * 4 + 255) / 256;
   constexpr int PARTS = 4 * NB;                                   // 16-byte parts per staged pixel
   constexpr int FLUSH = (MB * 32 * PARTS) / 64;                   // 16-byte stores per lane per tile
-  constexpr int kOOB = 0x7fffffff;                                // buffer offset past every range
   uint16_t *const patch = lds.patch, *const wl = lds.wl, *const ob = lds.ob;
   float* const bl = lds.bl;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -163,7 +164,8 @@ __device__ __forceinline__ void conv_block(const ConvArgs& a, unsigned block, un
   // step and none sits in a branch, so the wait before each LDS store counts exactly
   // the loads issued after it. Idle threads store to the spare slot.
   int pyx[PLOADS];  // patch position: row | column << 8
-  int prel[PLOADS], crel[PLOADS], plds[PLOADS];
+  uint32_t prel[PLOADS], crel[PLOADS];
+  int plds[PLOADS];
   uint32_t pidle = 0;
 #pragma unroll
   for (int k = 0; k < PLOADS; ++k) {
@@ -172,8 +174,8 @@ __device__ __forceinline__ void conv_block(const ConvArgs& a, unsigned block, un
     const bool ok = i < (NPOS << gs);
     pidle |= (ok ? 1u : 0u) << k;
     pyx[k] = py | (px << 8);
-    prel[k] = ((py * W + px) * a.cx + gi * 8) * 2;
-    crel[k] = (((py + 1) >> 1) * (W >> 1) + ((px + 1) >> 1)) * a.c1 * 2 + (gi * 8) * 2;
+    prel[k] = (static_cast<uint32_t>(py * W + px) * a.cx + gi * 8) * 2;
+    crel[k] = static_cast<uint32_t>(((py + 1) >> 1) * (W >> 1) + ((px + 1) >> 1)) * a.c1 * 2 + (gi * 8) * 2;
     plds[k] = ok ? py * kRowPitch + px * kPosStride + gi * 8 : PH * kRowPitch;
   }
   u32x4 prA[PLOADS], prB[PLOADS], wr[WLOADS];
@@ -189,8 +191,8 @@ __device__ __forceinline__ void conv_block(const ConvArgs& a, unsigned block, un
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(base), static_cast<short>(0), coarse ? cimg_bytes : img_bytes, kBufFlags);
     // byte offset of the patch corner (row y0 - 1, column x0 - 1)
-    const int corner = coarse ? (((s.y0 >> 1) - 1) * (W >> 1) + ((s.x0 >> 1) - 1)) * a.c1 * 2
-                              : ((s.y0 - 1) * W + (s.x0 - 1)) * a.cx * 2;
+    const uint32_t corner = coarse ? static_cast<uint32_t>(((s.y0 >> 1) - 1) * (W >> 1) + ((s.x0 >> 1) - 1)) * a.c1 * 2
+                                   : static_cast<uint32_t>((s.y0 - 1) * W + (s.x0 - 1)) * a.cx * 2;
     const bool interior = __builtin_amdgcn_readfirstlane(
         s.y0 >= 1 && s.y0 + PH - 1 <= H && s.x0 >= 1 && s.x0 + PW - 1 <= W ? 1 : 0);
     uint32_t okm = pidle;  // bit k: load k reads image data (else the zero padding)
@@ -207,9 +209,9 @@ __device__ __forceinline__ void conv_block(const ConvArgs& a, unsigned block, un
     }
 #pragma unroll
     for (int k = 0; k < PLOADS; ++k) {
-      int r0 = prel[k], r1 = crel[k];
+      uint32_t r0 = prel[k], r1 = crel[k];
       asm volatile("" : "+v"(r0), "+v"(r1));  // keep the per-load select a register select
-      const int off = (okm >> k) & 1u ? corner + (coarse ? r1 : r0) : kOOB;
+      const int off = (okm >> k) & 1u ? static_cast<int>(corner + (coarse ? r1 : r0)) : kOOB;
       pr[k] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
     }
   };
@@ -255,11 +257,11 @@ __device__ __forceinline__ void conv_block(const ConvArgs& a, unsigned block, un
   // following loads (one in-order counter tracks both) and never delay the wait for
   // them. The 2x2 pooling reads the staged bf16 values back.
   uint16_t* obw = ob + wave * OWAVE;
-  int orel[FLUSH];
+  uint32_t orel[FLUSH];
 #pragma unroll
   for (int k = 0; k < FLUSH; ++k) {
     const int c = lane + 64 * k, px = c / PARTS, part = c - px * PARTS, pi = px & 31;
-    orel[k] = (((2 * (wave * MB + (px >> 5)) + (pi >> 4)) * W + (pi & 15)) * Cout + part * 8) * 2;
+    orel[k] = (static_cast<uint32_t>((2 * (wave * MB + (px >> 5)) + (pi >> 4)) * W + (pi & 15)) * Cout + part * 8) * 2;
   }
   const uint32_t out_bytes = static_cast<uint32_t>(H) * W * Cout * 2;
   auto flush = [&](const Step& s) __attribute__((always_inline)) {
@@ -281,12 +283,12 @@ __device__ __forceinline__ void conv_block(const ConvArgs& a, unsigned block, un
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         static_cast<uint16_t*>(a.y) + static_cast<size_t>(s.n) * H * W * Cout + s.co0, static_cast<short>(0),
         out_bytes, kBufFlags);
-    const int corner = (s.y0 * W + s.x0) * Cout * 2;
+    const uint32_t corner = static_cast<uint32_t>(s.y0 * W + s.x0) * Cout * 2;
 #pragma unroll
     for (int k = 0; k < FLUSH; ++k) {
       const int c = lane + 64 * k, px = c / PARTS, part = c - px * PARTS;
       const u32x4 v = *reinterpret_cast<const u32x4*>(obw + px * OS + part * 8);
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u32_t, v), rs, corner + orel[k], 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u32_t, v), rs, static_cast<int>(corner + orel[k]), 0, 0);
     }
     if (EPI == kEpiReluPool) {  // H even: pooled rows are whole
       const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
@@ -309,8 +311,8 @@ __device__ __forceinline__ void conv_block(const ConvArgs& a, unsigned block, un
                            (__uint_as_float(v10[d] & 0xffff0000u) + __uint_as_float(v11[d] & 0xffff0000u));
           o[d] = pack_bf16(0.25f * lo, 0.25f * hi);
         }
-        const int off = (((yy >> 1) * (W >> 1) + (s.x0 >> 1) + (px >> 1)) * Cout + part * 8) * 2;
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u32_t, o), rp, off, 0, 0);
+        const uint32_t off = (static_cast<uint32_t>((yy >> 1) * (W >> 1) + (s.x0 >> 1) + (px >> 1)) * Cout + part * 8) * 2;
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u32_t, o), rp, static_cast<int>(off), 0, 0);
       }
     }
   };
@@ -501,8 +503,8 @@ __device__ __forceinline__ void wgrad_block(const WgradArgs& a, int chunk, int c
   // same eight buffer loads on every tile, padding and idle ones past the buffer's end (they
   // return zero): with loads in branches the wait before a tile's stores could not tell how
   // many later ones are in flight and drained them all.
-  constexpr int kOOB = 0x7fffffff;
-  int py[kWgItems], px[kWgItems], rel[kWgItems][4], to[kWgItems];  // first pixel, byte offsets from the tile's corner, place in LDS
+  int py[kWgItems], px[kWgItems], to[kWgItems];  // first pixel, place in LDS
+  uint32_t rel[kWgItems][4];                     // byte offsets from the tile's corner
   const bool z1 = __builtin_amdgcn_readfirstlane(ky) < 2;          // item 1 is one of dZ
   bool have[kWgItems];
 #pragma unroll
@@ -518,12 +520,13 @@ __device__ __forceinline__ void wgrad_block(const WgradArgs& a, int chunk, int c
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int y = py[k], x = px[k] + q;
-      rel[k][q] = z    ? (y * W + x) * Cout * 2 + part * 16
-                  : up ? ((y >> 1) * (W >> 1) + (x >> 1)) * c1 * 2 + part * 16
-                       : (y * W + x) * cx * 2 + part * 16;
+      rel[k][q] = z    ? static_cast<uint32_t>(y * W + x) * Cout * 2 + part * 16
+                  : up ? static_cast<uint32_t>((y >> 1) * (W >> 1) + (x >> 1)) * c1 * 2 + part * 16
+                       : static_cast<uint32_t>(y * W + x) * cx * 2 + part * 16;
     }
   }
-  const int x_bytes = up ? (H >> 1) * (W >> 1) * c1 * 2 : H * W * cx * 2, z_bytes = H * W * Cout * 2;
+  const uint32_t x_bytes = up ? static_cast<uint32_t>((H >> 1) * (W >> 1)) * c1 * 2 : static_cast<uint32_t>(H * W) * cx * 2;
+  const uint32_t z_bytes = static_cast<uint32_t>(H * W) * Cout * 2;
   u32x4 stage[kWgAhead][kWgItems][4];
   auto load_tile = [&](u32x4(&stage)[kWgItems][4], int tile) __attribute__((always_inline)) {
     const int n = tile / tiles_img, tr = tile - n * tiles_img;
@@ -534,17 +537,18 @@ __device__ __forceinline__ void wgrad_block(const WgradArgs& a, int chunk, int c
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(xb), static_cast<short>(0), x_bytes, kBufFlags);
     const __amdgpu_buffer_rsrc_t rz = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(dZ) + static_cast<size_t>(n) * H * W * Cout + cb * 32, static_cast<short>(0), z_bytes, kBufFlags);
-    const int xc = up ? ((y0 >> 1) * (W >> 1) + (x0 >> 1)) * c1 * 2 : (y0 * W + x0) * cx * 2;
-    const int zc = (y0 * W + x0) * Cout * 2;
+    const uint32_t xc = up ? static_cast<uint32_t>((y0 >> 1) * (W >> 1) + (x0 >> 1)) * c1 * 2
+                           : static_cast<uint32_t>(y0 * W + x0) * cx * 2;
+    const uint32_t zc = static_cast<uint32_t>(y0 * W + x0) * Cout * 2;
 #pragma unroll
     for (int k = 0; k < kWgItems; ++k) {
       const bool row_ok = have[k] && static_cast<unsigned>(y0 + py[k]) < static_cast<unsigned>(H);
-      const int corner = k == 1 && z1 ? zc : xc;
+      const uint32_t corner = k == 1 && z1 ? zc : xc;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int x = px[k] + q;
         const bool ok = row_ok && x <= kTileW && static_cast<unsigned>(x0 + x) < static_cast<unsigned>(W);
-        const int off = ok ? corner + rel[k][q] : kOOB;
+        const int off = ok ? static_cast<int>(corner + rel[k][q]) : kOOB;
         stage[k][q] = __builtin_bit_cast(
             u32x4, __builtin_amdgcn_raw_buffer_load_b128(k == 1 && z1 ? rz : rx, off, 0, 0));
       }
@@ -1016,13 +1020,12 @@ static bool plan_conv(const DnConv& c, ConvPlan& p) {
   if ((c.epi == kEpiReluPool || c.c1) && c.H % 2) return false;
   if (c.epi == kEpiRadiance && c.cout < 4) return false;
   if (c.c1 && !c.coarse) return false;
-  // element offsets inside one image are 32-bit
-  const long widest = c.cout > c.cx ? c.cout : c.cx;
-  if (long(c.H) * c.W * widest >= (1L << 31)) return false;
+  if (!dn_load_ok(c.H, c.W, c.cx) || !dn_load_ok(c.H / 2, c.W / 2, c.c1)) return false;
   if (c.epi == kEpiRadiance && Cin > 32) return false;  // feature prefetch assumes one chunk
   const long tiles16 = long(c.W / kTileW) * ((c.H + 15) / 16) * c.N;
   const int MB = p.MB = tiles16 >= 1024 ? 2 : 1;
   const long tiles = long(c.W / kTileW) * ((c.H + 8 * MB - 1) / (8 * MB)) * c.N;
+  if ((c.epi == kEpiRelu || c.epi == kEpiReluPool) && !dn_store_ok(c.H, c.W, c.cout, 8 * MB)) return false;
   const int NB = p.NB = MB == 1 && c.cout % 64 == 0 ? 2 : 1;  // MB = NB = 2 would need > 100 KB of LDS
   ConvArgs& a = p.a;
   a.x = c.x;
@@ -1112,6 +1115,7 @@ static void launch_conv_wgrad(const ConvPlan& p, const WgradArgs& w, unsigned wb
 bool dn_conv_wgrad(const uint16_t* X, const uint16_t* coarse, int c1, const uint16_t* dZ, int N, int H, int W, int Cin,
                    int Cout, float* wpartial, const uint16_t* Wd, float* gout, hipStream_t s) {
   const WgradArgs w{X, coarse, dZ, wpartial, c1, N, H, W, Cin, Cout, dn_wgrad_chunks(N, H, W)};
+  if (!dn_load_ok(H, W, Cin - c1) || !dn_load_ok(H / 2, W / 2, c1) || !dn_load_ok(H, W, Cout)) return false;
   const unsigned channels = (Cout / 32) * ((Cin + 31) / 32), wblocks = w.chunks * channels;
   DnConv c;
   ConvPlan p;
