@@ -30,6 +30,7 @@
 #include <algorithm>
 
 #include "device.h"
+#include "trt/segments.h"
 #include "trt/slab32.h"
 #include "trt/tonemap.h"
 
@@ -1049,7 +1050,7 @@ __device__ __forceinline__ void add_emission(const float4* __restrict__ emit, co
   for (uint32_t sgm = blockIdx.x % kSegs; sgm < kSegs; sgm += gridDim.x) {
     const uint32_t c = cnt[sgm * kLine];
     const uint32_t n = c < cap ? c : cap;
-    const uint32_t first = blockIdx.x / kSegs * kBlock, step = (gridDim.x - sgm + kSegs - 1) / kSegs * kBlock;
+    const uint32_t first = segment_place(blockIdx.x, kSegs) * kBlock, step = segment_blocks(sgm, gridDim.x, kSegs) * kBlock;
     const float4* seg = emit + static_cast<size_t>(sgm) * cap;
     uint32_t i = first + threadIdx.x;
     float4 e = make_float4(0.f, 0.f, 0.f, 0.f);
