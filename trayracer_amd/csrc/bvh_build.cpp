@@ -642,10 +642,16 @@ bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, N
       if (flat_run[k]) flat[flat_at[k]] += flat_run[k];
   };
   const size_t n_parts = std::min<size_t>(size_t(std::max(1, n_threads)), count / 16384 + 1);
+  auto pack_part = [&](size_t t) { pack_range(first + count * t / n_parts, first + count * (t + 1) / n_parts); };
   std::vector<std::thread> pool;
-  for (size_t t = 1; t < n_parts; ++t)
-    pool.emplace_back(pack_range, first + count * t / n_parts, first + count * (t + 1) / n_parts);
-  pack_range(first, first + count / n_parts);
+  size_t started = 1;
+  try {
+    pool.reserve(n_parts);
+    for (; started < n_parts; ++started) pool.emplace_back(pack_part, started);
+  } catch (...) {  // no more threads to be had: this one packs the rest
+  }
+  pack_part(0);
+  for (size_t t = started; t < n_parts; ++t) pack_part(t);
   for (std::thread& t : pool) t.join();
   size_t coplanar = 0;
   for (const std::atomic<uint32_t>& n : flat) coplanar += n >= kThickPlane ? n.load() : 0u;
