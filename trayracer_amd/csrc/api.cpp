@@ -73,6 +73,7 @@ struct Mesh {
 // memory; per ray: 32 B record, 16 B hit, 4 B instance, 1 B occlusion.
 constexpr uint32_t kSmallQuery = 4096;
 constexpr size_t kSmallQueryBytes = 32 + 16 + 4 + 1;
+constexpr size_t kReportBytes = size_t(kCtrSegBase) * 4;
 
 }  // namespace
 
@@ -130,7 +131,8 @@ struct trt_context {
   DevBuf tonemapped;  // RGBA8 display image
   DevBuf counters;
   DevBuf scratch_rays, scratch_hits, scratch_inst, scratch_occ;
-  void* frame_report = nullptr;  // pinned: a frame's counters, written by its last kernel
+  void* frame_report = nullptr;  // pinned: a frame's counters, written by its last kernel, or a ray query's
+  DevBuf report;                 // the same where no pinned memory is to be had
   void* small_query = nullptr;  // pinned host block of small ray queries
   void* read_stage = nullptr;   // pinned buffers of read_back's threads
   uint64_t path_capacity = 0;
@@ -396,6 +398,14 @@ RenderParams params_of_opts(const trt_context* ctx, const trt_render_opts& o) {
   return rp;
 }
 
+// Pinned host memory; null where none is to be had (the callers then do without).
+void* pinned(size_t bytes) {
+  void* p = nullptr;
+  if (hipHostMalloc(&p, bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  return nullptr;
+}
+
 // Grid of a persistent kernel over at most n queue items: every resident slot, but no more
 // than a wave per 64 items (idle waves cost launch time and failed queue fetches: 0.37 ->
 // 0.35 ms for a 640 x 360 frame; half as many waves again were slower) and at least a
@@ -412,9 +422,10 @@ trt_status run_frame(trt_context* ctx, const trt_render_opts& o, bool stats, boo
   const uint32_t n = o.width * o.height * o.spp;
   const DevAccel acc0 = accel_of(ctx);
   const SceneView sv = view_of(ctx);
-  if (!ctx->frame_report)
-    HIPC(hipHostMalloc(&ctx->frame_report, size_t(kCtrSegBase) * 4), "alloc frame report");
-  uint32_t* const hc = static_cast<uint32_t*>(ctx->frame_report);
+  uint32_t own_report[kCtrSegBase];
+  if (!ctx->frame_report) ctx->frame_report = pinned(kReportBytes);
+  if (!ctx->frame_report) HIPC(ctx->report.ensure(kReportBytes), "alloc frame report");
+  uint32_t* const report = ctx->frame_report ? static_cast<uint32_t*>(ctx->frame_report) : ctx->report.as<uint32_t>();
   uint32_t* ctr = ctx->counters.as<uint32_t>();
   FrameBuffers fb;
   fb.radiance = ctx->radiance.as<float4>();
@@ -511,12 +522,15 @@ trt_status run_frame(trt_context* ctx, const trt_render_opts& o, bool stats, boo
   if (timing) HIPC(hipEventRecord(ev[3], stm), "event");
   if (accumulate)
     launch_finalize(rp, fb.radiance, fb, ctx->sample_count == 0 ? 1u : 0u, ctx->aov_count == 0 ? 1u : 0u,
-                    ctx->aov_count + o.spp, ctr, cap, hc, stm);
+                    ctx->aov_count + o.spp, ctr, cap, report, stm);
   else
-    launch_report_counters(ctr, cap, hc, stm);
+    launch_report_counters(ctr, cap, report, stm);
   HIPC(hipEventRecord(ev[2], stm), "event");
   HIPC(hipGetLastError(), "kernel launch");
   HIPC(hipStreamSynchronize(stm), "frame");
+  if (!ctx->frame_report)
+    HIPC(hipMemcpy(own_report, ctx->report.p, sizeof(own_report), hipMemcpyDeviceToHost), "read frame report");
+  const uint32_t* const hc = ctx->frame_report ? report : own_report;
 
   ctx->last_paths = n;
   ctx->has_frame = true;
@@ -1075,23 +1089,22 @@ static void populate_pages(void* p, size_t bytes) {
 // the runtime, 1.11 with its copies into two threads' chunks, 0.87 with the kernel, 0.82 with
 // four threads; 133 MB: 12.8, 5.8, 5.8, 3.9; 7.6 MB after training: 1.07 by the runtime, 0.26.
 // 512 KB chunks are slower, 2 MB ones no faster. From kReadLarge bytes on, below which threads
-// cost more than they save. Returns when the copy is done. idle: nothing is queued on the
+// cost more than they save; by the runtime also with a budget of one thread and where there is
+// no pinned memory to be had. Returns when the copy is done. idle: nothing is queued on the
 // context's stream (a small copy then needs no stream: 39 us instead of 43 for 655 KB).
 constexpr size_t kReadLarge = size_t(4) << 20, kReadChunk = size_t(1) << 20;
 constexpr int kReadThreads = 4;
 static hipError_t read_back(trt_context* ctx, void* out, const void* src, size_t bytes, bool idle = false) {
   hipStream_t s = ctx->stream;
   const size_t parts = std::min<size_t>({size_t(kReadThreads), size_t(std::max(1, default_build_threads())), bytes / kReadChunk});
-  if (bytes < kReadLarge || parts < 2 || (reinterpret_cast<uintptr_t>(src) & 15)) {
+  const bool large = bytes >= kReadLarge && parts >= 2 && (reinterpret_cast<uintptr_t>(src) & 15) == 0;
+  if (large && !ctx->read_stage) ctx->read_stage = pinned(2 * kReadThreads * kReadChunk);
+  if (!large || !ctx->read_stage) {
     if (idle) return hipMemcpy(out, src, bytes, hipMemcpyDeviceToHost);
     const hipError_t e = hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, s);
     return e == hipSuccess ? hipStreamSynchronize(s) : e;
   }
-  if (!ctx->read_stage) {
-    const hipError_t e = hipHostMalloc(&ctx->read_stage, 2 * kReadThreads * kReadChunk);
-    if (e != hipSuccess) return e;
-  }
-  std::vector<hipError_t> result(parts, hipSuccess);
+  hipError_t result[kReadThreads] = {};
   auto read_part = [&](size_t t) {
     hipError_t& err = result[t];
     const size_t begin = bytes * t / parts & ~size_t(15), end = t + 1 == parts ? bytes : bytes * (t + 1) / parts & ~size_t(15);
@@ -1220,16 +1233,16 @@ static trt_status trace_common(trt_context* ctx, const float* rays, uint32_t n, 
   if (n == 0) return TRT_OK;
   HIPC(hipSetDevice(ctx->device), "hipSetDevice");
   hipStream_t s = ctx->stream;
-  const bool small = n <= kSmallQuery, want_inst = !any && inst && ctx->two_level;
+  if (n <= kSmallQuery && !ctx->small_query) ctx->small_query = pinned(size_t(kSmallQuery) * kSmallQueryBytes);
+  const bool small = n <= kSmallQuery && ctx->small_query, want_inst = !any && inst && ctx->two_level;
   HIPC(ctx->scratch_rays.ensure(size_t(n) * 32), "alloc rays");
-  if (!ctx->small_query) HIPC(hipHostMalloc(&ctx->small_query, size_t(kSmallQuery) * kSmallQueryBytes + 16), "alloc rays");
   if (!small && any) {
     HIPC(ctx->scratch_occ.ensure(n), "alloc hits");
   } else if (!small) {
     HIPC(ctx->scratch_hits.ensure(size_t(n) * 16), "alloc hits");
     HIPC(ctx->scratch_inst.ensure(size_t(n) * 4), "alloc hits");
   }
-  uint8_t* const block = static_cast<uint8_t*>(ctx->small_query);  // records, hits, instances, occlusion, status
+  uint8_t* const block = static_cast<uint8_t*>(ctx->small_query);  // records, hits, instances, occlusion
   float4* const rec = ctx->scratch_rays.as<float4>();
   const float4* src = rec;
   float4* d_hits = ctx->scratch_hits.as<float4>();
@@ -1256,7 +1269,9 @@ static trt_status trace_common(trt_context* ctx, const float* rays, uint32_t n, 
   else
     launch_extend(acc, q, HitBuf{d_hits, d_inst}, in, ctr, grid, false, s);
   HIPC(hipGetLastError(), "trace launch");
-  uint32_t* const status = reinterpret_cast<uint32_t*>(block + size_t(kSmallQuery) * kSmallQueryBytes);  // overflow, -, first invalid ray
+  uint32_t own_status[4];  // overflow, -, first invalid ray
+  if (!ctx->frame_report) ctx->frame_report = pinned(kReportBytes);
+  uint32_t* const status = ctx->frame_report ? static_cast<uint32_t*>(ctx->frame_report) : own_status;
   HIPC(hipMemcpyAsync(status, ctr + kCtrOverflow, 16, hipMemcpyDeviceToHost, s), "read status");
   HIPC(hipStreamSynchronize(s), "trace");
   uint64_t bad;
