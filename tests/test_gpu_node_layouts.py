@@ -83,3 +83,98 @@ def test_plates_off_the_grid(rend, axis, half):
     rays[1500:1800, 4 + axis] = 0.0
     _check_rays(rend, orc, rays)
     _check_frame(rend, sc, orc)
+
+
+def _cluster(n, radius, spread, at, seed):
+    """n instances (14 floats) of mesh 0 of the given radius within `spread` of a place."""
+    rng = np.random.default_rng(seed)
+    inst = np.zeros((n, 14), np.float32)
+    for i in range(n):
+        m = np.zeros((3, 4))
+        m[:, :3] = scenes._random_rotation(rng) * radius * rng.uniform(0.5, 1.0)
+        m[:, 3] = np.asarray(at) + rng.uniform(-spread, spread, 3)
+        inst[i, :12] = m.reshape(-1)
+        inst[i, 12:14] = np.array([0, i % 3], np.uint32).view(np.float32)
+    return inst
+
+
+def _two_level(refusing):
+    """A two-level scene that takes 48-byte nodes, by a mesh with a small detailed part in a large
+    one, or by a top level with small instances between far ones; seen from nearby."""
+    pos, _ = scenes.icosphere(1 if refusing == "top level" else 3)
+    if refusing == "top level":
+        at = np.array([600.0, 10.0, -300.0])
+        inst = np.concatenate([_cluster(150, 0.06, 0.5, at, 5), _cluster(4, 0.3, 2.0, at, 6), _cluster(2, 1.0, 1.0, (-3000, -3000, -3000), 7),
+                               _cluster(2, 1.0, 1.0, (3000, 3000, 2000), 8)])
+    else:
+        at = np.array([0.2, 0.1, 0.1]) * 3000.0 + [0.3, 0.2, 0.1]
+        pos = np.concatenate([pos * 0.5 + np.tile(at, 3),
+                              np.tile([-3000.0, -3000.0, -3000.0], 3)[None] + np.array([[0, 0, 0, 1, 0, 0, 0, 1, 0]]),
+                              np.tile([3000.0, 3000.0, 3000.0], 3)[None] + np.array([[0, 0, 0, 1, 0, 0, 0, 1, 0]])]).astype(np.float32)
+        inst = np.zeros((4, 14), np.float32)
+        for i in range(4):
+            m = np.zeros((3, 4))
+            m[:, :3] = np.eye(3)
+            m[:, 3] = [0.7 * (i % 2), 0.6 * (i // 2), 0.1 * i]
+            inst[i, :12] = m.reshape(-1)
+            inst[i, 12:14] = np.array([0, i % 3], np.uint32).view(np.float32)
+        at = at + [0.35, 0.3, 0.15]
+    mats = np.stack([scenes.material(c, roughness=r, metallic=m) for c, r, m in
+                     (((0.8, 0.3, 0.2), 0.4, 0.0), ((0.3, 0.7, 0.4), 0.7, 0.2), ((0.4, 0.4, 0.9), 0.3, 0.8))])
+    cam = dict(position=tuple(at + [0.0, 0.4, -3.0]), target=tuple(at), up=(0, 1, 0), fov=0.7, aperture=0.0, focal_dist=1.0,
+               distortion=0.0, bokeh_sides=0, bokeh_rotation=0.0)
+    return at, dict(positions=pos, normals=None, mat_ids=np.zeros(len(pos), np.uint32), meshes=[(0, len(pos))], materials=mats,
+                    instances=inst, camera=cam, sky=SKY,
+                    render=dict(width=24, height=24, spp=8, max_depth=3, rr_depth=3, seed=2, ray_epsilon=1e-3, clamp=0.0))
+
+
+def _check_backward(rend, sc):
+    """The gradient against the oracle's FP64 accumulation of the same float terms: the device
+    adds at most n = 24 x 24 x 8 x 3 per parameter in float, whose rounding is about
+    sqrt(n) 2^-24 ~ 7e-6 of the terms' magnitudes as it accumulates, below n 2^-24 ~ 8e-4 in the
+    worst case: 1e-3 of the largest gradient bounds it."""
+    theta = scenes.material_params(sc["materials"])
+    rend.set_material_params(theta, which=3)
+    rend.SetSettings(rend.settings.from_dict(sc["render"]))
+    assert rend.RenderFrame()["shadow_rays"] > 500
+    img = rend.color()[..., :3]
+    dldi = (2.0 * (img - 0.5 * img.mean())).astype(np.float32)
+    g = rend.backward(dldi)
+    orc = _oracle(sc)
+    orc.set_material_params(theta, which=3)
+    np.testing.assert_array_equal(img, orc.render()["image_f32"])
+    ref = orc.backward(dldi)
+    assert (np.abs(ref).max(axis=1) > 0).sum() >= 3
+    assert np.abs(g - ref).max() <= 1e-3 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("refusing", ["mesh", "top level"])
+def test_two_level_scenes_on_48_byte_nodes(rend, refusing):
+    """Hits, occlusion, a frame's paths and the gradient of two-level scenes whose trees do not
+    suit the 32-byte nodes."""
+    at, sc = _two_level(refusing)
+    rend.UpdateScene(sc)
+    assert _node_bytes(rend) == 48
+    orc = _oracle(sc)
+    rays = random_rays(3000, seed=11, lo=-2.0, hi=2.0, toward=(-0.6, 0.6))
+    rays[:, 0:3] += at.astype(np.float32)
+    rays[:300, 4:7] = 0.0
+    for k in range(3):  # parallel to an axis
+        rays[100 * k:100 * (k + 1), 4 + k] = 1.0
+    rays[300:600, 4:7] *= 1e4
+    _check_rays(rend, orc, rays)
+    _check_frame(rend, sc, orc)
+    _check_backward(rend, sc)
+
+
+def test_gradient_on_48_byte_nodes(rend):
+    """The adjoint's shadow rays through a single-level tree of 48-byte nodes."""
+    sc = scenes.soup(n_tris=6000, seed=12, width=24, height=24, spp=8, max_depth=3, n_emissive=6)
+    far = np.tile(np.array([[-3000.0], [2000.0]]), (1, 9)) + np.array([0, 0, 0, 1, 0, 0, 0, 1, 0])
+    sc["positions"] = np.concatenate([sc["positions"], far]).astype(np.float32)
+    sc["mat_ids"] = np.concatenate([sc["mat_ids"], np.zeros(2, np.uint32)])
+    sc["meshes"] = [(0, len(sc["positions"]))]
+    sc["sky"] = SKY
+    rend.UpdateScene(sc)
+    assert _node_bytes(rend) == 48
+    _check_backward(rend, sc)
