@@ -219,7 +219,8 @@ def denoise_metric(rend, steps):
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "k_extend_sl_soup1m_traffic.json")
 # the sources whose code the measured traffic belongs to
 TRAVERSAL_SOURCES = ["trayracer_amd/csrc/kernels.hip", "trayracer_amd/csrc/device.h", "trayracer_amd/csrc/bvh_build.cpp",
-                     "trayracer_amd/csrc/bvh_build.h", "trayracer_amd/csrc/api.cpp", "trayracer_amd/csrc/trt/intersect.h"]
+                     "trayracer_amd/csrc/bvh_build.h", "trayracer_amd/csrc/api.cpp", "trayracer_amd/csrc/trt/intersect.h",
+                     "trayracer_amd/csrc/trt/slab32.h", "trayracer_amd/csrc/trt/segments.h"]
 
 
 def traversal_source_hash():
@@ -268,7 +269,7 @@ def load_instruction_costs():
 
 
 def extend_roofline(tc, info, ext_rays, ext_ms, launches, workload):
-    """Two ceilings for the closest-hit traversal (Extend), per launch, from HIP-event
+    """Two yardsticks for the closest-hit traversal (Extend), per launch, from HIP-event
     launch times:
     * HBM: the bytes a launch must move at least, its rays' records (32 B ray in, 16 B hit
       out) plus every distinct node (32 or 48 B) and triangle record (48 B) it reads once
@@ -278,7 +279,9 @@ def extend_roofline(tc, info, ext_rays, ext_ms, launches, workload):
     * vector memory: the bytes every ray loads (ray and hit records, node visits x the
       node's bytes, triangle tests x 48 B) against the rate of independent random 48-byte gathers from
       an L1-resident buffer (trt_measure_gather), the fastest such loads go through the
-      CUs' load path (Extend's node loads mostly hit L1 and L2)."""
+      CUs' load path (Extend's node loads mostly hit L1 and L2). The gathers are of 48-byte
+      records, as 48-byte nodes and triangles are read; for the two-load 32-byte nodes the
+      rate is a comparison, not a bound."""
     n = max(1, launches)
     avg_s = ext_ms / n * 1e-3
     per_ray = 48 + tc["closest_nodes_per_ray"] * tc["node_bytes"] + tc["closest_tris_per_ray"] * tc["tri_bytes"]

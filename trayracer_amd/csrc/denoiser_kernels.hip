@@ -622,9 +622,10 @@ __global__ __launch_bounds__(kWgThreads) void k_wgrad(WgradArgs a) {
 // are independent and, at the sizes of training crops, each is a chain of load latencies
 // that leaves most of the chip idle (8 x 128 x 128: 12 and 16 us a layer on average one after
 // the other, 20 us together). The last conv_blocks workgroups convolve; the wave that the
-// weight gradient has no use for ends. Held to 168 VGPRs, 3 waves per SIMD, which two tiles
-// ahead in the weight gradient allow (a step at 8 x 128 x 128: 0.79 ms; with three tiles
-// ahead at 2 waves 0.82; convolution first 0.80).
+// weight gradient has no use for ends. With 32 output channels a group (NB = 1) held to 3 waves
+// per SIMD, 157 VGPRs, which two tiles ahead in the weight gradient allow (a step at 8 x 128 x
+// 128: 0.79 ms; with three tiles ahead at 2 waves 0.82; convolution first 0.80); with 64 the
+// convolution's 55 KB of LDS leave room for 2, of 179 VGPRs and 48 accumulators.
 template <int MB, int NB, bool SC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_conv_wgrad(ConvArgs c, unsigned conv_blocks,
                                                                                            WgradArgs w) {

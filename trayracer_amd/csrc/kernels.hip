@@ -22,9 +22,9 @@
 //  * No host synchronisation between bounces: queue sizes stay in device counters.
 //  * Radiance is accumulated per path (one writer per path per kernel) and reduced
 //    per pixel in a fixed sample order in Finalize, so images are deterministic. Shade
-//    lists emission rather than adding it; the emission and shadow launches of the
-//    shadow stream add every term in vertex order, and Shade runs beside the previous
-//    bounce's shadow launch.
+//    lists emission rather than adding it; the bounce's Shadow launch, on a stream of its
+//    own, adds first the listed emission and then its rays' contributions, so every term is
+//    added in vertex order while Shade runs beside the previous bounce's Shadow.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -270,10 +270,11 @@ struct Nodes48 {
 // to decode: v_fma_mix_f32 takes an fp16 operand as it is, so per axis
 //   ct = fma(c, step inv, (org - o) inv),  entry = ct - h |step inv|,  exit = ct + h |step inv|
 // are three instructions (six, plus six to gather the child references, with Nodes48).
-// The terms that cancel in ct have an error of up to 2u (|x| + R) |inv| (x the distance to
-// the box's centre, R the tree's half size): the part in |x| is relative to the distances,
-// and the half extents' margins (bvh_build.h) exceed the part in R. The per-ray
-// terms, and what they do with tiny direction components and extreme rays: slab32_ray.
+// The terms that cancel in ct have an error of up to 3u (|x| + R) |inv| (u = 2^-24, x the
+// distance to the box's centre, R the tree's half side on the axis): the part in |x| is
+// relative to the distances, and the half extents' margins (bvh_build.h) exceed the part in R.
+// The per-ray terms, and what they do with tiny direction components and extreme rays:
+// slab32_ray.
 struct Nodes32 {
   static constexpr uint32_t kBytes = sizeof(DevNode32);
   struct Ray {
@@ -1069,8 +1070,8 @@ __device__ __forceinline__ void add_emission(const float4* __restrict__ emit, co
   }
 }
 
-// Single-level scenes: Extend and Shadow through trace_queue, held to 72 VGPRs, 7 waves per
-// SIMD. They are bound by throughput, not latency (the texture data path is 91 % busy and
+// Single-level scenes: Extend and Shadow through trace_queue, held to 72 VGPRs (two spilled,
+// 12 bytes of scratch, with 32-byte nodes), 7 waves per SIMD. They are bound by throughput, not latency (the texture data path is 91 % busy and
 // VALU issue above its 4-cycle rate): 6 and 5 waves measured 11.98 and 12.01 ms a soup
 // frame against 11.82.
 template <class Nodes, bool STATS>
@@ -1123,9 +1124,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) voi
   }
 }
 
-// Two-level scenes: Extend and Shadow through trace_queue2, at 96 VGPRs, 5 waves per SIMD:
-// 11.8 ms per 4K frame of 1000 instances, against 12.5 at 6 waves and 13.2 at 7 (spilled
-// registers) and 11.9 at 4.
+// Two-level scenes: Extend and Shadow through trace_queue2, at 92 to 96 VGPRs, 5 waves per SIMD:
+// 11.8 ms per 4K frame of 1000 instances on 32-byte nodes, against 12.5 at 6 waves and 13.2 at 7
+// (spilled registers) and 11.9 at 4. On 48-byte nodes, 1280x720x4: 1000 spheres 2.71 ms, 2.91 at
+// 6 waves, 2.72 at 4; 300 on a ground plane 4.87, 5.13, 4.87.
 template <class Nodes, bool STATS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_extend_tl(DevAccel acc, RayQueue q, HitBuf h, SegIn in, uint32_t* ctr) {
   extern __shared__ uint32_t lds[];

@@ -1,16 +1,17 @@
 // Measurement hook: the vector-memory ceiling of the traversal kernels' loads.
 //
-// Extend and Shadow read 48-byte records (a node: three 16-byte rows; a triangle: three
-// 16-byte rows) at data-dependent addresses, one record per lane, and their rate is set
-// by how many such gathers the CUs' vector-memory path (address and data units, L1, L2)
+// Extend and Shadow read records (a triangle: three 16-byte rows, a node: two, or three
+// where the compact nodes do not fit) at data-dependent addresses, one record per lane, and
+// their rate is set by how many such gathers the CUs' vector-memory path (address and data units, L1, L2)
 // completes, not by HBM bandwidth: the working set is mostly served by the L2 and the
 // Infinity Cache. This kernel issues the same access pattern with nothing else in the
 // way: each lane reads 48-byte records at pseudo-random record indices of a buffer, the
 // loads independent of each other so that latency hides behind occupancy. Over a buffer
-// that fits the L2 it measures the highest rate such gathers reach, the ceiling that
-// the traversal's loaded bytes are compared with. A second entry times the same loads
-// per wave-level instruction with fewer active lanes, or with every lane of a wave at
-// one record, to show what a load instruction costs the load path when lanes idle.
+// that fits the L2 it measures the highest rate such gathers reach, which the traversal's
+// loaded bytes are compared with (a yardstick for the 32-byte nodes, not their ceiling). A
+// second entry times the same loads per wave-level instruction with fewer active lanes, or with
+// every lane of a wave at one record, to show what a load instruction costs the load path when
+// lanes idle.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
