@@ -1,7 +1,8 @@
 // Check of trt::pack_nodes32 on trees with finely divided axis-aligned surfaces. Prints "ok" or
 // the first violation and exits non-zero.
-//   1. the flat boxes of the two most divided planes of an axis stay thin, whatever the planes'
-//      heights, and every stored box contains the exact one;
+//   1. the flat boxes of the two most divided planes of an axis stay thin, of the most divided one
+//      where the grid has one step, whatever the planes' heights, and every stored box contains
+//      the exact one;
 //   2. rays that touch an exact box in FP64 pass the float slab test of the traversal, grazing
 //      rays among them;
 //   3. a tree with many flat boxes in further planes, off the grid, is refused, one with few is not.
@@ -78,8 +79,10 @@ int main() {
   };
   // (half side, heights): a floor, a hall, a hall about its centre, far from the origin
   const float scenes[][3] = {{5.f, -1.00317f, -1.00317f}, {50.f, -1.00317f, 3.7713f}, {3.f, -3.01f, 2.97f}, {700.f, -1.0003f, 44.123f}};
-  for (int axis = 0; axis < 3; ++axis)
+  for (int turn = 0; turn < 6; ++turn)
     for (const auto& sc : scenes) {
+      const int axis = turn % 3;
+      const bool stretch = turn < 3;
       std::vector<float> box;
       detail(box, std::min(1.f + sc[0] * 0.01f, 8.f));
       plane(box, axis, sc[1], sc[0], 100);
@@ -87,7 +90,9 @@ int main() {
       const std::vector<DevNode2> dn = tree(box);
       std::vector<DevNode32> pk(dn.size());
       NodeSpace g;
-      if (!pack_nodes32(dn, 0, dn.size(), g, pk.data(), 4)) return fail("planes refused", size_t(axis));
+      if (!pack_nodes32(dn, 0, dn.size(), g, pk.data(), 4, stretch)) return fail("planes refused", size_t(axis));
+      for (const float step : g.step)
+        if (!stretch && step != g.scale) return fail("more than one step", size_t(axis));
       double Rk = 0.0;  // the tree's half side on the axis
       {
         double lo = HUGE_VAL, hi = -HUGE_VAL;
@@ -106,7 +111,7 @@ int main() {
           for (int k = 0; k < 3; ++k) {
             const double cs = half_of(w[k] & 0xffffu) * g.step[k] + g.org[k], hs = half_of(w[k] >> 16) * g.step[k];
             if (!(cs - hs <= lo[k] && cs + hs >= hi[k])) return fail("box not contained", i);
-            if (k == axis && lo[k] == hi[k] && (lo[k] == sc[1] || lo[k] == sc[2]) && !(hs <= Rk * 0x1p-18))
+            if (k == axis && lo[k] == hi[k] && (lo[k] == sc[1] || (stretch && lo[k] == sc[2])) && !(hs <= Rk * 0x1p-18))
               return fail("thick box of a plane", i);
           }
           for (int r = 0; r < 8; ++r) {

@@ -59,9 +59,9 @@ def _plates(axis, heights, half, n=24):
     return np.concatenate(out).astype(np.float32)
 
 
-@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("axis,levels", [(0, 1), (1, 1), (2, 1), (1, 2)])
 @pytest.mark.parametrize("half", [2.0, 50.0])
-def test_plates_off_the_grid(rend, axis, half):
+def test_plates_off_the_grid(rend, axis, levels, half):
     """Finely divided plates whose heights the 32-byte nodes' grid is fitted to: rays from,
     along and grazing the plates as well as random ones equal brute force, and a frame's paths
     the oracle's."""
@@ -72,6 +72,9 @@ def test_plates_off_the_grid(rend, axis, half):
     sc["mat_ids"] = np.concatenate([sc["mat_ids"], np.full(len(plates), 7, np.uint32)])
     sc["meshes"] = [(0, len(sc["positions"]))]
     sc["sky"] = SKY
+    if levels == 2:
+        sc["instances"] = np.zeros((1, 14), np.float32)
+        sc["instances"][0, [0, 5, 10]] = 1.0
     rend.UpdateScene(sc)
     assert _node_bytes(rend) == 32
     orc = _oracle(sc)

@@ -907,9 +907,9 @@ trt_status trt_build(trt_context* ctx, const trt_build_opts* opts) {
   } else {
     for (size_t mi = 0; mi < ctx->meshes.size() && compact; ++mi) {
       const size_t end = mi + 1 < ctx->meshes.size() ? blas_root[mi + 1] : nodes.size();
-      compact = pack_nodes32(nodes, blas_root[mi], end - blas_root[mi], mesh_space[mi], nodes32.data(), threads);
+      compact = pack_nodes32(nodes, blas_root[mi], end - blas_root[mi], mesh_space[mi], nodes32.data(), threads, false);
     }
-    compact = compact && pack_nodes32(tlas_nodes, 0, tlas_nodes.size(), ctx->space, tlas32.data(), threads);
+    compact = compact && pack_nodes32(tlas_nodes, 0, tlas_nodes.size(), ctx->space, tlas32.data(), threads, false);
   }
   if (!compact && (!pack_nodes(nodes, nodes48) || !pack_nodes(tlas_nodes, tlas48)))
     return fail(ctx, TRT_UNSUPPORTED, "scene bounds too large for the node layout (infinite coordinates)");
@@ -921,7 +921,8 @@ trt_status trt_build(trt_context* ctx, const trt_build_opts* opts) {
     TlasInstance& t = inst_tlas[k];
     std::memset(&t, 0, sizeof(t));
     std::memcpy(t.w2o, in.w2o, sizeof(t.w2o));
-    t.space = grid_of(mesh_space[in.mesh]);
+    std::memcpy(t.org, mesh_space[in.mesh].org, sizeof(t.org));
+    t.step = mesh_space[in.mesh].scale;
     t.blas_root = blas_root[in.mesh] * ctx->node_bytes;  // a byte offset, like every node reference
     t.id = in.id;
   }

@@ -546,7 +546,7 @@ int flat_planes(const std::vector<DevNode2>& in, size_t first, size_t count, int
 }  // namespace
 
 bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, NodeSpace& space, DevNode32* out,
-                  int n_threads) {
+                  int n_threads, bool stretch) {
   static_assert(sizeof(DevNode32) == 32, "node size");
   double blo[3] = {HUGE_VAL, HUGE_VAL, HUGE_VAL}, bhi[3] = {-HUGE_VAL, -HUGE_VAL, -HUGE_VAL};
   for (int c = 0; c < 2; ++c) {  // the root's children bound the tree
@@ -569,7 +569,7 @@ bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, N
   if (R > 0.0) (void)std::frexp(R, &e);
   if (!std::isfinite(R) || e < -60 || e > 60) return false;
   space.scale = float(std::ldexp(1.0, e - 14));
-  // the two planes with the most flat boxes on each axis are put on the grid
+  // the planes with the most flat boxes on each axis, two or one, are put on the grid
   for (int k = 0; k < 3; ++k) {
     space.step[k] = space.scale;
     double at[2], c[2];
@@ -578,7 +578,7 @@ bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, N
       const double mid = (at[i] - space.org[k]) / space.scale;
       c[i] = half_value(half_bits(std::fabs(mid), false)) * (mid < 0.0 ? -1.0 : 1.0);
     }
-    if (n == 2 && c[0] != c[1]) {
+    if (stretch && n == 2 && c[0] != c[1]) {
       const double step = (at[1] - at[0]) / (c[1] - c[0]);
       if (std::fabs(step - space.scale) < kMaxStretch * space.scale) space.step[k] = float(step);
     }

@@ -122,8 +122,8 @@ bool pack_nodes(const std::vector<DevNode2>& in, std::vector<DevNode48>& out);
 // plane's distance from it. A ray that grazes the surface crosses hundreds of thick ones, one
 // after the other, while its launch waits for it. So org moves, by less than R / 128, and step,
 // by up to kMaxStretch, to put the two planes of each axis that have the most flat boxes on the
-// grid. (A 328 k-triangle ball on a floor of half side 20: 4.04 ms a frame, now 3.25, on 48-byte
-// nodes 3.28; with a plate above the floor 6.16, now 3.24, and 3.30.)
+// grid. (A 328 k-triangle ball on a floor of half side 20: 4.05 ms a frame, now 3.22, on 48-byte
+// nodes 3.29; with a plate above a floor of half side 5 6.17, now 3.22, and 3.32.)
 struct NodeSpace {
   float org[3];
   float scale;
@@ -135,7 +135,9 @@ struct alignas(16) DevNode32 {
 };
 
 // Converts nodes [first, first + count) of one tree (indices relative to the whole array) to
-// the compact layout. False, with the output unusable, when the tree does not suit it:
+// the compact layout. stretch: whether the steps may differ from `scale` (two-level trees keep
+// one step, and so only one plane per axis on the grid: an instance's set-up with three cost 1.6 %
+// of the frames of 1000 spheres). False, with the output unusable, when the tree does not suit it:
 //   a non-finite bound or one beyond the grid's range;
 //   more than kCoarseShare of the boxes grow by more than kCoarseGrowth (sum of half extents)
 // because the tree's detail is too fine for its extent (a small object in a large
@@ -154,7 +156,7 @@ constexpr double kThinHalf = 1.0 / (1 << 18);
 constexpr uint32_t kThickPlane = 1u << 12;
 constexpr size_t kMaxThickFlat = 1u << 15;
 bool pack_nodes32(const std::vector<DevNode2>& in, size_t first, size_t count, NodeSpace& space, DevNode32* out,
-                  int n_threads = 1);
+                  int n_threads = 1, bool stretch = true);
 
 // Converts a build tree into the device layout (depth-first order, node 0 = root).
 // Returns the device nodes; a root leaf is wrapped in a node with an empty second child.

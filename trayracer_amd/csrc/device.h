@@ -40,6 +40,9 @@ struct ShadowQueue {
 struct NodeGrid {
   float org[3], step[3];
 };
+TRT_FI NodeGrid grid_of(const float org[3], float step) {  // two-level scenes: one step per tree
+  return NodeGrid{{org[0], org[1], org[2]}, {step, step, step}};
+}
 inline NodeGrid grid_of(const NodeSpace& s) {
   return NodeGrid{{s.org[0], s.org[1], s.org[2]}, {s.step[0], s.step[1], s.step[2]}};
 }
@@ -47,9 +50,10 @@ inline NodeGrid grid_of(const NodeSpace& s) {
 // An instance as the two-level traversal reads it, in the top level's leaf order.
 struct alignas(16) TlasInstance {
   float w2o[12];
-  NodeGrid space;       // of the mesh's tree
+  float org[3], step;   // grid of the mesh's tree, of one step (NodeSpace)
   uint32_t blas_root;   // byte offset of the mesh's root in the node array
   uint32_t id;          // caller's instance index
+  uint32_t pad[2];
 };
 
 // Acceleration structure views.

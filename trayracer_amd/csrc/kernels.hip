@@ -769,7 +769,7 @@ __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& i
           slot = base + rank;
           float tmax;
           load(slot, ow, dw, tmin, tmax);
-          rb = Nodes::setup(acc.space, ow, dw);
+          rb = Nodes::setup(grid_of(acc.space.org, acc.space.step[0]), ow, dw);
           in_blas = false;
           r.t = tmax;
           r.prim = kNoHit;
@@ -846,7 +846,7 @@ __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& i
     const bool enters = !in_blas && node < 0 && node > kTravExit;
     if (leaves || enters) {
       V3 o = ow, d = dw;
-      NodeGrid space = acc.space;
+      NodeGrid space = grid_of(acc.space.org, acc.space.step[0]);
       if (enters) {
         const uint32_t c = ~static_cast<uint32_t>(node);
         const uint32_t first = c >> 3, cnt = c & 7u;
@@ -859,7 +859,7 @@ __device__ __forceinline__ void trace_queue2(const DevAccel& acc, const SegIn& i
         const TlasInstance& ins = acc.inst[first];
         o = xform_point(ins.w2o, ow);
         d = xform_vector(ins.w2o, dw);
-        space = ins.space;
+        space = grid_of(ins.org, ins.step);
         rs = ray_shear(d);
         cur_id = ins.id;
         in_blas = true;
