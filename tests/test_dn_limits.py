@@ -1,4 +1,4 @@
-"""Address limits of the denoiser's kernels (host code), and what their callers do with a refusal.
+"""Address limits of the denoiser's kernels (host code): what forward takes, backward takes.
 
 Compiles tests/native/dn_limits_check.cpp with g++ and runs it.
 """
